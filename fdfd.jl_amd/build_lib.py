@@ -19,8 +19,8 @@ LIBDIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIBDIR, "libfdfd.so")
 ARCH = "gfx950"
 
-SOURCES = ["k_operator.hip", "k_factor.hip", "k_bcr.hip", "k_mode.hip", "k_multi.hip",
-           "runtime.cpp", "bcr.cpp", "multi.cpp",
+SOURCES = ["k_operator.hip", "k_factor.hip", "k_bcr.hip", "k_mode.hip", "k_multi.hip", "k_nd.hip",
+           "runtime.cpp", "bcr.cpp", "nd.cpp", "multi.cpp",
            "eigen.cpp", "dense_eig.cpp", "batch.cpp", "mode.cpp", "modulated.cpp",
            "flux.cpp", "arnoldi.cpp", "vmode.cpp", "tune.cpp"]
 
@@ -70,6 +70,11 @@ ASAN_HOST = ["-Xarch_host", "-fsanitize=address", "-Xarch_host", "-fsanitize=und
              "-Xarch_host", "-fno-omit-frame-pointer", "-Xarch_host", "-fno-sanitize-recover=undefined"]
 ASAN_DIR = os.path.join(BUILD, "asan")
 ASAN_EXE = os.path.join(LIBDIR, "asan_driver")
+# Freed device memory passes through the sanitizer's quarantine too (256 MB by
+# default).  Once that is full, a free during the HIP runtime's own unloading
+# recycles device chunks and the sanitizer aborts on a check of its own, so
+# the quarantine is made larger than all the memory the driver frees.
+ASAN_DEFAULTS = 'extern "C" const char* __asan_default_options() { return "quarantine_size_mb=8192"; }\n'
 
 
 def _compile_asan(src: str) -> str:
@@ -96,8 +101,14 @@ def build_asan(jobs: int = 4, verbose: bool = False) -> str:
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"compile failed: {' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
+    osrc, oobj = os.path.join(ASAN_DIR, "options.cpp"), os.path.join(ASAN_DIR, "options.o")
+    with open(osrc, "w") as f:
+        f.write(ASAN_DEFAULTS)
+    r = subprocess.run([hipcc(), "-O1", "-x", "c++", "-c", osrc, "-o", oobj], capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"compile failed: {osrc}\n{r.stdout}\n{r.stderr}")
     tmp = ASAN_EXE + ".tmp"
-    cmd = [hipcc(), f"--offload-arch={ARCH}", *ASAN_HOST, dobj, *objs, "-o", tmp]
+    cmd = [hipcc(), f"--offload-arch={ARCH}", *ASAN_HOST, dobj, oobj, *objs, "-o", tmp]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"link failed: {' '.join(cmd)}\n{r.stdout}\n{r.stderr}")

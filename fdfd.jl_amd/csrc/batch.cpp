@@ -56,7 +56,7 @@ struct Builder {
             (void)hipStreamDestroy(b.stream);
         }
         for (void* p : {(void*)b.used, (void*)b.piv, (void*)b.win, (void*)b.verr, b.Vbuf, b.LU, b.Zb,
-                        (void*)b.eps})
+                        (void*)b.eps, b.nd_scratch})
             if (p) (void)hipFree(p);
         arena_clear(&b);
         buf_clear(&b);
@@ -87,6 +87,13 @@ int builder_init(Builder& B, Handle* h) {
     b.fuse_panels = h->fuse_panels;
     b.env_knobs = h->env_knobs;
     b.tuned_explicitly = h->tuned_explicitly;
+    b.nd_off = h->nd_off;
+    b.nd_plans = h->nd_plans;
+    // the dissection's build scratch moves to the builder for the batch
+    b.nd_scratch = h->nd_scratch;
+    b.nd_scratch_bytes = h->nd_scratch_bytes;
+    h->nd_scratch = nullptr;
+    h->nd_scratch_bytes = 0;
     b.work_N = h->work_N;  // borrowed: sized for the batch's largest grid
     b.g_mid = h->g_mid;
     b.x_out = h->x_out;
@@ -105,9 +112,13 @@ int builder_init(Builder& B, Handle* h) {
     return FDFD_OK;
 }
 
-// Borrowed pointers are cleared before the builder is destroyed.
-void builder_release_borrowed(Builder& B) {
+// Borrowed pointers are cleared before the builder is destroyed, and the
+// build scratch goes back to the batch's handle.
+void builder_release_borrowed(Builder& B, Handle* h) {
     Handle& b = B.H;
+    if (b.stream) (void)hipStreamSynchronize(b.stream);
+    std::swap(h->nd_scratch, b.nd_scratch);
+    std::swap(h->nd_scratch_bytes, b.nd_scratch_bytes);
     b.g_mid = b.x_out = b.V = b.Zk = b.tmp = b.tmp2 = b.bvec = b.xvec = b.hdev = nullptr;
     b.dpart = nullptr;
     b.rpart = nullptr;
@@ -200,6 +211,11 @@ int fdfd_batch_run(fdfd_batch* b, int precision, double tol, fdfd_stats* stats) 
     std::iota(order.begin(), order.end(), 0);
     auto fbytes = [&](const BatchJob& j) {
         const int n = std::min(j.g.Nx, j.g.Ny), m = std::max(j.g.Nx, j.g.Ny);
+        if (rt_nd_applies(h, j.g.Nx, j.g.Ny)) {
+            size_t arena = 0, scratch = 0;
+            rt_nd_bytes(j.g.Nx, j.g.Ny, &arena, &scratch);
+            return arena;
+        }
         return rt_factor_bytes(n, m, precision, h->gemm_b3 != 0);
     };
     std::stable_sort(order.begin(), order.end(),
@@ -249,12 +265,23 @@ int fdfd_batch_run(fdfd_batch* b, int precision, double tol, fdfd_stats* stats) 
         const BatchJob& job = b->jobs[ji];
         const int n = std::min(job.g.Nx, job.g.Ny), m = std::max(job.g.Nx, job.g.Ny);
         size_t sb = 0, ss = 0;
-        rt_factor_arena_sizes(n, m, precision, h->gemm_b3 != 0, &sb, &ss);
+        size_t scratch = 0;
+        if (rt_nd_applies(h, job.g.Nx, job.g.Ny)) {
+            rt_nd_bytes(job.g.Nx, job.g.Ny, &sb, &scratch);
+            if ((rc = rt_nd_prepare(h, job.g.Nx, job.g.Ny))) {
+                free_results(b);
+                return rc;
+            }
+        } else {
+            rt_factor_arena_sizes(n, m, precision, h->gemm_b3 != 0, &sb, &ss);
+        }
         arena_bytes[ji] = ((sb + 255) & ~(size_t)255) + ((ss + 255) & ~(size_t)255);
         // per frequency: the arenas plus the operator, Gauss-Jordan work and
-        // tables allocated beside them (about 96 B and 2 GJ channels per cell)
+        // tables allocated beside them (about 96 B and 2 GJ channels per cell,
+        // or the dissection's scratch)
         const double N = (double)job.g.Nx * job.g.Ny;
-        const double per = (double)arena_bytes[ji] + 96.0 * N + 64.0 * N * (double)VMAX / n;
+        const double per = (double)arena_bytes[ji] + 96.0 * N +
+                           (scratch ? (double)scratch : 64.0 * N * (double)VMAX / n);
         int B = (int)std::floor(usable / per);
         B = std::max(1, std::min<int>({B, (int)job.omegas.size(), 64}));
         group[ji] = B;
@@ -457,7 +484,7 @@ int fdfd_batch_run(fdfd_batch* b, int precision, double tol, fdfd_stats* stats) 
     release(0);
     release(1);
     if (dsrc) (void)hipFree(dsrc);
-    builder_release_borrowed(bld);
+    builder_release_borrowed(bld, h);
     (void)hipStreamSynchronize(h->stream);
     h->slab = nullptr;  // the slab itself stays with the handle (bslab)
     h->slab_size = h->slab_used = 0;

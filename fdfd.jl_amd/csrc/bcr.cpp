@@ -158,6 +158,119 @@ static int* blk_e(const Factor* F, int id) {
     return (int*)((char*)blk_b(F, id) + 4 * (size_t)b3_plane(F->n) * 2);
 }
 
+// Batched Gauss-Jordan inversion of nj blocks of n rows (k_factor.hip).
+// Panels of NB columns.  With the windowed search, two panels are factored
+// before one trailing pass applies both (the second panel's columns, as the
+// first panel leaves them, are formed by the window panel for its window and
+// by the Z build's check blocks for every row, and its pivot rows by the Z
+// build); the full search runs single panels.
+void rt_launch_gj(Handle* h, const LineJob* J, int nj, int n, bool fp64, bool h3, bool full, bool prof) {
+    hipStream_t st = h->stream;
+    const size_t elem = fp64 ? sizeof(double2) : sizeof(float2);
+    const int NB = h->panel_width ? h->panel_width : PMAX;
+    auto scope = [&](int id, double fl, double by) {
+        return prof ? new ProfScope(h, id, fl, by, st) : nullptr;
+    };
+    for (int k0 = 0; k0 < n;) {
+        int nb1, nb2 = 0;
+        const int fresh = std::min(n, WIN + k0);
+        {
+            ProfScope* ps = scope(P_PANEL, 0, 0);
+            if (!full) {
+                nb1 = std::min(NB, n - k0);
+                if (fp64) launch_wpanel<double>(st, J, nj, n, k0, nb1, fresh, 0);
+                else launch_wpanel<float>(st, J, nj, n, k0, nb1, fresh, 0);
+            } else {
+                // full-search panel width: powers of two (16 columns of
+                // complex128 per thread would not fit 1024 threads' registers)
+                nb1 = fp64 ? 8 : 16;
+                while (nb1 > n - k0) nb1 >>= 1;
+                if (fp64) launch_panel<double>(st, J, nj, n, k0, nb1);
+                else launch_panel<float>(st, J, nj, n, k0, nb1);
+            }
+            delete ps;
+        }
+        {
+            ProfScope* ps = scope(P_ZBUILD, 0, 0);
+            if (fp64) launch_zbuild<double>(st, J, nj, n, k0, nb1, fresh, !full, 0, 0, 0);
+            else launch_zbuild<float>(st, J, nj, n, k0, nb1, fresh, !full, 0, 0, 0);
+            delete ps;
+        }
+        if (!full && nb1 == PMAX && k0 + nb1 < n && h->fuse_panels) {
+            const int k2 = k0 + nb1;
+            nb2 = std::min(NB, n - k2);
+            const int fresh2 = std::min(n, WIN + k2);
+            // (the second panel's values as the first panel leaves
+            // them are formed by the window panel, for its window,
+            // and by the Z build's check blocks, for every row)
+            ProfScope* ps = scope(P_PANEL, 0, 0);
+            if (fp64) launch_wpanel<double>(st, J, nj, n, k2, nb2, fresh2, 1);
+            else launch_wpanel<float>(st, J, nj, n, k2, nb2, fresh2, 1);
+            delete ps;
+            ps = scope(P_ZBUILD, 0, 0);
+            if (fp64) launch_zbuild<double>(st, J, nj, n, k2, nb2, fresh2, 1, 1, k0, nb1);
+            else launch_zbuild<float>(st, J, nj, n, k2, nb2, fresh2, 1, 1, k0, nb1);
+            delete ps;
+        }
+        {
+            ProfScope* ps = scope(P_TRAIL, 8.0 * n * (double)n * (nb1 + nb2) * nj,
+                                  2.0 * n * (double)n * elem * nj);
+            if (fp64) launch_trailing<double>(st, J, nj, n, k0, nb1, nb2);
+            else if (h3 && n % 4 == 0) launch_trailing_h3(st, J, nj, n, k0, nb1, nb2);
+            else launch_trailing<float>(st, J, nj, n, k0, nb1, nb2);
+            delete ps;
+        }
+        k0 += nb1 + nb2;
+    }
+}
+
+// Rebuilds the factors Fs[bad[..]] by the line reduction, with the full-column
+// pivot search when `full` (fresh factors, swapped in; the others keep their
+// storage)
+static int rebuild(Handle* h, const std::vector<Factor*>& Fs, const std::vector<int>& bad, bool full, float* ms) {
+    if (bad.empty()) return FDFD_OK;
+    std::vector<Factor*> sub;
+    for (int f : bad) {
+        Factor* G = new Factor();
+        G->pol = Fs[f]->pol;
+        G->omega = Fs[f]->omega;
+        G->omega_pml = Fs[f]->omega_pml;
+        G->shift = Fs[f]->shift;
+        G->form = Fs[f]->form;
+        G->precision = Fs[f]->precision;
+        sub.push_back(G);
+    }
+    const bool was_full = h->full_pivot_search, was_off = h->nd_off;
+    h->full_pivot_search = was_full || full;
+    h->nd_off = true;
+    const int rc = rt_build_factors(h, sub);
+    h->full_pivot_search = was_full;
+    h->nd_off = was_off;
+    if (rc) {
+        for (Factor* G : sub) rt_free_factor(h, G);
+        return rc;
+    }
+    *ms = sub[0]->t_factor_ms;
+    for (size_t q = 0; q < bad.size(); ++q) {
+        Factor* F = Fs[bad[q]];
+        const int id = F->id;
+        rt_release_factor_storage(h, F);
+        *F = *sub[q];           // takes over the rebuilt factor's storage
+        F->id = id;
+        F->pivot_fallback = 1;
+        delete sub[q];          // the struct only: its storage now belongs to F
+    }
+    return FDFD_OK;
+}
+
+int rt_rebuild_by_lines(Handle* h, const std::vector<Factor*>& Fs) {
+    std::vector<int> dissected;
+    for (int f = 0; f < (int)Fs.size(); ++f)
+        if (Fs[f]->nd) dissected.push_back(f);
+    float ms = 0;
+    return rebuild(h, Fs, dissected, false, &ms);
+}
+
 int rt_build_factors(Handle* h, const std::vector<Factor*>& Fs) {
     const GridDesc& g = h->g;
     const long N = (long)g.Nx * g.Ny;
@@ -188,6 +301,18 @@ int rt_build_factors(Handle* h, const std::vector<Factor*>& Fs) {
         h->inject = 0;
     if (inject == FDFD_INJECT_OOM)
         return fail(h, FDFD_ERR_OOM, "factor storage allocation failed (injected)");
+    bool forms01 = true;
+    for (Factor* F : Fs) forms01 = forms01 && F->form <= 1;
+    if (forms01 && inject != FDFD_INJECT_SINGULAR && rt_nd_applies(h, g.Nx, g.Ny)) {
+        std::vector<int> bad;
+        if ((rc = rt_build_nd(h, Fs, bad))) return rc;
+        if (inject == FDFD_INJECT_PIVOT_FALLBACK && (bad.empty() || bad[0] != 0)) bad.insert(bad.begin(), 0);
+        const double ms_nd = Fs[0]->t_factor_ms;
+        float ms_redo = 0;
+        if ((rc = rebuild(h, Fs, bad, true, &ms_redo))) return rc;
+        for (Factor* F : Fs) F->t_factor_ms = ms_nd + ms_redo;
+        return FDFD_OK;
+    }
     if ((rc = ensure_factor_work(h, n, std::max(1, P.max_gj * B)))) return rc;
     if ((rc = ensure_solve_work(h, N))) return rc;
     if (trisolve_prepare(n) != (int)hipSuccess)
@@ -360,7 +485,6 @@ int rt_build_factors(Handle* h, const std::vector<Factor*>& Fs) {
     }
 
     const bool fp64 = (prec == FDFD_FP64);
-    const int NB = h->panel_width ? h->panel_width : PMAX;
     auto launch_all = [&](bool full, bool prof) {
         hipStream_t st = h->stream;
         auto scope = [&](int id, double fl, double by) {
@@ -414,65 +538,8 @@ int rt_build_factors(Handle* h, const std::vector<Factor*>& Fs) {
                     og += nj;
                 }
             } else {
-                const LineJob* J = T.lj + ol;
-                launch_gjreset(st, J, nj, n);
-                // Panels of NB columns.  With the windowed search, two panels are
-                // factored before one trailing pass applies both (the second panel's
-                // columns, as the first panel leaves them, are formed by the window
-                // panel for its window and by the Z build's check blocks for every
-                // row, and its pivot rows by the Z build); the full search runs
-                // single panels.
-                for (int k0 = 0; k0 < n;) {
-                    int nb1, nb2 = 0;
-                    const int fresh = std::min(n, WIN + k0);
-                    {
-                        ProfScope* ps = scope(P_PANEL, 0, 0);
-                        if (!full) {
-                            nb1 = std::min(NB, n - k0);
-                            if (fp64) launch_wpanel<double>(st, J, nj, n, k0, nb1, fresh, 0);
-                            else launch_wpanel<float>(st, J, nj, n, k0, nb1, fresh, 0);
-                        } else {
-                            // full-search panel width: powers of two (16 columns of
-                            // complex128 per thread would not fit 1024 threads' registers)
-                            nb1 = fp64 ? 8 : 16;
-                            while (nb1 > n - k0) nb1 >>= 1;
-                            if (fp64) launch_panel<double>(st, J, nj, n, k0, nb1);
-                            else launch_panel<float>(st, J, nj, n, k0, nb1);
-                        }
-                        delete ps;
-                    }
-                    {
-                        ProfScope* ps = scope(P_ZBUILD, 0, 0);
-                        if (fp64) launch_zbuild<double>(st, J, nj, n, k0, nb1, fresh, !full, 0, 0, 0);
-                        else launch_zbuild<float>(st, J, nj, n, k0, nb1, fresh, !full, 0, 0, 0);
-                        delete ps;
-                    }
-                    if (!full && nb1 == PMAX && k0 + nb1 < n && h->fuse_panels) {
-                        const int k2 = k0 + nb1;
-                        nb2 = std::min(NB, n - k2);
-                        const int fresh2 = std::min(n, WIN + k2);
-                        // (the second panel's values as the first panel leaves
-                        // them are formed by the window panel, for its window,
-                        // and by the Z build's check blocks, for every row)
-                        ProfScope* ps = scope(P_PANEL, 0, 0);
-                        if (fp64) launch_wpanel<double>(st, J, nj, n, k2, nb2, fresh2, 1);
-                        else launch_wpanel<float>(st, J, nj, n, k2, nb2, fresh2, 1);
-                        delete ps;
-                        ps = scope(P_ZBUILD, 0, 0);
-                        if (fp64) launch_zbuild<double>(st, J, nj, n, k2, nb2, fresh2, 1, 1, k0, nb1);
-                        else launch_zbuild<float>(st, J, nj, n, k2, nb2, fresh2, 1, 1, k0, nb1);
-                        delete ps;
-                    }
-                    {
-                        ProfScope* ps = scope(P_TRAIL, 8.0 * n * (double)n * (nb1 + nb2) * nj,
-                                              2.0 * n * (double)n * elem * nj);
-                        if (fp64) launch_trailing<double>(st, J, nj, n, k0, nb1, nb2);
-                        else if (h->trail_h3 && n % 4 == 0) launch_trailing_h3(st, J, nj, n, k0, nb1, nb2);
-                        else launch_trailing<float>(st, J, nj, n, k0, nb1, nb2);
-                        delete ps;
-                    }
-                    k0 += nb1 + nb2;
-                }
+                launch_gjreset(st, T.lj + ol, nj, n);
+                rt_launch_gj(h, T.lj + ol, nj, n, fp64, h->trail_h3 != 0, full, prof);
                 ol += nj;
             }
         }
@@ -507,38 +574,12 @@ int rt_build_factors(Handle* h, const std::vector<Factor*>& Fs) {
         if (full || bad.empty()) break;
         if ((int)bad.size() < B) {
             HIPCHK(h, hipEventElapsedTime(&ms, e0, e1));
-            std::vector<Factor*> sub;
-            for (int f : bad) {
-                Factor* G = new Factor();
-                G->pol = Fs[f]->pol;
-                G->omega = Fs[f]->omega;
-                G->omega_pml = Fs[f]->omega_pml;
-                G->shift = Fs[f]->shift;
-                G->form = Fs[f]->form;
-                G->precision = Fs[f]->precision;
-                sub.push_back(G);
-            }
-            const bool was_full = h->full_pivot_search;
-            h->full_pivot_search = true;
-            rc = rt_build_factors(h, sub);
-            h->full_pivot_search = was_full;
-            if (rc) {
-                for (Factor* G : sub) rt_free_factor(h, G);
+            if ((rc = rebuild(h, Fs, bad, true, &ms_redo))) {
                 (void)hipEventDestroy(e0);
                 (void)hipEventDestroy(e1);
                 return rc;
             }
-            ms_redo = sub[0]->t_factor_ms;
-            for (size_t q = 0; q < bad.size(); ++q) {
-                Factor* F = Fs[bad[q]];
-                const int id = F->id;
-                rt_release_factor_storage(h, F);
-                *F = *sub[q];           // takes over the rebuilt factor's storage
-                F->id = id;
-                F->pivot_fallback = 1;
-                delete sub[q];          // the struct only: its storage now belongs to F
-                redo.push_back(bad[q]);
-            }
+            redo = bad;
             break;
         }
     }
@@ -683,6 +724,7 @@ static void launch_solve(Handle* h, Factor* F, bool prof) {
 // (direct launches while per-kernel profiling is on).
 int rt_prec_apply(Handle* h, Factor* F, int trans, const double2* in, double2* out) {
     const GridDesc& g = h->g;
+    if (F->nd) return rt_nd_solve(h, F, trans, in, out, 0, nullptr, 1, h->prof.enabled);
     const long N = (long)g.Nx * g.Ny;
     // A'^T = W^-1 A' W with W = sxf (x) syf (driven form) or sxb (x) syb
     // (sideband form): the periodic differences satisfy dxf^T = -dxb

@@ -146,8 +146,8 @@ static void launch_solve_multi(Handle* h, Factor* F, long rs, const int* ridx, i
     }
 }
 
-int rt_gmres_multi(Handle* h, Factor* F, int nr, const double2* B, double2* X, double tol,
-                   int* iters, double* worst) {
+static int gmres_multi(Handle* h, Factor* F, int nr, const double2* B, double2* X, double tol,
+                       int* iters, double* worst) {
     if (nr < 1 || nr > KMULTI) return fail(h, FDFD_ERR_INVALID, "1 <= sources <= 16 per multi solve");
     if (F->form != 0 && F->form != 1)
         return fail(h, FDFD_ERR_INVALID, "multi-source solves take driven or sideband factors");
@@ -290,7 +290,11 @@ int rt_gmres_multi(Handle* h, Factor* F, int nr, const double2* B, double2* X, d
             // Z_j = M^-1 V_j (through the x_out slots of the reduced solve)
             std::vector<double2> one(ni, make_double2(1.0, 0.0));
             if ((rc = scale(h->x_out, Vj, one))) return rc;
-            launch_solve_multi(h, F, N, m.ridx, ni, prof);
+            if (F->nd) {
+                if ((rc = rt_nd_solve(h, F, 0, h->x_out, h->x_out, N, m.ridx, ni, prof))) return rc;
+            } else {
+                launch_solve_multi(h, F, N, m.ridx, ni, prof);
+            }
             if ((rc = scale(Zj, h->x_out, one))) return rc;
             // W = A' Z_j, then CGS2 against V_0..V_j
             apply(W, Zj, nullptr, ni);
@@ -387,6 +391,22 @@ int rt_gmres_multi(Handle* h, Factor* F, int nr, const double2* B, double2* X, d
         return fail(h, FDFD_ERR_NOCONV, buf);
     }
     return FDFD_OK;
+}
+
+// The lockstep solve; a dissected factor on which a source fails is rebuilt by
+// the line reduction and the solve repeated.
+int rt_gmres_multi(Handle* h, Factor* F, int nr, const double2* B, double2* X, double tol,
+                   int* iters, double* worst) {
+    const double before = *worst;
+    int rc = gmres_multi(h, F, nr, B, X, tol, iters, worst);
+    if (rc == FDFD_ERR_NOCONV && F->nd) {
+        if ((rc = rt_rebuild_by_lines(h, {F}))) return rc;
+        const long N = (long)h->g.Nx * h->g.Ny;
+        launch_zero(h->stream, X, N * nr);
+        *worst = before;
+        rc = gmres_multi(h, F, nr, B, X, tol, iters, worst);
+    }
+    return rc;
 }
 
 }  // namespace fdfd

@@ -1,0 +1,68 @@
+// Arguments of the nested-dissection kernels (k_nd.hip), filled by nd.cpp.
+#pragma once
+
+#include "fdfd_common.h"
+#include "nd_plan.h"
+
+namespace fdfd {
+
+// one level of the tree on the device; offsets are in complex entries
+struct NdLev {
+    int kind, nch, cnt, p, b;
+    int cb;           // boundary size of the child level
+    int stat;         // first pivot-statistics slot of the level
+    const int* node;  // cnt x (p + b) cells, -1 padding
+    const short* cm;  // cnt x 2 x (p + b) positions in the children's boundaries
+    long offX, offQ;        // X (cnt x p x p) and Q (cnt x p x b) in the arena
+    long offV, offU, offUc; // solve vectors: separator values, boundary updates, children's updates
+};
+
+struct NdMapArgs {
+    int kind, nch, cnt, p, b, wrapx, wrapy, cwrapx, cwrapy, Nx, Ny;
+    const nd::Box *box, *cbox;
+};
+
+// per factor
+struct NdFac {
+    const double2* coef;  // symmetrised operator planes (CC, CE, CN)
+    void* arena;
+    double* pivstat;      // 3 per front
+};
+
+// Gauss-Jordan scratch of a level, one slot per (factor, front)
+struct NdGj {
+    void *Y, *F12, *Vbuf, *LU, *Z;
+    int *used, *prow, *iprow, *piv, *win, *verr;
+    LineJob* jobs;
+};
+
+// vectors of a reduced solve: source ridx[s] (0 without a list) at in / out
+// + ridx * rs, one source's work vectors, and the scaling of the input
+// (six (x) siy) and output (sox (x) soy)
+struct NdVec {
+    const double2* in;
+    double2* out;
+    long rs;
+    const int* ridx;
+    double2 *v, *u, *x;
+    const double2 *six, *siy, *sox, *soy;
+};
+
+void launch_nd_maps(hipStream_t s, const NdMapArgs& a, int* node, short* cm);
+void launch_nd_symmetrise(hipStream_t s, double2* coef, double2* us, const double2* wx,
+                          const double2* wy, int Nx, int Ny);
+void launch_nd_leaf(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, int Nx, int Ny, void* S);
+void launch_nd_asm(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, int Nx, int Ny,
+                   const void* Sc, const NdGj& w);
+void launch_nd_unperm(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, const NdGj& w);
+void launch_nd_gemm(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, const void* F12,
+                    const void* Sc, void* S, bool schur);
+void launch_nd_stat(hipStream_t s, const NdFac* fac, int B, int nfronts, double* out);
+void launch_nd_up(hipStream_t s, const NdLev& lv, const void* arena, const NdVec& z, int Nx);
+void launch_nd_down(hipStream_t s, const NdLev& lv, const void* arena, const NdVec& z, int Nx);
+// several sources (at most 16): pack / unpack, one level up, one level down
+void launch_ndm_io(hipStream_t s, const NdVec& z, void* x, long N, int Nx, int na, bool pack);
+void launch_ndm_up(hipStream_t s, const NdLev& lv, const void* arena, void* vp, void* up, const void* x);
+void launch_ndm_down(hipStream_t s, const NdLev& lv, const void* arena, const void* vp, void* x);
+
+}  // namespace fdfd

@@ -220,7 +220,8 @@ void rt_release_factor_storage(Handle* h, Factor* F) {
     if (!F) return;
     (void)hipStreamSynchronize(h->stream);  // the arena may be reused by the next factor
     for (void* b : {(void*)F->coef, (void*)F->sxf, (void*)F->sxb, (void*)F->syf, (void*)F->syb,
-                    (void*)F->prow, (void*)F->iprow, (void*)F->pivstat, F->tabs, (void*)F->triw})
+                    (void*)F->prow, (void*)F->iprow, (void*)F->pivstat, F->tabs, (void*)F->triw,
+                    (void*)F->ndu})
         buf_free(h, b);
     arena_give(h, F->blocks, F->blocks_bytes);
     arena_give(h, F->blocks_b, F->blocks_b_bytes);
@@ -235,6 +236,8 @@ void rt_release_factor_storage(Handle* h, Factor* F) {
     F->trs_tab = nullptr;
     F->triw = nullptr;
     F->solve_exec = nullptr;
+    F->ndu = nullptr;
+    F->nd.reset();
 }
 
 static void free_factor(Handle* h, Factor* F) {
@@ -446,9 +449,11 @@ int rt_gmres_op(Handle* h, long N,
     return fail(h, FDFD_ERR_NOCONV, buf);
 }
 
-// FGMRES on one factor's operator A' (or A'^T), preconditioned by the factor
+// FGMRES on one factor's operator A' (or A'^T), preconditioned by the factor.
+// A dissected factor on which it fails above the residual `accept` (that the
+// caller would take) is rebuilt by the line reduction and the solve repeated.
 static int gmres(Handle* h, Factor* F, int trans, const double2* b, double2* x, double tol,
-                 int max_restarts, SolveStats& st) {
+                 int max_restarts, SolveStats& st, double accept = 0) {
     const GridDesc& g = h->g;
     const long N = (long)g.Nx * g.Ny;
     auto apply = [&](const double2* xx, double2* yy, const double2* bb) -> int {
@@ -458,8 +463,20 @@ static int gmres(Handle* h, Factor* F, int trans, const double2* b, double2* x, 
         return FDFD_OK;
     };
     auto prec = [&](const double2* v, double2* z) -> int { return rt_prec_apply(h, F, trans, v, z); };
-    return rt_gmres_op(h, N, apply, prec, h->V, h->Zk, b, x, tol, max_restarts, &st.iters,
-                       &st.restarts, &st.resid);
+    const bool injected = h->inject == FDFD_INJECT_NOCONV;
+    int rc = rt_gmres_op(h, N, apply, prec, h->V, h->Zk, b, x, tol, max_restarts, &st.iters,
+                         &st.restarts, &st.resid);
+    // an injected cut is a failure also where the few iterations suffice, as
+    // one does with dissected (complex128) factors
+    if (rc == FDFD_OK && injected && F->nd)
+        return fail(h, FDFD_ERR_NOCONV, "refinement did not reach the tolerance (injected)");
+    if (rc == FDFD_ERR_NOCONV && F->nd && !injected && st.resid > accept) {
+        if ((rc = rt_rebuild_by_lines(h, {F}))) return rc;
+        launch_zero(h->stream, x, N);
+        rc = rt_gmres_op(h, N, apply, prec, h->V, h->Zk, b, x, tol, max_restarts, &st.iters,
+                         &st.restarts, &st.resid);
+    }
+    return rc;
 }
 
 }  // namespace fdfd
@@ -519,6 +536,8 @@ int fdfd_create(int device_ordinal, fdfd_handle** out) {
     const char* ef = std::getenv("FDFD_FUSE_PANELS");
     hh->impl.fuse_panels = (ef && ef[0] == '0') ? 0 : 1;
     hh->impl.env_knobs = e3 || ew || eb || et || ef;
+    const char* emeth = std::getenv("FDFD_METHOD");
+    hh->impl.nd_off = emeth && std::strcmp(emeth, "bcr") == 0;
     const char* em = std::getenv("FDFD_MV_MFMA");
     hh->impl.mv_mfma = (em && em[0] == '0') ? 0 : 1;
     if (hipStreamCreateWithFlags(&hh->impl.stream, hipStreamNonBlocking) != hipSuccess) {
@@ -546,7 +565,7 @@ int fdfd_destroy(fdfd_handle* hh) {
     free_multi_work(h);
     void* bufs[] = {h->eps, h->used, h->piv, h->win, h->verr, h->Vbuf, h->LU, h->Zb,
                     h->g_mid, h->x_out, h->V, h->Zk, h->tmp, h->tmp2, h->bvec, h->xvec,
-                    h->dpart, h->rpart, h->hdev, h->bslab, h->io};
+                    h->dpart, h->rpart, h->hdev, h->bslab, h->io, h->nd_scratch, h->nd_vec};
     for (void* b : bufs) dfree(b);
     if (h->tstage) (void)hipHostFree(h->tstage);
     if (h->tstage_ev) (void)hipEventDestroy(h->tstage_ev);
@@ -983,7 +1002,7 @@ namespace fdfd {
 int rt_gmres(Handle* h, Factor* F, int trans, const double2* b, double2* x, double tol, int* iters,
              double* resid) {
     SolveStats st;
-    int rc = gmres(h, F, trans, b, x, tol, MAX_RESTARTS, st);
+    int rc = gmres(h, F, trans, b, x, tol, MAX_RESTARTS, st, 1e-8);
     if (iters) *iters += st.iters;
     if (resid) *resid = st.resid;
     return rc;

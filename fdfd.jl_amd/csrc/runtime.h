@@ -6,6 +6,7 @@
 #include <complex>
 #include <functional>
 #include <map>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -15,6 +16,8 @@
 namespace fdfd {
 
 using cd = std::complex<double>;
+
+struct NdPlan;
 
 // per-kernel profile slots: Gauss-Jordan trailing update, panel, block
 // formation, reduced-solve steps, stencil/residual, Z build, complex GEMM,
@@ -73,6 +76,11 @@ struct Factor {
     double pivot_growth = 0;
     int singular_line = -1;
     int pivot_fallback = 0;   // 1 if the full-column pivot search was used
+    // nested dissection (nd.cpp): the tree the factor was built on (null: line
+    // reduction) and the symmetrising vectors ux, 1/ux, uy, 1/uy; the factor
+    // entries are in `blocks`
+    std::shared_ptr<NdPlan> nd;
+    double2* ndu = nullptr;
 };
 
 struct Handle {
@@ -99,6 +107,7 @@ struct Handle {
     int gemm_b3 = 1;                   // mixed path: three-product fp16 GEMMs (FDFD_MIXED_GEMM=fp32: FP32)
     int trail_h3 = 1;                  // mixed path: three-product fp16 trailing updates (FDFD_MIXED_TRAIL=fp32: FP32)
     int fuse_panels = 1;               // two Gauss-Jordan panels per trailing pass (FDFD_FUSE_PANELS=0)
+    bool nd_off = false;               // line reduction only (FDFD_METHOD=bcr)
     bool env_knobs = false;            // a variant switch above came from the environment
     bool tuned_explicitly = false;     // fdfd_autotune chose the variants (no cache lookup)
     // sweep / Krylov work
@@ -150,6 +159,13 @@ struct Handle {
     void* io = nullptr;
     size_t io_bytes = 0;
     long eps_n = 0;      // cells the eps buffer holds
+    // nested dissection: plans of the last few grid shapes, build scratch and
+    // solve vectors (grown as needed)
+    std::vector<std::shared_ptr<NdPlan>> nd_plans;
+    void* nd_scratch = nullptr;
+    size_t nd_scratch_bytes = 0;
+    void* nd_vec = nullptr;
+    size_t nd_vec_bytes = 0;
 };
 
 // error helper: record message, return code
@@ -256,6 +272,17 @@ int rt_gmres_op(Handle* h, long N, const std::function<int(const double2*, doubl
 int rt_build_factors(Handle* h, const std::vector<Factor*>& Fs);
 int rt_build_factor(Handle* h, Factor* F);
 int rt_prec_apply(Handle* h, Factor* F, int trans, const double2* in, double2* out);
+// nested dissection (nd.cpp)
+constexpr int ND_MIN_LINE = 16;  // shorter lines: line reduction
+bool rt_nd_applies(const Handle* h, int Nx, int Ny);
+void rt_nd_bytes(int Nx, int Ny, size_t* arena, size_t* scratch);
+int rt_nd_prepare(Handle* h, int Nx, int Ny);
+// rebuilds the dissected factors among Fs by the line reduction (a solve whose
+// refinement failed on them is then tried once more)
+int rt_rebuild_by_lines(Handle* h, const std::vector<Factor*>& Fs);
+int rt_build_nd(Handle* h, const std::vector<Factor*>& Fs, std::vector<int>& bad);
+int rt_nd_solve(Handle* h, Factor* F, int trans, const double2* in, double2* out, long rs,
+                const int* ridx, int na, bool prof);
 size_t rt_factor_bytes(int n, int m, int precision, bool b3);
 void rt_factor_arena_sizes(int n, int m, int precision, bool b3, size_t* blocks, size_t* split);
 

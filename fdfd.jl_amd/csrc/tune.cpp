@@ -146,6 +146,8 @@ extern "C" int fdfd_autotune(fdfd_handle* hh, int pol, double omega, int precisi
     const Knobs start = get_knobs(h);
     Knobs best = start;
     double best_ms = 1e300;
+    const bool nd_was_off = h->nd_off;
+    h->nd_off = true;  // the variants are the line reduction's
     for (const Knobs& k : candidates(precision)) {
         if (rc) break;
         set_knobs(h, k);
@@ -173,6 +175,7 @@ extern "C" int fdfd_autotune(fdfd_handle* hh, int pol, double omega, int precisi
             best = k;
         }
     }
+    h->nd_off = nd_was_off;
     (void)hipFree(dsrc);
     (void)hipFree(dout);
     set_knobs(h, rc ? start : best);

@@ -48,7 +48,12 @@ typedef struct {
 /* Polarization: src/types.jl:20 (@enum Polarization TM=1 TE=2). */
 enum { FDFD_TM = 1, FDFD_TE = 2 };
 
-/* Factor precision.  FDFD_FP64: complex128 block factors (the plain path).
+/* Factor precision.  Driven and sideband operators on grids of at least 16
+ * lines (min(Nx, Ny) >= 16) are factored by nested dissection, with
+ * complex128 entries under either option.  Other operators and grids, and
+ * every factorization of a handle created with FDFD_METHOD=bcr (or any of the
+ * variant switches) in the environment, use the reduction of the grid's lines:
+ * FDFD_FP64: complex128 block factors (the plain path).
  * FDFD_FP32_IR: complex64 block factors, accuracy restored by FP64 flexible
  * GMRES on the exact FP64 operator.  The complex64 products run by default as
  * fp16x3 MFMA products of row-scaled split operands (about 22-bit products,
@@ -379,8 +384,9 @@ int fdfd_get_tuning(fdfd_handle* h, int* knobs, int nknobs);
  *   FDFD_INJECT_SINGULAR        next factorization reports a zero pivot in
  *                               line block `arg` (FDFD_ERR_SINGULAR)
  *   FDFD_INJECT_NOCONV          next refined solve runs at most `arg` FGMRES
- *                               iterations and no restart (FDFD_ERR_NOCONV
- *                               unless that reaches the tolerance)
+ *                               iterations and no restart (FDFD_ERR_NOCONV;
+ *                               on factors of the line reduction unless that
+ *                               reaches the tolerance)
  *   FDFD_INJECT_OOM             next factorization fails its storage
  *                               allocation (FDFD_ERR_OOM) */
 enum {
