@@ -121,108 +121,327 @@ __device__ inline double2 nd_entry(const double2* coef, long N, int Nx, int Ny, 
 }
 
 // ---------------------------------------------------------------------------
-// Leaves: one workgroup per leaf, the whole front (p + b <= 16 T) in
-// registers as a 16 x 16 cyclic distribution (thread (ti, tj) holds entries
-// (ti + 16 a, tj + 16 c)), eliminated cell by cell in place (a sweep): the
-// pivot row goes through LDS, double-buffered, one barrier per cell.  By
-// symmetry the pivot column is the pivot row with the sign of the already
-// swept rows flipped.
+// In-place inversion by sweeps.  Sweeping cell k of a symmetric matrix M replaces
+//   M_ij -= M_ik M_kj / d,  M_kj /= d,  M_ik /= -d,  M_kk = 1 / d,  d = M_kk,
+// and sweeping the first np cells leaves M_ss^-1, Q = M_ss^-1 M_su above -Q^T,
+// and the Schur complement.  Entries between swept and unswept cells are
+// antisymmetric, all others symmetric, so only one triangle is kept; sweeps
+// commute, so nothing is permuted.
+//
+// A matrix of 16 T cells is held in registers by the four waves of a
+// workgroup, lower 16 x 16 tiles (I, J) in the MFMA accumulator layout, tile
+// number I (I + 1) / 2 + J on wave (number % 4).  A block of 16 cells is swept at
+// once:
+//   a  the wave of tile (k, k) sweeps it on its own (nd_sweep16), the others put
+//      the block row R_J = M_kJ into LDS;
+//   b  Z_J = D^-1 R_J on MFMA, replacing tiles (k, J) by Z_J, (I, k) by -Z_I^T;
+//   c  M_IJ -= sigma_I R_I^T Z_J on the other tiles, sigma = -1 for swept I;
+//      the wave of the next diagonal tile goes on to its sweep meanwhile.
+// Cells are taken in order: with FP64 fronts and refinement the growth this
+// allows (1e4 .. 1e5, like the near-resonances of the boxes) costs nothing that
+// pivoting inside a separator would save.  What bounds a small inversion is the
+// instruction count of its chain (a wave issues one in four cycles or more, an
+// FP64 operation takes 16 from operand to result): sweeping 64 cells one by one
+// with diagonal pivoting took 55 us on all four waves and 38 us in 16-cell
+// tiles, four by four on all waves (817 instructions a step) 28 us.
 // ---------------------------------------------------------------------------
-template <int T>
-__global__ __launch_bounds__(256) void k_nd_leaf(NdLev lv, const NdFac* fac, int Nx, int Ny, void* Sv) {
-    const NdFac F = fac[blockIdx.y];
-    const int p = lv.p, b = lv.b, f = p + b, fr = blockIdx.x;
-    const long N = (long)Nx * Ny;
-    __shared__ int nd[16 * T];
-    __shared__ C row[2][16 * T];
-    const int t = threadIdx.x, ti = t >> 4, tj = t & 15;
-    for (int i = t; i < 16 * T; i += 256) nd[i] = i < f ? lv.node[(long)fr * f + i] : -1;
-    __syncthreads();
-    C A[T][T];
+__device__ inline C nd_rcp(C z) {
+    // 1 / z from one hardware reciprocal of |z|^2 (about half the bits) and one
+    // step r (1 + e + e^2), e = 1 - n r (the entries are scaled to O(1) and grow
+    // by 1e6 or so: no range handling)
+    const double n = fma(z.x, z.x, z.y * z.y), r0 = rcp_hw(n);
+    const double e = fma(-n, r0, 1.0), r = fma(r0, fma(e, e, e), r0);
+    return mk<C>(z.x * r, -z.y * r);
+}
+// a b + c in four fused steps
+__device__ inline C cfma(C a, C b, C c) {
+    return mk<C>(fma(a.x, b.x, fma(-a.y, b.y, c.x)), fma(a.x, b.y, fma(a.y, b.x, c.y)));
+}
+
+using F64 = mfma_t<double>;
+
+// smallest and largest 2 x 2 pivot determinant (|re| + |im|), and whether one was
+// zero or not finite
+struct NdPiv {
+    double mn = 1e300, mx = 0;
+    bool bad = false;
+    __device__ inline void add(C det) {
+        const double m = cabs1(det);
+        mn = fmin(mn, m);
+        mx = fmax(mx, m);
+        bad = bad || !(m > 0 && m < 1e300);
+    }
+};
+
+// inverse of a symmetric 2 x 2 block [a b; b c]
+__device__ inline void nd_inv2(C a, C b, C c, C& x, C& y, C& z, NdPiv& pv) {
+    const C det = cfma(a, c, cneg(cmul(b, b)));
+    pv.add(det);
+    const C r = nd_rcp(det);
+    x = cmul(c, r);
+    y = cneg(cmul(b, r));
+    z = cmul(a, r);
+}
+
+// One wave sweeps the first kw cells (a multiple of 4) of its 16 x 16 tile, four
+// at a time, the K of one 16 x 16 x 4 product: rows 4 v .. 4 v + 3 are entry v
+// of the lanes, so the pivot rows are both operands as they stand,
+//   M -= sigma R^T Z,  Z = D^-1 R,
+// with the 4 x 4 pivot block D inverted by every lane (two 2 x 2 blocks, two
+// reciprocals), pivot rows replaced by Z and pivot columns by -sigma R^T D^-1.
+__device__ __attribute__((always_inline)) inline void nd_sweep16(d4v& mr, d4v& mi, int kw, C (*R)[17], NdPiv& pv) {
+    const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+    static_for<0, 4>([&](auto vc) {
+        constexpr int v = decltype(vc)::value, k0 = 4 * v;
+        if (k0 < kw) {  // uniform
+            const bool quad = (l16 >> 2) == v;
+            C a = mk<C>(mr[v], mi[v]);
+            R[g][l16] = a;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            auto D = [&](int i, int j) { return R[i][k0 + j]; };
+            const C d00 = D(0, 0), d01 = D(0, 1), d11 = D(1, 1), a0 = D(0, 2), a1 = D(0, 3), a2 = D(1, 2),
+                    a3 = D(1, 3), d22 = D(2, 2), d23 = D(2, 3), d33 = D(3, 3);
+            const C b0 = R[0][l16], b1 = R[1][l16], b2 = R[2][l16], b3 = R[3][l16];
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            // D^-1 = [P + X S^-1 X^T, -X S^-1; ., S^-1], P = D11^-1, X = P D12,
+            // S = D22 - D12^T X
+            C p0, p1, p2, s0, s1, s2;
+            nd_inv2(d00, d01, d11, p0, p1, p2, pv);
+            const C x0 = cfma(p0, a0, cmul(p1, a2)), x1 = cfma(p0, a1, cmul(p1, a3));
+            const C x2 = cfma(p1, a0, cmul(p2, a2)), x3 = cfma(p1, a1, cmul(p2, a3));
+            const C na0 = cneg(a0), na1 = cneg(a1), na2 = cneg(a2), na3 = cneg(a3);
+            nd_inv2(cfma(na0, x0, cfma(na2, x2, d22)), cfma(na0, x1, cfma(na2, x3, d23)),
+                    cfma(na1, x1, cfma(na3, x3, d33)), s0, s1, s2, pv);
+            const C y0 = cfma(x0, s0, cmul(x1, s1)), y1 = cfma(x0, s1, cmul(x1, s2));  // X S^-1
+            const C y2 = cfma(x2, s0, cmul(x3, s1)), y3 = cfma(x2, s1, cmul(x3, s2));
+            const C q0 = cfma(y0, x0, cfma(y1, x1, p0)), q1 = cfma(y0, x2, cfma(y1, x3, p1)),
+                    q2 = cfma(y2, x2, cfma(y3, x3, p2));
+            // this lane group's row of D^-1, and the entry for a pivot column
+            auto pick = [&](int i, C a, C b, C c, C e) {
+                const C lo = csel((i & 1) != 0, b, a), hi = csel((i & 1) != 0, e, c);
+                return csel((i & 2) != 0, hi, lo);
+            };
+            const C n0 = cneg(y0), n1 = cneg(y1), n2 = cneg(y2), n3 = cneg(y3);
+            const C r0 = pick(g, q0, q1, n0, n1), r1 = pick(g, q1, q2, n2, n3), r2 = pick(g, n0, n2, s0, s1),
+                    r3 = pick(g, n1, n3, s1, s2);
+            C z = cfma(r0, b0, cfma(r1, b1, cfma(r2, b2, cmul(r3, b3))));
+            z = csel(quad, pick(l16, r0, r1, r2, r3), z);
+            a = csel(l16 < k0, a, cneg(a));  // antisymmetric to swept cells
 #pragma unroll
-    for (int a = 0; a < T; ++a)
-#pragma unroll
-        for (int c = 0; c < T; ++c) {
-            const int i = ti + 16 * a, j = tj + 16 * c;
-            const int ki = nd[i], kj = nd[j];
-            A[a][c] = mk<C>(R(0), R(0));
-            if (i < p || j < p) {
-                if (ki >= 0 && kj >= 0) A[a][c] = (nd_entry(F.coef, N, Nx, Ny, ki, kj));
-                else if (i == j) A[a][c] = mk<C>(R(1), R(0));
+            for (int w = 0; w < 4; ++w) {
+                mr[w] = quad ? 0.0 : mr[w];
+                mi[w] = quad ? 0.0 : mi[w];
             }
-        }
-    R mn = R(1e30), mx = R(0);
-    bool zero = false;
-    static_for<0, T>([&](auto ac) {
-        constexpr int ka = decltype(ac)::value;
-        for (int kk = 0; kk < 16; ++kk) {
-            const int k = 16 * ka + kk;
-            if (k >= p) break;  // uniform
-            C* rb = row[kk & 1];
-            if (ti == kk) {
-#pragma unroll
-                for (int c = 0; c < T; ++c) rb[tj + 16 * c] = A[ka][c];
-            }
-            __syncthreads();
-            const C d = rb[k];
-            const C r = crcp_scaled(d);
-            if (nd[k] >= 0) {
-                const R m = cabs1(d);
-                mn = m < mn ? m : mn;
-                mx = m > mx ? m : mx;
-                if (!(m > R(0))) zero = true;
-            }
-            C ci[T], rj[T];
-#pragma unroll
-            for (int a = 0; a < T; ++a) {
-                const int i = ti + 16 * a;
-                const C v = cmul(rb[i], r);           // F[k][i] / d
-                ci[a] = i < k ? v : cneg(v);          // -F[i][k] / d
-                rj[a] = rb[tj + 16 * a];
-            }
-#pragma unroll
-            for (int a = 0; a < T; ++a)
-#pragma unroll
-                for (int c = 0; c < T; ++c) A[a][c] = cadd(A[a][c], cmul(ci[a], rj[c]));
-            // pivot column and row (overwrite the update of their entries)
-            if (tj == kk) {
-#pragma unroll
-                for (int a = 0; a < T; ++a) A[a][ka] = ci[a];
-            }
-            if (ti == kk) {
-#pragma unroll
-                for (int c = 0; c < T; ++c) A[ka][c] = cmul(rj[c], r);
-                if (tj == kk) A[ka][ka] = r;
-            }
+            mr = F64::run(a.x, z.x, mr);
+            mi = F64::run(a.x, z.y, mi);
+            mr = F64::run(-a.y, z.y, mr);
+            mi = F64::run(a.y, z.x, mi);
+            mr[v] = z.x;
+            mi[v] = z.y;
         }
     });
-    C* X = (C*)F.arena + lv.offX + (long)fr * p * p;
-    C* Q = (C*)F.arena + lv.offQ + (long)fr * p * b;
-    C* S = (C*)Sv + ((long)blockIdx.y * lv.cnt + fr) * b * b;
+}
+
+// DB: the block row is double-buffered (one barrier less a block, more LDS)
+template <int T> struct NdSweep {
+    static constexpr int NTL = T * (T + 1) / 2, NS = (NTL + 3) / 4;  // tiles, slots per wave
+    static constexpr bool DB = T <= 4;
+    C R[DB ? 2 : 1][T][16][17];
+    C Z[T][16][17];
+    C D[16][17];
+    double pv[4][3];
+};
+
+// f(slot, I, J) for the tiles of this wave (I, J wave-uniform)
+template <int T, typename F> __device__ __attribute__((always_inline)) inline void nd_each_tile(F&& f) {
+    const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    static_for<0, NdSweep<T>::NS>([&](auto sc) {
+        const int e = 4 * decltype(sc)::value + wv;
+        if (e < NdSweep<T>::NTL) {
+            int I = 0;
 #pragma unroll
-    for (int a = 0; a < T; ++a)
-#pragma unroll
-        for (int c = 0; c < T; ++c) {
-            const int i = ti + 16 * a, j = tj + 16 * c;
-            if (i < p && j < p) gstore(X + i * p + j, A[a][c]);
-            else if (i < p && j < f) gstore(Q + i * b + (j - p), A[a][c]);
-            else if (i >= p && i < f && j >= p && j < f) gstore(S + (i - p) * b + (j - p), A[a][c]);
+            for (int q = 1; q < T; ++q) I += e >= q * (q + 1) / 2;
+            f(sc, I, e - I * (I + 1) / 2);
         }
-    if (t == 0) {
-        double* ps = F.pivstat + 3 * (long)(lv.stat + fr);
-        ps[0] = (double)mn;
-        ps[1] = (double)mx;
-        ps[2] = zero ? 1.0 : 0.0;
+    });
+}
+// f(slot, v, i, j, off) for the entries of this thread (off: an off-diagonal
+// tile, whose mirror image is not stored)
+template <int T, typename F> __device__ __attribute__((always_inline)) inline void nd_each_entry(F&& f) {
+    const int lane = threadIdx.x & 63;
+    nd_each_tile<T>([&](auto sc, int I, int J) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) f(sc, v, 16 * I + F64::row(lane, v), 16 * J + (lane & 15), I != J);
+    });
+}
+
+// sweeps the first np cells (a multiple of 4); pst: pivot statistics, combined
+// with what is there when `add`
+template <int T>
+__device__ __attribute__((always_inline)) inline void nd_sweep(d4v (&mr)[NdSweep<T>::NS], d4v (&mi)[NdSweep<T>::NS],
+                                                               int np, NdSweep<T>& s, double* pst, bool add) {
+    const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+    NdPiv pv;
+#pragma unroll 1
+    for (int kb = 0; 16 * kb < np; ++kb) {
+        const int kw = min(16, np - 16 * kb);
+        C(*R)[16][17] = s.R[NdSweep<T>::DB ? kb & 1 : 0];
+        // the diagonal tile of block kb is in slot e / 4 of wave e % 4
+        const int e = kb * (kb + 3) / 2;
+        nd_each_tile<T>([&](auto sc, int I, int J) {
+            if (I != J && I == kb) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) R[J][F64::row(lane, v)][l16] = mk<C>(mr[sc][v], mi[sc][v]);
+            } else if (I != J && J == kb) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) R[I][l16][F64::row(lane, v)] = mk<C>(mr[sc][v], mi[sc][v]);
+            }
+        });
+        if ((e & 3) == __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6)) {
+            // one copy of the sweep's code for all slots
+            d4v xr = mr[0], xi = mi[0];
+#pragma unroll
+            for (int q = 1; q < NdSweep<T>::NS; ++q)
+                if ((e >> 2) == q) {
+                    xr = mr[q];
+                    xi = mi[q];
+                }
+            nd_sweep16(xr, xi, kw, s.D, pv);
+#pragma unroll
+            for (int q = 0; q < NdSweep<T>::NS; ++q)
+                if ((e >> 2) == q) {
+                    mr[q] = xr;
+                    mi[q] = xi;
+                }
+#pragma unroll
+            for (int v = 0; v < 4; ++v) s.D[F64::row(lane, v)][l16] = mk<C>(xr[v], xi[v]);
+        }
+        if (T == 1) break;
+        __syncthreads();
+        const int kq = kw >> 2;  // K steps
+        nd_each_tile<T>([&](auto sc, int I, int J) {
+            if ((I == kb) == (J == kb)) return;
+            const bool rowt = I == kb;  // tile (k, J), else (I, k)
+            // (k, J): D^-1 R_J; (I, k): R_I^T D^-1 (D^-1 is symmetric)
+            const C(*Ap)[17] = rowt ? s.D : R[I];
+            const C(*Bp)[17] = rowt ? R[J] : s.D;
+            d4v xr = {0, 0, 0, 0}, xi = {0, 0, 0, 0}, yr = {0, 0, 0, 0}, yi = {0, 0, 0, 0};
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (q < kq) {
+                    const C av = Ap[4 * q + g][l16], bv = Bp[4 * q + g][l16];
+                    xr = F64::run(av.x, bv.x, xr);
+                    xi = F64::run(av.x, bv.y, xi);
+                    yr = F64::run(av.y, bv.y, yr);
+                    yi = F64::run(av.y, bv.x, yi);
+                }
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const C z = mk<C>(xr[v] - yr[v], xi[v] + yi[v]);
+                if (rowt) s.Z[J][F64::row(lane, v)][l16] = z;
+                else s.Z[I][l16][F64::row(lane, v)] = z;
+                mr[sc][v] = rowt ? z.x : -z.x;
+                mi[sc][v] = rowt ? z.y : -z.y;
+            }
+        });
+        __syncthreads();
+        nd_each_tile<T>([&](auto sc, int I, int J) {
+            if (I == kb || J == kb) return;
+            const C(*Ap)[17] = R[I];
+            const C(*Bp)[17] = s.Z[J];
+            const unsigned long long sg = I > kb ? 0x8000000000000000ull : 0ull;  // subtract unless swept
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (q < kq) {
+                    C av = Ap[4 * q + g][l16];
+                    const C bv = Bp[4 * q + g][l16];
+                    av.x = __longlong_as_double(__double_as_longlong(av.x) ^ (long long)sg);
+                    av.y = __longlong_as_double(__double_as_longlong(av.y) ^ (long long)sg);
+                    mr[sc] = F64::run(av.x, bv.x, mr[sc]);
+                    mi[sc] = F64::run(av.x, bv.y, mi[sc]);
+                    mr[sc] = F64::run(-av.y, bv.y, mr[sc]);
+                    mi[sc] = F64::run(av.y, bv.x, mi[sc]);
+                }
+        });
+        if (!NdSweep<T>::DB) __syncthreads();
+    }
+    // every lane of a wave has the same pivots
+    if (lane == 0) {
+        double* w = s.pv[threadIdx.x >> 6];
+        w[0] = pv.mn;
+        w[1] = pv.mx;
+        w[2] = pv.bad ? 1.0 : 0.0;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double lo = add ? pst[0] : 1e300, hi = add ? pst[1] : 0.0, bad = add ? pst[2] : 0.0;
+        for (int w = 0; w < 4; ++w) {
+            lo = fmin(lo, s.pv[w][0]);
+            hi = fmax(hi, s.pv[w][1]);
+            bad = fmax(bad, s.pv[w][2]);
+        }
+        pst[0] = lo;
+        pst[1] = hi;
+        pst[2] = bad;
     }
 }
 
+// Leaves: one workgroup per leaf, its whole front swept in registers (the
+// separator padded to whole tiles with unit rows, then the boundary).
+template <int T>
+__global__ __launch_bounds__(256, 2) void k_nd_leaf(NdLev lv, const NdFac* fac, int Nx, int Ny, void* Sv) {
+    const NdFac F = fac[blockIdx.y];
+    const int p = lv.p, b = lv.b, p16 = (p + 15) & ~15, fr = blockIdx.x;
+    const long N = (long)Nx * Ny;
+    __shared__ NdSweep<T> s;
+    __shared__ int nd[16 * T];
+    const int t = threadIdx.x;
+    for (int i = t; i < 16 * T; i += 256) {
+        const int e = i < p ? i : (i >= p16 && i < p16 + b ? p + i - p16 : -1);
+        nd[i] = e >= 0 ? lv.node[(long)fr * (p + b) + e] : -1;
+    }
+    __syncthreads();
+    constexpr int NS = NdSweep<T>::NS;
+    d4v mr[NS], mi[NS];
+    nd_each_entry<T>([&](auto sc, int v, int i, int j, bool) {
+        C z = mk<C>(0, 0);
+        const int ki = nd[i], kj = nd[j];
+        if (i < p16 || j < p16) {
+            if (ki >= 0 && kj >= 0) z = nd_entry(F.coef, N, Nx, Ny, ki, kj);
+            else if (i == j) z = mk<C>(1, 0);
+        }
+        mr[sc][v] = z.x;
+        mi[sc][v] = z.y;
+    });
+    nd_sweep<T>(mr, mi, p, s, F.pivstat + 3 * (long)(lv.stat + fr), false);
+    C* X = (C*)F.arena + lv.offX + (long)fr * p * p;
+    C* Q = (C*)F.arena + lv.offQ + (long)fr * p * b;
+    C* S = (C*)Sv + ((long)blockIdx.y * lv.cnt + fr) * b * b;
+    nd_each_entry<T>([&](auto sc, int v, int i, int j, bool off) {
+        const C z = mk<C>(mr[sc][v], mi[sc][v]);
+        const int ib = i - p16, jb = j - p16;
+        if (i < p && j < p) {
+            gstore(X + i * p + j, z);
+            if (off) gstore(X + j * p + i, z);
+        } else if (ib >= 0 && ib < b && j < p) {
+            gstore(Q + j * b + ib, cneg(z));
+        } else if (ib >= 0 && ib < b && jb >= 0 && jb < b) {
+            gstore(S + ib * b + jb, z);
+            if (off) gstore(S + jb * b + ib, z);
+        }
+    });
+}
+
 void launch_nd_leaf(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, int Nx, int Ny, void* S) {
-    const int f = lv.p + lv.b;
+    const int f = ((lv.p + 15) & ~15) + lv.b;
     const dim3 g(lv.cnt, B);
     if (f <= 32) k_nd_leaf<2><<<g, 256, 0, s>>>(lv, fac, Nx, Ny, S);
     else if (f <= 48) k_nd_leaf<3><<<g, 256, 0, s>>>(lv, fac, Nx, Ny, S);
     else if (f <= 64) k_nd_leaf<4><<<g, 256, 0, s>>>(lv, fac, Nx, Ny, S);
-    else k_nd_leaf<5><<<g, 256, 0, s>>>(lv, fac, Nx, Ny, S);
+    else if (f <= 80) k_nd_leaf<5><<<g, 256, 0, s>>>(lv, fac, Nx, Ny, S);
+    else k_nd_leaf<6><<<g, 256, 0, s>>>(lv, fac, Nx, Ny, S);
 }
 
 // children's contribution to entry (i, j) of a front, i, j front indices
@@ -239,93 +458,350 @@ __device__ inline C nd_gather(const NdLev& lv, const C* Sc, const short* cm, int
 }
 
 // ---------------------------------------------------------------------------
-// Assembly of [F11 | F12] of a level: operator entries plus the children's
-// Schur complements, padded separator cells as unit rows.  The first
-// workgroup of a front also writes its Gauss-Jordan job and start state.
+// Assembly of a level's fronts (operator entries plus the children's Schur
+// complements, padded separator cells as unit rows) and the start of their
+// inversion, in one launch:
+//   blocks [0, cnt):  the leading 16 T <= 64 separator cells are gathered into
+//                     registers and swept; the inverse goes to X when that is
+//                     the whole separator, else to D (64 x 64, zero-padded);
+//   blocks [cnt, ..): ASM_ROWS rows of F12, and of the lower triangle of F11
+//                     when the separator is longer than 64 cells.
 // ---------------------------------------------------------------------------
 constexpr int ASM_ROWS = 8;
+constexpr int NB = 64;  // block of the inversion
 
-__global__ __launch_bounds__(256) void k_nd_asm(NdLev lv, const NdFac* fac, int Nx, int Ny,
-                                                const void* Scv, NdGj w, int nchunk) {
-    const int fr = blockIdx.x / nchunk, ch = blockIdx.x % nchunk, q = blockIdx.y;
+template <int T>
+__global__ __launch_bounds__(256, 2) void k_nd_front(NdLev lv, const NdFac* fac, int Nx, int Ny, const void* Scv,
+                                                  NdInv w, int nchunk) {
+    const int q = blockIdx.y, p = lv.p, b = lv.b, f = p + b;
     const NdFac F = fac[q];
-    const int p = lv.p, b = lv.b, f = p + b;
-    const long N = (long)Nx * Ny, job = (long)q * lv.cnt + fr;
+    const long N = (long)Nx * Ny;
+    const bool inv = (int)blockIdx.x < lv.cnt;
+    const int e = (int)blockIdx.x - lv.cnt;
+    const int fr = inv ? (int)blockIdx.x : e / nchunk;
+    const long job = (long)q * lv.cnt + fr;
     const int* node = lv.node + (long)fr * f;
     const short* cm = lv.cm + (long)fr * 2 * f;
     const C* Sc = (const C*)Scv + ((long)q * lv.cnt * lv.nch + (long)fr * lv.nch) * lv.cb * lv.cb;
+    auto entry = [&](int i, int j) {
+        const int ki = node[i], kj = node[j];
+        C v = mk<C>(0, 0);
+        if (ki >= 0 && kj >= 0) v = cadd(nd_entry(F.coef, N, Nx, Ny, ki, kj), nd_gather(lv, Sc, cm, i, j));
+        else if (i == j) v = mk<C>(1, 0);
+        return v;
+    };
+    if (inv) {
+        __shared__ NdSweep<T> s;
+        const int np = min(p, NB);
+        constexpr int NS = NdSweep<T>::NS;
+        d4v mr[NS], mi[NS];
+        nd_each_entry<T>([&](auto sc, int v, int i, int j, bool) {
+            const C z = i < np && j < np ? entry(i, j) : mk<C>(i == j ? 1 : 0, 0);
+            mr[sc][v] = z.x;
+            mi[sc][v] = z.y;
+        });
+        nd_sweep<T>(mr, mi, np, s, F.pivstat + 3 * (long)(lv.stat + fr), false);
+        const bool whole = p <= NB;
+        C* out = whole ? (C*)F.arena + lv.offX + (long)fr * p * p : (C*)w.D + job * 2 * NB * NB;
+        const int ld = whole ? p : NB;
+        nd_each_entry<T>([&](auto sc, int v, int i, int j, bool off) {
+            const C z = mk<C>(mr[sc][v], mi[sc][v]);
+            if (i < np && j < np) {
+                gstore(out + i * ld + j, z);
+                if (off) gstore(out + j * ld + i, z);
+            }
+        });
+        return;
+    }
+    const int ch = e % nchunk, j0 = p > NB ? 0 : p;
     C* Y = (C*)w.Y + job * p * p;
     C* G = (C*)w.F12 + job * p * b;
-    const int t = threadIdx.x;
     for (int r = 0; r < ASM_ROWS; ++r) {
         const int i = ch * ASM_ROWS + r;
         if (i >= p) break;
-        const int ki = node[i];
-        for (int j = t; j < f; j += 256) {
-            const int kj = node[j];
-            C v = mk<C>(R(0), R(0));
-            if (ki >= 0 && kj >= 0) {
-                v = (nd_entry(F.coef, N, Nx, Ny, ki, kj));
-                v = cadd(v, nd_gather(lv, Sc, cm, i, j));
-            } else if (i == j) {
-                v = mk<C>(R(1), R(0));
+        for (int j = j0 + (int)threadIdx.x; j < f; j += 256) {
+            if (j < p) {
+                if (j <= (i | (NB - 1))) gstore(Y + (long)i * p + j, entry(i, j));
+            } else {
+                gstore(G + (long)i * b + (j - p), entry(i, j));
             }
-            if (j < p) gstore(Y + (long)i * p + j, v);
-            else gstore(G + (long)i * b + (j - p), v);
         }
     }
-    if (ch != 0) return;
-    for (int i = t; i < p; i += 256) {
-        w.used[job * p + i] = 0;
-        w.iprow[job * p + i] = -1;
-    }
-    for (int i = t; i < 64; i += 256) w.win[job * 64 + i] = i < p ? i : -1;
-    if (t == 0) {
-        LineJob J;
-        J.Y = Y;
-        J.used = w.used + job * p;
-        J.prow = w.prow + job * p;
-        J.iprow = w.iprow + job * p;
-        J.Vbuf = (C*)w.Vbuf + job * p * VMAX;
-        J.LU = (C*)w.LU + job * 2 * PMAX * PMAX;
-        J.piv = w.piv + job * VMAX;
-        J.Z = (C*)w.Z + job * VMAX * p;
-        J.win = w.win + job * 64;
-        J.verr = w.verr + q;
-        J.pivstat = F.pivstat + 3 * (long)(lv.stat + fr);
-        J.n = p;
-        J.pivstat[0] = __builtin_huge_val();
-        J.pivstat[1] = 0;
-        J.pivstat[2] = 0;
-        w.jobs[job] = J;
-    }
 }
 
-void launch_nd_asm(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, int Nx, int Ny,
-                   const void* Sc, const NdGj& w) {
-    const int nch = (lv.p + ASM_ROWS - 1) / ASM_ROWS;
-    k_nd_asm<<<dim3(lv.cnt * nch, B), 256, 0, s>>>(lv, fac, Nx, Ny, Sc, w, nch);
+void launch_nd_front(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, int Nx, int Ny, const void* Sc,
+                     const NdInv& w) {
+    const int nch = (lv.b == 0 && lv.p <= NB) ? 0 : (lv.p + ASM_ROWS - 1) / ASM_ROWS;
+    const dim3 g(lv.cnt * (1 + nch), B);
+    if (lv.p <= 16) k_nd_front<1><<<g, 256, 0, s>>>(lv, fac, Nx, Ny, Sc, w, nch);
+    else if (lv.p <= 32) k_nd_front<2><<<g, 256, 0, s>>>(lv, fac, Nx, Ny, Sc, w, nch);
+    else if (lv.p <= 48) k_nd_front<3><<<g, 256, 0, s>>>(lv, fac, Nx, Ny, Sc, w, nch);
+    else k_nd_front<4><<<g, 256, 0, s>>>(lv, fac, Nx, Ny, Sc, w, nch);
 }
 
-// X[a][c] = Y[prow[a]][iprow[c]] (natural order) into the factor's arena
-__global__ __launch_bounds__(256) void k_nd_unperm(NdLev lv, const NdFac* fac, NdGj w, int nchunk) {
-    const int fr = blockIdx.x / nchunk, ch = blockIdx.x % nchunk, q = blockIdx.y;
-    const int p = lv.p;
+// ---------------------------------------------------------------------------
+// Separators longer than 64 cells: block sweeps of 64 on the lower tiles of Y.
+// For block k with inverse D^-1 and block row R_J = M_kJ (stored as tile
+// (k, J), or transposed as tile (J, k) for J > k):
+//   k_nd_bz : Z_J = D^-1 R_J; tile (k, J) <- Z_J, tile (J, k) <- -Z_J^T, and
+//             the workgroup of block k + 1 goes on to M_JJ - R_J^T Z_J and
+//             sweeps it, so the next D^-1 is ready when the level's other
+//             tiles are;
+//   k_nd_bu : M_IJ -= sigma_I R_I^T Z_J on the other lower tiles, sigma = -1 for
+//             swept blocks I < k.
+// ---------------------------------------------------------------------------
+// 64 x 64 x 64 complex product by four waves of 32 x 32, operands staged 16 K
+// rows at a time; la(k, i) and lb(k, j) give the entries (KB: neighbouring
+// threads read neighbouring k of B).  Three real products per complex one.
+struct NdTile {
+    using M = mfma_t<double>;
+    double sAr[16][NB + 16], sAi[16][NB + 16], sBr[16][NB + 16], sBi[16][NB + 16];
+};
+struct NdAcc {
+    mfma_t<double>::acc c1[2][2], c2[2][2], c3[2][2];
+};
+template <bool KB, typename LA, typename LB>
+__device__ __attribute__((always_inline)) inline void nd_tile_product(NdTile& s, NdAcc& A, LA&& la, LB&& lb) {
+    using M = mfma_t<double>;
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6, wr = wv >> 1, wc = wv & 1;
+    const int lr = lane & 15, lk = lane >> 4;
+    C ra[4], rb[4];
+    auto load = [&](int k0) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int id = t + 256 * e;
+            ra[e] = la(k0 + (id >> 6), id & 63);
+            rb[e] = KB ? lb(k0 + (id & 15), id >> 4) : lb(k0 + (id >> 6), id & 63);
+        }
+    };
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y) {
+            A.c1[x][y] = M::acc{0, 0, 0, 0};
+            A.c2[x][y] = M::acc{0, 0, 0, 0};
+            A.c3[x][y] = M::acc{0, 0, 0, 0};
+        }
+    load(0);
+    for (int k0 = 0; k0 < NB; k0 += 16) {
+        __syncthreads();  // the previous stage (or the caller's use of s) is consumed
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int id = t + 256 * e;
+            s.sAr[id >> 6][id & 63] = ra[e].x;
+            s.sAi[id >> 6][id & 63] = ra[e].y;
+            const int k = KB ? id & 15 : id >> 6, j = KB ? id >> 4 : id & 63;
+            s.sBr[k][j] = rb[e].x;
+            s.sBi[k][j] = rb[e].y;
+        }
+        __syncthreads();
+        if (k0 + 16 < NB) load(k0 + 16);
+#pragma unroll
+        for (int kk = 0; kk < 16; kk += 4) {
+            double ar[2], ai[2], as[2], br[2], bi[2], bs[2];
+#pragma unroll
+            for (int x = 0; x < 2; ++x) {
+                ar[x] = s.sAr[kk + lk][wr * 32 + x * 16 + lr];
+                ai[x] = s.sAi[kk + lk][wr * 32 + x * 16 + lr];
+                as[x] = ar[x] + ai[x];
+                br[x] = s.sBr[kk + lk][wc * 32 + x * 16 + lr];
+                bi[x] = s.sBi[kk + lk][wc * 32 + x * 16 + lr];
+                bs[x] = br[x] + bi[x];
+            }
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+#pragma unroll
+                for (int y = 0; y < 2; ++y) A.c1[x][y] = M::run(ar[x], br[y], A.c1[x][y]);
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+#pragma unroll
+                for (int y = 0; y < 2; ++y) A.c2[x][y] = M::run(ai[x], bi[y], A.c2[x][y]);
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+#pragma unroll
+                for (int y = 0; y < 2; ++y) A.c3[x][y] = M::run(as[x], bs[y], A.c3[x][y]);
+        }
+    }
+}
+// f(i, j, value) for this thread's entries of the product
+template <typename F> __device__ inline void nd_each_acc(const NdAcc& A, F&& f) {
+    using M = mfma_t<double>;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, wr = wv >> 1, wc = wv & 1;
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                f(wr * 32 + x * 16 + M::row(lane, v), wc * 32 + y * 16 + (lane & 15),
+                  mk<C>(A.c1[x][y][v] - A.c2[x][y][v], A.c3[x][y][v] - A.c1[x][y][v] - A.c2[x][y][v]));
+}
+
+__global__ __launch_bounds__(256, 2) void k_nd_bz(NdLev lv, const NdFac* fac, NdInv w, int k, int nb) {
+    __shared__ union {
+        NdTile s;
+        NdSweep<4> w;
+    } u;
+    NdTile& s = u.s;
+    const int per = max(nb - 1, 1), fr = blockIdx.x / per, q = blockIdx.y, p = lv.p;
+    const long job = (long)q * lv.cnt + fr;
+    const int J = (k + 1 + (int)blockIdx.x % per) % nb;  // block k + 1 first
+    const int kw = min(NB, p - k * NB), jw = min(NB, p - J * NB);
+    C* Y = (C*)w.Y + job * p * p;
+    C* Rb = (C*)w.R + job * NB * p + J * NB;
+    C* Zb = (C*)w.Z + job * NB * p + J * NB;
+    const C* D = (const C*)w.D + (job * 2 + (k & 1)) * NB * NB;
+    const C zero = mk<C>(0, 0);
+    auto ld = [&](const C* ptr, bool ok) {
+        const C v = gload(ok ? ptr : D);
+        return csel(ok, v, zero);
+    };
+    auto dv = [&](int kk, int i) { return ld(D + kk * NB + i, kk < kw && i < kw); };
+    if (blockIdx.x % per == 0) {  // tile (k, k) <- D^-1
+        for (int e = threadIdx.x; e < NB * NB; e += 256) {
+            const int i = e >> 6, j = e & 63;
+            if (i < kw && j < kw) gstore(Y + (long)(k * NB + i) * p + k * NB + j, gload(D + e));
+        }
+    }
+    NdAcc A;
+    if (J < k) {
+        const C* T = Y + (long)k * NB * p + J * NB;
+        auto rv = [&](int kk, int j) { return ld(T + (long)kk * p + j, kk < kw && j < jw); };
+        nd_tile_product<false>(s, A, dv, rv);
+        for (int e = threadIdx.x; e < NB * NB; e += 256) {
+            const int kk = e >> 6, j = e & 63;
+            if (j < jw) gstore(Rb + (long)kk * p + j, rv(kk, j));
+        }
+        __syncthreads();  // the tile is read before it is overwritten
+        nd_each_acc(A, [&](int i, int j, C z) {
+            if (j < jw) {
+                gstore(Zb + (long)i * p + j, i < kw ? z : zero);
+                if (i < kw) gstore(Y + (long)(k * NB + i) * p + J * NB + j, z);
+            }
+        });
+    } else {
+        const C* T = Y + (long)J * NB * p + k * NB;
+        auto rv = [&](int kk, int j) { return ld(T + (long)j * p + kk, kk < kw && j < jw); };
+        nd_tile_product<true>(s, A, dv, rv);
+        for (int e = threadIdx.x; e < NB * NB; e += 256) {
+            const int kk = e & 63, j = e >> 6;
+            if (j < jw) gstore(Rb + (long)kk * p + j, rv(kk, j));
+        }
+        __syncthreads();
+        nd_each_acc(A, [&](int i, int j, C z) {
+            if (j < jw) {
+                gstore(Zb + (long)i * p + j, i < kw ? z : zero);
+                if (i < kw) gstore(Y + (long)(J * NB + j) * p + k * NB + i, cneg(z));
+            }
+        });
+    }
+    if (J != k + 1) return;
+    // M_JJ - R_J^T Z_J, swept: the next block's inverse (R and Z come back
+    // through global memory, written by this workgroup)
+    __threadfence_block();
+    __syncthreads();
+    auto rr = [&](int kk, int i) { return ld(Rb + (long)kk * p + i, i < jw); };
+    auto zz = [&](int kk, int j) { return ld(Zb + (long)kk * p + j, j < jw); };
+    nd_tile_product<false>(s, A, rr, zz);
+    __syncthreads();
+    C* P = (C*)&u.s;  // the product as a 64 x 64 tile, in two halves
+    static_assert(sizeof(NdTile) >= sizeof(C) * NB * NB / 2, "half a product tile fits the stages");
+    constexpr int NS = NdSweep<4>::NS;
+    d4v mr[NS], mi[NS];
+    for (int hf = 0; hf < 2; ++hf) {
+        nd_each_acc(A, [&](int i, int j, C z) {
+            if ((i >> 5) == hf) P[(i & 31) * NB + j] = z;
+        });
+        __syncthreads();
+        nd_each_entry<4>([&](auto sc, int v, int i, int j, bool) {
+            if ((i >> 5) == hf) {
+                const bool ok = i < jw && j < jw;
+                const C old = ld(Y + (long)(J * NB + i) * p + J * NB + j, ok);
+                const C z = csel(ok, csub(old, P[(i & 31) * NB + j]), mk<C>(i == j ? 1 : 0, 0));
+                mr[sc][v] = z.x;
+                mi[sc][v] = z.y;
+            }
+        });
+        __syncthreads();
+    }
+    nd_sweep<4>(mr, mi, jw, u.w, fac[q].pivstat + 3 * (long)(lv.stat + fr), true);
+    C* Dn = (C*)w.D + (job * 2 + ((k + 1) & 1)) * NB * NB;
+    nd_each_entry<4>([&](auto sc, int v, int i, int j, bool off) {
+        const C z = mk<C>(mr[sc][v], mi[sc][v]);
+        gstore(Dn + i * NB + j, z);
+        if (off) gstore(Dn + j * NB + i, z);
+    });
+}
+
+__global__ __launch_bounds__(256, 2) void k_nd_bu(NdLev lv, NdInv w, int k, int nb, int ntile) {
+    __shared__ NdTile s;
+    const int fr = blockIdx.x / ntile, q = blockIdx.y, p = lv.p;
+    const long job = (long)q * lv.cnt + fr;
+    // tile number -> (I, J), I >= J, over the blocks other than k
+    const int e = blockIdx.x % ntile;
+    int I = (int)((sqrtf(8.0f * e + 1.0f) - 1.0f) * 0.5f);
+    while ((I + 1) * (I + 2) / 2 <= e) ++I;
+    while (I * (I + 1) / 2 > e) --I;
+    int J = e - I * (I + 1) / 2;
+    I += I >= k;
+    J += J >= k;
+    if (I == k + 1 && J == k + 1) return;  // done by k_nd_bz
+    const int iw = min(NB, p - I * NB), jw = min(NB, p - J * NB);
+    C* Y = (C*)w.Y + job * p * p + (long)I * NB * p + J * NB;
+    const C* Rb = (const C*)w.R + job * NB * p + I * NB;
+    const C* Zb = (const C*)w.Z + job * NB * p + J * NB;
+    const C zero = mk<C>(0, 0);
+    auto ld = [&](const C* ptr, const C* safe, bool ok) {
+        const C v = gload(ok ? ptr : safe);
+        return csel(ok, v, zero);
+    };
+    NdAcc A;
+    nd_tile_product<false>(
+        s, A, [&](int kk, int i) { return ld(Rb + (long)kk * p + i, Rb, i < iw); },
+        [&](int kk, int j) { return ld(Zb + (long)kk * p + j, Zb, j < jw); });
+    const double sg = I < k ? 1.0 : -1.0;
+    nd_each_acc(A, [&](int i, int j, C z) {
+        if (i < iw && j < jw) {
+            C* y = Y + (long)i * p + j;
+            gstore(y, cadd(gload(y), cscale(z, sg)));
+        }
+    });
+}
+
+// X (whole) from the lower tiles of Y
+__global__ __launch_bounds__(256) void k_nd_mirror(NdLev lv, const NdFac* fac, NdInv w, int nb) {
+    __shared__ C tile[32][33];
+    const int q = blockIdx.y, p = lv.p, np = (p + 31) / 32;
+    const int fr = blockIdx.x / (np * np), e = blockIdx.x % (np * np), I = e / np, J = e % np;
+    if (J > I) return;
     const long job = (long)q * lv.cnt + fr;
     const C* Y = (const C*)w.Y + job * p * p;
-    const int *pr = w.prow + job * p, *ip = w.iprow + job * p;
     C* X = (C*)fac[q].arena + lv.offX + (long)fr * p * p;
-    for (int r = 0; r < ASM_ROWS; ++r) {
-        const int a = ch * ASM_ROWS + r;
-        if (a >= p) break;
-        const C* y = Y + (long)pr[a] * p;
-        for (int c = threadIdx.x; c < p; c += 256) gstore(X + (long)a * p + c, gload(y + ip[c]));
+    const int c = threadIdx.x & 31, r0 = threadIdx.x >> 5;
+    for (int r = r0; r < 32; r += 8) {
+        const int i = I * 32 + r, j = J * 32 + c;
+        if (i < p && j < p) {
+            const C v = gload(Y + (long)i * p + j);
+            tile[r][c] = v;
+            gstore(X + (long)i * p + j, v);
+        }
+    }
+    if (I == J) return;
+    __syncthreads();
+    for (int r = r0; r < 32; r += 8) {
+        const int i = J * 32 + r, j = I * 32 + c;
+        if (i < p && j < p) gstore(X + (long)i * p + j, tile[c][r]);
     }
 }
 
-void launch_nd_unperm(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, const NdGj& w) {
-    const int nch = (lv.p + ASM_ROWS - 1) / ASM_ROWS;
-    k_nd_unperm<<<dim3(lv.cnt * nch, B), 256, 0, s>>>(lv, fac, w, nch);
+void launch_nd_invert(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, const NdInv& w) {
+    if (lv.p <= NB) return;
+    const int nb = (lv.p + NB - 1) / NB, nt = (nb - 1) * nb / 2, np = (lv.p + 31) / 32;
+    for (int k = 0; k < nb; ++k) {
+        k_nd_bz<<<dim3(lv.cnt * (nb - 1), B), 256, 0, s>>>(lv, fac, w, k, nb);
+        k_nd_bu<<<dim3(lv.cnt * nt, B), 256, 0, s>>>(lv, w, k, nb, nt);
+    }
+    k_nd_mirror<<<dim3(lv.cnt * np * np, B), 256, 0, s>>>(lv, fac, w, nb);
 }
 
 // ---------------------------------------------------------------------------

@@ -3,15 +3,14 @@
 // The torus of cells is dissected by nd_plan.h; every tree level is one batch
 // of equal-sized fronts (k_nd.hip).  Leaves are eliminated in registers; a
 // level above assembles [F11 | F12] from the operator and its children's
-// Schur complements, inverts F11 by the batched Gauss-Jordan kernels of the
-// line reduction (window pivoting inside the separator, verified), and forms
-// Q = X F12 and the Schur complement F22 - F12^T Q on MFMA.
+// Schur complements, inverts F11 by symmetric block sweeps, and forms Q = X F12 and the Schur complement
+// F22 - F12^T Q on MFMA.
 //
 // Against the block cyclic reduction of the lines (bcr.cpp) this takes of
 // the order of N^1.5 operations and N log N storage instead of n^3 m and
-// n^2 m, at the price of pivoting only inside a separator.  A factor whose
-// pivots fail their check (zero, not finite, or beaten by a row outside the
-// window) is rebuilt by the line reduction.
+// n^2 m, at the price of a fixed pivot order (4 x 4 blocks).  A factor with a
+// pivot that is zero or not finite is rebuilt by the line reduction, and so is
+// one on which the refinement does not converge.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -26,7 +25,6 @@
 namespace fdfd {
 
 int rt_assemble(Handle* h, Factor* F);
-void rt_launch_gj(Handle* h, const LineJob* J, int nj, int n, bool fp64, bool h3, bool full, bool prof);
 
 // Tree and index maps of one grid shape on the device, shared by the factors
 // built with it; lev[0] is the root.
@@ -70,9 +68,9 @@ void size_plan(NdPlan& P, const std::vector<nd::Level>& L) {
         P.ulen += cnt * b;
         P.fronts += (int)cnt;
         P.maxS[i & 1] = std::max(P.maxS[i & 1], cnt * b * b);
-        if (L[i].nch > 0) {
+        if (L[i].nch > 0) P.maxF12 = std::max(P.maxF12, cnt * p * b);
+        if (L[i].nch > 0 && p > 64) {  // separators inverted in blocks
             P.maxY = std::max(P.maxY, cnt * p * p);
-            P.maxF12 = std::max(P.maxF12, cnt * p * b);
             P.maxp = std::max(P.maxp, cnt * p);
             P.maxcnt = std::max(P.maxcnt, cnt);
         }
@@ -89,27 +87,19 @@ void size_plan(NdPlan& P, const std::vector<nd::Level>& L) {
 // level and the Schur complements of two neighbouring levels
 struct Scratch {
     size_t bytes = 0;
-    size_t oY, oF12, oV, oLU, oZ, oused, oprow, oiprow, opiv, owin, overr, ojobs, oS[2], ofac, ostat;
+    size_t oY, oF12, oR, oZ, oD, oS[2], ofac, ostat;
     Scratch(const NdPlan& P, int B) {
-        const size_t elem = ELEM;
         auto take = [&](size_t n) {
             const size_t o = bytes;
             bytes += (n + 255) & ~(size_t)255;
             return o;
         };
-        oY = take(elem * P.maxY * B);
-        oF12 = take(elem * P.maxF12 * B);
-        oV = take(elem * P.maxp * VMAX * B);
-        oLU = take(elem * P.maxcnt * 2 * PMAX * PMAX * B);
-        oZ = take(elem * P.maxp * VMAX * B);
-        oused = take(sizeof(int) * P.maxp * B);
-        oprow = take(sizeof(int) * P.maxp * B);
-        oiprow = take(sizeof(int) * P.maxp * B);
-        opiv = take(sizeof(int) * P.maxcnt * VMAX * B);
-        owin = take(sizeof(int) * P.maxcnt * WIN * B);
-        overr = take(sizeof(int) * B);
-        ojobs = take(sizeof(LineJob) * P.maxcnt * B);
-        for (int k = 0; k < 2; ++k) oS[k] = take(elem * P.maxS[k] * B);
+        oY = take(ELEM * P.maxY * B);
+        oF12 = take(ELEM * P.maxF12 * B);
+        oR = take(ELEM * P.maxp * 64 * B);
+        oZ = take(ELEM * P.maxp * 64 * B);
+        oD = take(ELEM * P.maxcnt * 2 * 64 * 64 * B);
+        for (int k = 0; k < 2; ++k) oS[k] = take(ELEM * P.maxS[k] * B);
         ofac = take(sizeof(NdFac) * B);
         ostat = take(sizeof(double) * 3 * B);
     }
@@ -248,11 +238,7 @@ int rt_build_nd(Handle* h, const std::vector<Factor*>& Fs, std::vector<int>& bad
     }
     NdFac* dfac = (NdFac*)(w + sc.ofac);
     COPY(h, dfac, fac.data(), sizeof(NdFac) * B, hipMemcpyHostToDevice);
-    int* verr = (int*)(w + sc.overr);
-    HIPCHK(h, hipMemsetAsync(verr, 0, sizeof(int) * B, st));
-    const NdGj gj{w + sc.oY, w + sc.oF12, w + sc.oV, w + sc.oLU, w + sc.oZ,
-                  (int*)(w + sc.oused), (int*)(w + sc.oprow), (int*)(w + sc.oiprow),
-                  (int*)(w + sc.opiv), (int*)(w + sc.owin), verr, (LineJob*)(w + sc.ojobs)};
+    const NdInv iw{w + sc.oY, w + sc.oF12, w + sc.oR, w + sc.oZ, w + sc.oD};
     hipEvent_t e0, e1;
     HIPCHK(h, hipEventCreate(&e0));
     HIPCHK(h, hipEventCreate(&e1));
@@ -269,18 +255,17 @@ int rt_build_nd(Handle* h, const std::vector<Factor*>& Fs, std::vector<int>& bad
             delete ps;
             continue;
         }
-        launch_nd_asm(st, v, dfac, B, g.Nx, g.Ny, Sc, gj);
+        launch_nd_front(st, v, dfac, B, g.Nx, g.Ny, Sc, iw);
         delete ps;
-        rt_launch_gj(h, gj.jobs, v.cnt * B, v.p, true, false, false, prof);
-        ps = scope(P_SCHUR, 0, 2 * p * p * nj * ELEM);
-        launch_nd_unperm(st, v, dfac, B, gj);
+        ps = scope(P_PANEL, 4 * p * p * p * nj, 0);
+        launch_nd_invert(st, v, dfac, B, iw);
         delete ps;
         if (v.b == 0) continue;
         ps = scope(P_GEMM, 8 * p * p * b * nj, 0);
-        launch_nd_gemm(st, v, dfac, B, gj.F12, nullptr, nullptr, false);
+        launch_nd_gemm(st, v, dfac, B, iw.F12, nullptr, nullptr, false);
         delete ps;
         ps = scope(P_GEMM, 4 * p * b * b * nj, 0);
-        launch_nd_gemm(st, v, dfac, B, gj.F12, Sc, S, true);
+        launch_nd_gemm(st, v, dfac, B, iw.F12, Sc, S, true);
         delete ps;
     }
     double* dstat = (double*)(w + sc.ostat);
@@ -288,10 +273,8 @@ int rt_build_nd(Handle* h, const std::vector<Factor*>& Fs, std::vector<int>& bad
     hipError_t le = hipGetLastError();
     (void)hipEventRecord(e1, st);
     std::vector<double> stat(3 * (size_t)B);
-    std::vector<int> vh(B);
     rc = le == hipSuccess ? FDFD_OK : fail(h, FDFD_ERR_HIP, std::string("dissection kernels: ") + hipGetErrorString(le));
     if (!rc) rc = stream_copy(h, stat.data(), dstat, sizeof(double) * stat.size(), hipMemcpyDeviceToHost);
-    if (!rc) rc = stream_copy(h, vh.data(), verr, sizeof(int) * B, hipMemcpyDeviceToHost);
     float ms = 0;
     if (!rc) (void)hipEventElapsedTime(&ms, e0, e1);
     (void)hipEventDestroy(e0);
@@ -305,8 +288,9 @@ int rt_build_nd(Handle* h, const std::vector<Factor*>& Fs, std::vector<int>& bad
         F->t_factor_ms = ms;
         F->singular_line = -1;
         F->pivot_fallback = 0;
-        F->pivot_growth = mn > 0 ? mx / mn : std::numeric_limits<double>::infinity();
-        if (vh[f] || stat[3 * f + 2] != 0 || !(mn > 0) || !std::isfinite(mx)) bad.push_back(f);
+        // (the statistics are of 2 x 2 determinants)
+        F->pivot_growth = mn > 0 ? std::sqrt(mx / mn) : std::numeric_limits<double>::infinity();
+        if (stat[3 * f + 2] != 0 || !(mn > 0) || !std::isfinite(mx)) bad.push_back(f);
     }
     return FDFD_OK;
 }

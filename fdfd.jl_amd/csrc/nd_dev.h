@@ -29,11 +29,11 @@ struct NdFac {
     double* pivstat;      // 3 per front
 };
 
-// Gauss-Jordan scratch of a level, one slot per (factor, front)
-struct NdGj {
-    void *Y, *F12, *Vbuf, *LU, *Z;
-    int *used, *prow, *iprow, *piv, *win, *verr;
-    LineJob* jobs;
+// inversion scratch of a level, one slot per (factor, front): the separator
+// block, F12, the block row and its product of a block sweep (64 x p each) and
+// two 64 x 64 block inverses
+struct NdInv {
+    void *Y, *F12, *R, *Z, *D;
 };
 
 // vectors of a reduced solve: source ridx[s] (0 without a list) at in / out
@@ -52,9 +52,9 @@ void launch_nd_maps(hipStream_t s, const NdMapArgs& a, int* node, short* cm);
 void launch_nd_symmetrise(hipStream_t s, double2* coef, double2* us, const double2* wx,
                           const double2* wy, int Nx, int Ny);
 void launch_nd_leaf(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, int Nx, int Ny, void* S);
-void launch_nd_asm(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, int Nx, int Ny,
-                   const void* Sc, const NdGj& w);
-void launch_nd_unperm(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, const NdGj& w);
+void launch_nd_front(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, int Nx, int Ny, const void* Sc,
+                     const NdInv& w);
+void launch_nd_invert(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, const NdInv& w);
 void launch_nd_gemm(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, const void* F12,
                     const void* Sc, void* S, bool schur);
 void launch_nd_stat(hipStream_t s, const NdFac* fac, int B, int nfronts, double* out);
