@@ -105,6 +105,9 @@ void launch_nd_symmetrise(hipStream_t s, double2* coef, double2* us, const doubl
 // entry (k, l) of the symmetrised operator (coupling planes of k_nd_coef)
 __device__ inline double2 nd_entry(const double2* coef, long N, int Nx, int Ny, int k, int l) {
     double2 v = make_double2(0, 0);
+    // most pairs of a front are no neighbours on the torus
+    const int dk = k > l ? k - l : l - k;
+    if (dk > 1 && dk != Nx && dk != Nx - 1 && dk != (int)N - Nx) return v;
     const int xk = k % Nx, yk = k / Nx, xl = l % Nx, yl = l / Nx;
     const int xke = xk + 1 == Nx ? 0 : xk + 1, xle = xl + 1 == Nx ? 0 : xl + 1;
     const int ykn = yk + 1 == Ny ? 0 : yk + 1, yln = yl + 1 == Ny ? 0 : yl + 1;
@@ -502,7 +505,7 @@ __global__ __launch_bounds__(256, 2) void k_nd_front(NdLev lv, const NdFac* fac,
         });
         nd_sweep<T>(mr, mi, np, s, F.pivstat + 3 * (long)(lv.stat + fr), false);
         const bool whole = p <= NB;
-        C* out = whole ? (C*)F.arena + lv.offX + (long)fr * p * p : (C*)w.D + job * 2 * NB * NB;
+        C* out = whole ? (C*)F.arena + lv.offX + (long)fr * p * p : (C*)w.D + job * NB * NB;
         const int ld = whole ? p : NB;
         nd_each_entry<T>([&](auto sc, int v, int i, int j, bool off) {
             const C z = mk<C>(mr[sc][v], mi[sc][v]);
@@ -513,17 +516,31 @@ __global__ __launch_bounds__(256, 2) void k_nd_front(NdLev lv, const NdFac* fac,
         });
         return;
     }
-    const int ch = e % nchunk, j0 = p > NB ? 0 : p;
+    const int r0 = (e % nchunk) * ASM_ROWS, j0 = p > NB ? 0 : p, nr = min(ASM_ROWS, p - r0);
     C* Y = (C*)w.Y + job * p * p;
     C* G = (C*)w.F12 + job * p * b;
-    for (int r = 0; r < ASM_ROWS; ++r) {
-        const int i = ch * ASM_ROWS + r;
-        if (i >= p) break;
-        for (int j = j0 + (int)threadIdx.x; j < f; j += 256) {
-            if (j < p) {
-                if (j <= (i | (NB - 1))) gstore(Y + (long)i * p + j, entry(i, j));
-            } else {
-                gstore(G + (long)i * b + (j - p), entry(i, j));
+    for (int j = j0 + (int)threadIdx.x; j < f; j += 256) {
+        const int kj = node[j], c0 = cm[j], c1 = lv.nch > 1 ? cm[f + j] : -1;
+        // every row's contributions are loaded before the first is used
+        C v0[ASM_ROWS], v1[ASM_ROWS];
+#pragma unroll
+        for (int r = 0; r < ASM_ROWS; ++r) {
+            const int i = r0 + min(r, nr - 1), m0 = cm[i], m1 = lv.nch > 1 ? cm[f + i] : -1;
+            const bool k0 = m0 >= 0 && c0 >= 0, k1 = m1 >= 0 && c1 >= 0;
+            v0[r] = gload(Sc + (k0 ? (long)m0 * lv.cb + c0 : 0));
+            v1[r] = gload(Sc + (k1 ? ((long)lv.cb + m1) * lv.cb + c1 : 0));
+        }
+#pragma unroll
+        for (int r = 0; r < ASM_ROWS; ++r) {
+            const int i = r0 + min(r, nr - 1), ki = node[i], m0 = cm[i], m1 = lv.nch > 1 ? cm[f + i] : -1;
+            C v = mk<C>(0, 0);
+            if (ki >= 0 && kj >= 0) v = nd_entry(F.coef, N, Nx, Ny, ki, kj);
+            else if (i == j) v = mk<C>(1, 0);
+            v = cadd(v, csel(m0 >= 0 && c0 >= 0, v0[r], mk<C>(0, 0)));
+            v = cadd(v, csel(m1 >= 0 && c1 >= 0, v1[r], mk<C>(0, 0)));
+            if (r < nr) {
+                if (j >= p) gstore(G + (long)i * b + (j - p), v);
+                else if (j <= (i | (NB - 1))) gstore(Y + (long)i * p + j, v);
             }
         }
     }
@@ -543,228 +560,230 @@ void launch_nd_front(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, in
 // Separators longer than 64 cells: block sweeps of 64 on the lower tiles of Y.
 // For block k with inverse D^-1 and block row R_J = M_kJ (stored as tile
 // (k, J), or transposed as tile (J, k) for J > k):
-//   k_nd_bz : Z_J = D^-1 R_J; tile (k, J) <- Z_J, tile (J, k) <- -Z_J^T, and
-//             the workgroup of block k + 1 goes on to M_JJ - R_J^T Z_J and
-//             sweeps it, so the next D^-1 is ready when the level's other
-//             tiles are;
+//   k_nd_bz : Z_J = D^-1 R_J; tile (k, J) <- Z_J, tile (J, k) <- -Z_J^T;
 //   k_nd_bu : M_IJ -= sigma_I R_I^T Z_J on the other lower tiles, sigma = -1 for
-//             swept blocks I < k.
+//             swept blocks I < k; the first workgroup goes on to sweep tile
+//             (k + 1, k + 1), so the next D^-1 is ready when the other tiles
+//             are.
+// The chain of a block is the product for Z (by halves of a tile, 64 x 32), the
+// product on tile (k + 1, k + 1), on its lower 16 x 16 tiles in the layout of the
+// sweep, and the sweep (23 us).  It bounds a level of few fronts: 47 us a block
+// of the 1024-cell separators of a 1024 x 1024 grid, against 76 us with both
+// products and the sweep in k_nd_bz and the second product on the whole tile.
 // ---------------------------------------------------------------------------
-// 64 x 64 x 64 complex product by four waves of 32 x 32, operands staged 16 K
-// rows at a time; la(k, i) and lb(k, j) give the entries (KB: neighbouring
-// threads read neighbouring k of B).  Three real products per complex one.
+// The operands of a product over 64 K rows, 64 rows by TN columns, staged 16 K
+// rows at a time through LDS; mm(kk) multiplies K rows kk .. kk + 3 of a stage.
+// pa(k, i) and pb(k, j) give an entry's address, clamped where oka / okb, which
+// zero it at the store to LDS, are false; keep(k, j, v) sees every entry of B
+// (KB: neighbouring threads read neighbouring k of B).
 struct NdTile {
-    using M = mfma_t<double>;
     double sAr[16][NB + 16], sAi[16][NB + 16], sBr[16][NB + 16], sBi[16][NB + 16];
 };
-struct NdAcc {
-    mfma_t<double>::acc c1[2][2], c2[2][2], c3[2][2];
-};
-template <bool KB, typename LA, typename LB>
-__device__ __attribute__((always_inline)) inline void nd_tile_product(NdTile& s, NdAcc& A, LA&& la, LB&& lb) {
-    using M = mfma_t<double>;
-    const int t = threadIdx.x, lane = t & 63, wv = t >> 6, wr = wv >> 1, wc = wv & 1;
-    const int lr = lane & 15, lk = lane >> 4;
-    C ra[4], rb[4];
+template <bool KB, int TN, typename PA, typename PB, typename OA, typename OB, typename KP, typename MM>
+__device__ __attribute__((always_inline)) inline void nd_staged(NdTile& s, PA&& pa, PB&& pb, OA&& oka, OB&& okb,
+                                                                KP&& keep, MM&& mm) {
+    constexpr int NE = TN / 16;
+    const int t = threadIdx.x;
+    C ra[4], rb[NE];
+    auto kB = [&](int e) { return KB ? t & 15 : (t + 256 * e) / TN; };
+    auto jB = [&](int e) { return KB ? (t + 256 * e) >> 4 : (t + 256 * e) % TN; };
     auto load = [&](int k0) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int id = t + 256 * e;
-            ra[e] = la(k0 + (id >> 6), id & 63);
-            rb[e] = KB ? lb(k0 + (id & 15), id >> 4) : lb(k0 + (id >> 6), id & 63);
-        }
+        for (int e = 0; e < 4; ++e) ra[e] = gload(pa(k0 + ((t + 256 * e) >> 6), t & 63));
+#pragma unroll
+        for (int e = 0; e < NE; ++e) rb[e] = gload(pb(k0 + kB(e), jB(e)));
     };
-#pragma unroll
-    for (int x = 0; x < 2; ++x)
-#pragma unroll
-        for (int y = 0; y < 2; ++y) {
-            A.c1[x][y] = M::acc{0, 0, 0, 0};
-            A.c2[x][y] = M::acc{0, 0, 0, 0};
-            A.c3[x][y] = M::acc{0, 0, 0, 0};
-        }
     load(0);
     for (int k0 = 0; k0 < NB; k0 += 16) {
         __syncthreads();  // the previous stage (or the caller's use of s) is consumed
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const int id = t + 256 * e;
-            s.sAr[id >> 6][id & 63] = ra[e].x;
-            s.sAi[id >> 6][id & 63] = ra[e].y;
-            const int k = KB ? id & 15 : id >> 6, j = KB ? id >> 4 : id & 63;
-            s.sBr[k][j] = rb[e].x;
-            s.sBi[k][j] = rb[e].y;
+            const int k = (t + 256 * e) >> 6, i = t & 63;
+            const bool oa = oka(k0 + k, i);
+            s.sAr[k][i] = oa ? ra[e].x : 0.0;
+            s.sAi[k][i] = oa ? ra[e].y : 0.0;
+        }
+#pragma unroll
+        for (int e = 0; e < NE; ++e) {
+            const int k = kB(e), j = jB(e);
+            const C v = csel(okb(k0 + k, j), rb[e], mk<C>(0, 0));
+            s.sBr[k][j] = v.x;
+            s.sBi[k][j] = v.y;
+            keep(k0 + k, j, v);
         }
         __syncthreads();
         if (k0 + 16 < NB) load(k0 + 16);
 #pragma unroll
-        for (int kk = 0; kk < 16; kk += 4) {
-            double ar[2], ai[2], as[2], br[2], bi[2], bs[2];
-#pragma unroll
-            for (int x = 0; x < 2; ++x) {
-                ar[x] = s.sAr[kk + lk][wr * 32 + x * 16 + lr];
-                ai[x] = s.sAi[kk + lk][wr * 32 + x * 16 + lr];
-                as[x] = ar[x] + ai[x];
-                br[x] = s.sBr[kk + lk][wc * 32 + x * 16 + lr];
-                bi[x] = s.sBi[kk + lk][wc * 32 + x * 16 + lr];
-                bs[x] = br[x] + bi[x];
-            }
-#pragma unroll
-            for (int x = 0; x < 2; ++x)
-#pragma unroll
-                for (int y = 0; y < 2; ++y) A.c1[x][y] = M::run(ar[x], br[y], A.c1[x][y]);
-#pragma unroll
-            for (int x = 0; x < 2; ++x)
-#pragma unroll
-                for (int y = 0; y < 2; ++y) A.c2[x][y] = M::run(ai[x], bi[y], A.c2[x][y]);
-#pragma unroll
-            for (int x = 0; x < 2; ++x)
-#pragma unroll
-                for (int y = 0; y < 2; ++y) A.c3[x][y] = M::run(as[x], bs[y], A.c3[x][y]);
-        }
+        for (int kk = 0; kk < 16; kk += 4) mm(kk);
     }
 }
-// f(i, j, value) for this thread's entries of the product
-template <typename F> __device__ inline void nd_each_acc(const NdAcc& A, F&& f) {
-    using M = mfma_t<double>;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, wr = wv >> 1, wc = wv & 1;
+// Accumulators of a 64 x TN tile on four waves of 32 x TN / 2, three real products
+// per complex one
+template <int TN> struct NdAcc {
+    static constexpr int BN = TN / 32;
+    d4v c1[2][BN] = {}, c2[2][BN] = {}, c3[2][BN] = {};
+    __device__ __attribute__((always_inline)) inline void mul(const NdTile& s, int kk) {
+        const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, wr = wv >> 1, wc = wv & 1;
+        const int lr = lane & 15, lk = lane >> 4;
+        double ar[2], ai[2], as[2], br[BN], bi[BN], bs[BN];
 #pragma unroll
-    for (int x = 0; x < 2; ++x)
+        for (int x = 0; x < 2; ++x) {
+            ar[x] = s.sAr[kk + lk][wr * 32 + x * 16 + lr];
+            ai[x] = s.sAi[kk + lk][wr * 32 + x * 16 + lr];
+            as[x] = ar[x] + ai[x];
+        }
 #pragma unroll
-        for (int y = 0; y < 2; ++y)
+        for (int y = 0; y < BN; ++y) {
+            br[y] = s.sBr[kk + lk][wc * (TN / 2) + y * 16 + lr];
+            bi[y] = s.sBi[kk + lk][wc * (TN / 2) + y * 16 + lr];
+            bs[y] = br[y] + bi[y];
+        }
 #pragma unroll
-            for (int v = 0; v < 4; ++v)
-                f(wr * 32 + x * 16 + M::row(lane, v), wc * 32 + y * 16 + (lane & 15),
-                  mk<C>(A.c1[x][y][v] - A.c2[x][y][v], A.c3[x][y][v] - A.c1[x][y][v] - A.c2[x][y][v]));
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < BN; ++y) c1[x][y] = F64::run(ar[x], br[y], c1[x][y]);
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < BN; ++y) c2[x][y] = F64::run(ai[x], bi[y], c2[x][y]);
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < BN; ++y) c3[x][y] = F64::run(as[x], bs[y], c3[x][y]);
+    }
+    // f(i, j, value) for this thread's entries of the product
+    template <typename F> __device__ __attribute__((always_inline)) inline void each(F&& f) const {
+        const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, wr = wv >> 1, wc = wv & 1;
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < BN; ++y)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    f(wr * 32 + x * 16 + F64::row(lane, v), wc * (TN / 2) + y * 16 + (lane & 15),
+                      mk<C>(c1[x][y][v] - c2[x][y][v], c3[x][y][v] - c1[x][y][v] - c2[x][y][v]));
+    }
+};
+
+constexpr int ZC = 32;  // columns of Z per workgroup
+
+__global__ __launch_bounds__(256, 2) void k_nd_bz(NdLev lv, NdInv w, int k, int nb) {
+    __shared__ NdTile s;
+    const int per = (nb - 1) * (NB / ZC), fr = blockIdx.x / per, q = blockIdx.y, p = lv.p;
+    const int e = (int)blockIdx.x % per, Jb = e / (NB / ZC), J = Jb + (Jb >= k);
+    const long job = (long)q * lv.cnt + fr;
+    const int jc = J * NB + (e % (NB / ZC)) * ZC;  // first column
+    const int kw = min(NB, p - k * NB), jw = min(ZC, p - jc);
+    C* Y = (C*)w.Y + job * p * p;
+    C* Rb = (C*)w.R + job * NB * p + jc;
+    C* Zb = (C*)w.Z + job * NB * p + jc;
+    const C* D = (const C*)w.D + job * NB * NB;
+    const C zero = mk<C>(0, 0);
+    if (e == 0) {  // tile (k, k) <- D^-1
+        for (int i = threadIdx.x; i < NB * NB; i += 256) {
+            const int r = i >> 6, j = i & 63;
+            if (r < kw && j < kw) gstore(Y + (long)(k * NB + r) * p + k * NB + j, gload(D + i));
+        }
+    }
+    if (jw <= 0) return;
+    auto pd = [&](int kk, int i) { return D + kk * NB + i; };
+    auto okd = [&](int kk, int i) { return kk < kw && i < kw; };
+    auto okr = [&](int kk, int j) { return kk < kw && j < jw; };
+    auto keep = [&](int kk, int j, C v) {
+        if (j < jw) gstore(Rb + (long)kk * p + j, v);
+    };
+    NdAcc<ZC> A;
+    auto mm = [&](int kk) { A.mul(s, kk); };
+    const bool lower = J < k;
+    C* T = lower ? Y + (long)k * NB * p + jc : Y + (long)jc * p + k * NB;
+    if (lower)
+        nd_staged<false, ZC>(s, pd, [&](int kk, int j) { return T + (long)min(kk, kw - 1) * p + min(j, jw - 1); }, okd,
+                             okr, keep, mm);
+    else
+        nd_staged<true, ZC>(s, pd, [&](int kk, int j) { return T + (long)min(j, jw - 1) * p + min(kk, kw - 1); }, okd,
+                            okr, keep, mm);
+    // (the tile was read, by this workgroup alone, before the last barrier)
+    A.each([&](int i, int j, C z) {
+        if (j >= jw) return;
+        gstore(Zb + (long)i * p + j, i < kw ? z : zero);
+        if (i < kw) {
+            if (lower) gstore(T + (long)i * p + j, z);
+            else gstore(T + (long)j * p + i, cneg(z));
+        }
+    });
 }
 
-__global__ __launch_bounds__(256, 2) void k_nd_bz(NdLev lv, const NdFac* fac, NdInv w, int k, int nb) {
+__global__ __launch_bounds__(256, 2) void k_nd_bu(NdLev lv, const NdFac* fac, NdInv w, int k, int nb, int ntile) {
     __shared__ union {
         NdTile s;
         NdSweep<4> w;
     } u;
     NdTile& s = u.s;
-    const int per = max(nb - 1, 1), fr = blockIdx.x / per, q = blockIdx.y, p = lv.p;
-    const long job = (long)q * lv.cnt + fr;
-    const int J = (k + 1 + (int)blockIdx.x % per) % nb;  // block k + 1 first
-    const int kw = min(NB, p - k * NB), jw = min(NB, p - J * NB);
-    C* Y = (C*)w.Y + job * p * p;
-    C* Rb = (C*)w.R + job * NB * p + J * NB;
-    C* Zb = (C*)w.Z + job * NB * p + J * NB;
-    const C* D = (const C*)w.D + (job * 2 + (k & 1)) * NB * NB;
-    const C zero = mk<C>(0, 0);
-    auto ld = [&](const C* ptr, bool ok) {
-        const C v = gload(ok ? ptr : D);
-        return csel(ok, v, zero);
-    };
-    auto dv = [&](int kk, int i) { return ld(D + kk * NB + i, kk < kw && i < kw); };
-    if (blockIdx.x % per == 0) {  // tile (k, k) <- D^-1
-        for (int e = threadIdx.x; e < NB * NB; e += 256) {
-            const int i = e >> 6, j = e & 63;
-            if (i < kw && j < kw) gstore(Y + (long)(k * NB + i) * p + k * NB + j, gload(D + e));
-        }
-    }
-    NdAcc A;
-    if (J < k) {
-        const C* T = Y + (long)k * NB * p + J * NB;
-        auto rv = [&](int kk, int j) { return ld(T + (long)kk * p + j, kk < kw && j < jw); };
-        nd_tile_product<false>(s, A, dv, rv);
-        for (int e = threadIdx.x; e < NB * NB; e += 256) {
-            const int kk = e >> 6, j = e & 63;
-            if (j < jw) gstore(Rb + (long)kk * p + j, rv(kk, j));
-        }
-        __syncthreads();  // the tile is read before it is overwritten
-        nd_each_acc(A, [&](int i, int j, C z) {
-            if (j < jw) {
-                gstore(Zb + (long)i * p + j, i < kw ? z : zero);
-                if (i < kw) gstore(Y + (long)(k * NB + i) * p + J * NB + j, z);
-            }
-        });
-    } else {
-        const C* T = Y + (long)J * NB * p + k * NB;
-        auto rv = [&](int kk, int j) { return ld(T + (long)j * p + kk, kk < kw && j < jw); };
-        nd_tile_product<true>(s, A, dv, rv);
-        for (int e = threadIdx.x; e < NB * NB; e += 256) {
-            const int kk = e & 63, j = e >> 6;
-            if (j < jw) gstore(Rb + (long)kk * p + j, rv(kk, j));
-        }
-        __syncthreads();
-        nd_each_acc(A, [&](int i, int j, C z) {
-            if (j < jw) {
-                gstore(Zb + (long)i * p + j, i < kw ? z : zero);
-                if (i < kw) gstore(Y + (long)(J * NB + j) * p + k * NB + i, cneg(z));
-            }
-        });
-    }
-    if (J != k + 1) return;
-    // M_JJ - R_J^T Z_J, swept: the next block's inverse (R and Z come back
-    // through global memory, written by this workgroup)
-    __threadfence_block();
-    __syncthreads();
-    auto rr = [&](int kk, int i) { return ld(Rb + (long)kk * p + i, i < jw); };
-    auto zz = [&](int kk, int j) { return ld(Zb + (long)kk * p + j, j < jw); };
-    nd_tile_product<false>(s, A, rr, zz);
-    __syncthreads();
-    C* P = (C*)&u.s;  // the product as a 64 x 64 tile, in two halves
-    static_assert(sizeof(NdTile) >= sizeof(C) * NB * NB / 2, "half a product tile fits the stages");
-    constexpr int NS = NdSweep<4>::NS;
-    d4v mr[NS], mi[NS];
-    for (int hf = 0; hf < 2; ++hf) {
-        nd_each_acc(A, [&](int i, int j, C z) {
-            if ((i >> 5) == hf) P[(i & 31) * NB + j] = z;
-        });
-        __syncthreads();
-        nd_each_entry<4>([&](auto sc, int v, int i, int j, bool) {
-            if ((i >> 5) == hf) {
-                const bool ok = i < jw && j < jw;
-                const C old = ld(Y + (long)(J * NB + i) * p + J * NB + j, ok);
-                const C z = csel(ok, csub(old, P[(i & 31) * NB + j]), mk<C>(i == j ? 1 : 0, 0));
-                mr[sc][v] = z.x;
-                mi[sc][v] = z.y;
-            }
-        });
-        __syncthreads();
-    }
-    nd_sweep<4>(mr, mi, jw, u.w, fac[q].pivstat + 3 * (long)(lv.stat + fr), true);
-    C* Dn = (C*)w.D + (job * 2 + ((k + 1) & 1)) * NB * NB;
-    nd_each_entry<4>([&](auto sc, int v, int i, int j, bool off) {
-        const C z = mk<C>(mr[sc][v], mi[sc][v]);
-        gstore(Dn + i * NB + j, z);
-        if (off) gstore(Dn + j * NB + i, z);
-    });
-}
-
-__global__ __launch_bounds__(256, 2) void k_nd_bu(NdLev lv, NdInv w, int k, int nb, int ntile) {
-    __shared__ NdTile s;
     const int fr = blockIdx.x / ntile, q = blockIdx.y, p = lv.p;
     const long job = (long)q * lv.cnt + fr;
-    // tile number -> (I, J), I >= J, over the blocks other than k
-    const int e = blockIdx.x % ntile;
+    // tile number -> (I, J), I >= J, over the blocks other than k; number 0 and
+    // that of (k + 1, k + 1) change places
+    int e = blockIdx.x % ntile;
+    const int en = k + 1 < nb ? k * (k + 3) / 2 : 0;
+    e = e == 0 ? en : e == en ? 0 : e;
     int I = (int)((sqrtf(8.0f * e + 1.0f) - 1.0f) * 0.5f);
     while ((I + 1) * (I + 2) / 2 <= e) ++I;
     while (I * (I + 1) / 2 > e) --I;
     int J = e - I * (I + 1) / 2;
     I += I >= k;
     J += J >= k;
-    if (I == k + 1 && J == k + 1) return;  // done by k_nd_bz
     const int iw = min(NB, p - I * NB), jw = min(NB, p - J * NB);
     C* Y = (C*)w.Y + job * p * p + (long)I * NB * p + J * NB;
     const C* Rb = (const C*)w.R + job * NB * p + I * NB;
     const C* Zb = (const C*)w.Z + job * NB * p + J * NB;
-    const C zero = mk<C>(0, 0);
-    auto ld = [&](const C* ptr, const C* safe, bool ok) {
-        const C v = gload(ok ? ptr : safe);
-        return csel(ok, v, zero);
-    };
-    NdAcc A;
-    nd_tile_product<false>(
-        s, A, [&](int kk, int i) { return ld(Rb + (long)kk * p + i, Rb, i < iw); },
-        [&](int kk, int j) { return ld(Zb + (long)kk * p + j, Zb, j < jw); });
-    const double sg = I < k ? 1.0 : -1.0;
-    nd_each_acc(A, [&](int i, int j, C z) {
-        if (i < iw && j < jw) {
-            C* y = Y + (long)i * p + j;
-            gstore(y, cadd(gload(y), cscale(z, sg)));
-        }
+    auto pa = [&](int kk, int i) { return Rb + (long)kk * p + min(i, iw - 1); };
+    auto pb = [&](int kk, int j) { return Zb + (long)kk * p + min(j, jw - 1); };
+    auto oka = [&](int, int i) { return i < iw; };
+    auto okb = [&](int, int j) { return j < jw; };
+    auto keep = [](int, int, C) {};
+    if (I != k + 1 || J != k + 1) {
+        NdAcc<NB> A;
+        nd_staged<false, NB>(s, pa, pb, oka, okb, keep, [&](int kk) { A.mul(s, kk); });
+        const double sg = I < k ? 1.0 : -1.0;
+        A.each([&](int i, int j, C z) {
+            if (i < iw && j < jw) {
+                C* y = Y + (long)i * p + j;
+                gstore(y, cadd(gload(y), cscale(z, sg)));
+            }
+        });
+        return;
+    }
+    // the lower 16 x 16 tiles in the layout of the sweep
+    constexpr int NS = NdSweep<4>::NS;
+    const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
+    d4v mr[NS], mi[NS], c1[NS] = {}, c2[NS] = {}, c3[NS] = {};
+    nd_each_entry<4>([&](auto sc, int v, int i, int j, bool) {
+        const C y = gload(Y + (long)min(i, iw - 1) * p + min(j, iw - 1));
+        mr[sc][v] = y.x;
+        mi[sc][v] = y.y;
+    });
+    nd_staged<false, NB>(s, pa, pb, oka, okb, keep, [&](int kk) {
+        nd_each_tile<4>([&](auto sc, int ti, int tj) {
+            const double ar = s.sAr[kk + lk][16 * ti + lr], ai = s.sAi[kk + lk][16 * ti + lr];
+            const double br = s.sBr[kk + lk][16 * tj + lr], bi = s.sBi[kk + lk][16 * tj + lr];
+            c1[sc] = F64::run(ar, br, c1[sc]);
+            c2[sc] = F64::run(ai, bi, c2[sc]);
+            c3[sc] = F64::run(ar + ai, br + bi, c3[sc]);
+        });
+    });
+    nd_each_entry<4>([&](auto sc, int v, int i, int j, bool) {
+        const bool ok = i < iw && j < iw;
+        const double re = c1[sc][v] - c2[sc][v], im = c3[sc][v] - c1[sc][v] - c2[sc][v];
+        mr[sc][v] = ok ? mr[sc][v] - re : (i == j ? 1.0 : 0.0);
+        mi[sc][v] = ok ? mi[sc][v] - im : 0.0;
+    });
+    __syncthreads();
+    nd_sweep<4>(mr, mi, iw, u.w, fac[q].pivstat + 3 * (long)(lv.stat + fr), true);
+    C* Dn = (C*)w.D + job * NB * NB;
+    nd_each_entry<4>([&](auto sc, int v, int i, int j, bool off) {
+        const C z = mk<C>(mr[sc][v], mi[sc][v]);
+        gstore(Dn + i * NB + j, z);
+        if (off) gstore(Dn + j * NB + i, z);
     });
 }
 
@@ -798,8 +817,8 @@ void launch_nd_invert(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, c
     if (lv.p <= NB) return;
     const int nb = (lv.p + NB - 1) / NB, nt = (nb - 1) * nb / 2, np = (lv.p + 31) / 32;
     for (int k = 0; k < nb; ++k) {
-        k_nd_bz<<<dim3(lv.cnt * (nb - 1), B), 256, 0, s>>>(lv, fac, w, k, nb);
-        k_nd_bu<<<dim3(lv.cnt * nt, B), 256, 0, s>>>(lv, w, k, nb, nt);
+        k_nd_bz<<<dim3(lv.cnt * (nb - 1) * (NB / ZC), B), 256, 0, s>>>(lv, w, k, nb);
+        k_nd_bu<<<dim3(lv.cnt * nt, B), 256, 0, s>>>(lv, fac, w, k, nb, nt);
     }
     k_nd_mirror<<<dim3(lv.cnt * np * np, B), 256, 0, s>>>(lv, fac, w, nb);
 }
@@ -812,9 +831,16 @@ void launch_nd_invert(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, c
 // the latter only on tiles that meet the lower triangle; entries below the
 // diagonal are written to both halves.  Operands are staged KT rows of K at a
 // time through LDS, the next stage loading into registers meanwhile.
+//
+// Tiles of 32 x 32, one accumulator set per wave: with few fronts (512 x 2048
+// at four of them) larger tiles leave CUs without work, and with many the
+// epilogue of S (gathers from two children and two writes of each entry)
+// dominates and wants workgroups to overlap with.  All levels of a 1024 x 1024
+// grid, S and Q: 128 x 64 tiles 5.04 + 1.53 ms, 64 x 64 4.33 + 1.26, 64 x 32
+// 4.05 + 1.32, 32 x 32 3.98 + 1.25; of a 200 x 120 grid 152 + 95 us against 89 + 53.
 // ---------------------------------------------------------------------------
 template <int TM, int TN, int KT, int WR, int WC, bool SCHUR>
-__global__ __launch_bounds__(64 * WR * WC) void k_nd_gemm(NdLev lv, const NdFac* fac, const void* F12v,
+__global__ __launch_bounds__(64 * WR * WC, 2) void k_nd_gemm(NdLev lv, const NdFac* fac, const void* F12v,
                                                         const void* Scv, void* Sv, int ntm, int ntn) {
     using M = mfma_t<R>;
     using acc_t = typename M::acc;
@@ -823,7 +849,11 @@ __global__ __launch_bounds__(64 * WR * WC) void k_nd_gemm(NdLev lv, const NdFac*
     constexpr int PA = TM + 16, PB = TN + 16;
     constexpr int AE = TM * KT / NT, BE = TN * KT / NT;
     static_assert(AE >= 1 && BE >= 1 && BM >= 1 && BN >= 1, "tile shape");
-    __shared__ R sAr[KT][PA], sAi[KT][PA], sBr[KT][PB], sBi[KT][PB];
+    __shared__ struct {
+        double ar[KT][PA], ai[KT][PA], br[KT][PB], bi[KT][PB];
+    } sh;
+    auto &sAr = sh.ar, &sAi = sh.ai;
+    auto &sBr = sh.br, &sBi = sh.bi;
     const int q = blockIdx.y, tiles = ntm * ntn;
     const int fr = blockIdx.x / tiles, tile = blockIdx.x % tiles;
     const int i0 = (tile / ntn) * TM, j0 = (tile % ntn) * TN;
@@ -838,45 +868,36 @@ __global__ __launch_bounds__(64 * WR * WC) void k_nd_gemm(NdLev lv, const NdFac*
     const int wr = wv / WC, wc = wv % WC, lr = lane & 15, lk = lane >> 4;
     const C* Bg = SCHUR ? Q : F12;
     C ra[AE], rb[BE];
-    const C zero = mk<C>(R(0), R(0));
+    // clamped addresses; entries outside are zeroed when they are stored to LDS
+    // (a select here would wait for the load)
+    const C* Ag = SCHUR ? F12 : X;
+    const int lda = SCHUR ? b : p;  // X is symmetric: read along its rows
     auto load = [&](int kb) {
 #pragma unroll
         for (int e = 0; e < AE; ++e) {
-            const int id = t + NT * e;
-            if (SCHUR) {
-                const int k = kb + id / TM, i = i0 + id % TM;
-                const bool ok = k < p && i < b;
-                ra[e] = gload(F12 + (ok ? (long)k * b + i : 0));
-                if (!ok) ra[e] = zero;
-            } else {
-                const int i = i0 + id / KT, k = kb + id % KT;
-                const bool ok = k < p && i < p;
-                ra[e] = gload(X + (ok ? (long)i * p + k : 0));
-                if (!ok) ra[e] = zero;
-            }
+            const int id = t + NT * e, k = kb + id / TM, i = i0 + id % TM;
+            ra[e] = gload(Ag + (long)min(k, p - 1) * lda + min(i, Mr - 1));
         }
 #pragma unroll
         for (int e = 0; e < BE; ++e) {
-            const int id = t + NT * e;
-            const int k = kb + id / TN, j = j0 + id % TN;
-            const bool ok = k < p && j < b;
-            rb[e] = gload(Bg + (ok ? (long)k * b + j : 0));
-            if (!ok) rb[e] = zero;
+            const int id = t + NT * e, k = kb + id / TN, j = j0 + id % TN;
+            rb[e] = gload(Bg + (long)min(k, p - 1) * b + min(j, b - 1));
         }
     };
-    auto store = [&]() {
+    auto store = [&](int kb) {
 #pragma unroll
         for (int e = 0; e < AE; ++e) {
-            const int id = t + NT * e;
-            const int k = SCHUR ? id / TM : id % KT, i = SCHUR ? id % TM : id / KT;
-            sAr[k][i] = ra[e].x;
-            sAi[k][i] = ra[e].y;
+            const int id = t + NT * e, k = id / TM, i = id % TM;
+            const bool ok = kb + k < p && i0 + i < Mr;
+            sAr[k][i] = ok ? ra[e].x : 0.0;
+            sAi[k][i] = ok ? ra[e].y : 0.0;
         }
 #pragma unroll
         for (int e = 0; e < BE; ++e) {
-            const int id = t + NT * e;
-            sBr[id / TN][id % TN] = rb[e].x;
-            sBi[id / TN][id % TN] = rb[e].y;
+            const int id = t + NT * e, k = id / TN, j = id % TN;
+            const bool ok = kb + k < p && j0 + j < b;
+            sBr[k][j] = ok ? rb[e].x : 0.0;
+            sBi[k][j] = ok ? rb[e].y : 0.0;
         }
     };
     acc_t c1[BM][BN], c2[BM][BN], c3[BM][BN];
@@ -890,7 +911,7 @@ __global__ __launch_bounds__(64 * WR * WC) void k_nd_gemm(NdLev lv, const NdFac*
         }
     load(0);
     for (int kb = 0; kb < p; kb += KT) {
-        store();
+        store(kb);
         __syncthreads();
         if (kb + KT < p) load(kb + KT);
 #pragma unroll
@@ -923,32 +944,73 @@ __global__ __launch_bounds__(64 * WR * WC) void k_nd_gemm(NdLev lv, const NdFac*
         }
         __syncthreads();
     }
-    const short* cm = lv.cm + (long)fr * 2 * (p + b);
-    const C* Sc = SCHUR ? (const C*)Scv + ((long)q * lv.cnt * lv.nch + (long)fr * lv.nch) * lv.cb * lv.cb
-                        : nullptr;
-    C* S = SCHUR ? (C*)Sv + job * b * b : nullptr;
+    if (!SCHUR) {
 #pragma unroll
-    for (int x = 0; x < BM; ++x)
+        for (int x = 0; x < BM; ++x)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int i = i0 + wr * WM + x * 16 + M::row(lane, v);
-            if (i >= Mr) continue;
+            for (int v = 0; v < 4; ++v) {
+                const int i = i0 + wr * WM + x * 16 + M::row(lane, v);
 #pragma unroll
-            for (int y = 0; y < BN; ++y) {
-                const int j = j0 + wc * WN + y * 16 + lr;
-                if (j >= b) continue;
-                const R re = c1[x][y][v] - c2[x][y][v];
-                const R im = c3[x][y][v] - c1[x][y][v] - c2[x][y][v];
-                if (!SCHUR) {
-                    gstore(Q + (long)i * b + j, mk<C>(re, im));
-                } else if (i >= j) {
-                    const C o = nd_gather(lv, Sc, cm, p + i, p + j);
-                    const C z = mk<C>(o.x - re, o.y - im);
-                    gstore(S + (long)i * b + j, z);
-                    if (i > j) gstore(S + (long)j * b + i, z);
+                for (int y = 0; y < BN; ++y) {
+                    const int j = j0 + wc * WN + y * 16 + lr;
+                    if (i < p && j < b)
+                        gstore(Q + (long)i * b + j, mk<C>(c1[x][y][v] - c2[x][y][v], c3[x][y][v] - c1[x][y][v] - c2[x][y][v]));
                 }
             }
+        return;
+    }
+    // S: the children's entries of a 16 x 16 block are loaded before they are
+    // used (entry 0 where there is none), the block is written row by row, and
+    // its mirror image row by row after a transpose through the wave's LDS
+    const short *cm = lv.cm + (long)fr * 2 * (p + b) + p, *cm1 = cm + (p + b);
+    const C* Sc = (const C*)Scv + ((long)q * lv.cnt * lv.nch + (long)fr * lv.nch) * lv.cb * lv.cb;
+    C* S = (C*)Sv + job * b * b;
+    const bool two = lv.nch > 1;
+    C(*tr)[17] = (C(*)[17])((C*)&sAr[0][0] + wv * 16 * 17);  // (the stages are consumed)
+    static_assert(sizeof(C) * WR * WC * 16 * 17 <= sizeof(double) * 2 * KT * (PA + PB), "transpose tiles fit the stages");
+#pragma unroll
+    for (int x = 0; x < BM; ++x) {
+        const int ib = i0 + wr * WM + x * 16;
+        int m0[4], m1[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int i = min(ib + M::row(lane, v), b - 1);
+            m0[v] = cm[i];
+            m1[v] = two ? cm1[i] : -1;
         }
+#pragma unroll
+        for (int y = 0; y < BN; ++y) {
+            const int jb = j0 + wc * WN + y * 16, j = jb + lr;
+            if (jb > ib || jb >= b) continue;  // uniform: above the diagonal, or outside
+            const int n0 = cm[min(j, b - 1)], n1 = two ? cm1[min(j, b - 1)] : -1;
+            C o0[4], o1[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                o0[v] = gload(Sc + (m0[v] >= 0 && n0 >= 0 ? (long)m0[v] * lv.cb + n0 : 0));
+                o1[v] = gload(Sc + (m1[v] >= 0 && n1 >= 0 ? ((long)lv.cb + m1[v]) * lv.cb + n1 : 0));
+            }
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const bool k0 = m0[v] >= 0 && n0 >= 0, k1 = m1[v] >= 0 && n1 >= 0;
+                const double re = c1[x][y][v] - c2[x][y][v], im = c3[x][y][v] - c1[x][y][v] - c2[x][y][v];
+                const C z = mk<C>((k0 ? o0[v].x : 0.0) + (k1 ? o1[v].x : 0.0) - re,
+                                  (k0 ? o0[v].y : 0.0) + (k1 ? o1[v].y : 0.0) - im);
+                const int i = ib + M::row(lane, v);
+                if (i < b && j < b) gstore(S + (long)i * b + j, z);
+                tr[M::row(lane, v)][lr] = z;
+            }
+            if (ib == jb) continue;  // a diagonal block is whole
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int jj = jb + M::row(lane, v), i = ib + lr;
+                if (i < b && jj < b) gstore(S + (long)jj * b + i, tr[lr][M::row(lane, v)]);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
 }
 
 void launch_nd_gemm(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, const void* F12,
@@ -957,14 +1019,8 @@ void launch_nd_gemm(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, con
         const int ntm = ((schur ? lv.b : lv.p) + TM - 1) / TM, ntn = (lv.b + TN - 1) / TN;
         kern<<<dim3(lv.cnt * ntm * ntn, B), NT, 0, s>>>(lv, fac, F12, Sc, S, ntm, ntn);
     };
-    constexpr int TN = 64;
-    if (lv.b >= 256 && lv.p >= 96) {
-        if (schur) go(k_nd_gemm<128, TN, 16, 4, 2, true>, 128, TN, 512);
-        else go(k_nd_gemm<128, TN, 16, 4, 2, false>, 128, TN, 512);
-    } else {
-        if (schur) go(k_nd_gemm<64, 64, 8, 2, 2, true>, 64, 64, 256);
-        else go(k_nd_gemm<64, 64, 8, 2, 2, false>, 64, 64, 256);
-    }
+    if (schur) go(k_nd_gemm<32, 32, 16, 2, 2, true>, 32, 32, 256);
+    else go(k_nd_gemm<32, 32, 16, 2, 2, false>, 32, 32, 256);
 }
 
 // smallest and largest pivot and zero-pivot flag of each factor's fronts

@@ -98,7 +98,7 @@ struct Scratch {
         oF12 = take(ELEM * P.maxF12 * B);
         oR = take(ELEM * P.maxp * 64 * B);
         oZ = take(ELEM * P.maxp * 64 * B);
-        oD = take(ELEM * P.maxcnt * 2 * 64 * 64 * B);
+        oD = take(ELEM * P.maxcnt * 64 * 64 * B);
         for (int k = 0; k < 2; ++k) oS[k] = take(ELEM * P.maxS[k] * B);
         ofac = take(sizeof(NdFac) * B);
         ostat = take(sizeof(double) * 3 * B);
