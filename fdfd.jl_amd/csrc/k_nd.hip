@@ -140,6 +140,8 @@ __device__ inline double2 nd_entry(const double2* coef, long N, int Nx, int Ny, 
 //   b  Z_J = D^-1 R_J on MFMA, replacing tiles (k, J) by Z_J, (I, k) by -Z_I^T;
 //   c  M_IJ -= sigma_I R_I^T Z_J on the other tiles, sigma = -1 for swept I;
 //      the wave of the next diagonal tile goes on to its sweep meanwhile.
+// The last block may end inside its tile: with its swept rows s and the others u,
+// D holds D_ss^-1 and E = D_ss^-1 M_su, and b leaves R_uJ - E^T R_sJ in rows u.
 // Cells are taken in order: with FP64 fronts and refinement the growth this
 // allows (1e4 .. 1e5, like the near-resonances of the boxes) costs nothing that
 // pivoting inside a separator would save.  What bounds a small inversion is the
@@ -247,12 +249,13 @@ __device__ __attribute__((always_inline)) inline void nd_sweep16(d4v& mr, d4v& m
     });
 }
 
-// DB: the block row is double-buffered (one barrier less a block, more LDS)
+// DB: the block row is double-buffered (one barrier less a block, more LDS).
+// R and Z leave out the block being swept.
 template <int T> struct NdSweep {
     static constexpr int NTL = T * (T + 1) / 2, NS = (NTL + 3) / 4;  // tiles, slots per wave
     static constexpr bool DB = T <= 4;
-    C R[DB ? 2 : 1][T][16][17];
-    C Z[T][16][17];
+    C R[DB ? 2 : 1][T > 1 ? T - 1 : 1][16][17];
+    C Z[T > 1 ? T - 1 : 1][16][17];
     C D[16][17];
     double pv[4][3];
 };
@@ -291,15 +294,16 @@ __device__ __attribute__((always_inline)) inline void nd_sweep(d4v (&mr)[NdSweep
     for (int kb = 0; 16 * kb < np; ++kb) {
         const int kw = min(16, np - 16 * kb);
         C(*R)[16][17] = s.R[NdSweep<T>::DB ? kb & 1 : 0];
+        auto at = [&](int I) { return I - (I > kb); };
         // the diagonal tile of block kb is in slot e / 4 of wave e % 4
         const int e = kb * (kb + 3) / 2;
         nd_each_tile<T>([&](auto sc, int I, int J) {
             if (I != J && I == kb) {
 #pragma unroll
-                for (int v = 0; v < 4; ++v) R[J][F64::row(lane, v)][l16] = mk<C>(mr[sc][v], mi[sc][v]);
+                for (int v = 0; v < 4; ++v) R[at(J)][F64::row(lane, v)][l16] = mk<C>(mr[sc][v], mi[sc][v]);
             } else if (I != J && J == kb) {
 #pragma unroll
-                for (int v = 0; v < 4; ++v) R[I][l16][F64::row(lane, v)] = mk<C>(mr[sc][v], mi[sc][v]);
+                for (int v = 0; v < 4; ++v) R[at(I)][l16][F64::row(lane, v)] = mk<C>(mr[sc][v], mi[sc][v]);
             }
         });
         if ((e & 3) == __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6)) {
@@ -319,7 +323,7 @@ __device__ __attribute__((always_inline)) inline void nd_sweep(d4v (&mr)[NdSweep
                     mi[q] = xi;
                 }
 #pragma unroll
-            for (int v = 0; v < 4; ++v) s.D[F64::row(lane, v)][l16] = mk<C>(xr[v], xi[v]);
+            for (int v = 0; v < 4; ++v) s.D[F64::row(lane, v)][l16] = mk<C>(l16 < kw ? xr[v] : -xr[v], l16 < kw ? xi[v] : -xi[v]);
         }
         if (T == 1) break;
         __syncthreads();
@@ -328,9 +332,18 @@ __device__ __attribute__((always_inline)) inline void nd_sweep(d4v (&mr)[NdSweep
             if ((I == kb) == (J == kb)) return;
             const bool rowt = I == kb;  // tile (k, J), else (I, k)
             // (k, J): D^-1 R_J; (I, k): R_I^T D^-1 (D^-1 is symmetric)
-            const C(*Ap)[17] = rowt ? s.D : R[I];
-            const C(*Bp)[17] = rowt ? R[J] : s.D;
+            const C(*Ap)[17] = rowt ? s.D : R[at(I)];
+            const C(*Bp)[17] = rowt ? R[at(J)] : s.D;
             d4v xr = {0, 0, 0, 0}, xi = {0, 0, 0, 0}, yr = {0, 0, 0, 0}, yi = {0, 0, 0, 0};
+            if (kw < 16) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const bool un = (rowt ? F64::row(lane, v) : l16) >= kw;
+                    xr[v] = un ? mr[sc][v] : 0.0;
+                    xi[v] = un ? mi[sc][v] : 0.0;
+                }
+            }
+            const bool ng = !rowt && l16 < kw;
 #pragma unroll
             for (int q = 0; q < 4; ++q)
                 if (q < kq) {
@@ -343,17 +356,17 @@ __device__ __attribute__((always_inline)) inline void nd_sweep(d4v (&mr)[NdSweep
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 const C z = mk<C>(xr[v] - yr[v], xi[v] + yi[v]);
-                if (rowt) s.Z[J][F64::row(lane, v)][l16] = z;
-                else s.Z[I][l16][F64::row(lane, v)] = z;
-                mr[sc][v] = rowt ? z.x : -z.x;
-                mi[sc][v] = rowt ? z.y : -z.y;
+                if (rowt) s.Z[at(J)][F64::row(lane, v)][l16] = z;
+                else s.Z[at(I)][l16][F64::row(lane, v)] = z;
+                mr[sc][v] = ng ? -z.x : z.x;
+                mi[sc][v] = ng ? -z.y : z.y;
             }
         });
         __syncthreads();
         nd_each_tile<T>([&](auto sc, int I, int J) {
             if (I == kb || J == kb) return;
-            const C(*Ap)[17] = R[I];
-            const C(*Bp)[17] = s.Z[J];
+            const C(*Ap)[17] = R[at(I)];
+            const C(*Bp)[17] = s.Z[at(J)];
             const unsigned long long sg = I > kb ? 0x8000000000000000ull : 0ull;  // subtract unless swept
 #pragma unroll
             for (int q = 0; q < 4; ++q)
@@ -391,40 +404,67 @@ __device__ __attribute__((always_inline)) inline void nd_sweep(d4v (&mr)[NdSweep
     }
 }
 
-// Leaves: one workgroup per leaf, its whole front swept in registers (the
-// separator padded to whole tiles with unit rows, then the boundary).
+// Leaves: one workgroup per leaf, its whole front, the separator and then the
+// boundary, swept in registers.  The chain of the sweep bounds a workgroup (some
+// 50 us for 52 cells), so what counts is how many share a compute unit: a leaf
+// of 7 x 7 cells is 80 rows, 15 tiles, 166 VGPRs and 39 kB of LDS, three
+// workgroups.  The 16384 leaves of a 1024 x 1024 grid take 1.09 ms; 1.71 ms with
+// the boundary behind whole tiles of separator (96 rows, 21 tiles, two
+// workgroups), 1.19 ms with the entries gathered one by one from memory.
 template <int T>
-__global__ __launch_bounds__(256, 2) void k_nd_leaf(NdLev lv, const NdFac* fac, int Nx, int Ny, void* Sv) {
+__global__ __launch_bounds__(256, 3) void k_nd_leaf(NdLev lv, const NdFac* fac, int Nx, int Ny, void* Sv) {
     const NdFac F = fac[blockIdx.y];
-    const int p = lv.p, b = lv.b, p16 = (p + 15) & ~15, fr = blockIdx.x;
+    const int p = lv.p, b = lv.b, fr = blockIdx.x;
     const long N = (long)Nx * Ny;
-    __shared__ NdSweep<T> s;
-    __shared__ int nd[16 * T];
-    const int t = threadIdx.x;
-    for (int i = t; i < 16 * T; i += 256) {
-        const int e = i < p ? i : (i >= p16 && i < p16 + b ? p + i - p16 : -1);
-        nd[i] = e >= 0 ? lv.node[(long)fr * (p + b) + e] : -1;
+    constexpr int NF = 16 * T;
+    // the operator at the front's cells, for the gather below: one load a thread
+    // in place of a branch and a load for each entry that is not zero
+    __shared__ union {
+        NdSweep<T> w;
+        struct {
+            C cc[NF], ce[NF], cn[NF];
+            int x[NF], y[NF];  // x < 0: no cell
+        } g;
+    } s;
+    for (int e = threadIdx.x; e < 3 * NF; e += 256) {
+        const int i = e % NF, pl = e / NF;
+        const int k = i < p + b ? lv.node[(long)fr * (p + b) + i] : -1, kk = max(k, 0);
+        const C c = gload(F.coef + (long)(pl == 0 ? CC : pl == 1 ? CE : CN) * N + kk);
+        (pl == 0 ? s.g.cc : pl == 1 ? s.g.ce : s.g.cn)[i] = c;
+        if (pl == 0) {
+            s.g.x[i] = k < 0 ? -1 : k % Nx;
+            s.g.y[i] = kk / Nx;
+        }
     }
     __syncthreads();
     constexpr int NS = NdSweep<T>::NS;
     d4v mr[NS], mi[NS];
     nd_each_entry<T>([&](auto sc, int v, int i, int j, bool) {
         C z = mk<C>(0, 0);
-        const int ki = nd[i], kj = nd[j];
-        if (i < p16 || j < p16) {
-            if (ki >= 0 && kj >= 0) z = nd_entry(F.coef, N, Nx, Ny, ki, kj);
-            else if (i == j) z = mk<C>(1, 0);
+        const int xi = s.g.x[i], xj = s.g.x[j], yi = s.g.y[i], yj = s.g.y[j];
+        if (i < p || j < p) {
+            if (xi < 0 || xj < 0) {
+                z = mk<C>(i == j ? 1 : 0, 0);
+            } else if (yi == yj) {
+                if (i == j) z = s.g.cc[i];
+                if (xj == (xi + 1 == Nx ? 0 : xi + 1)) z = cadd(z, s.g.ce[i]);
+                if (xi == (xj + 1 == Nx ? 0 : xj + 1)) z = cadd(z, s.g.ce[j]);
+            } else if (xi == xj) {
+                if (yj == (yi + 1 == Ny ? 0 : yi + 1)) z = cadd(z, s.g.cn[i]);
+                if (yi == (yj + 1 == Ny ? 0 : yj + 1)) z = cadd(z, s.g.cn[j]);
+            }
         }
         mr[sc][v] = z.x;
         mi[sc][v] = z.y;
     });
-    nd_sweep<T>(mr, mi, p, s, F.pivstat + 3 * (long)(lv.stat + fr), false);
+    __syncthreads();
+    nd_sweep<T>(mr, mi, p, s.w, F.pivstat + 3 * (long)(lv.stat + fr), false);
     C* X = (C*)F.arena + lv.offX + (long)fr * p * p;
     C* Q = (C*)F.arena + lv.offQ + (long)fr * p * b;
     C* S = (C*)Sv + ((long)blockIdx.y * lv.cnt + fr) * b * b;
     nd_each_entry<T>([&](auto sc, int v, int i, int j, bool off) {
         const C z = mk<C>(mr[sc][v], mi[sc][v]);
-        const int ib = i - p16, jb = j - p16;
+        const int ib = i - p, jb = j - p;
         if (i < p && j < p) {
             gstore(X + i * p + j, z);
             if (off) gstore(X + j * p + i, z);
@@ -437,14 +477,14 @@ __global__ __launch_bounds__(256, 2) void k_nd_leaf(NdLev lv, const NdFac* fac, 
     });
 }
 
+static_assert(nd::LEAF_FRONT <= 80, "a leaf fits the largest kernel");
 void launch_nd_leaf(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, int Nx, int Ny, void* S) {
-    const int f = ((lv.p + 15) & ~15) + lv.b;
+    const int f = lv.p + lv.b;
     const dim3 g(lv.cnt, B);
     if (f <= 32) k_nd_leaf<2><<<g, 256, 0, s>>>(lv, fac, Nx, Ny, S);
     else if (f <= 48) k_nd_leaf<3><<<g, 256, 0, s>>>(lv, fac, Nx, Ny, S);
     else if (f <= 64) k_nd_leaf<4><<<g, 256, 0, s>>>(lv, fac, Nx, Ny, S);
-    else if (f <= 80) k_nd_leaf<5><<<g, 256, 0, s>>>(lv, fac, Nx, Ny, S);
-    else k_nd_leaf<6><<<g, 256, 0, s>>>(lv, fac, Nx, Ny, S);
+    else k_nd_leaf<5><<<g, 256, 0, s>>>(lv, fac, Nx, Ny, S);
 }
 
 // children's contribution to entry (i, j) of a front, i, j front indices

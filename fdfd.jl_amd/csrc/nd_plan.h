@@ -38,10 +38,10 @@ struct Box {
     int x0, w, y0, h;
 };
 
-// largest leaf: cells, and front size of the leaf kernel (separator in whole
-// tiles of 16, then the boundary)
+// largest leaf: cells, and rows of the leaf kernel's front (cells and boundary,
+// each padded to a multiple of 4)
 constexpr int LEAF_CELLS = 49;
-constexpr int LEAF_FRONT = 96;
+constexpr int LEAF_FRONT = 80;
 
 // sides of a box: the columns left and right of it (nx of them: none when it
 // wraps in x, one when both are the same column) and the rows below and above
@@ -158,7 +158,7 @@ inline std::vector<Level> make_plan(int Nx, int Ny) {
         }
         const bool open = !cur.wrapx && !cur.wrapy;
         const bool canx = cur.wrapx ? wmin >= 2 : wmin >= 3, cany = cur.wrapy ? hmin >= 2 : hmin >= 3;
-        if ((open && W * H <= LEAF_CELLS && ((W * H + 15) & ~15) + 2 * (W + H) + 3 <= LEAF_FRONT) || (!canx && !cany)) {
+        if ((open && W * H <= LEAF_CELLS && ((W * H + 3) & ~3) + ((2 * (W + H) + 3) & ~3) <= LEAF_FRONT) || (!canx && !cany)) {
             cur.kind = ND_LEAF;
         } else {
             const double ex = cur.wrapx ? 0.5 * W : W, ey = cur.wrapy ? 0.5 * H : H;

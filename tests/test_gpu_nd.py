@@ -84,3 +84,26 @@ def test_several_grids_share_a_handle(monkeypatch):
             assert np.linalg.norm(b - O.assemble(g, d.eps_r, om, O.TM) @ x) <= 1e-12 * np.linalg.norm(b)
     finally:
         e.close()
+
+
+@pytest.mark.parametrize("Nx,Ny", [(16, 16), (18, 18), (20, 20), (22, 22), (24, 24), (28, 28), (19, 30), (16, 27)])
+def test_leaf_fronts_of_every_size(monkeypatch, Nx, Ny):
+    """Leaves of 20 to 49 cells with boundaries of 16 to 32: the last swept block
+    ends inside its 16-cell tile after 4, 8, 12 or 16 cells, with boundary rows
+    behind it.  FP64 factors leave a relative residual near 1e-13 after one
+    application, so a sound one needs at most two iterations for 1e-13 (a wrong
+    entry costs many or never converges)."""
+    d = _device(Nx, Ny, 2, Nx * 31 + Ny)
+    om = float(d.omega[0])
+    b = O.rhs(om, d.src)
+    e = _engine(monkeypatch, "nd", d)
+    try:
+        for pol in (O.TM, O.TE):
+            fid, fst = e.factor(pol, om, "fp64")
+            x, st = e.linsolve(fid, b, tol=1e-13)
+            res = np.linalg.norm(b - O.assemble(d.grid, d.eps_r, om, pol) @ x) / np.linalg.norm(b)
+            print(f"{Nx}x{Ny} pol={pol}: res={res:.1e} its={st['iterations']}", flush=True)
+            assert fst["pivot_fallback"] == 0 and st["iterations"] <= 2 and res <= 1e-12
+            e.release(fid)
+    finally:
+        e.close()
