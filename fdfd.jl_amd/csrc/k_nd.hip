@@ -1092,157 +1092,221 @@ void launch_nd_stat(hipStream_t s, const NdFac* fac, int B, int nfronts, double*
 }
 
 // ---------------------------------------------------------------------------
-// Reduced solve.  Upward step of a level: the separator values
+// Reduced solve for one right-hand side: a launch per level and direction,
+// memory-bound on the leaves and bound by latency on all levels above, so a
+// kernel keeps its chain short: what addresses the matrix does not depend on the
+// vectors, and its loads are issued before the gathers (list, then value) that
+// the vectors take; no workgroup barrier comes before the products; edges are
+// clamped addresses against a zero operand, not branches.  A solve on a 512 x 512
+// grid: 295 us in 30 launches (leaves 17 up and 58 down, 4.7 TB/s; the levels above
+// 3 to 11 each), against 490 us with v staged by the workgroup before it loads Q
+// and rows of X and Q in turn (leaves 26 and 111, levels 9 to 19).
+//
+// Upward step of a level: the separator values
 //   v = scaled right-hand side + children's updates
-// and the boundary update u = children's updates - Q^T v.  A workgroup takes
-// CW boundary columns; 256 / CW row groups split the separator.
+// and the boundary update u = children's updates - Q^T v.  A task is CL boundary
+// columns of one front: the lanes of a wave are CL columns by 64 / CL rows, and
+// KW waves take a part of the separator each.
 // ---------------------------------------------------------------------------
-template <int CW>
-__global__ __launch_bounds__(256) void k_nd_up(NdLev lv, const void* arena, NdVec z, int Nx, int nchunk) {
-    constexpr int RG = 256 / CW;
-    extern __shared__ char nd_lds[];
-    C* vs = (C*)nd_lds;
-    __shared__ C red[RG][CW];
-    const int fr = blockIdx.x / nchunk, ch = blockIdx.x % nchunk;
-    const int p = lv.p, b = lv.b, f = p + b;
+constexpr int UP_MU = 8;  // rows of Q a lane loads at a time
+
+template <int CL, int KW>
+__global__ __launch_bounds__(KW > 4 ? 64 * KW : 256) void k_nd_up(NdLev lv, const void* arena, NdVec z, int Nx,
+                                                                 int nchunk) {
+    constexpr int RG = 64 / CL, NW = KW > 4 ? KW : 4;  // row groups of a wave, waves
+    __shared__ C vs[NW][64];
+    __shared__ C red[KW > 1 ? KW : 1][CL];
+    const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wk = KW > 1 ? wv : 0;
+    const int task = KW > 1 ? (int)blockIdx.x : (int)blockIdx.x * NW + wv;
+    if (KW == 1 && task >= lv.cnt * nchunk) return;  // (no barrier follows)
+    const int fr = task / nchunk, ch = task % nchunk;
+    const int p = lv.p, b = lv.b, f = p + b, nch = lv.nch;
     const int src = z.ridx ? z.ridx[0] : 0;
     const double2* in = z.in + (long)src * z.rs;
-    double2* vb = z.v + lv.offV + (long)fr * p;
-    double2* ub = z.u + lv.offU + (long)fr * b;
-    const double2* uc = z.u + lv.offUc + (long)fr * lv.nch * lv.cb;
+    const double2* uc = z.u + lv.offUc + (long)fr * nch * lv.cb;
     const int* node = lv.node + (long)fr * f;
     const short* cm = lv.cm + (long)fr * 2 * f;
-    const int t = threadIdx.x;
-    auto kids = [&](int i) {
-        double2 a = make_double2(0, 0);
-        if (lv.nch > 0) {
-            const int m0 = cm[i];
-            if (m0 >= 0) a = uc[m0];
-            if (lv.nch > 1) {
-                const int m1 = cm[f + i];
-                if (m1 >= 0) a = cadd(a, uc[lv.cb + m1]);
+    const int col = lane % CL, rg = lane / CL, j = ch * CL + col;
+    const C* Q = (const C*)arena + lv.offQ + (long)fr * p * b + min(j, b - 1);
+    auto kids = [&](int m0, int m1) {
+        C a = mk<C>(0, 0);
+        if (nch > 0) {
+            const C a0 = uc[max(m0, 0)];
+            a = csel(m0 >= 0, a0, a);
+            if (nch > 1) {
+                const C a1 = uc[lv.cb + max(m1, 0)];
+                a = cadd(a, csel(m1 >= 0, a1, mk<C>(0, 0)));
             }
         }
         return a;
     };
-    for (int i = t; i < p; i += 256) {
-        const int k = node[i];
-        double2 v = make_double2(0, 0);
-        if (k >= 0) {
-            v = cmul(in[k], cmul(z.six[k % Nx], z.siy[k / Nx]));
-            v = cadd(v, kids(i));
+    // children's share of this task's columns, for the first lane group
+    const bool fin = wk == 0 && rg == 0 && j < b;
+    int n0 = -1, n1 = -1;
+    if (nch > 0 && b > 0) n0 = cm[p + min(j, b - 1)];
+    if (nch > 1 && b > 0) n1 = cm[f + p + min(j, b - 1)];
+    const int PW = KW > 1 ? (p + KW - 1) / KW : p, ib = wk * PW, ie = min(p, ib + PW);
+    C acc = mk<C>(0, 0);
+    for (int i0 = ib; i0 < ie; i0 += 64) {
+        const int n = min(64, ie - i0), i = i0 + min(lane, n - 1);
+        const int k = node[i], m0 = nch > 0 ? cm[i] : -1, m1 = nch > 1 ? cm[f + i] : -1;
+        C q[UP_MU];
+        auto load = [&](int r0) {
+#pragma unroll
+            for (int m = 0; m < UP_MU; ++m) q[m] = gload(Q + (long)(i0 + min(r0 + rg + RG * m, n - 1)) * b);
+        };
+        if (b > 0) load(0);
+        const int kk = max(k, 0);
+        C v = cadd(cmul(in[kk], cmul(z.six[kk % Nx], z.siy[kk / Nx])), kids(m0, m1));
+        v = csel(k >= 0 && lane < n, v, mk<C>(0, 0));
+        if (ch == 0 && lane < n) z.v[lv.offV + (long)fr * p + i] = v;
+        if (b == 0) continue;
+        __builtin_amdgcn_wave_barrier();
+        vs[wv][lane] = v;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        for (int r0 = 0; r0 < n; r0 += UP_MU * RG) {
+            if (r0 > 0) load(r0);
+#pragma unroll
+            for (int m = 0; m < UP_MU; ++m) {
+                const int r = r0 + rg + RG * m;
+                const C x = csel(r < n, vs[wv][min(r, 63)], mk<C>(0, 0));
+                acc = cfma(q[m], x, acc);
+            }
         }
-        vs[i] = (v);
-        if (ch == 0) vb[i] = v;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
     if (b == 0) return;
-    __syncthreads();
-    const int c = t % CW, rg = t / CW, j = ch * CW + c;
-    C acc = mk<C>(R(0), R(0));
-    if (j < b) {
-        const C* Q = (const C*)arena + lv.offQ + (long)fr * p * b + j;
-        int i = rg;
-        for (; i + 3 * RG < p; i += 4 * RG) {
-            const C q0 = gload(Q + (long)i * b), q1 = gload(Q + (long)(i + RG) * b),
-                    q2 = gload(Q + (long)(i + 2 * RG) * b), q3 = gload(Q + (long)(i + 3 * RG) * b);
-            acc = cadd(acc, cmul(q0, vs[i]));
-            acc = cadd(acc, cmul(q1, vs[i + RG]));
-            acc = cadd(acc, cmul(q2, vs[i + 2 * RG]));
-            acc = cadd(acc, cmul(q3, vs[i + 3 * RG]));
-        }
-        for (; i < p; i += RG) acc = cadd(acc, cmul(gload(Q + (long)i * b), vs[i]));
+    const C own = kids(n0, n1);
+#pragma unroll
+    for (int o = CL; o < 64; o <<= 1) {
+        acc.x += shfl_x(acc.x, o);
+        acc.y += shfl_x(acc.y, o);
     }
-    red[rg][c] = acc;
-    __syncthreads();
-    if (t < CW && j < b) {
-#pragma unroll 4
-        for (int r = 1; r < RG; ++r) acc = cadd(acc, red[r][c]);
-        ub[j] = csub(kids(p + j), (acc));
+    if (KW > 1) {
+        if (rg == 0) red[wk][col] = acc;
+        __syncthreads();
+        if (!fin) return;
+#pragma unroll
+        for (int w = 1; w < KW; ++w) acc = cadd(acc, red[w][col]);
     }
+    if (fin) z.u[lv.offU + (long)fr * b + j] = csub(own, acc);
 }
 
-// Downward step: x = X v - Q x_boundary, one wave per row (RPW rows at a
-// time), the vector staged through LDS in pieces.
-constexpr int DN_PIECE = 512;
-
-template <int RPW>
+// Downward step: x = X v - Q x_boundary.  A task is RW rows of one front, whose
+// columns (of X, then of Q) are spread over the lanes of KW waves; the sums over
+// the lanes are folded so that each exchange halves the rows a lane holds.
+template <int RW, int KW>
 __global__ __launch_bounds__(256) void k_nd_down(NdLev lv, const void* arena, NdVec z, int Nx, int nchunk) {
-    __shared__ C xs[DN_PIECE];
-    const int fr = blockIdx.x / nchunk, ch = blockIdx.x % nchunk;
+    constexpr int MU = RW >= 8 ? 2 : 8 / RW;  // columns a lane takes at a time
+    __shared__ C red[KW][RW];
+    const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wk = KW > 1 ? wv : 0;
+    const int task = KW > 1 ? (int)blockIdx.x : (int)blockIdx.x * 4 + wv;
+    if (KW == 1 && task >= lv.cnt * nchunk) return;  // (no barrier follows)
+    const int fr = task / nchunk, r0 = (task % nchunk) * RW;
     const int p = lv.p, b = lv.b, f = p + b;
     const int src = z.ridx ? z.ridx[0] : 0;
     double2* out = z.out + (long)src * z.rs;
     double2* xg = z.x;
     const double2* vb = z.v + lv.offV + (long)fr * p;
     const int* node = lv.node + (long)fr * f;
-    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
     const C* X = (const C*)arena + lv.offX + (long)fr * p * p;
     const C* Q = (const C*)arena + lv.offQ + (long)fr * p * b;
-    const int r0 = (ch * 4 + wv) * RPW;
-    C acc[RPW];
+    // the row that the folds leave in this lane, its cell and scaling
+    constexpr int FB = RW == 8 ? 3 : RW == 4 ? 2 : RW == 2 ? 1 : 0;  // folds
+    const int row = lane >> (6 - FB), ni = node[min(r0 + row, p - 1)];
+    C acc[RW];
 #pragma unroll
-    for (int r = 0; r < RPW; ++r) acc[r] = mk<C>(R(0), R(0));
-    for (int part = 0; part < 2; ++part) {
-        const int len = part ? b : p;
-        const C* Mt = part ? Q : X;
-        for (int k0 = 0; k0 < len; k0 += DN_PIECE) {
-            const int n = min(DN_PIECE, len - k0);
-            __syncthreads();
-            for (int k = t; k < n; k += 256) {
-                if (part) {
-                    const int kk = node[p + k0 + k];
-                    xs[k] = kk >= 0 ? (cneg(xg[kk])) : mk<C>(R(0), R(0));
-                } else {
-                    xs[k] = (vb[k0 + k]);
-                }
-            }
-            __syncthreads();
-            for (int k = lane; k < n; k += 64) {
-                const C x = xs[k];
+    for (int r = 0; r < RW; ++r) acc[r] = mk<C>(0, 0);
+    for (int k0 = wk * 64 + lane; __any(k0 < f); k0 += 64 * KW * MU) {
+        C a[MU][RW], x[MU];
+        int kn[MU];
 #pragma unroll
-                for (int r = 0; r < RPW; ++r) {
-                    const int i = min(r0 + r, p - 1);
-                    acc[r] = cadd(acc[r], cmul(gload(Mt + (long)i * len + k0 + k), x));
-                }
-            }
+        for (int m = 0; m < MU; ++m) {
+            const int k = min(k0 + 64 * KW * m, f - 1);
+            kn[m] = node[k];
+            x[m] = vb[min(k, p - 1)];
+        }
+#pragma unroll
+        for (int m = 0; m < MU; ++m) {
+            const int k = min(k0 + 64 * KW * m, f - 1);
+            const bool q = k >= p;
+            const C* M = q ? Q + (k - p) : X + k;
+            const int ld = q ? b : p;
+#pragma unroll
+            for (int r = 0; r < RW; ++r) a[m][r] = gload(M + (long)min(r0 + r, p - 1) * ld);
+        }
+#pragma unroll
+        for (int m = 0; m < MU; ++m) {
+            const int k = k0 + 64 * KW * m;
+            const C xb = xg[max(kn[m], 0)];
+            C y = csel(k < p, x[m], csel(kn[m] >= 0, cneg(xb), mk<C>(0, 0)));
+            y = csel(k < f, y, mk<C>(0, 0));
+#pragma unroll
+            for (int r = 0; r < RW; ++r) acc[r] = cfma(a[m][r], y, acc[r]);
         }
     }
+    const int nc = max(ni, 0);
+    const C sc = cmul(z.sox[nc % Nx], z.soy[nc / Nx]);
+    static_for<0, FB>([&](auto s) {
+        constexpr int h = RW >> (decltype(s)::value + 1), o = 32 >> decltype(s)::value;
+        const bool up = (lane & o) != 0;
 #pragma unroll
-    for (int r = 0; r < RPW; ++r) {
-        for (int o = 32; o > 0; o >>= 1) {
-            acc[r].x += shfl_x(acc[r].x, o);
-            acc[r].y += shfl_x(acc[r].y, o);
+        for (int r = 0; r < h; ++r) {
+            const C keep = csel(up, acc[r + h], acc[r]), give = csel(up, acc[r], acc[r + h]);
+            acc[r] = mk<C>(keep.x + shfl_x(give.x, o), keep.y + shfl_x(give.y, o));
         }
-        const int i = r0 + r;
-        if (lane == 0 && i < p) {
-            const int k = node[i];
-            if (k >= 0) {
-                const double2 x = (acc[r]);
-                xg[k] = x;
-                out[k] = cmul(x, cmul(z.sox[k % Nx], z.soy[k / Nx]));
-            }
-        }
+    });
+#pragma unroll
+    for (int o = 32 >> FB; o > 0; o >>= 1) {
+        acc[0].x += shfl_x(acc[0].x, o);
+        acc[0].y += shfl_x(acc[0].y, o);
+    }
+    const bool head = (lane & ((64 >> FB) - 1)) == 0;
+    C y = acc[0];
+    if (KW > 1) {
+        if (head) red[wk][row] = y;
+        __syncthreads();
+        if (wk > 0 || !head) return;
+#pragma unroll
+        for (int w = 1; w < KW; ++w) y = cadd(y, red[w][row]);
+    }
+    if (head && r0 + row < p && ni >= 0) {
+        xg[ni] = y;
+        out[ni] = cmul(y, sc);
     }
 }
 
+// The widest task that still makes ND_WAVES waves (8 on each compute unit);
+// below, narrower ones with the sums split over the waves of a workgroup.
+constexpr long ND_WAVES = 2048;
+
 void launch_nd_up(hipStream_t s, const NdLev& lv, const void* arena, const NdVec& z, int Nx) {
-    const size_t lds = sizeof(C) * lv.p;
-    auto go = [&](auto kern, int CW) {
-        const int nch = std::max(1, (lv.b + CW - 1) / CW);
-        kern<<<dim3(lv.cnt * nch), 256, lds, s>>>(lv, arena, z, Nx, nch);
+    auto tasks = [&](int CL) { return (long)lv.cnt * std::max(1, (lv.b + CL - 1) / CL); };
+    auto go = [&](auto kern, int CL, int KW) {
+        const long n = tasks(CL);
+        const int per = KW > 1 ? 1 : 4, NT = KW > 4 ? 64 * KW : 256;
+        kern<<<(unsigned)((n + per - 1) / per), NT, 0, s>>>(lv, arena, z, Nx, (int)(n / lv.cnt));
     };
-    // few fronts: narrow column groups, so that more workgroups share a front
-    if ((long)lv.cnt * lv.b < 64 * 512) go(k_nd_up<4>, 4);
-    else if (lv.b <= 32 || (long)lv.cnt * lv.b < 64 * 2048) go(k_nd_up<16>, 16);
-    else go(k_nd_up<64>, 64);
+    if (lv.p <= 16 && tasks(64) >= ND_WAVES) go(k_nd_up<64, 1>, 64, 1);
+    else if (tasks(32) >= ND_WAVES) go(k_nd_up<32, 1>, 32, 1);
+    else if (tasks(16) >= ND_WAVES) go(k_nd_up<16, 1>, 16, 1);
+    else if (lv.p <= 64 || tasks(16) * 4 >= ND_WAVES) go(k_nd_up<16, 4>, 16, 4);
+    else go(k_nd_up<8, 16>, 8, 16);
 }
 void launch_nd_down(hipStream_t s, const NdLev& lv, const void* arena, const NdVec& z, int Nx) {
-    auto go = [&](auto kern, int RPW) {
-        const int nch = (lv.p + 4 * RPW - 1) / (4 * RPW);
-        kern<<<dim3(lv.cnt * nch), 256, 0, s>>>(lv, arena, z, Nx, nch);
+    auto tasks = [&](int RW) { return (long)lv.cnt * ((lv.p + RW - 1) / RW); };
+    auto go = [&](auto kern, int RW, int KW) {
+        const long n = tasks(RW);
+        const int per = KW > 1 ? 1 : 4;
+        kern<<<(unsigned)((n + per - 1) / per), 256, 0, s>>>(lv, arena, z, Nx, (int)(n / lv.cnt));
     };
-    if ((long)lv.cnt * lv.p < 4096) go(k_nd_down<1>, 1);
-    else go(k_nd_down<4>, 4);
+    if (tasks(8) >= ND_WAVES) go(k_nd_down<8, 1>, 8, 1);
+    else if (tasks(4) * 4 >= ND_WAVES) go(k_nd_down<4, 4>, 4, 4);
+    else if (tasks(2) * 4 >= ND_WAVES) go(k_nd_down<2, 4>, 2, 4);
+    else go(k_nd_down<1, 4>, 1, 4);
 }
 
 // ---------------------------------------------------------------------------
