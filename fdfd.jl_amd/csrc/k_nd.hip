@@ -1279,9 +1279,11 @@ __global__ __launch_bounds__(256) void k_nd_down(NdLev lv, const void* arena, Nd
     }
 }
 
-// The widest task that still makes ND_WAVES waves (8 on each compute unit);
-// below, narrower ones with the sums split over the waves of a workgroup.
-constexpr long ND_WAVES = 2048;
+// The widest task that still makes ND_WAVES waves (one for each SIMD); below,
+// narrower ones with the sums split over the waves of a workgroup.  Some 390
+// applications on a 512 x 512 grid with 512 / 1024 / 2048 / 4096 waves: 158 / 146 /
+// 160 / 186 ms; a modulated device of 500 x 200: 10.6 / 10.5 / 11.4 / 11.8 ms.
+constexpr long ND_WAVES = 1024;
 
 void launch_nd_up(hipStream_t s, const NdLev& lv, const void* arena, const NdVec& z, int Nx) {
     auto tasks = [&](int CL) { return (long)lv.cnt * std::max(1, (lv.b + CL - 1) / CL); };
