@@ -17,8 +17,8 @@
 namespace fdfd {
 
 int rt_norm(Handle* h, const double2* x, long N, double* out);
-int rt_multidot(Handle* h, const double2* V, long N, int k, const double2* w, cd* out);
-int rt_update(Handle* h, double2* w, const double2* V, long N, int k, const cd* c, double sign);
+int rt_orth(Handle* h, const double2* V, long N, int k, double2* w, cd* c, double* norm);
+void rt_update(Handle* h, double2* w, const double2* V, long N, int k, const cd* c);
 int small_eig(int n, std::vector<cd> A, std::vector<cd>& evals, std::vector<cd>& evecs);
 
 int rt_arnoldi(Handle* h, long N, int nev, int ncv, int which, double tol, int maxiter,
@@ -60,7 +60,7 @@ int rt_arnoldi(Handle* h, long N, int nev, int ncv, int which, double tol, int m
     const int m = ncv;
     std::vector<cd> H((size_t)(m + 1) * m, 0.0);  // row-major (m+1) x m
     auto Hat = [&](int i, int j) -> cd& { return H[(size_t)i * m + j]; };
-    std::vector<cd> hc(m + 1), hc2(m + 1);
+    std::vector<cd> hc(m + 1);
     int start = 0, nconv = 0, restarts = 0;
     std::vector<cd> theta, Y;
     std::vector<int> order;
@@ -69,13 +69,9 @@ int rt_arnoldi(Handle* h, long N, int nev, int ncv, int which, double tol, int m
         for (int j = start; j < m; ++j) {
             double2* w = vec(j + 1);
             if ((rc = op(vec(j), w))) { cleanup(); return rc; }
-            if ((rc = rt_multidot(h, Vb, N, j + 1, w, hc.data()))) { cleanup(); return rc; }
-            if ((rc = rt_update(h, w, Vb, N, j + 1, hc.data(), -1.0))) { cleanup(); return rc; }
-            if ((rc = rt_multidot(h, Vb, N, j + 1, w, hc2.data()))) { cleanup(); return rc; }
-            if ((rc = rt_update(h, w, Vb, N, j + 1, hc2.data(), -1.0))) { cleanup(); return rc; }
-            for (int i = 0; i <= j; ++i) Hat(i, j) = hc[i] + hc2[i];
             double hn;
-            if ((rc = rt_norm(h, w, N, &hn))) { cleanup(); return rc; }
+            if ((rc = rt_orth(h, Vb, N, j + 1, w, hc.data(), &hn))) { cleanup(); return rc; }
+            for (int i = 0; i <= j; ++i) Hat(i, j) = hc[i];
             Hat(j + 1, j) = hn;
             if (hn > 0) launch_scale_copy(h->stream, w, w, make_double2(1.0 / hn, 0), N);
         }
@@ -126,7 +122,7 @@ int rt_arnoldi(Handle* h, long N, int nev, int ncv, int which, double tol, int m
             std::vector<cd> col(m);
             for (int i = 0; i < m; ++i) col[i] = Qk[(size_t)i * keep + q];
             launch_zero(h->stream, Wb + (long)q * N, N);
-            if ((rc = rt_update(h, Wb + (long)q * N, Vb, N, m, col.data(), 1.0))) { cleanup(); return rc; }
+            rt_update(h, Wb + (long)q * N, Vb, N, m, col.data());
         }
         if (hipMemcpyAsync(vec(keep), vec(m), sizeof(double2) * N, hipMemcpyDeviceToDevice, h->stream) !=
                 hipSuccess ||
@@ -162,7 +158,7 @@ int rt_arnoldi(Handle* h, long N, int nev, int ncv, int which, double tol, int m
             for (int i = 0; i < m; ++i) col[i] = Y[(size_t)i * m + order[q]];
             double2* x = ritz + (long)q * N;
             launch_zero(h->stream, x, N);
-            if ((rc = rt_update(h, x, Vb, N, m, col.data(), 1.0))) { cleanup(); return rc; }
+            rt_update(h, x, Vb, N, m, col.data());
             if ((rc = stream_copy(h, hx.data(), x, sizeof(double2) * N, hipMemcpyDeviceToHost))) {
                 cleanup();
                 return rc;

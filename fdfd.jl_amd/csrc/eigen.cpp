@@ -25,9 +25,6 @@ namespace fdfd {
 int rt_gmres(Handle* h, Factor* F, int trans, const double2* b, double2* x, double tol, int* iters,
              double* resid);
 int rt_build_factor(Handle* h, Factor* F);
-int rt_norm(Handle* h, const double2* x, long N, double* out);
-int rt_multidot(Handle* h, const double2* V, long N, int k, const double2* w, cd* out);
-int rt_update(Handle* h, double2* w, const double2* V, long N, int k, const cd* c, double sign);
 int small_eig(int n, std::vector<cd> A, std::vector<cd>& evals, std::vector<cd>& evecs);
 int rt_arnoldi(Handle* h, long N, int nev, int ncv, int which, double tol, int maxiter,
                const std::function<int(const double2*, double2*)>& op, double2* ritz,

@@ -295,27 +295,29 @@ void launch_diag_multi(hipStream_t s, const DiagJob* jobs_d, int njobs, int n, l
 int trisolve_multi_prepare(int n);
 void launch_trisolve_multi(hipStream_t s, const TrsJob* jobs_d, int njobs, int n, long rs,
                            const int* ridx, int na);
-void launch_multidot_b(hipStream_t s, const double2* V, long ldv, long rs, int k, const double2* w,
-                       long wrs, long n, double2* partial, double2* out, int nblk,
-                       const int* ridx, int na);
 void launch_gemv_update_b(hipStream_t s, double2* w, long wrs, const double2* V, long ldv, long rs,
                           const int* kcnt, const double2* h, int kstride, double sign, long n,
                           const int* ridx, int na);
-void launch_norm2_b(hipStream_t s, const double2* x, long rs, long n, double* partial, double* out,
-                    int nblk, const int* ridx, int na);
 void launch_scale_b(hipStream_t s, double2* y, long yrs, const double2* x, long xrs, const double2* a,
                     long n, const int* ridx, int na);
 void launch_apply(hipStream_t s, double2* y, const double2* x, const double2* coef,
                   int Nx, int Ny, int transpose, const double2* b /*nullable: r=b-Ax*/);
 void launch_scale_copy(hipStream_t s, double2* y, const double2* x, double2 a, long n);
 void launch_zero(hipStream_t s, double2* y, long n);
-void launch_multidot(hipStream_t s, const double2* V, long ldv, int k, const double2* w,
-                     long n, double2* partial, int nblk);
-void launch_reduce_partials(hipStream_t s, const double2* partial, int nblk, int k, double2* out);
-void launch_gemv_update(hipStream_t s, double2* w, const double2* V, long ldv, int k,
-                        const double2* h, double sign, long n);
-void launch_norm2(hipStream_t s, const double2* x, long n, double* partial, int nblk);
-void launch_reduce_real(hipStream_t s, const double* partial, int nblk, double* out);
+// For na sources (ridx, rs apart; one without a list): w -= V (V^H w) twice, the
+// coefficients' sum in pin (pinned, 32 a source), the squared norm in pin_norm2;
+// h: device, 2 x 32 coefficients a source; k <= ORTH_MAXK vectors
+constexpr int ORTH_MAXK = 32;
+void launch_orth(hipStream_t s, const double2* V, long ldv, int k, double2* w, long n, long rs, const int* ridx,
+                 int na, double2* h, double2* partial, double* rpartial, int nblk, double2* pin,
+                 double* pin_norm2);
+// h = pin = V^H w
+void launch_dots(hipStream_t s, const double2* V, long ldv, int k, const double2* w, long n, double2* h,
+                 double2* partial, int nblk, double2* pin);
+void launch_combine(hipStream_t s, double2* w, const double2* V, long ldv, int k, const double2* c, long n);
+// out[y] = |x_r|^2
+void launch_norm2(hipStream_t s, const double2* x, long n, long rs, const int* ridx, int na, double* partial,
+                  int nblk, double* out);
 void launch_fields(hipStream_t s, double2* out, const double2* x, const double2* eps,
                    const double2* sxf, const double2* sxb, const double2* syf,
                    const double2* syb, const GridDesc& g, int pol, double2 w,

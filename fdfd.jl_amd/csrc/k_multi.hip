@@ -536,77 +536,6 @@ void launch_trisolve_multi(hipStream_t s, const TrsJob* jobs_d, int njobs, int n
 // Krylov building blocks over the active sources (grid row y -> source
 // ridx[y]).  Basis vector j of source r sits at V + j * ldv + r * rs.
 // ---------------------------------------------------------------------------
-constexpr int MB_MAXK = 32;
-
-// partial[y][blk][i] = sum over this block's cells of conj(V_{i,r}) w_r
-__global__ __launch_bounds__(256) void k_multidot_b(const double2* V, long ldv, long rs, int k,
-                                                    const double2* w, long wrs, long n,
-                                                    double2* partial, const int* ridx) {
-    __shared__ double2 red[4][MB_MAXK];
-    const long r = ridx[blockIdx.y];
-    const double2* Vr = V + r * rs;
-    const double2* wr = w + r * wrs;
-    double2 acc[MB_MAXK];
-#pragma unroll
-    for (int i = 0; i < MB_MAXK; ++i) acc[i] = make_double2(0, 0);
-    for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < n;
-         e += (long)gridDim.x * blockDim.x) {
-        const double2 we = wr[e];
-#pragma unroll
-        for (int i = 0; i < MB_MAXK; ++i)
-            if (i < k) acc[i] = cadd(acc[i], cconjmul(Vr[i * ldv + e], we));
-    }
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-#pragma unroll
-    for (int i = 0; i < MB_MAXK; ++i) {
-        if (i < k) {
-            double re = acc[i].x, im = acc[i].y;
-            for (int o = 32; o > 0; o >>= 1) {
-                re += __shfl_xor(re, o, 64);
-                im += __shfl_xor(im, o, 64);
-            }
-            if (lane == 0) red[wv][i] = make_double2(re, im);
-        }
-    }
-    __syncthreads();
-    if (threadIdx.x < k) {
-        double2 s = red[0][threadIdx.x];
-        for (int q = 1; q < 4; ++q) s = cadd(s, red[q][threadIdx.x]);
-        partial[((long)blockIdx.y * gridDim.x + blockIdx.x) * k + threadIdx.x] = s;
-    }
-}
-
-// out[y][i] = sum_blk partial[y][blk][i]: thread t adds column t % 32 over
-// rows t / 32 + 32 q (fixed order), then the 32 row groups in LDS
-__global__ __launch_bounds__(1024) void k_reduce_partials_b(const double2* partial, int nblk, int k,
-                                                            double2* out) {
-    __shared__ double2 acc[32][32];
-    const int y = blockIdx.x;
-    const double2* P = partial + (long)y * nblk * k;
-    const int c = threadIdx.x % 32, grp = threadIdx.x / 32;
-    for (int c0 = 0; c0 < k; c0 += 32) {
-        const int i = c0 + c;
-        double2 s = make_double2(0, 0);
-        if (i < k)
-            for (int b = grp; b < nblk; b += 32) s = cadd(s, P[b * (long)k + i]);
-        acc[grp][c] = s;
-        __syncthreads();
-        if (grp == 0 && i < k) {
-            double2 t = acc[0][c];
-            for (int g2 = 1; g2 < 32; ++g2) t = cadd(t, acc[g2][c]);
-            out[(long)y * k + i] = t;
-        }
-        __syncthreads();
-    }
-}
-
-void launch_multidot_b(hipStream_t s, const double2* V, long ldv, long rs, int k, const double2* w,
-                       long wrs, long n, double2* partial, double2* out, int nblk,
-                       const int* ridx, int na) {
-    k_multidot_b<<<dim3(nblk, na), 256, 0, s>>>(V, ldv, rs, k, w, wrs, n, partial, ridx);
-    k_reduce_partials_b<<<na, 1024, 0, s>>>(partial, nblk, k, out);
-}
-
 // w_r += sign * sum_{i < kcnt[y]} h[y][i] V_{i,r}   (h has kstride entries per source)
 __global__ void k_gemv_update_b(double2* w, long wrs, const double2* V, long ldv, long rs,
                                 const int* kcnt, const double2* h, int kstride, double sign,
@@ -632,39 +561,6 @@ void launch_gemv_update_b(hipStream_t s, double2* w, long wrs, const double2* V,
                           const int* ridx, int na) {
     const unsigned nb = (unsigned)std::max<long>(1, std::min<long>((n + 255) / 256, 2048 / na + 1));
     k_gemv_update_b<<<dim3(nb, na), 256, 0, s>>>(w, wrs, V, ldv, rs, kcnt, h, kstride, sign, n, ridx);
-}
-
-// out[y] = ||x_r||^2
-__global__ __launch_bounds__(256) void k_norm2_b(const double2* x, long rs, long n, double* partial,
-                                                 const int* ridx) {
-    __shared__ double red[4];
-    const double2* xr = x + (long)ridx[blockIdx.y] * rs;
-    double acc = 0;
-    for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < n;
-         e += (long)gridDim.x * blockDim.x)
-        acc += cnorm2(xr[e]);
-    for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
-    __syncthreads();
-    if (threadIdx.x == 0) partial[(long)blockIdx.y * gridDim.x + blockIdx.x] = red[0] + red[1] + red[2] + red[3];
-}
-__global__ __launch_bounds__(256) void k_reduce_real_b(const double* partial, int nblk, double* out) {
-    __shared__ double acc[256];
-    const double* P = partial + (long)blockIdx.x * nblk;
-    double s = 0;
-    for (int b = threadIdx.x; b < nblk; b += 256) s += P[b];
-    acc[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) acc[threadIdx.x] += acc[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[blockIdx.x] = acc[0];
-}
-void launch_norm2_b(hipStream_t s, const double2* x, long rs, long n, double* partial, double* out,
-                    int nblk, const int* ridx, int na) {
-    k_norm2_b<<<dim3(nblk, na), 256, 0, s>>>(x, rs, n, partial, ridx);
-    k_reduce_real_b<<<na, 256, 0, s>>>(partial, nblk, out);
 }
 
 // y_r = a[y] * x_r

@@ -377,106 +377,37 @@ template <> __device__ inline double wave_sum<double>(double v) {
     return v;
 }
 
-// partial[blk*k + i] = sum_{e in blk} conj(V_i[e]) w[e]   (k <= 32)
-constexpr int MD_MAXK = 32;
-__global__ __launch_bounds__(256) void k_multidot(const double2* V, long ldv, int k,
-                                                  const double2* w, long n, double2* partial) {
-    __shared__ double2 red[4][MD_MAXK];
-    double2 acc[MD_MAXK];
-    for (int i = 0; i < MD_MAXK; ++i) acc[i] = make_double2(0, 0);
-    for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < n;
-         e += (long)gridDim.x * blockDim.x) {
-        double2 we = w[e];
-#pragma unroll
-        for (int i = 0; i < MD_MAXK; ++i)
-            if (i < k) acc[i] = cadd(acc[i], cconjmul(V[i * ldv + e], we));
-    }
-    int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-#pragma unroll
-    for (int i = 0; i < MD_MAXK; ++i) {
-        if (i < k) {
-            double re = wave_sum(acc[i].x), im = wave_sum(acc[i].y);
-            if (lane == 0) red[wv][i] = make_double2(re, im);
-        }
-    }
-    __syncthreads();
-    if (threadIdx.x < k) {
-        double2 s = red[0][threadIdx.x];
-        for (int q = 1; q < 4; ++q) s = cadd(s, red[q][threadIdx.x]);
-        partial[blockIdx.x * (long)k + threadIdx.x] = s;
-    }
-}
+// sources by grid row: ridx[y] (0 without a list), rs apart
+__device__ inline long source_offset(const int* ridx, long rs) { return ridx ? ridx[blockIdx.y] * rs : 0; }
 
-void launch_multidot(hipStream_t s, const double2* V, long ldv, int k, const double2* w, long n,
-                     double2* partial, int nblk) {
-    k_multidot<<<nblk, 256, 0, s>>>(V, ldv, k, w, n, partial);
-}
-
-// Final sums of per-block partials, one workgroup of 1024 threads: thread t
-// adds column t % 32 over the rows t / 32, t / 32 + 32, ... (a fixed order, so
-// results are reproducible), then the 32 row groups of a column are added in
-// LDS.  (One thread per column walking all rows waited out one load latency
-// per row: 77 us for 512 rows.)
-constexpr int RP_COLS = 32, RP_GROUPS = 32;
-__device__ inline void reduce_columns(const double2* partial, int nblk, int k, double2* out) {
-    __shared__ double2 acc[RP_GROUPS][RP_COLS];
-    const int c = threadIdx.x % RP_COLS, grp = threadIdx.x / RP_COLS;
-    for (int c0 = 0; c0 < k; c0 += RP_COLS) {
-        const int i = c0 + c;
-        double2 s = make_double2(0, 0);
-        if (i < k)
-            for (int b = grp; b < nblk; b += RP_GROUPS) s = cadd(s, partial[b * (long)k + i]);
-        acc[grp][c] = s;
-        __syncthreads();
-        if (grp == 0 && i < k) {
-            double2 t = acc[0][c];
-            for (int g2 = 1; g2 < RP_GROUPS; ++g2) t = cadd(t, acc[g2][c]);
-            out[i] = t;
-        }
-        __syncthreads();
-    }
-}
-__global__ __launch_bounds__(1024) void k_reduce_partials(const double2* partial, int nblk, int k,
-                                                          double2* out) {
-    reduce_columns(partial, nblk, k, out);
-}
-void launch_reduce_partials(hipStream_t s, const double2* partial, int nblk, int k,
-                            double2* out) {
-    k_reduce_partials<<<1, RP_COLS * RP_GROUPS, 0, s>>>(partial, nblk, k, out);
-}
-
-// w += sign * sum_i h_i V_i
-__global__ void k_gemv_update(double2* w, const double2* V, long ldv, int k, const double2* h,
-                              double sign, long n) {
-    __shared__ double2 hs[64];
-    if (threadIdx.x < k) hs[threadIdx.x] = cscale(h[threadIdx.x], sign);
-    __syncthreads();
-    for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < n;
-         e += (long)gridDim.x * blockDim.x) {
+// w += sum_i c_i V_i, the coefficients (k <= 32) by value
+struct Coef32 {
+    double2 c[ORTH_MAXK];
+};
+__global__ __launch_bounds__(256) void k_combine(double2* w, const double2* V, long ldv, int k, Coef32 h, long n) {
+    for (long e = blockIdx.x * 256L + threadIdx.x; e < n; e += 256L * gridDim.x) {
         double2 acc = w[e];
-        for (int i = 0; i < k; ++i) acc = cadd(acc, cmul(hs[i], V[i * ldv + e]));
+#pragma unroll 4
+        for (int i = 0; i < k; ++i) acc = cadd(acc, cmul(h.c[i], V[i * ldv + e]));
         w[e] = acc;
     }
 }
-void launch_gemv_update(hipStream_t s, double2* w, const double2* V, long ldv, int k,
-                        const double2* h, double sign, long n) {
-    unsigned nb = (unsigned)std::min<long>((n + 255) / 256, 2048);
-    k_gemv_update<<<nb, 256, 0, s>>>(w, V, ldv, k, h, sign, n);
+void launch_combine(hipStream_t s, double2* w, const double2* V, long ldv, int k, const double2* c, long n) {
+    Coef32 h{};
+    for (int i = 0; i < k; ++i) h.c[i] = c[i];
+    const unsigned nb = (unsigned)std::min<long>((n + 255) / 256, 2048);
+    k_combine<<<nb, 256, 0, s>>>(w, V, ldv, k, h, n);
 }
 
-__global__ __launch_bounds__(256) void k_norm2(const double2* x, long n, double* partial) {
+__global__ __launch_bounds__(256) void k_norm2(const double2* x, long n, long rs, const int* ridx, double* partial) {
     __shared__ double red[4];
+    x += source_offset(ridx, rs);
     double acc = 0;
-    for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < n;
-         e += (long)gridDim.x * blockDim.x)
-        acc += cnorm2(x[e]);
+    for (long e = blockIdx.x * 256L + threadIdx.x; e < n; e += 256L * gridDim.x) acc += cnorm2(x[e]);
     acc = wave_sum(acc);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
     __syncthreads();
-    if (threadIdx.x == 0) partial[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
-}
-void launch_norm2(hipStream_t s, const double2* x, long n, double* partial, int nblk) {
-    k_norm2<<<nblk, 256, 0, s>>>(x, n, partial);
+    if (threadIdx.x == 0) partial[(long)blockIdx.y * gridDim.x + blockIdx.x] = red[0] + red[1] + red[2] + red[3];
 }
 // sum of nblk partials: 256 threads, fixed strided order, then a fixed tree
 __device__ inline void reduce_real(const double* partial, int nblk, double* out) {
@@ -492,10 +423,134 @@ __device__ inline void reduce_real(const double* partial, int nblk, double* out)
     if (threadIdx.x == 0) *out = acc[0];
 }
 __global__ __launch_bounds__(256) void k_reduce_real(const double* partial, int nblk, double* out) {
-    reduce_real(partial, nblk, out);
+    reduce_real(partial + (long)blockIdx.x * nblk, nblk, out + blockIdx.x);
 }
-void launch_reduce_real(hipStream_t s, const double* partial, int nblk, double* out) {
-    k_reduce_real<<<1, 256, 0, s>>>(partial, nblk, out);
+void launch_norm2(hipStream_t s, const double2* x, long n, long rs, const int* ridx, int na, double* partial,
+                  int nblk, double* out) {
+    nblk = (int)std::min<long>(nblk, (n + 255) / 256);
+    k_norm2<<<dim3(nblk, na), 256, 0, s>>>(x, n, rs, ridx, partial);
+    k_reduce_real<<<na, 256, 0, s>>>(partial, nblk, out);
+}
+
+// ---------------------------------------------------------------------------
+// Orthogonalisation of w against k <= 32 vectors, twice, with the coefficients
+// kept on the device (h1, h2) and their sum and the squared norm of the result
+// written to pinned host memory: one synchronisation in place of five, each of
+// which left the device idle for 20 to 40 us, and six launches for nine (390
+// solves and 196 Arnoldi steps on 512 x 512: 233 -> 159 ms).
+//   k_orth<false>: partial sums of h1 = V^H w
+//   k_orth<true> : w -= V h1 and the partial sums of h2 = V^H w, reading V once
+//   k_orth_norm  : w -= V h2 and the partial sums of |w|^2
+// Grid row y does this for source ridx[y] (0 without a list), rs further on in V
+// and w.  KM bounds k: small bases keep few accumulators, and many waves in
+// flight.
+// ---------------------------------------------------------------------------
+template <int KM, bool UPD>
+__global__ __launch_bounds__(256) void k_orth(const double2* V, long ldv, int k, double2* w, long n, long rs,
+                                              const int* ridx, const double2* h, double2* partial) {
+    __shared__ double2 red[4][KM];
+    const long off = source_offset(ridx, rs);
+    V += off;
+    w += off;
+    double2 acc[KM], hs[KM];
+#pragma unroll
+    for (int i = 0; i < KM; ++i) {
+        acc[i] = make_double2(0, 0);
+        hs[i] = UPD && i < k ? h[(long)blockIdx.y * 2 * ORTH_MAXK + i] : make_double2(0, 0);
+    }
+    for (long e = blockIdx.x * 256L + threadIdx.x; e < n; e += 256L * gridDim.x) {
+        double2 we = w[e], v[KM];
+#pragma unroll
+        for (int i = 0; i < KM; ++i)
+            if (i < k) v[i] = V[i * ldv + e];
+        if (UPD) {
+#pragma unroll
+            for (int i = 0; i < KM; ++i)
+                if (i < k) we = csub(we, cmul(hs[i], v[i]));
+            w[e] = we;
+        }
+#pragma unroll
+        for (int i = 0; i < KM; ++i)
+            if (i < k) acc[i] = cadd(acc[i], cconjmul(v[i], we));
+    }
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+#pragma unroll
+    for (int i = 0; i < KM; ++i) {
+        if (i < k) {
+            const double re = wave_sum(acc[i].x), im = wave_sum(acc[i].y);
+            if (lane == 0) red[wv][i] = make_double2(re, im);
+        }
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < k) {
+        double2 s = red[0][threadIdx.x];
+        for (int q = 1; q < 4; ++q) s = cadd(s, red[q][threadIdx.x]);
+        partial[((long)blockIdx.y * k + threadIdx.x) * gridDim.x + blockIdx.x] = s;
+    }
+}
+__global__ __launch_bounds__(256) void k_orth_norm(const double2* V, long ldv, int k, double2* w, long n, long rs,
+                                                   const int* ridx, const double2* h, double* partial) {
+    __shared__ double red[4];
+    const long off = source_offset(ridx, rs);
+    V += off;
+    w += off;
+    h += (long)blockIdx.y * 2 * ORTH_MAXK;
+    double acc = 0;
+    for (long e = blockIdx.x * 256L + threadIdx.x; e < n; e += 256L * gridDim.x) {
+        double2 we = w[e];
+#pragma unroll 4
+        for (int i = 0; i < k; ++i) we = csub(we, cmul(h[i], V[i * ldv + e]));
+        w[e] = we;
+        acc += cnorm2(we);
+    }
+    acc = wave_sum(acc);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0) partial[(long)blockIdx.y * gridDim.x + blockIdx.x] = red[0] + red[1] + red[2] + red[3];
+}
+// coefficient blockIdx.x of source y from its nblk partial sums: h, and in `pin`
+// its sum with `first` when there is one
+__global__ __launch_bounds__(256) void k_orth_sum(const double2* partial, int nblk, double2* h, const double2* first,
+                                                  double2* pin) {
+    __shared__ double2 red[4];
+    const int i = blockIdx.x, y = blockIdx.y, t = threadIdx.x;
+    partial += ((long)y * gridDim.x + i) * nblk;
+    double2 s = make_double2(0, 0);
+    for (int b = t; b < nblk; b += 256) s = cadd(s, partial[b]);
+    s.x = wave_sum(s.x);
+    s.y = wave_sum(s.y);
+    if ((t & 63) == 0) red[t >> 6] = s;
+    __syncthreads();
+    if (t == 0) {
+        s = cadd(cadd(red[0], red[1]), cadd(red[2], red[3]));
+        h[(long)y * 2 * ORTH_MAXK + i] = s;
+        if (pin) pin[(long)y * ORTH_MAXK + i] = first ? cadd(s, first[(long)y * 2 * ORTH_MAXK + i]) : s;
+    }
+}
+void launch_dots(hipStream_t s, const double2* V, long ldv, int k, const double2* w, long n, double2* h,
+                 double2* partial, int nblk, double2* pin) {
+    nblk = (int)std::min<long>(nblk, (n + 255) / 256);
+    k_orth<ORTH_MAXK, false><<<nblk, 256, 0, s>>>(V, ldv, k, (double2*)w, n, 0, nullptr, nullptr, partial);
+    k_orth_sum<<<k, 256, 0, s>>>(partial, nblk, h, nullptr, pin);
+}
+void launch_orth(hipStream_t s, const double2* V, long ldv, int k, double2* w, long n, long rs, const int* ridx,
+                 int na, double2* h, double2* partial, double* rpartial, int nblk, double2* pin,
+                 double* pin_norm2) {
+    nblk = (int)std::min<long>(nblk, (n + 255) / 256);
+    double2 *h1 = h, *h2 = h + ORTH_MAXK;
+    const dim3 g(nblk, na), gs(k, na);
+    auto dots = [&](auto km) {
+        constexpr int KM = decltype(km)::value;
+        k_orth<KM, false><<<g, 256, 0, s>>>(V, ldv, k, w, n, rs, ridx, nullptr, partial);
+        k_orth_sum<<<gs, 256, 0, s>>>(partial, nblk, h1, nullptr, nullptr);
+        k_orth<KM, true><<<g, 256, 0, s>>>(V, ldv, k, w, n, rs, ridx, h1, partial);
+        k_orth_sum<<<gs, 256, 0, s>>>(partial, nblk, h2, h1, pin);
+    };
+    if (k <= 2) dots(std::integral_constant<int, 2>{});
+    else if (k <= 8) dots(std::integral_constant<int, 8>{});
+    else dots(std::integral_constant<int, ORTH_MAXK>{});
+    k_orth_norm<<<g, 256, 0, s>>>(V, ldv, k, w, n, rs, ridx, h2, rpartial);
+    k_reduce_real<<<na, 256, 0, s>>>(rpartial, nblk, pin_norm2);
 }
 
 // ---------------------------------------------------------------------------

@@ -27,21 +27,20 @@ namespace {
 
 constexpr int K = GMRES_KDIM;
 constexpr int MNBLK = 256;  // reduction blocks per source
-constexpr int PIN_SLOTS = 4;
+constexpr int PIN_SLOTS = 8;  // more than the uploads between two synchronisations
 
 // per-source device scratch: ridx | kcnt | coefficients | reduced values | partials
 struct MSmall {
     int* ridx;
     int* kcnt;
     double2* coef;     // KMULTI x (K + 2)
-    double2* outc;     // KMULTI x (K + 2)
-    double* outr;      // KMULTI
+    double2* orth;     // KMULTI x 2 ORTH_MAXK
     double2* part;     // KMULTI x MNBLK x (K + 2)
     double* partr;     // KMULTI x MNBLK
 };
 size_t msmall_bytes() {
-    return sizeof(int) * 2 * KMULTI + sizeof(double2) * 2 * KMULTI * (K + 2) +
-           sizeof(double) * KMULTI + sizeof(double2) * (size_t)KMULTI * MNBLK * (K + 2) +
+    return sizeof(int) * 2 * KMULTI + sizeof(double2) * KMULTI * (K + 2 + 2 * ORTH_MAXK) +
+           sizeof(double2) * (size_t)KMULTI * MNBLK * (K + 2) +
            sizeof(double) * KMULTI * MNBLK + 1024;
 }
 MSmall msmall(void* base) {
@@ -51,8 +50,7 @@ MSmall msmall(void* base) {
     m.kcnt = (int*)p; p += sizeof(int) * KMULTI;
     p = (char*)(((uintptr_t)p + 255) & ~(uintptr_t)255);
     m.coef = (double2*)p; p += sizeof(double2) * KMULTI * (K + 2);
-    m.outc = (double2*)p; p += sizeof(double2) * KMULTI * (K + 2);
-    m.outr = (double*)p; p += sizeof(double) * KMULTI;
+    m.orth = (double2*)p; p += sizeof(double2) * KMULTI * 2 * ORTH_MAXK;
     m.part = (double2*)p; p += sizeof(double2) * (size_t)KMULTI * MNBLK * (K + 2);
     m.partr = (double*)p;
     return m;
@@ -71,12 +69,27 @@ PinSlot pin_slot(void* base, int i) {
     return s;
 }
 
+// behind the slots, what kernels leave for the host: orthogonalisation
+// coefficients, norms of the right-hand sides and of the last vectors
+struct PinOut {
+    double2* c;          // KMULTI x ORTH_MAXK
+    double *nb, *nv;     // KMULTI each
+};
+size_t pin_bytes() { return pin_slot_bytes() * PIN_SLOTS + sizeof(double2) * KMULTI * (ORTH_MAXK + 1) + 64; }
+PinOut pin_out(void* base) {
+    PinOut o;
+    o.c = (double2*)(((uintptr_t)base + pin_slot_bytes() * PIN_SLOTS + 15) & ~(uintptr_t)15);
+    o.nb = (double*)(o.c + KMULTI * ORTH_MAXK);
+    o.nv = o.nb + KMULTI;
+    return o;
+}
+
 }  // namespace
 
 int ensure_multi_work(Handle* h, long N, int k) {
     if (!h->msmall) {
         HIPCHK(h, hipMalloc(&h->msmall, msmall_bytes()));
-        HIPCHK(h, hipHostMalloc(&h->mpin, pin_slot_bytes() * PIN_SLOTS, hipHostMallocDefault));
+        HIPCHK(h, hipHostMalloc(&h->mpin, pin_bytes(), hipHostMallocDefault));
     }
     if (h->multi_N >= N && h->multi_k >= k) return FDFD_OK;
     N = std::max(N, h->multi_N);
@@ -195,13 +208,10 @@ static int gmres_multi(Handle* h, Factor* F, int nr, const double2* B, double2* 
                                      hipMemcpyHostToDevice, st));
         return FDFD_OK;
     };
-    auto norms = [&](const double2* x, long rs, int na, std::vector<double>& out) -> int {
-        launch_norm2_b(st, x, rs, N, m.partr, m.outr, MNBLK, m.ridx, na);
+    const PinOut po = pin_out(h->mpin);
+    auto host_norms = [](const double* v, int na, std::vector<double>& out) {
         out.resize(na);
-        HIPCHK(h, hipMemcpyAsync(out.data(), m.outr, sizeof(double) * na, hipMemcpyDeviceToHost, st));
-        HIPCHK(h, hipStreamSynchronize(st));
-        for (auto& v : out) v = std::sqrt(v);
-        return FDFD_OK;
+        for (int q = 0; q < na; ++q) out[q] = std::sqrt(((const volatile double*)v)[q]);
     };
     // scale source slots: y_r = a_r x_r
     auto scale = [&](double2* y, const double2* x, const std::vector<double2>& a) -> int {
@@ -222,17 +232,7 @@ static int gmres_multi(Handle* h, Factor* F, int nr, const double2* B, double2* 
     act.resize(nr);
     for (int r = 0; r < nr; ++r) act[r] = r;
     if ((rc = upload_list(act, nullptr))) return rc;
-    {
-        std::vector<double> nb;
-        if ((rc = norms(B, N, nr, nb))) return rc;
-        for (int r = 0; r < nr; ++r) bnorm[r] = nb[r];
-    }
-    for (int r = 0; r < nr; ++r)
-        if (bnorm[r] == 0) {
-            launch_zero(st, X + (long)r * N, N);
-            state[r] = 1;
-            resid[r] = 0;
-        }
+    launch_norm2(st, B, N, N, m.ridx, nr, m.partr, MNBLK, po.nb);  // arrives with the first residuals
     struct Src {
         std::vector<std::complex<double>> H, gv, sn, y;
         std::vector<double> cs;
@@ -253,16 +253,25 @@ static int gmres_multi(Handle* h, Factor* F, int nr, const double2* B, double2* 
         for (int r = 0; r < nr; ++r)
             if (state[r] == 0) act.push_back(r);
         if (act.empty()) break;
-        if ((rc = upload_list(act, nullptr))) return rc;
+        if (rs > 0 && (rc = upload_list(act, nullptr))) return rc;
         const int na = (int)act.size();
         // V_0,r = B_r - A' X_r, beta_r = ||V_0,r||
         apply(V, X, B, na);
         std::vector<double> beta;
-        if ((rc = norms(V, N, na, beta))) return rc;
+        launch_norm2(st, V, N, N, m.ridx, na, m.partr, MNBLK, po.nv);
+        HIPCHK(h, hipStreamSynchronize(st));
+        host_norms(po.nv, na, beta);
+        if (rs == 0) host_norms(po.nb, nr, bnorm);
         std::vector<int> cyc;
         std::vector<double2> inv;
         for (int q = 0; q < na; ++q) {
             const int r = act[q];
+            if (bnorm[r] == 0) {
+                launch_zero(st, X + (long)r * N, N);
+                state[r] = 1;
+                resid[r] = 0;
+                continue;
+            }
             resid[r] = beta[q] / bnorm[r];
             if (resid[r] <= tol) { state[r] = 1; continue; }
             // no restart left, or a whole cycle that gained less than 10%: the
@@ -287,47 +296,30 @@ static int gmres_multi(Handle* h, Factor* F, int nr, const double2* B, double2* 
             double2* Vj = V + (long)j * ldv;
             double2* Zj = Z + (long)j * ldv;
             double2* W = V + (long)(j + 1) * ldv;
-            // Z_j = M^-1 V_j (through the x_out slots of the reduced solve)
-            std::vector<double2> one(ni, make_double2(1.0, 0.0));
-            if ((rc = scale(h->x_out, Vj, one))) return rc;
+            // Z_j = M^-1 V_j (by lines through the x_out slots of the reduced solve)
             if (F->nd) {
-                if ((rc = rt_nd_solve(h, F, 0, h->x_out, h->x_out, N, m.ridx, ni, prof))) return rc;
+                if ((rc = rt_nd_solve(h, F, 0, Vj, Zj, N, m.ridx, ni, prof))) return rc;
             } else {
+                const std::vector<double2> one(ni, make_double2(1.0, 0.0));
+                if ((rc = scale(h->x_out, Vj, one))) return rc;
                 launch_solve_multi(h, F, N, m.ridx, ni, prof);
+                if ((rc = scale(Zj, h->x_out, one))) return rc;
             }
-            if ((rc = scale(Zj, h->x_out, one))) return rc;
             // W = A' Z_j, then CGS2 against V_0..V_j
             apply(W, Zj, nullptr, ni);
-            std::vector<std::vector<std::complex<double>>> hsum(ni, std::vector<std::complex<double>>(j + 1, 0));
-            for (int pass = 0; pass < 2; ++pass) {
-                launch_multidot_b(st, V, ldv, N, j + 1, W, N, N, m.part, m.outc, MNBLK, m.ridx, ni);
-                PinSlot s = next_slot();
-                HIPCHK(h, hipMemcpyAsync(s.c, m.outc, sizeof(double2) * ni * (j + 1),
-                                         hipMemcpyDeviceToHost, st));
-                HIPCHK(h, hipStreamSynchronize(st));
-                std::vector<int> cnt(ni, j + 1);
-                PinSlot u = next_slot();
-                for (int q = 0; q < ni; ++q)
-                    for (int i = 0; i <= j; ++i) {
-                        hsum[q][i] += std::complex<double>(s.c[q * (j + 1) + i].x, s.c[q * (j + 1) + i].y);
-                        u.c[q * (K + 2) + i] = s.c[q * (j + 1) + i];
-                    }
-                for (int q = 0; q < ni; ++q) u.ints[KMULTI + q] = j + 1;
-                HIPCHK(h, hipMemcpyAsync(m.kcnt, u.ints + KMULTI, sizeof(int) * ni, hipMemcpyHostToDevice, st));
-                HIPCHK(h, hipMemcpyAsync(m.coef, u.c, sizeof(double2) * ni * (K + 2), hipMemcpyHostToDevice, st));
-                launch_gemv_update_b(st, W, N, V, ldv, N, m.kcnt, m.coef, K + 2, -1.0, N, m.ridx, ni);
-            }
+            launch_orth(st, V, ldv, j + 1, W, N, N, m.ridx, ni, m.orth, m.part, m.partr, MNBLK, po.c, po.nv);
+            HIPCHK(h, hipStreamSynchronize(st));
             std::vector<double> hn;
-            if ((rc = norms(W, N, ni, hn))) return rc;
+            host_norms(po.nv, ni, hn);
             std::vector<double2> hinv(ni);
             for (int q = 0; q < ni; ++q) hinv[q] = make_double2(hn[q] > 0 ? 1.0 / hn[q] : 1.0, 0.0);
-            if ((rc = scale(W, W, hinv))) return rc;
             std::vector<int> still;
             for (int q = 0; q < ni; ++q) {
                 const int r = it[q];
                 Src& s = S[r];
                 auto Hij = [&](int i, int jj) -> std::complex<double>& { return s.H[(size_t)i * K + jj]; };
-                for (int i = 0; i <= j; ++i) Hij(i, j) = hsum[q][i];
+                const volatile double* hc = (const volatile double*)(po.c + q * ORTH_MAXK);
+                for (int i = 0; i <= j; ++i) Hij(i, j) = std::complex<double>(hc[2 * i], hc[2 * i + 1]);
                 Hij(j + 1, j) = hn[q];
                 for (int i = 0; i < j; ++i) {
                     const std::complex<double> a = Hij(i, j), bb = Hij(i + 1, j);
@@ -354,6 +346,7 @@ static int gmres_multi(Handle* h, Factor* F, int nr, const double2* B, double2* 
                 const double est = std::abs(s.gv[j + 1]) / bnorm[r];
                 if (!(est <= 0.5 * tol || hn[q] == 0)) still.push_back(r);
             }
+            if (!still.empty() && (rc = scale(W, W, hinv))) return rc;
             it = still;
         }
         // y = H^-1 g and X_r += Z_r y_r for every source of the cycle

@@ -107,7 +107,8 @@ int ensure_solve_work(Handle* h, long N) {
         h->nblk = 512;
         HIPCHK(h, hipMalloc(&h->dpart, sizeof(double2) * h->nblk * (KDIM + 2)));
         HIPCHK(h, hipMalloc(&h->rpart, sizeof(double) * h->nblk));
-        HIPCHK(h, hipMalloc(&h->hdev, sizeof(double2) * (KDIM + 2)));
+        HIPCHK(h, hipMalloc(&h->hdev, sizeof(double2) * 2 * (KDIM + 2)));
+        HIPCHK(h, hipHostMalloc(&h->hpin, sizeof(double2) * (KDIM + 4)));
     }
     h->work_N = N;
     h->kdim = KDIM;
@@ -312,41 +313,62 @@ void rt_apply(Handle* h, const Factor* F, double2* y, const double2* x, int tran
 // ---------------------------------------------------------------------------
 // FP64 Krylov building blocks
 // ---------------------------------------------------------------------------
+// |x|^2 into scalar i of the pinned buffer, without waiting
+static volatile double* start_norm(Handle* h, const double2* x, long N, int i) {
+    double* out = (double*)h->hpin + i;
+    launch_norm2(h->stream, x, N, 0, nullptr, 1, h->rpart, h->nblk, out);
+    return out;
+}
 static int dev_norm(Handle* h, const double2* x, long N, double* out) {
-    launch_norm2(h->stream, x, N, h->rpart, h->nblk);
-    launch_reduce_real(h->stream, h->rpart, h->nblk, (double*)h->hdev);
-    double v = 0;
-    HIPCHK(h, hipMemcpyAsync(&v, h->hdev, sizeof(double), hipMemcpyDeviceToHost, h->stream));
+    volatile double* v = start_norm(h, x, N, 0);
     HIPCHK(h, hipStreamSynchronize(h->stream));
-    *out = std::sqrt(v);
+    *out = std::sqrt(*v);
     return FDFD_OK;
 }
 
 // h[0..k-1] = V[0..k-1]^H w
-// (in chunks of at most 32 vectors, the multidot kernel's register budget)
+// (in chunks of at most 32 vectors, the kernel's register budget)
 static int dev_multidot(Handle* h, const double2* V, long N, int k, const double2* w, cd* out) {
     for (int c0 = 0; c0 < k; c0 += 32) {
         const int kc = std::min(32, k - c0);
-        launch_multidot(h->stream, V + (long)c0 * N, N, kc, w, N, h->dpart, h->nblk);
-        launch_reduce_partials(h->stream, h->dpart, h->nblk, kc, h->hdev);
-        HIPCHK(h, hipMemcpyAsync(out + c0, h->hdev, sizeof(double2) * kc, hipMemcpyDeviceToHost,
-                                 h->stream));
+        launch_dots(h->stream, V + (long)c0 * N, N, kc, w, N, h->hdev, h->dpart, h->nblk, h->hpin);
         HIPCHK(h, hipStreamSynchronize(h->stream));
+        const volatile double* v = (const volatile double*)h->hpin;
+        for (int i = 0; i < kc; ++i) out[c0 + i] = cd(v[2 * i], v[2 * i + 1]);
     }
     return FDFD_OK;
 }
 
-// w += sign * V[0..k-1] c   (in chunks of at most 32 vectors)
-static int dev_update(Handle* h, double2* w, const double2* V, long N, int k, const cd* c,
-                      double sign) {
-    for (int c0 = 0; c0 < k; c0 += 32) {
-        const int kc = std::min(32, k - c0);
-        HIPCHK(h, hipMemcpyAsync(h->hdev, c + c0, sizeof(double2) * kc, hipMemcpyHostToDevice,
-                                 h->stream));
-        launch_gemv_update(h->stream, w, V + (long)c0 * N, N, kc, h->hdev, sign, N);
-        HIPCHK(h, hipStreamSynchronize(h->stream));  // c lives in host memory
+// w += V[0..k-1] c   (in chunks of at most 32 vectors)
+static void dev_update(Handle* h, double2* w, const double2* V, long N, int k, const cd* c) {
+    for (int c0 = 0; c0 < k; c0 += 32)
+        launch_combine(h->stream, w, V + (long)c0 * N, N, std::min(32, k - c0), (const double2*)(c + c0), N);
+}
+
+// w orthogonalised against V[0..k-1] by two passes of classical Gram-Schmidt:
+// c = their coefficients, norm = |w| after
+static int dev_orth(Handle* h, const double2* V, long N, int k, double2* w, cd* c, double* norm) {
+    if (k <= 32) {
+        launch_orth(h->stream, V, N, k, w, N, 0, nullptr, 1, h->hdev, h->dpart, h->rpart, h->nblk, h->hpin,
+                    (double*)(h->hpin + 32));
+        HIPCHK(h, hipStreamSynchronize(h->stream));
+        const volatile double* v = (const volatile double*)h->hpin;
+        for (int i = 0; i < k; ++i) c[i] = cd(v[2 * i], v[2 * i + 1]);
+        *norm = std::sqrt(v[64]);
+        return FDFD_OK;
     }
-    return FDFD_OK;
+    std::vector<cd> d(k);
+    std::fill(c, c + k, cd(0));
+    for (int pass = 0; pass < 2; ++pass) {
+        int rc = dev_multidot(h, V, N, k, w, d.data());
+        if (rc) return rc;
+        for (int i = 0; i < k; ++i) {
+            c[i] += d[i];
+            d[i] = -d[i];
+        }
+        dev_update(h, w, V, N, k, d.data());
+    }
+    return dev_norm(h, w, N, norm);
 }
 
 struct SolveStats { int iters = 0, restarts = 0; double resid = 0; };
@@ -366,19 +388,20 @@ int rt_gmres_op(Handle* h, long N,
         K = std::min(std::max(h->inject_arg, 0), GMRES_KDIM);
         max_restarts = K > 0 ? 1 : 0;
     }
-    if ((rc = dev_norm(h, b, N, &bnorm))) return rc;
-    if (bnorm == 0) {
-        launch_zero(h->stream, x, N);
-        *resid_out = 0;
-        return FDFD_OK;
-    }
-    std::vector<cd> H((size_t)(K + 1) * K), gv(K + 1), sn(K), hc(K + 1), hc2(K + 1), y(K);
+    volatile double* bn2 = start_norm(h, b, N, 1);  // arrives with the first residual
+    std::vector<cd> H((size_t)(K + 1) * K), gv(K + 1), sn(K), hc(K + 1), y(K);
     std::vector<double> cs(K);
     double resid = 1, prev = 2;
     for (int rs = 0; rs <= max_restarts; ++rs) {
         if ((rc = apply(x, V, b))) return rc;
         double beta;
         if ((rc = dev_norm(h, V, N, &beta))) return rc;
+        if (rs == 0) bnorm = std::sqrt(*bn2);
+        if (bnorm == 0) {
+            launch_zero(h->stream, x, N);
+            *resid_out = 0;
+            return FDFD_OK;
+        }
         resid = beta / bnorm;
         *resid_out = resid;
         if (resid <= tol) return FDFD_OK;
@@ -398,16 +421,10 @@ int rt_gmres_op(Handle* h, long N,
             double2* w = V + (long)(j + 1) * N;
             if ((rc = prec(vj, zj))) return rc;
             if ((rc = apply(zj, w, nullptr))) return rc;
-            // CGS2
-            if ((rc = dev_multidot(h, V, N, j + 1, w, hc.data()))) return rc;
-            if ((rc = dev_update(h, w, V, N, j + 1, hc.data(), -1.0))) return rc;
-            if ((rc = dev_multidot(h, V, N, j + 1, w, hc2.data()))) return rc;
-            if ((rc = dev_update(h, w, V, N, j + 1, hc2.data(), -1.0))) return rc;
-            for (int i = 0; i <= j; ++i) H[(size_t)i * K + j] = hc[i] + hc2[i];
             double hn;
-            if ((rc = dev_norm(h, w, N, &hn))) return rc;
+            if ((rc = dev_orth(h, V, N, j + 1, w, hc.data(), &hn))) return rc;
+            for (int i = 0; i <= j; ++i) H[(size_t)i * K + j] = hc[i];
             H[(size_t)(j + 1) * K + j] = hn;
-            if (hn > 0) launch_scale_copy(h->stream, w, w, make_double2(1.0 / hn, 0), N);
             // Givens
             for (int i = 0; i < j; ++i) {
                 cd a = H[(size_t)i * K + j], bb = H[(size_t)(i + 1) * K + j];
@@ -433,6 +450,7 @@ int rt_gmres_op(Handle* h, long N,
             jdone = j + 1;
             double est = std::abs(gv[j + 1]) / bnorm;
             if (est <= 0.5 * tol || hn == 0) break;
+            launch_scale_copy(h->stream, w, w, make_double2(1.0 / hn, 0), N);
         }
         // y = H^-1 g, x += Z y
         for (int i = jdone - 1; i >= 0; --i) {
@@ -440,7 +458,7 @@ int rt_gmres_op(Handle* h, long N,
             for (int l = i + 1; l < jdone; ++l) s -= H[(size_t)i * K + l] * y[l];
             y[i] = s / H[(size_t)i * K + i];
         }
-        if ((rc = dev_update(h, x, Zk, N, jdone, y.data(), 1.0))) return rc;
+        dev_update(h, x, Zk, N, jdone, y.data());
     }
     *resid_out = resid;
     char buf[160];
@@ -568,6 +586,7 @@ int fdfd_destroy(fdfd_handle* hh) {
                     h->dpart, h->rpart, h->hdev, h->bslab, h->io, h->nd_scratch, h->nd_vec};
     for (void* b : bufs) dfree(b);
     if (h->tstage) (void)hipHostFree(h->tstage);
+    if (h->hpin) (void)hipHostFree(h->hpin);
     if (h->tstage_ev) (void)hipEventDestroy(h->tstage_ev);
     prof_resolve(h->prof);
     for (auto e : h->prof.pool) (void)hipEventDestroy(e);
@@ -1009,10 +1028,8 @@ int rt_gmres(Handle* h, Factor* F, int trans, const double2* b, double2* x, doub
 }
 void rt_free_factor(Handle* h, Factor* F) { free_factor(h, F); }
 int rt_norm(Handle* h, const double2* x, long N, double* out) { return dev_norm(h, x, N, out); }
-int rt_multidot(Handle* h, const double2* V, long N, int k, const double2* w, cd* out) {
-    return dev_multidot(h, V, N, k, w, out);
+int rt_orth(Handle* h, const double2* V, long N, int k, double2* w, cd* c, double* norm) {
+    return dev_orth(h, V, N, k, w, c, norm);
 }
-int rt_update(Handle* h, double2* w, const double2* V, long N, int k, const cd* c, double sign) {
-    return dev_update(h, w, V, N, k, c, sign);
-}
+void rt_update(Handle* h, double2* w, const double2* V, long N, int k, const cd* c) { dev_update(h, w, V, N, k, c); }
 }  // namespace fdfd

@@ -128,6 +128,7 @@ struct Handle {
     double2* dpart = nullptr;   // multidot partials
     double* rpart = nullptr;    // norm partials
     double2* hdev = nullptr;    // small device vector of coefficients
+    double2* hpin = nullptr;    // pinned: scalars that kernels leave for the host
     int nblk = 0;
     Prof prof;
     // released factor arenas kept for reuse (at most ARENA_POOL), freed by
