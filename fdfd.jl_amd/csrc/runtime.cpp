@@ -777,6 +777,17 @@ int fdfd_solve_d(fdfd_handle* hh, int factor_id, int nrhs, const void* d_src, vo
     return FDFD_OK;
 }
 
+// the handle's staging buffer, grown, not reallocated per call
+static int ensure_io(Handle* h, size_t need) {
+    if (h->io_bytes >= need) return FDFD_OK;
+    dfree(h->io);
+    h->io = nullptr;
+    h->io_bytes = 0;
+    HIPCHK(h, hipMalloc(&h->io, need));
+    h->io_bytes = need;
+    return FDFD_OK;
+}
+
 int fdfd_solve(fdfd_handle* hh, int factor_id, int nrhs, const fdfd_complex* src,
                fdfd_complex* out, double tol, fdfd_stats* stats) {
     Handle* h = H(hh);
@@ -784,19 +795,12 @@ int fdfd_solve(fdfd_handle* hh, int factor_id, int nrhs, const fdfd_complex* src
     if (!find_factor(h, factor_id)) return fail(h, FDFD_ERR_NOTFOUND, "unknown factor id");
     (void)hipSetDevice(h->device);
     const long N = (long)h->g.Nx * h->g.Ny;
-    // device staging: sources then fields, in the handle's buffer (grown, not
-    // reallocated per call)
-    const size_t need = sizeof(double2) * N * 4 * (size_t)nrhs;
-    if (h->io_bytes < need) {
-        dfree(h->io);
-        h->io = nullptr;
-        h->io_bytes = 0;
-        HIPCHK(h, hipMalloc(&h->io, need));
-        h->io_bytes = need;
-    }
+    // device staging: sources then fields
+    int rc = ensure_io(h, sizeof(double2) * N * 4 * (size_t)nrhs);
+    if (rc) return rc;
     double2* ds = (double2*)h->io;
     double2* dout = ds + N * nrhs;
-    int rc = stream_copy(h, ds, src, sizeof(double2) * N * nrhs, hipMemcpyHostToDevice);
+    rc = stream_copy(h, ds, src, sizeof(double2) * N * nrhs, hipMemcpyHostToDevice);
     if (!rc) rc = fdfd_solve_d(hh, factor_id, nrhs, ds, dout, tol, stats);
     if (!rc) rc = stream_copy(h, out, dout, sizeof(double2) * N * 3 * nrhs, hipMemcpyDeviceToHost);
     return rc;
@@ -950,16 +954,16 @@ int fdfd_solve_pullback(fdfd_handle* hh, int factor_id, const fdfd_complex* ez,
     if (!find_factor(h, factor_id)) return fail(h, FDFD_ERR_NOTFOUND, "unknown factor id");
     (void)hipSetDevice(h->device);
     const long N = (long)h->g.Nx * h->g.Ny;
-    void* buf = nullptr;  // ez | dfields (3N) | grad
-    HIPCHK(h, hipMalloc(&buf, sizeof(double2) * 4 * N + sizeof(double) * N));
-    double2* dez = (double2*)buf;
+    // ez | dfields (3N) | grad, in the handle's staging buffer
+    int rc = ensure_io(h, sizeof(double2) * 4 * N + sizeof(double) * N);
+    if (rc) return rc;
+    double2* dez = (double2*)h->io;
     double2* ddf = dez + N;
     double* dg = (double*)(ddf + 3 * N);
-    int rc = stream_copy(h, dez, ez, sizeof(double2) * N, hipMemcpyHostToDevice);
+    rc = stream_copy(h, dez, ez, sizeof(double2) * N, hipMemcpyHostToDevice);
     if (!rc) rc = stream_copy(h, ddf, dfields, sizeof(double2) * 3 * N, hipMemcpyHostToDevice);
     if (!rc) rc = fdfd_solve_pullback_d(hh, factor_id, dez, ddf, tol, dg, stats);
     if (!rc) rc = stream_copy(h, grad, dg, sizeof(double) * N, hipMemcpyDeviceToHost);
-    dfree(buf);
     return rc;
 }
 

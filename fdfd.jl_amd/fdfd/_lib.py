@@ -64,6 +64,7 @@ _PS = C.POINTER(fdfd_stats)
 # name -> (restype, argtypes)
 PROTOTYPES = {
     "fdfd_version": (_I, [_PI, _PI, _PI]),
+    "fdfd_pack": (_I, [_P, C.c_longlong, C.c_longlong, C.c_longlong, _I, _I, _I, _P]),
     "fdfd_last_error": (C.c_char_p, [_P]),
     "fdfd_arch": (C.c_char_p, []),
     "fdfd_create": (_I, [_I, C.POINTER(_P)]),

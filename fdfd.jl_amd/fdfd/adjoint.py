@@ -27,7 +27,7 @@ import numpy as np
 
 from . import _lib
 from .core import TM, Device, FieldTM
-from .solve import _flat, _ptr, engine
+from .solve import _flat, _pack, _ptr, engine
 
 
 def _field_cotangent(df, shape) -> np.ndarray:
@@ -36,12 +36,12 @@ def _field_cotangent(df, shape) -> np.ndarray:
     Nx, Ny = shape
     df = np.asarray(df, dtype=np.complex128)
     if df.shape == (Nx, Ny):
-        full = np.zeros((Nx, Ny, 3), dtype=np.complex128)
-        full[:, :, 0] = df
-        df = full
+        full = np.zeros((3, Nx * Ny), dtype=np.complex128)
+        full[0] = _flat(df)
+        return full.reshape(-1)
     if df.shape != (Nx, Ny, 3):
         raise ValueError(f"field cotangent must be {Nx}x{Ny}x3 or {Nx}x{Ny}, got {df.shape}")
-    return np.ascontiguousarray(df.transpose(2, 1, 0)).ravel()
+    return _pack(df).reshape(-1)
 
 
 class _Pullback:
@@ -129,10 +129,13 @@ def objective_and_gradient(d: Device, m: np.ndarray, precision="fp64", tol: floa
     mode-overlap objective of an inverse-design step.  m: Nx x Ny weights."""
     f, pb = solve_rrule(d, TM, precision, tol, eng)
     try:
-        ez = f.data[:, :, 0]
-        s = np.sum(np.asarray(m) * ez)
+        if np.shape(m) != tuple(d.grid.N):
+            raise ValueError(f"m must be {d.grid.N[0]}x{d.grid.N[1]}, got {np.shape(m)}")
+        # both in the solver's order: no strided passes
+        mf = _flat(m)
+        s = np.dot(mf, _flat(f.data[:, :, 0]))
         # dJ/dRe ez + i dJ/dIm ez = 2 s conj(m)
-        grad = pb(2 * s * np.conj(m))
+        grad = pb((2 * s * np.conj(mf)).reshape(d.grid.N, order="F"))
     finally:
         pb.release()
     return float(abs(s) ** 2), grad, f

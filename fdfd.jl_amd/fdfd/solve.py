@@ -24,9 +24,27 @@ PRECISIONS = {"fp64": FDFD_FP64, "mixed": FDFD_FP32_IR, "fp32": FDFD_FP32_IR,
               FDFD_FP64: FDFD_FP64, FDFD_FP32_IR: FDFD_FP32_IR}
 
 
+def _pack(a: np.ndarray) -> np.ndarray:
+    """Nx x Ny x n in any order -> contiguous complex128 [n, Ny, Nx]."""
+    a = np.asarray(a, dtype=np.complex128)
+    if a.ndim != 3:  # further axes of length 1
+        return np.stack([a[:, :, r].ravel(order="F") for r in range(a.shape[2])])
+    # numpy's own transposition is as good for small arrays and arrays in order
+    if a.size < 4096 or a.flags.f_contiguous or not a.flags.aligned or any(s % 16 for s in a.strides):
+        return np.ascontiguousarray(a.transpose(2, 1, 0))
+    out = np.empty(a.shape[::-1], dtype=np.complex128)
+    sx, sy, sr = (s // 16 for s in a.strides)
+    if _lib.load().fdfd_pack(_ptr(a), sx, sy, sr, a.shape[0], a.shape[1], a.shape[2], _ptr(out)) != 0:
+        raise ValueError("fdfd_pack refused the array")
+    return out
+
+
 def _flat(a: np.ndarray) -> np.ndarray:
     """Nx x Ny (x fastest) -> contiguous complex128 vector."""
-    return np.ascontiguousarray(np.asarray(a, dtype=np.complex128).ravel(order="F"))
+    a = np.asarray(a, dtype=np.complex128)
+    if a.ndim != 2:
+        return np.ascontiguousarray(a.ravel(order="F"))
+    return _pack(a[:, :, None]).reshape(-1)
 
 
 def _ptr(a: np.ndarray):
@@ -88,7 +106,7 @@ class Engine:
         if srcs.ndim == 2:
             srcs = srcs[:, :, None]
         nrhs = srcs.shape[2]
-        s = np.ascontiguousarray(np.stack([_flat(srcs[:, :, r]) for r in range(nrhs)]))
+        s = _pack(srcs)
         out = np.empty((nrhs, 3, len(g)), dtype=np.complex128)
         st = fdfd_stats()
         self._chk(self.lib.fdfd_solve(self.h, fid, nrhs, _ptr(s), _ptr(out), tol, C.byref(st)))
@@ -158,8 +176,7 @@ class Engine:
                 srcs = np.asarray(srcs, dtype=np.complex128)
                 if srcs.ndim == 2:
                     srcs = srcs[:, :, None]
-                ss = np.ascontiguousarray(np.stack([_flat(srcs[:, :, r])
-                                                    for r in range(srcs.shape[2])]))
+                ss = _pack(srcs)
                 jid = C.c_int()
                 self._chk(self.lib.fdfd_batch_add(
                     b, g.N[0], g.N[1], g.dx, g.dy, g.Npml[0], g.Npml[1], g.L0, int(pol),

@@ -108,6 +108,12 @@ int fdfd_destroy(fdfd_handle* h);
 int fdfd_set_grid(fdfd_handle* h, int Nx, int Ny, double dx, double dy,
                   int npml_x, int npml_y, double L0);
 
+/* Host arrays into this layout: dst[(r Ny + y) Nx + x] =
+ * src[x sx + y sy + r sr], strides in complex values (r < nr: sources).
+ * Needs no handle. */
+int fdfd_pack(const fdfd_complex* src, long long sx, long long sy, long long sr, int Nx, int Ny,
+              int nr, fdfd_complex* dst);
+
 /* Relative permittivity Device.eps_r (src/device.jl:21), Nx*Ny complex. */
 int fdfd_set_eps(fdfd_handle* h, const fdfd_complex* eps);
 int fdfd_set_eps_d(fdfd_handle* h, const void* d_eps);
