@@ -17,7 +17,7 @@
 using namespace fdfd;
 
 namespace {
-constexpr int MODE_MAX_N = 16384;  // longest slice (one lane runs the O(n) solves)
+constexpr int MODE_MAX_N = 16384;  // longest slice (one wave runs the O(n) solves)
 }
 
 extern "C" int fdfd_eigenmode(fdfd_handle* hh, int nprob, const fdfd_mode_problem* probs,
@@ -52,35 +52,32 @@ extern "C" int fdfd_eigenmode(fdfd_handle* hh, int nprob, const fdfd_mode_proble
     }
     (void)hipSetDevice(h->device);
     const size_t ntot = off[nprob];
-    // one device buffer: eps | V | W | vec | beta (double2), tri work (double), info (int)
+    // one device buffer: jobs | eps, written by one copy, V | W | tri work, and
+    // vec | beta | info, read by one
     size_t nV = 0, nW = 0, nT = 0;
     for (int p = 0; p < nprob; ++p) {
         nV += (size_t)(mp[p] + 1) * probs[p].n;
         nW += (size_t)mp[p] * probs[p].n;
         nT += (size_t)tri::work_doubles(probs[p].n);
     }
-    const size_t n2 = ntot + nV + nW + ntot * nev + (size_t)nprob * nev;
-    const size_t bytes = n2 * sizeof(double2) + nT * sizeof(double) + (size_t)nprob * 4 * sizeof(int) +
-                         (size_t)nprob * sizeof(ModeJob) + alignof(ModeJob);
-    char* buf = nullptr;
-    if (hipMalloc(&buf, bytes) != hipSuccess) return fail(h, FDFD_ERR_OOM, "mode workspace allocation failed");
-    struct Free {
-        char* p;
-        ~Free() { (void)hipFree(p); }
-    } guard{buf};
-    double2* d_eps = (double2*)buf;
+    static_assert(alignof(ModeJob) <= 16, "the job table starts the buffer");
+    const size_t bjobs = ((size_t)nprob * sizeof(ModeJob) + 15) & ~(size_t)15, bin = bjobs + ntot * sizeof(double2);
+    const size_t bout = (ntot * nev + (size_t)nprob * nev) * sizeof(double2) + (size_t)nprob * 4 * sizeof(int);
+    const size_t bytes = bin + (nV + nW) * sizeof(double2) + nT * sizeof(double) + 16 + bout;
+    int rc = rt_ensure_io(h, bytes);
+    if (rc) return rc;
+    char* buf = (char*)h->io;
+    ModeJob* d_jobs = (ModeJob*)buf;
+    double2* d_eps = (double2*)(buf + bjobs);
     double2* d_V = d_eps + ntot;
     double2* d_W = d_V + nV;
-    double2* d_vec = d_W + nW;
+    double* d_trw = (double*)(d_W + nW);
+    double2* d_vec = (double2*)(d_trw + ((nT + 1) & ~(size_t)1));
     double2* d_beta = d_vec + ntot * nev;
-    double* d_trw = (double*)(d_beta + (size_t)nprob * nev);
-    int* d_info = (int*)(d_trw + nT);
-    ModeJob* d_jobs = (ModeJob*)(d_info + (size_t)nprob * 4);
-    // ModeJob holds doubles: keep the table 8-byte aligned
-    if (((uintptr_t)d_jobs) % alignof(ModeJob) != 0)
-        d_jobs = (ModeJob*)(((uintptr_t)d_jobs + alignof(ModeJob) - 1) & ~(uintptr_t)(alignof(ModeJob) - 1));
-    std::vector<double2> heps(ntot);
-    std::vector<ModeJob> jobs(nprob);
+    int* d_info = (int*)(d_beta + (size_t)nprob * nev);
+    std::vector<char> hin(bin);
+    ModeJob* jobs = (ModeJob*)hin.data();
+    double2* heps = (double2*)(hin.data() + bjobs);
     size_t oV = 0, oW = 0, oT = 0;
     for (int p = 0; p < nprob; ++p) {
         const fdfd_mode_problem& P = probs[p];
@@ -106,8 +103,7 @@ extern "C" int fdfd_eigenmode(fdfd_handle* hh, int nprob, const fdfd_mode_proble
         oW += (size_t)mp[p] * P.n;
         oT += (size_t)tri::work_doubles(P.n);
     }
-    COPY(h, d_eps, heps.data(), ntot * sizeof(double2), hipMemcpyHostToDevice);
-    COPY(h, d_jobs, jobs.data(), nprob * sizeof(ModeJob), hipMemcpyHostToDevice);
+    COPY(h, buf, hin.data(), bin, hipMemcpyHostToDevice);
     hipEvent_t e0, e1;
     HIPCHK(h, hipEventCreate(&e0));
     HIPCHK(h, hipEventCreate(&e1));
@@ -120,18 +116,19 @@ extern "C" int fdfd_eigenmode(fdfd_handle* hh, int nprob, const fdfd_mode_proble
         (void)hipEventDestroy(e1);
         return fail(h, FDFD_ERR_HIP, std::string("k_mode launch: ") + hipGetErrorString(le));
     }
-    std::vector<int> info((size_t)nprob * 4);
-    std::vector<double2> hb((size_t)nprob * nev);
-    int rc = stream_copy(h, info.data(), d_info, info.size() * sizeof(int), hipMemcpyDeviceToHost);
-    if (!rc) rc = stream_copy(h, hb.data(), d_beta, hb.size() * sizeof(double2), hipMemcpyDeviceToHost);
-    if (!rc && vectors)
-        rc = stream_copy(h, vectors, d_vec, ntot * nev * sizeof(double2), hipMemcpyDeviceToHost);
+    // (the vectors lead the block: without them the copy starts at beta)
+    const size_t skip = vectors ? 0 : ntot * nev * sizeof(double2);
+    std::vector<char> hout(bout);
+    rc = stream_copy(h, hout.data() + skip, (char*)d_vec + skip, bout - skip, hipMemcpyDeviceToHost);
+    const double2* hb = (const double2*)hout.data() + ntot * nev;
+    const int* info = (const int*)(hb + (size_t)nprob * nev);
     float ms = 0;
     (void)hipEventElapsedTime(&ms, e0, e1);
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     if (rc) return rc;
-    for (size_t i = 0; i < hb.size(); ++i) {
+    if (vectors) std::memcpy(vectors, hout.data(), ntot * nev * sizeof(double2));
+    for (size_t i = 0; i < (size_t)nprob * nev; ++i) {
         beta[i].re = hb[i].x;
         beta[i].im = hb[i].y;
     }

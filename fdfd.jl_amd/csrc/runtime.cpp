@@ -89,6 +89,17 @@ int ensure_factor_work(Handle* h, int n, int nch) {
 
 static const int KDIM = GMRES_KDIM;
 
+// the handle's staging buffer, grown, not reallocated per call
+int rt_ensure_io(Handle* h, size_t need) {
+    if (h->io_bytes >= need) return FDFD_OK;
+    dfree(h->io);
+    h->io = nullptr;
+    h->io_bytes = 0;
+    HIPCHK(h, hipMalloc(&h->io, need));
+    h->io_bytes = need;
+    return FDFD_OK;
+}
+
 int ensure_solve_work(Handle* h, long N) {
     if (h->work_N >= N) return FDFD_OK;
     void** bufs[] = {(void**)&h->g_mid, (void**)&h->x_out, (void**)&h->V,
@@ -777,17 +788,6 @@ int fdfd_solve_d(fdfd_handle* hh, int factor_id, int nrhs, const void* d_src, vo
     return FDFD_OK;
 }
 
-// the handle's staging buffer, grown, not reallocated per call
-static int ensure_io(Handle* h, size_t need) {
-    if (h->io_bytes >= need) return FDFD_OK;
-    dfree(h->io);
-    h->io = nullptr;
-    h->io_bytes = 0;
-    HIPCHK(h, hipMalloc(&h->io, need));
-    h->io_bytes = need;
-    return FDFD_OK;
-}
-
 int fdfd_solve(fdfd_handle* hh, int factor_id, int nrhs, const fdfd_complex* src,
                fdfd_complex* out, double tol, fdfd_stats* stats) {
     Handle* h = H(hh);
@@ -796,7 +796,7 @@ int fdfd_solve(fdfd_handle* hh, int factor_id, int nrhs, const fdfd_complex* src
     (void)hipSetDevice(h->device);
     const long N = (long)h->g.Nx * h->g.Ny;
     // device staging: sources then fields
-    int rc = ensure_io(h, sizeof(double2) * N * 4 * (size_t)nrhs);
+    int rc = rt_ensure_io(h, sizeof(double2) * N * 4 * (size_t)nrhs);
     if (rc) return rc;
     double2* ds = (double2*)h->io;
     double2* dout = ds + N * nrhs;
@@ -955,7 +955,7 @@ int fdfd_solve_pullback(fdfd_handle* hh, int factor_id, const fdfd_complex* ez,
     (void)hipSetDevice(h->device);
     const long N = (long)h->g.Nx * h->g.Ny;
     // ez | dfields (3N) | grad, in the handle's staging buffer
-    int rc = ensure_io(h, sizeof(double2) * 4 * N + sizeof(double) * N);
+    int rc = rt_ensure_io(h, sizeof(double2) * 4 * N + sizeof(double) * N);
     if (rc) return rc;
     double2* dez = (double2*)h->io;
     double2* ddf = dez + N;

@@ -190,6 +190,7 @@ int fail(Handle* h, int code, const std::string& msg);
 // streams are non-blocking, so a plain hipMemcpy (null stream) would not wait
 // for kernels still queued on them; every host<->device transfer of the
 // library goes through here instead.
+int rt_ensure_io(Handle* h, size_t need);
 int stream_copy(Handle* h, void* dst, const void* src, size_t bytes, hipMemcpyKind kind);
 
 

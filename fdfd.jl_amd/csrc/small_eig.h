@@ -1,8 +1,7 @@
 // Small dense complex eigensolver (host/device, FP64), used for the
-// projected matrices of the Arnoldi drivers: the 2-D eigenfrequency driver
-// on the host (eigen.cpp) and the batched 1-D mode kernel on the device
-// (k_mode.hip).  Storage is supplied by the caller, so the device version
-// can run on LDS-resident arrays.
+// projected matrix of the 2-D eigenfrequency driver (eigen.cpp).  The batched 1-D
+// mode kernel runs the same algorithm on a wave (wave_eig, k_mode.hip) with the
+// complex helpers below.  Storage is supplied by the caller.
 //
 // A = Q T Q^H: Householder reduction to Hessenberg form, then implicit
 // single-shift QR with Wilkinson shifts (exceptional shift every 11th
