@@ -444,19 +444,13 @@ int fdfd_batch_run(fdfd_batch* b, int precision, double tol, fdfd_stats* stats) 
                 // lockstep FGMRES on the factor
                 for (int s0 = 0; s0 < job.nsrc && rc == FDFD_OK; s0 += KMULTI) {
                     const int ns = std::min(KMULTI, job.nsrc - s0);
-                    for (int k = 0; k < ns; ++k) {
-                        // b' = scale * (i omega) * src   (driven.jl:36,46)
-                        launch_scale_copy(h->stream, h->mB + (long)k * N, dsrc + (long)(s0 + k) * N,
-                                          make_double2(0.0, F->scale * F->omega), N);
-                        launch_zero(h->stream, h->mX + (long)k * N, N);
-                    }
+                    // b' = scale * (i omega) * src   (driven.jl:36,46)
+                    launch_scale_copy(h->stream, h->mB, dsrc + (long)s0 * N,
+                                      make_double2(0.0, F->scale * F->omega), N * ns);
                     rc = rt_gmres_multi(h, F, ns, h->mB, h->mX, tol, &iters, &worst);
                     if (rc) break;
-                    for (int k = 0; k < ns; ++k) {
-                        double2* out = job.result + ((long)(G.o0 + q) * job.nsrc + s0 + k) * 3 * N;
-                        launch_fields(h->stream, out, h->mX + (long)k * N, h->eps, F->sxf, F->sxb,
-                                      F->syf, F->syb, g, F->pol, w, 0);
-                    }
+                    launch_fields(h->stream, job.result + ((long)(G.o0 + q) * job.nsrc + s0) * 3 * N, h->mX, h->eps,
+                                  F->sxf, F->sxb, F->syf, F->syb, g, F->pol, w, 0, ns);
                 }
             }
             (void)hipEventRecord(e1, h->stream);

@@ -80,7 +80,6 @@ extern "C" int fdfd_eigenfrequency(fdfd_handle* hh, int pol, double omega0, int 
     auto op = [&](const double2* x, double2* y) -> int {
         if (pol == FDFD_TM) launch_mul_eps(h->stream, h->tmp, x, h->eps, make_double2(opscale, 0), N);
         else launch_scale_copy(h->stream, h->tmp, x, make_double2(opscale, 0), N);
-        launch_zero(h->stream, y, N);
         double res = 0;
         int r = rt_gmres(h, F, 0, h->tmp, y, inner_tol, &iters, &res);
         if (r == FDFD_ERR_NOCONV && res <= 1e-8) r = FDFD_OK;

@@ -295,9 +295,9 @@ void launch_diag_multi(hipStream_t s, const DiagJob* jobs_d, int njobs, int n, l
 int trisolve_multi_prepare(int n);
 void launch_trisolve_multi(hipStream_t s, const TrsJob* jobs_d, int njobs, int n, long rs,
                            const int* ridx, int na);
-void launch_gemv_update_b(hipStream_t s, double2* w, long wrs, const double2* V, long ldv, long rs,
-                          const int* kcnt, const double2* h, int kstride, double sign, long n,
-                          const int* ridx, int na);
+void launch_combine_b(hipStream_t s, double2* w, long wrs, const double2* V, long ldv, long rs,
+                      const int* kcnt, const double2* h, int kstride, long n, const int* ridx, int na,
+                      bool add);
 void launch_scale_b(hipStream_t s, double2* y, long yrs, const double2* x, long xrs, const double2* a,
                     long n, const int* ridx, int na);
 void launch_apply(hipStream_t s, double2* y, const double2* x, const double2* coef,
@@ -314,14 +314,18 @@ void launch_orth(hipStream_t s, const double2* V, long ldv, int k, double2* w, l
 // h = pin = V^H w
 void launch_dots(hipStream_t s, const double2* V, long ldv, int k, const double2* w, long n, double2* h,
                  double2* partial, int nblk, double2* pin);
-void launch_combine(hipStream_t s, double2* w, const double2* V, long ldv, int k, const double2* c, long n);
+// v = x / |x|, out[y] = |x|^2
+void launch_normalise(hipStream_t s, double2* v, const double2* x, long n, long rs, const int* ridx, int na,
+                      double* partial, int nblk, double* out);
+void launch_combine(hipStream_t s, double2* w, const double2* V, long ldv, int k, const double2* c, long n,
+                    bool add);
 // out[y] = |x_r|^2
 void launch_norm2(hipStream_t s, const double2* x, long n, long rs, const int* ridx, int na, double* partial,
                   int nblk, double* out);
 void launch_fields(hipStream_t s, double2* out, const double2* x, const double2* eps,
                    const double2* sxf, const double2* sxb, const double2* syf,
                    const double2* syb, const GridDesc& g, int pol, double2 w,
-                   int eigen_mode);
+                   int eigen_mode, int count = 1);
 void launch_mul_eps(hipStream_t s, double2* y, const double2* x, const double2* eps,
                     double2 a, long n);
 void launch_grad(hipStream_t s, double* grad, const double2* e, const double2* lam,

@@ -536,31 +536,30 @@ void launch_trisolve_multi(hipStream_t s, const TrsJob* jobs_d, int njobs, int n
 // Krylov building blocks over the active sources (grid row y -> source
 // ridx[y]).  Basis vector j of source r sits at V + j * ldv + r * rs.
 // ---------------------------------------------------------------------------
-// w_r += sign * sum_{i < kcnt[y]} h[y][i] V_{i,r}   (h has kstride entries per source)
-__global__ void k_gemv_update_b(double2* w, long wrs, const double2* V, long ldv, long rs,
-                                const int* kcnt, const double2* h, int kstride, double sign,
-                                long n, const int* ridx) {
+// w_r = [w_r +] sum_{i < kcnt[y]} h[y][i] V_{i,r}   (h has kstride entries per source)
+__global__ void k_combine_b(double2* w, long wrs, const double2* V, long ldv, long rs, const int* kcnt,
+                            const double2* h, int kstride, long n, const int* ridx, bool add) {
     __shared__ double2 hs[64];
     const int y = blockIdx.y;
     const long r = ridx[y];
     const int k = kcnt[y];
-    if (threadIdx.x < k) hs[threadIdx.x] = cscale(h[(long)y * kstride + threadIdx.x], sign);
+    if ((int)threadIdx.x < k) hs[threadIdx.x] = h[(long)y * kstride + threadIdx.x];
     __syncthreads();
     double2* wr = w + r * wrs;
     const double2* Vr = V + r * rs;
     for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < n;
          e += (long)gridDim.x * blockDim.x) {
-        double2 acc = wr[e];
+        double2 acc = add ? wr[e] : make_double2(0, 0);
         for (int i = 0; i < k; ++i) acc = cadd(acc, cmul(hs[i], Vr[i * ldv + e]));
         wr[e] = acc;
     }
 }
 
-void launch_gemv_update_b(hipStream_t s, double2* w, long wrs, const double2* V, long ldv, long rs,
-                          const int* kcnt, const double2* h, int kstride, double sign, long n,
-                          const int* ridx, int na) {
+void launch_combine_b(hipStream_t s, double2* w, long wrs, const double2* V, long ldv, long rs,
+                      const int* kcnt, const double2* h, int kstride, long n, const int* ridx, int na,
+                      bool add) {
     const unsigned nb = (unsigned)std::max<long>(1, std::min<long>((n + 255) / 256, 2048 / na + 1));
-    k_gemv_update_b<<<dim3(nb, na), 256, 0, s>>>(w, wrs, V, ldv, rs, kcnt, h, kstride, sign, n, ridx);
+    k_combine_b<<<dim3(nb, na), 256, 0, s>>>(w, wrs, V, ldv, rs, kcnt, h, kstride, n, ridx, add);
 }
 
 // y_r = a[y] * x_r

@@ -380,23 +380,24 @@ template <> __device__ inline double wave_sum<double>(double v) {
 // sources by grid row: ridx[y] (0 without a list), rs apart
 __device__ inline long source_offset(const int* ridx, long rs) { return ridx ? ridx[blockIdx.y] * rs : 0; }
 
-// w += sum_i c_i V_i, the coefficients (k <= 32) by value
+// w = [w +] sum_i c_i V_i, the coefficients (k <= 32) by value
 struct Coef32 {
     double2 c[ORTH_MAXK];
 };
-__global__ __launch_bounds__(256) void k_combine(double2* w, const double2* V, long ldv, int k, Coef32 h, long n) {
+__global__ __launch_bounds__(256) void k_combine(double2* w, const double2* V, long ldv, int k, Coef32 h, long n, bool add) {
     for (long e = blockIdx.x * 256L + threadIdx.x; e < n; e += 256L * gridDim.x) {
-        double2 acc = w[e];
+        double2 acc = add ? w[e] : make_double2(0, 0);
 #pragma unroll 4
         for (int i = 0; i < k; ++i) acc = cadd(acc, cmul(h.c[i], V[i * ldv + e]));
         w[e] = acc;
     }
 }
-void launch_combine(hipStream_t s, double2* w, const double2* V, long ldv, int k, const double2* c, long n) {
+void launch_combine(hipStream_t s, double2* w, const double2* V, long ldv, int k, const double2* c, long n,
+                    bool add) {
     Coef32 h{};
     for (int i = 0; i < k; ++i) h.c[i] = c[i];
     const unsigned nb = (unsigned)std::min<long>((n + 255) / 256, 2048);
-    k_combine<<<nb, 256, 0, s>>>(w, V, ldv, k, h, n);
+    k_combine<<<nb, 256, 0, s>>>(w, V, ldv, k, h, n, add);
 }
 
 __global__ __launch_bounds__(256) void k_norm2(const double2* x, long n, long rs, const int* ridx, double* partial) {
@@ -527,6 +528,29 @@ __global__ __launch_bounds__(256) void k_orth_sum(const double2* partial, int nb
         if (pin) pin[(long)y * ORTH_MAXK + i] = first ? cadd(s, first[(long)y * 2 * ORTH_MAXK + i]) : s;
     }
 }
+// v = x / |x| (0 of x = 0) and |x|^2 in out[y] (pinned), the norm from k_norm2's
+// partial sums in every workgroup
+__global__ __launch_bounds__(256) void k_normalise(double2* v, const double2* x, long n, long rs, const int* ridx,
+                                                   const double* partial, int nblk, double* out) {
+    __shared__ double red[4];
+    const int t = threadIdx.x;
+    double s = 0;
+    for (int b = t; b < nblk; b += 256) s += partial[(long)blockIdx.y * nblk + b];
+    s = wave_sum(s);
+    if ((t & 63) == 0) red[t >> 6] = s;
+    __syncthreads();
+    s = red[0] + red[1] + red[2] + red[3];
+    if (blockIdx.x == 0 && t == 0) out[blockIdx.y] = s;
+    const double a = s == 0 ? 0.0 : 1.0 / sqrt(s);
+    const long off = source_offset(ridx, rs);
+    for (long e = blockIdx.x * 256L + t; e < n; e += 256L * gridDim.x) v[off + e] = cscale(x[off + e], a);
+}
+void launch_normalise(hipStream_t s, double2* v, const double2* x, long n, long rs, const int* ridx, int na,
+                      double* partial, int nblk, double* out) {
+    nblk = (int)std::min<long>(nblk, (n + 255) / 256);
+    k_norm2<<<dim3(nblk, na), 256, 0, s>>>(x, n, rs, ridx, partial);
+    k_normalise<<<dim3(nblk, na), 256, 0, s>>>(v, x, n, rs, ridx, partial, nblk, out);
+}
 void launch_dots(hipStream_t s, const double2* V, long ldv, int k, const double2* w, long n, double2* h,
                  double2* partial, int nblk, double2* pin) {
     nblk = (int)std::min<long>(nblk, (n + 255) / 256);
@@ -564,12 +588,15 @@ void launch_orth(hipStream_t s, const double2* V, long ldv, int k, double2* w, l
 // eigen TE (eigen.jl:108-109): Ex uses Texi, Ey uses Teyi.
 // eigen_mode: 0 driven, 1 eigen.  The eps0' of TE is folded into w by the host.
 // ---------------------------------------------------------------------------
+// (grid row y: vector y of x, fields y of out)
 __global__ void k_fields(double2* out, const double2* x, const double2* eps, const double2* sxf,
                          const double2* sxb, const double2* syf, const double2* syb, int Nx,
                          int Ny, double dx, double dy, int pol, double2 w, int eigen_mode) {
     long N = (long)Nx * Ny;
     long k = blockIdx.x * (long)blockDim.x + threadIdx.x;
     if (k >= N) return;
+    out += blockIdx.y * 3 * N;
+    x += blockIdx.y * N;
     int i = (int)(k % Nx), j = (int)(k / Nx);
     long kw = (i == 0) ? k + Nx - 1 : k - 1;
     long ke = (i + 1 == Nx) ? k - (Nx - 1) : k + 1;
@@ -605,9 +632,9 @@ __global__ void k_fields(double2* out, const double2* x, const double2* eps, con
 void launch_fields(hipStream_t s, double2* out, const double2* x, const double2* eps,
                    const double2* sxf, const double2* sxb, const double2* syf,
                    const double2* syb, const GridDesc& g, int pol, double2 w,
-                   int eigen_mode) {
+                   int eigen_mode, int count) {
     long N = (long)g.Nx * g.Ny;
-    k_fields<<<(unsigned)((N + 255) / 256), 256, 0, s>>>(out, x, eps, sxf, sxb, syf, syb, g.Nx,
+    k_fields<<<dim3((unsigned)((N + 255) / 256), count), 256, 0, s>>>(out, x, eps, sxf, sxb, syf, syb, g.Nx,
                                                          g.Ny, g.dx, g.dy, pol, w, eigen_mode);
 }
 

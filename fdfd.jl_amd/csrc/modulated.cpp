@@ -111,7 +111,6 @@ extern "C" int fdfd_modulated_solve(fdfd_handle* hh, double omega, double Omega,
     launch_zero(h->stream, b, NF);
     if ((rc = stream_copy(h, fld, src, sizeof(double2) * N, hipMemcpyHostToDevice))) return done(rc);
     launch_scale_copy(h->stream, b + (long)K * N, fld, make_double2(0.0, scale * omega), N);
-    launch_zero(h->stream, x, NF);
 
     auto apply = [&](const double2* xx, double2* yy, const double2* bb) -> int {
         for (int j = 0; j < nf; ++j)
@@ -132,7 +131,6 @@ extern "C" int fdfd_modulated_solve(fdfd_handle* hh, double omega, double Omega,
     rc = rt_gmres_op(h, NF, apply, prec, V, Zk, b, x, tol, MF_MAX_RESTARTS, &iters, &restarts, &resid);
     if (rc == FDFD_ERR_NOCONV && Fs[0]->nd && !injected) {  // once more on line-reduction factors
         if ((rc = rt_rebuild_by_lines(h, Fs))) return done(rc);
-        launch_zero(h->stream, x, NF);
         rc = rt_gmres_op(h, NF, apply, prec, V, Zk, b, x, tol, MF_MAX_RESTARTS, &iters, &restarts, &resid);
     }
     if (rc == FDFD_OK) {

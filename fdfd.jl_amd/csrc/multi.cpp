@@ -232,12 +232,18 @@ static int gmres_multi(Handle* h, Factor* F, int nr, const double2* B, double2* 
     act.resize(nr);
     for (int r = 0; r < nr; ++r) act[r] = r;
     if ((rc = upload_list(act, nullptr))) return rc;
-    launch_norm2(st, B, N, N, m.ridx, nr, m.partr, MNBLK, po.nb);  // arrives with the first residuals
+    if (!(tol < 1)) {  // no iterations asked for
+        launch_zero(st, X, N * nr);
+        launch_norm2(st, B, N, N, m.ridx, nr, m.partr, MNBLK, po.nb);
+        HIPCHK(h, hipStreamSynchronize(st));
+        host_norms(po.nb, nr, bnorm);
+        for (double v : bnorm) *worst = std::max(*worst, v > 0 ? 1.0 : 0.0);
+        return FDFD_OK;
+    }
     struct Src {
         std::vector<std::complex<double>> H, gv, sn, y;
         std::vector<double> cs;
         int jdone = 0;
-        bool ext = false;
     };
     std::vector<Src> S(nr);
     for (auto& s : S) {
@@ -255,44 +261,46 @@ static int gmres_multi(Handle* h, Factor* F, int nr, const double2* B, double2* 
         if (act.empty()) break;
         if (rs > 0 && (rc = upload_list(act, nullptr))) return rc;
         const int na = (int)act.size();
-        // V_0,r = B_r - A' X_r, beta_r = ||V_0,r||
-        apply(V, X, B, na);
-        std::vector<double> beta;
-        launch_norm2(st, V, N, N, m.ridx, na, m.partr, MNBLK, po.nv);
-        HIPCHK(h, hipStreamSynchronize(st));
-        host_norms(po.nv, na, beta);
-        if (rs == 0) host_norms(po.nb, nr, bnorm);
+        // V_0,r = (B_r - A' X_r) / |.|; the first time X = 0 and V_0,r = B_r / |B_r|, whose
+        // norms arrive with the first coefficients (residuals are relative to them)
         std::vector<int> cyc;
         std::vector<double2> inv;
-        for (int q = 0; q < na; ++q) {
-            const int r = act[q];
-            if (bnorm[r] == 0) {
-                launch_zero(st, X + (long)r * N, N);
-                state[r] = 1;
-                resid[r] = 0;
-                continue;
+        if (rs == 0) {
+            launch_normalise(st, V, B, N, N, m.ridx, nr, m.partr, MNBLK, po.nb);
+        } else {
+            apply(V, X, B, na);
+            std::vector<double> beta;
+            launch_norm2(st, V, N, N, m.ridx, na, m.partr, MNBLK, po.nv);
+            HIPCHK(h, hipStreamSynchronize(st));
+            host_norms(po.nv, na, beta);
+            for (int q = 0; q < na; ++q) {
+                const int r = act[q];
+                resid[r] = beta[q] / bnorm[r];
+                if (resid[r] <= tol) state[r] = 1;
+                // no restart left, or a whole cycle that gained less than 10%: the
+                // rounding floor of the operator
+                else if (rs == max_restarts || resid[r] > 0.9 * prev[r]) state[r] = 2;
+                if (state[r] == 0) inv.push_back(make_double2(1.0 / beta[q], 0.0));
             }
-            resid[r] = beta[q] / bnorm[r];
-            if (resid[r] <= tol) { state[r] = 1; continue; }
-            // no restart left, or a whole cycle that gained less than 10%: the
-            // rounding floor of the operator
-            if (rs == max_restarts || (rs > 0 && resid[r] > 0.9 * prev[r])) { state[r] = 2; continue; }
+        }
+        for (int r : act) {
+            if (state[r] != 0) continue;
             prev[r] = resid[r];
             cyc.push_back(r);
-            inv.push_back(make_double2(1.0 / beta[q], 0.0));
             Src& s = S[r];
             std::fill(s.gv.begin(), s.gv.end(), 0.0);
-            s.gv[0] = beta[q];
+            s.gv[0] = resid[r];
             s.jdone = 0;
-            s.ext = true;
         }
         if (cyc.empty()) continue;
-        if ((rc = upload_list(cyc, nullptr))) return rc;
-        if ((rc = scale(V, V, inv))) return rc;
+        if (rs > 0) {
+            if ((rc = upload_list(cyc, nullptr))) return rc;
+            if ((rc = scale(V, V, inv))) return rc;
+        }
         std::vector<int> it = cyc;
         for (int j = 0; j < K && !it.empty(); ++j) {
             const int ni = (int)it.size();
-            if ((rc = upload_list(it, nullptr))) return rc;
+            if (rs + j > 0 && (rc = upload_list(it, nullptr))) return rc;
             double2* Vj = V + (long)j * ldv;
             double2* Zj = Z + (long)j * ldv;
             double2* W = V + (long)(j + 1) * ldv;
@@ -311,12 +319,18 @@ static int gmres_multi(Handle* h, Factor* F, int nr, const double2* B, double2* 
             HIPCHK(h, hipStreamSynchronize(st));
             std::vector<double> hn;
             host_norms(po.nv, ni, hn);
+            if (rs == 0 && j == 0) host_norms(po.nb, nr, bnorm);
             std::vector<double2> hinv(ni);
             for (int q = 0; q < ni; ++q) hinv[q] = make_double2(hn[q] > 0 ? 1.0 / hn[q] : 1.0, 0.0);
             std::vector<int> still;
             for (int q = 0; q < ni; ++q) {
                 const int r = it[q];
                 Src& s = S[r];
+                if (bnorm[r] == 0) {  // x = 0: its update has no terms
+                    state[r] = 1;
+                    resid[r] = 0;
+                    continue;
+                }
                 auto Hij = [&](int i, int jj) -> std::complex<double>& { return s.H[(size_t)i * K + jj]; };
                 const volatile double* hc = (const volatile double*)(po.c + q * ORTH_MAXK);
                 for (int i = 0; i <= j; ++i) Hij(i, j) = std::complex<double>(hc[2 * i], hc[2 * i + 1]);
@@ -343,7 +357,7 @@ static int gmres_multi(Handle* h, Factor* F, int nr, const double2* B, double2* 
                 s.gv[j] = s.cs[j] * s.gv[j];
                 ++*iters;
                 s.jdone = j + 1;
-                const double est = std::abs(s.gv[j + 1]) / bnorm[r];
+                const double est = std::abs(s.gv[j + 1]);
                 if (!(est <= 0.5 * tol || hn[q] == 0)) still.push_back(r);
             }
             if (!still.empty() && (rc = scale(W, W, hinv))) return rc;
@@ -358,14 +372,14 @@ static int gmres_multi(Handle* h, Factor* F, int nr, const double2* B, double2* 
                 for (int l = i + 1; l < s.jdone; ++l) v -= s.H[(size_t)i * K + l] * s.y[l];
                 s.y[i] = v / s.H[(size_t)i * K + i];
             }
-            for (int i = 0; i < s.jdone; ++i) u.c[q * (K + 2) + i] = make_double2(s.y[i].real(), s.y[i].imag());
+            for (int i = 0; i < s.jdone; ++i) u.c[q * (K + 2) + i] = make_double2(bnorm[cyc[q]] * s.y[i].real(), bnorm[cyc[q]] * s.y[i].imag());
             u.ints[q] = cyc[q];
             u.ints[KMULTI + q] = s.jdone;
         }
         HIPCHK(h, hipMemcpyAsync(m.ridx, u.ints, sizeof(int) * cyc.size(), hipMemcpyHostToDevice, st));
         HIPCHK(h, hipMemcpyAsync(m.kcnt, u.ints + KMULTI, sizeof(int) * cyc.size(), hipMemcpyHostToDevice, st));
         HIPCHK(h, hipMemcpyAsync(m.coef, u.c, sizeof(double2) * cyc.size() * (K + 2), hipMemcpyHostToDevice, st));
-        launch_gemv_update_b(st, X, N, Z, ldv, N, m.kcnt, m.coef, K + 2, 1.0, N, m.ridx, (int)cyc.size());
+        launch_combine_b(st, X, N, Z, ldv, N, m.kcnt, m.coef, K + 2, N, m.ridx, (int)cyc.size(), rs > 0);
         HIPCHK(h, hipStreamSynchronize(st));  // the pinned slots are reused next cycle
     }
     double w = 0;
@@ -394,8 +408,6 @@ int rt_gmres_multi(Handle* h, Factor* F, int nr, const double2* B, double2* X, d
     int rc = gmres_multi(h, F, nr, B, X, tol, iters, worst);
     if (rc == FDFD_ERR_NOCONV && F->nd) {
         if ((rc = rt_rebuild_by_lines(h, {F}))) return rc;
-        const long N = (long)h->g.Nx * h->g.Ny;
-        launch_zero(h->stream, X, N * nr);
         *worst = before;
         rc = gmres_multi(h, F, nr, B, X, tol, iters, worst);
     }

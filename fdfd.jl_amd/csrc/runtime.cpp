@@ -119,7 +119,7 @@ int ensure_solve_work(Handle* h, long N) {
         HIPCHK(h, hipMalloc(&h->dpart, sizeof(double2) * h->nblk * (KDIM + 2)));
         HIPCHK(h, hipMalloc(&h->rpart, sizeof(double) * h->nblk));
         HIPCHK(h, hipMalloc(&h->hdev, sizeof(double2) * 2 * (KDIM + 2)));
-        HIPCHK(h, hipHostMalloc(&h->hpin, sizeof(double2) * (KDIM + 4)));
+        HIPCHK(h, hipHostMalloc(&h->hpin, sizeof(double2) * (ORTH_MAXK + 2)));
     }
     h->work_N = N;
     h->kdim = KDIM;
@@ -324,16 +324,10 @@ void rt_apply(Handle* h, const Factor* F, double2* y, const double2* x, int tran
 // ---------------------------------------------------------------------------
 // FP64 Krylov building blocks
 // ---------------------------------------------------------------------------
-// |x|^2 into scalar i of the pinned buffer, without waiting
-static volatile double* start_norm(Handle* h, const double2* x, long N, int i) {
-    double* out = (double*)h->hpin + i;
-    launch_norm2(h->stream, x, N, 0, nullptr, 1, h->rpart, h->nblk, out);
-    return out;
-}
 static int dev_norm(Handle* h, const double2* x, long N, double* out) {
-    volatile double* v = start_norm(h, x, N, 0);
+    launch_norm2(h->stream, x, N, 0, nullptr, 1, h->rpart, h->nblk, (double*)h->hpin);
     HIPCHK(h, hipStreamSynchronize(h->stream));
-    *out = std::sqrt(*v);
+    *out = std::sqrt(*(const volatile double*)h->hpin);
     return FDFD_OK;
 }
 
@@ -350,10 +344,11 @@ static int dev_multidot(Handle* h, const double2* V, long N, int k, const double
     return FDFD_OK;
 }
 
-// w += V[0..k-1] c   (in chunks of at most 32 vectors)
-static void dev_update(Handle* h, double2* w, const double2* V, long N, int k, const cd* c) {
+// w = [w +] V[0..k-1] c   (in chunks of at most 32 vectors)
+static void dev_update(Handle* h, double2* w, const double2* V, long N, int k, const cd* c, bool add = true) {
     for (int c0 = 0; c0 < k; c0 += 32)
-        launch_combine(h->stream, w, V + (long)c0 * N, N, std::min(32, k - c0), (const double2*)(c + c0), N);
+        launch_combine(h->stream, w, V + (long)c0 * N, N, std::min(32, k - c0), (const double2*)(c + c0), N,
+                       add || c0 > 0);
 }
 
 // w orthogonalised against V[0..k-1] by two passes of classical Gram-Schmidt:
@@ -385,7 +380,10 @@ static int dev_orth(Handle* h, const double2* V, long N, int k, double2* w, cd* 
 struct SolveStats { int iters = 0, restarts = 0; double resid = 0; };
 
 // Right-preconditioned flexible GMRES(KDIM) on A' x = b (or A'^T x = b) in
-// FP64, preconditioned by the block factors.  x is the initial guess on entry.
+// FP64, preconditioned by the block factors.  It starts from x = 0, so the first
+// cycle's residual is b: it is normalised on the device, the cycle's small
+// problem is scaled by |b| (known with its first coefficients), and x is written
+// by the first update.
 int rt_gmres_op(Handle* h, long N,
                 const std::function<int(const double2*, double2*, const double2*)>& apply,
                 const std::function<int(const double2*, double2*)>& prec, double2* V, double2* Zk,
@@ -399,32 +397,38 @@ int rt_gmres_op(Handle* h, long N,
         K = std::min(std::max(h->inject_arg, 0), GMRES_KDIM);
         max_restarts = K > 0 ? 1 : 0;
     }
-    volatile double* bn2 = start_norm(h, b, N, 1);  // arrives with the first residual
+    if (!(tol < 1) || K == 0) {  // no iterations asked for, or none allowed
+        launch_zero(h->stream, x, N);
+        if ((rc = dev_norm(h, b, N, &bnorm))) return rc;
+        *resid_out = bnorm > 0 ? 1 : 0;
+        if (*resid_out <= tol) return FDFD_OK;
+        max_restarts = -1;
+    }
+    const volatile double* bn2 = (const volatile double*)(h->hpin + 33);
     std::vector<cd> H((size_t)(K + 1) * K), gv(K + 1), sn(K), hc(K + 1), y(K);
     std::vector<double> cs(K);
     double resid = 1, prev = 2;
     for (int rs = 0; rs <= max_restarts; ++rs) {
-        if ((rc = apply(x, V, b))) return rc;
-        double beta;
-        if ((rc = dev_norm(h, V, N, &beta))) return rc;
-        if (rs == 0) bnorm = std::sqrt(*bn2);
-        if (bnorm == 0) {
-            launch_zero(h->stream, x, N);
-            *resid_out = 0;
-            return FDFD_OK;
+        // (residuals are relative to |b| from here on)
+        if (rs == 0) {
+            launch_normalise(h->stream, V, b, N, 0, nullptr, 1, h->rpart, h->nblk, (double*)(h->hpin + 33));
+        } else {
+            if ((rc = apply(x, V, b))) return rc;
+            double beta;
+            if ((rc = dev_norm(h, V, N, &beta))) return rc;
+            resid = beta / bnorm;
+            *resid_out = resid;
+            if (resid <= tol) return FDFD_OK;
+            if (rs == max_restarts) break;
+            // a whole restart cycle that gains less than 10% has reached the
+            // rounding floor of the operator: stop instead of cycling
+            if (resid > 0.9 * prev) break;
+            ++*restarts;
+            launch_scale_copy(h->stream, V, V, make_double2(1.0 / beta, 0), N);
         }
-        resid = beta / bnorm;
-        *resid_out = resid;
-        if (resid <= tol) return FDFD_OK;
-        if (rs == max_restarts) break;
-        // a whole restart cycle that gains less than 10% has reached the
-        // rounding floor of the operator: stop instead of cycling
-        if (rs > 0 && resid > 0.9 * prev) break;
         prev = resid;
-        if (rs > 0) ++*restarts;
-        launch_scale_copy(h->stream, V, V, make_double2(1.0 / beta, 0), N);
         std::fill(gv.begin(), gv.end(), cd(0));
-        gv[0] = beta;
+        gv[0] = resid;
         int jdone = 0;
         for (int j = 0; j < K; ++j) {
             double2* vj = V + (long)j * N;
@@ -434,6 +438,14 @@ int rt_gmres_op(Handle* h, long N,
             if ((rc = apply(zj, w, nullptr))) return rc;
             double hn;
             if ((rc = dev_orth(h, V, N, j + 1, w, hc.data(), &hn))) return rc;
+            if (rs == 0 && j == 0) {
+                bnorm = std::sqrt(*bn2);
+                if (bnorm == 0) {
+                    launch_zero(h->stream, x, N);
+                    *resid_out = 0;
+                    return FDFD_OK;
+                }
+            }
             for (int i = 0; i <= j; ++i) H[(size_t)i * K + j] = hc[i];
             H[(size_t)(j + 1) * K + j] = hn;
             // Givens
@@ -459,7 +471,7 @@ int rt_gmres_op(Handle* h, long N,
             gv[j] = cs[j] * gv[j];
             ++*iters;
             jdone = j + 1;
-            double est = std::abs(gv[j + 1]) / bnorm;
+            const double est = std::abs(gv[j + 1]);
             if (est <= 0.5 * tol || hn == 0) break;
             launch_scale_copy(h->stream, w, w, make_double2(1.0 / hn, 0), N);
         }
@@ -469,7 +481,8 @@ int rt_gmres_op(Handle* h, long N,
             for (int l = i + 1; l < jdone; ++l) s -= H[(size_t)i * K + l] * y[l];
             y[i] = s / H[(size_t)i * K + i];
         }
-        dev_update(h, x, Zk, N, jdone, y.data());
+        for (int i = 0; i < jdone; ++i) y[i] *= bnorm;
+        dev_update(h, x, Zk, N, jdone, y.data(), rs > 0);
     }
     *resid_out = resid;
     char buf[160];
@@ -501,7 +514,6 @@ static int gmres(Handle* h, Factor* F, int trans, const double2* b, double2* x, 
         return fail(h, FDFD_ERR_NOCONV, "refinement did not reach the tolerance (injected)");
     if (rc == FDFD_ERR_NOCONV && F->nd && !injected && st.resid > accept) {
         if ((rc = rt_rebuild_by_lines(h, {F}))) return rc;
-        launch_zero(h->stream, x, N);
         rc = rt_gmres_op(h, N, apply, prec, h->V, h->Zk, b, x, tol, max_restarts, &st.iters,
                          &st.restarts, &st.resid);
     }
@@ -737,16 +749,12 @@ int fdfd_solve_d(fdfd_handle* hh, int factor_id, int nrhs, const void* d_src, vo
         for (int s0 = 0; s0 < nrhs && rc == FDFD_OK; s0 += KMULTI) {
             const int ns = std::min(KMULTI, nrhs - s0);
             if ((rc = ensure_multi_work(h, N, ns))) break;
-            for (int k = 0; k < ns; ++k) {
-                launch_scale_copy(h->stream, h->mB + (long)k * N, (const double2*)d_src + (long)(s0 + k) * N,
-                                  make_double2(0.0, F->scale * F->omega), N);
-                launch_zero(h->stream, h->mX + (long)k * N, N);
-            }
+            launch_scale_copy(h->stream, h->mB, (const double2*)d_src + (long)s0 * N,
+                              make_double2(0.0, F->scale * F->omega), N * ns);
             rc = rt_gmres_multi(h, F, ns, h->mB, h->mX, tol, &st.iters, &worst);
             if (rc) break;
-            for (int k = 0; k < ns; ++k)
-                launch_fields(h->stream, (double2*)d_out + (long)(s0 + k) * 3 * N, h->mX + (long)k * N,
-                              h->eps, F->sxf, F->sxb, F->syf, F->syb, g, F->pol, wf, 0);
+            launch_fields(h->stream, (double2*)d_out + (long)s0 * 3 * N, h->mX, h->eps, F->sxf, F->sxb, F->syf,
+                          F->syb, g, F->pol, wf, 0, ns);
         }
     }
     for (int r = 0; r < nrhs && nrhs == 1 && rc == FDFD_OK; ++r) {
@@ -754,7 +762,6 @@ int fdfd_solve_d(fdfd_handle* hh, int factor_id, int nrhs, const void* d_src, vo
         double2* out = (double2*)d_out + (long)r * 3 * N;
         // b' = scale * (i omega) * src   (driven.jl:36,46)
         launch_scale_copy(h->stream, h->bvec, src, make_double2(0.0, F->scale * F->omega), N);
-        launch_zero(h->stream, h->xvec, N);
         SolveStats s1;
         rc = gmres(h, F, 0, h->bvec, h->xvec, tol, MAX_RESTARTS, s1);
         st.iters += s1.iters;
@@ -820,7 +827,6 @@ int fdfd_linsolve(fdfd_handle* hh, int factor_id, int transpose, int nrhs, const
     for (int r = 0; r < nrhs; ++r) {
         COPY(h, h->tmp, b + (long)r * N, sizeof(double2) * N, hipMemcpyHostToDevice);
         launch_scale_copy(h->stream, h->bvec, h->tmp, make_double2(F->scale, 0), N);
-        launch_zero(h->stream, h->xvec, N);
         SolveStats s1;
         int rc = gmres(h, F, transpose ? 1 : 0, h->bvec, h->xvec, tol, MAX_RESTARTS, s1);
         st.iters += s1.iters;
@@ -918,7 +924,6 @@ int fdfd_solve_pullback_d(fdfd_handle* hh, int factor_id, const void* d_ez, cons
     // scale * conj(bar Ez + Mx^H bar Hx + My^H bar Hy), c = 1/(i w mu0')
     launch_field_adjoint(h->stream, h->bvec, (const double2*)d_dfields, F->sxb, F->syb, g,
                          make_double2(0.0, -1.0 / (F->omega * mu0n)), F->scale);
-    launch_zero(h->stream, h->xvec, N);
     SolveStats st;
     int rc = gmres(h, F, 1, h->bvec, h->xvec, tol, MAX_RESTARTS, st);
     if (rc == FDFD_OK) {

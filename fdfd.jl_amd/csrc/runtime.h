@@ -262,7 +262,8 @@ void rt_apply(Handle* h, const Factor* F, double2* y, const double2* x, int tran
 // Right-preconditioned FGMRES(30) in FP64 on an operator given by callbacks:
 //   apply(x, y, b): y = b - A x if b != nullptr, else y = A x
 //   prec(v, z):     z = M^-1 v
-// V ((30 + 1) * N) and Zk (30 * N) are the caller's device workspace.  Stops
+// V ((30 + 1) * N) and Zk (30 * N) are the caller's device workspace.  Starts from
+// x = 0 (x is only written).  Stops
 // at ||b - A x|| <= tol ||b|| (FDFD_ERR_NOCONV after max_restarts restarts).
 constexpr int GMRES_KDIM = 30;
 int rt_gmres_op(Handle* h, long N, const std::function<int(const double2*, double2*, const double2*)>& apply,

@@ -110,7 +110,6 @@ extern "C" int fdfd_vector_eigenmode(fdfd_handle* hh, double omega, fdfd_complex
     // follows its error.
     auto op = [&](const double2* x, double2* y) -> int {
         launch_scale_copy(h->stream, bb, x, make_double2(s, 0), N2);
-        launch_zero(h->stream, y, N2);
         double res = 0;
         int r = rt_gmres_op(h, N2, apply, prec, V, Zk, bb, y, inner_tol, VM_MAX_RESTARTS, &inner_its,
                             &inner_restarts, &res);
