@@ -404,6 +404,41 @@ __device__ __attribute__((always_inline)) inline void nd_sweep(d4v (&mr)[NdSweep
     }
 }
 
+// The operator at up to NF cells of a front, in LDS: one load a thread in place
+// of a branch and a load for each entry that is not zero
+template <int NF> struct NdCells {
+    C cc[NF], ce[NF], cn[NF];
+    int x[NF], y[NF];  // x < 0: no cell
+    __device__ inline void load(const int* node, int n, const double2* coef, long N, int Nx) {
+        for (int e = threadIdx.x; e < 3 * NF; e += 256) {
+            const int i = e % NF, pl = e / NF;
+            const int k = i < n ? node[i] : -1, kk = max(k, 0);
+            const C c = gload(coef + (long)(pl == 0 ? CC : pl == 1 ? CE : CN) * N + kk);
+            (pl == 0 ? cc : pl == 1 ? ce : cn)[i] = c;
+            if (pl == 0) {
+                x[i] = k < 0 ? -1 : k % Nx;
+                y[i] = kk / Nx;
+            }
+        }
+    }
+    // entry (i, j) of the symmetrised operator, a unit row where there is no cell
+    __device__ inline C entry(int i, int j, int Nx, int Ny) const {
+        C z = mk<C>(0, 0);
+        const int xi = x[i], xj = x[j], yi = y[i], yj = y[j];
+        if (xi < 0 || xj < 0) {
+            z = mk<C>(i == j ? 1 : 0, 0);
+        } else if (yi == yj) {
+            if (i == j) z = cc[i];
+            if (xj == (xi + 1 == Nx ? 0 : xi + 1)) z = cadd(z, ce[i]);
+            if (xi == (xj + 1 == Nx ? 0 : xj + 1)) z = cadd(z, ce[j]);
+        } else if (xi == xj) {
+            if (yj == (yi + 1 == Ny ? 0 : yi + 1)) z = cadd(z, cn[i]);
+            if (yi == (yj + 1 == Ny ? 0 : yj + 1)) z = cadd(z, cn[j]);
+        }
+        return z;
+    }
+};
+
 // Leaves: one workgroup per leaf, its whole front, the separator and then the
 // boundary, swept in registers.  The chain of the sweep bounds a workgroup (some
 // 50 us for 52 cells), so what counts is how many share a compute unit: a leaf
@@ -417,43 +452,17 @@ __global__ __launch_bounds__(256, 3) void k_nd_leaf(NdLev lv, const NdFac* fac, 
     const int p = lv.p, b = lv.b, fr = blockIdx.x;
     const long N = (long)Nx * Ny;
     constexpr int NF = 16 * T;
-    // the operator at the front's cells, for the gather below: one load a thread
-    // in place of a branch and a load for each entry that is not zero
     __shared__ union {
         NdSweep<T> w;
-        struct {
-            C cc[NF], ce[NF], cn[NF];
-            int x[NF], y[NF];  // x < 0: no cell
-        } g;
+        NdCells<NF> g;
     } s;
-    for (int e = threadIdx.x; e < 3 * NF; e += 256) {
-        const int i = e % NF, pl = e / NF;
-        const int k = i < p + b ? lv.node[(long)fr * (p + b) + i] : -1, kk = max(k, 0);
-        const C c = gload(F.coef + (long)(pl == 0 ? CC : pl == 1 ? CE : CN) * N + kk);
-        (pl == 0 ? s.g.cc : pl == 1 ? s.g.ce : s.g.cn)[i] = c;
-        if (pl == 0) {
-            s.g.x[i] = k < 0 ? -1 : k % Nx;
-            s.g.y[i] = kk / Nx;
-        }
-    }
+    s.g.load(lv.node + (long)fr * (p + b), p + b, F.coef, N, Nx);
     __syncthreads();
     constexpr int NS = NdSweep<T>::NS;
     d4v mr[NS], mi[NS];
     nd_each_entry<T>([&](auto sc, int v, int i, int j, bool) {
         C z = mk<C>(0, 0);
-        const int xi = s.g.x[i], xj = s.g.x[j], yi = s.g.y[i], yj = s.g.y[j];
-        if (i < p || j < p) {
-            if (xi < 0 || xj < 0) {
-                z = mk<C>(i == j ? 1 : 0, 0);
-            } else if (yi == yj) {
-                if (i == j) z = s.g.cc[i];
-                if (xj == (xi + 1 == Nx ? 0 : xi + 1)) z = cadd(z, s.g.ce[i]);
-                if (xi == (xj + 1 == Nx ? 0 : xj + 1)) z = cadd(z, s.g.ce[j]);
-            } else if (xi == xj) {
-                if (yj == (yi + 1 == Ny ? 0 : yi + 1)) z = cadd(z, s.g.cn[i]);
-                if (yi == (yj + 1 == Ny ? 0 : yj + 1)) z = cadd(z, s.g.cn[j]);
-            }
-        }
+        if (i < p || j < p) z = s.g.entry(i, j, Nx, Ny);
         mr[sc][v] = z.x;
         mi[sc][v] = z.y;
     });
@@ -487,19 +496,6 @@ void launch_nd_leaf(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, int
     else k_nd_leaf<5><<<g, 256, 0, s>>>(lv, fac, Nx, Ny, S);
 }
 
-// children's contribution to entry (i, j) of a front, i, j front indices
-__device__ inline C nd_gather(const NdLev& lv, const C* Sc, const short* cm, int i, int j) {
-    const int f = lv.p + lv.b;
-    C v = mk<C>(0, 0);
-    const int i0 = cm[i], j0 = cm[j];
-    if (i0 >= 0 && j0 >= 0) v = gload(Sc + (long)i0 * lv.cb + j0);
-    if (lv.nch > 1) {
-        const int i1 = cm[f + i], j1 = cm[f + j];
-        if (i1 >= 0 && j1 >= 0) v = cadd(v, gload(Sc + (long)lv.cb * lv.cb + (long)i1 * lv.cb + j1));
-    }
-    return v;
-}
-
 // ---------------------------------------------------------------------------
 // Assembly of a level's fronts (operator entries plus the children's Schur
 // complements, padded separator cells as unit rows) and the start of their
@@ -526,24 +522,40 @@ __global__ __launch_bounds__(256, 2) void k_nd_front(NdLev lv, const NdFac* fac,
     const int* node = lv.node + (long)fr * f;
     const short* cm = lv.cm + (long)fr * 2 * f;
     const C* Sc = (const C*)Scv + ((long)q * lv.cnt * lv.nch + (long)fr * lv.nch) * lv.cb * lv.cb;
-    auto entry = [&](int i, int j) {
-        const int ki = node[i], kj = node[j];
-        C v = mk<C>(0, 0);
-        if (ki >= 0 && kj >= 0) v = cadd(nd_entry(F.coef, N, Nx, Ny, ki, kj), nd_gather(lv, Sc, cm, i, j));
-        else if (i == j) v = mk<C>(1, 0);
-        return v;
-    };
     if (inv) {
-        __shared__ NdSweep<T> s;
-        const int np = min(p, NB);
+        constexpr int NF = 16 * T;
+        __shared__ union {
+            NdSweep<T> w;
+            struct {
+                NdCells<NF> c;
+                short m[2][NF];  // the cells' places in the children
+            } g;
+        } s;
+        const int np = min(p, NB), two = lv.nch > 1 ? 1 : 0;
+        s.g.c.load(node, np, F.coef, N, Nx);
+        for (int i = threadIdx.x; i < 2 * NF; i += 256) {
+            const int c = i / NF, k = i % NF;
+            s.g.m[c][k] = k < np && c <= two ? cm[c * f + k] : -1;
+        }
+        __syncthreads();
         constexpr int NS = NdSweep<T>::NS;
         d4v mr[NS], mi[NS];
+        // the children's entries are all loaded before the first is used (entry 0
+        // where there is none)
+        C o0[NS][4], o1[NS][4];
         nd_each_entry<T>([&](auto sc, int v, int i, int j, bool) {
-            const C z = i < np && j < np ? entry(i, j) : mk<C>(i == j ? 1 : 0, 0);
-            mr[sc][v] = z.x;
-            mi[sc][v] = z.y;
+            const int i0 = s.g.m[0][i], j0 = s.g.m[0][j], i1 = s.g.m[1][i], j1 = s.g.m[1][j];
+            o0[sc][v] = gload(Sc + (i0 >= 0 && j0 >= 0 ? (long)i0 * lv.cb + j0 : 0));
+            o1[sc][v] = gload(Sc + (i1 >= 0 && j1 >= 0 ? ((long)lv.cb + i1) * lv.cb + j1 : 0));
         });
-        nd_sweep<T>(mr, mi, np, s, F.pivstat + 3 * (long)(lv.stat + fr), false);
+        nd_each_entry<T>([&](auto sc, int v, int i, int j, bool) {
+            const bool k0 = s.g.m[0][i] >= 0 && s.g.m[0][j] >= 0, k1 = s.g.m[1][i] >= 0 && s.g.m[1][j] >= 0;
+            const C z = s.g.c.entry(i, j, Nx, Ny);
+            mr[sc][v] = z.x + (k0 ? o0[sc][v].x : 0.0) + (k1 ? o1[sc][v].x : 0.0);
+            mi[sc][v] = z.y + (k0 ? o0[sc][v].y : 0.0) + (k1 ? o1[sc][v].y : 0.0);
+        });
+        __syncthreads();
+        nd_sweep<T>(mr, mi, np, s.w, F.pivstat + 3 * (long)(lv.stat + fr), false);
         const bool whole = p <= NB;
         C* out = whole ? (C*)F.arena + lv.offX + (long)fr * p * p : (C*)w.D + job * NB * NB;
         const int ld = whole ? p : NB;
