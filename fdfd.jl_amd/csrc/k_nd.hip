@@ -1398,17 +1398,23 @@ struct ndm_acc {
     }
 };
 
-// sum of the KS waves' tiles through LDS (valid in wave 0)
-template <int KS>
-__device__ inline void ndm_reduce(C (&z)[4], C (*red)[4][64], int wv, int lane) {
-    if constexpr (KS > 1) {
+// f(r, value) for the tile's entries v = r of this wave's lanes; with KS waves their
+// tiles are added through LDS, entry r by wave r
+template <int KS, typename F>
+__device__ __attribute__((always_inline)) inline void ndm_finish(const C (&z)[4], C (*red)[4][64], int wv, int lane,
+                                                                 F&& f) {
+    if constexpr (KS == 1) {
 #pragma unroll
-        for (int v = 0; v < 4; ++v) red[wv][v][lane] = z[v];
+        for (int r = 0; r < 4; ++r) f(r, z[r]);
+    } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) red[wv][r][lane] = z[r];
         __syncthreads();
-        if (wv == 0)
-            for (int w = 1; w < KS; ++w)
+        if (wv >= 4) return;
+        C s = red[0][wv][lane];
 #pragma unroll
-                for (int v = 0; v < 4; ++v) z[v] = cadd(z[v], red[w][v][lane]);
+        for (int w = 1; w < KS; ++w) s = cadd(s, red[w][wv][lane]);
+        f(0, s);
     }
 }
 
@@ -1427,6 +1433,16 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS) void k_ndm_up(NdLev lv, co
     const int p = lv.p, b = lv.b, l16 = lane & 15, kg = lane >> 4;
     const C* Q = (const C*)arena + lv.offQ + (long)fr * p * b + min(j0 + l16, b - 1);
     const C* v = vp + (lv.offV + (long)fr * p) * 16 + l16;
+    // what this wave's entries are subtracted from
+    C* u = up + (lv.offU + (long)fr * b) * 16 + l16;
+    constexpr int NR = KS == 1 ? 4 : 1;
+    int row[NR];
+    C old[NR];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+        row[r] = j0 + M::row(lane, KS == 1 ? r : wv & 3);
+        old[r] = gload(u + (long)min(row[r], b - 1) * 16);
+    }
     ndm_acc A;
     const int nst = p / 4;
     for (int s0 = KS == 1 ? 0 : wv * NDM_U; s0 < nst; s0 += KS * NDM_U) {
@@ -1444,22 +1460,18 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS) void k_ndm_up(NdLev lv, co
     C z[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) z[r] = mk<C>(A.rr[r] - A.ii[r], A.ri[r]);
-    ndm_reduce<KS>(z, red, wv, lane);
-    if (KS > 1 && wv != 0) return;
-    C* u = up + (lv.offU + (long)fr * b) * 16 + l16;
-    C old[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) old[r] = gload(u + (long)min(j0 + M::row(lane, r), b - 1) * 16);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int j = j0 + M::row(lane, r);
-        if (j < b) gstore(u + (long)j * 16, csub(old[r], z[r]));
-    }
+    ndm_finish<KS>(z, red, wv, lane, [&](int r, C s) {
+        if (row[r] < b) gstore(u + (long)row[r] * 16, csub(old[r], s));
+    });
 }
 
 // x = X v - Q x_boundary, 16 separator cells a tile.  X is symmetric, so its
 // operand is read along rows (16 neighbouring columns); a lane reads four
 // neighbouring entries of its row of Q and the K order is permuted to match.
+// A level of few tiles is bound by the chain list, value, product: the list is read
+// two groups ahead, and the waves' tiles are added by four of them (13 us for 256 x
+// 1020 on two fronts, 23 us with the list read in turn and one wave adding; 16
+// sources on 384 x 512 1.66 -> 1.49 ms).
 template <int KS>
 __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS) void k_ndm_down(NdLev lv, const void* arena, const C* vp,
                                                                  C* xp, int nt) {
@@ -1475,6 +1487,14 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS) void k_ndm_down(NdLev lv, 
     const C* X = (const C*)arena + lv.offX + (long)fr * p * p + row;
     const C* Q = (const C*)arena + lv.offQ + (long)fr * p * b + (long)row * b;
     const C* v = vp + (lv.offV + (long)fr * p) * 16 + l16;
+    // the cells of this wave's entries (-1: none)
+    constexpr int NR = KS == 1 ? 4 : 1;
+    int cell[NR];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+        const int i = i0 + M::row(lane, KS == 1 ? r : wv & 3);
+        cell[r] = i < p ? node[i] : -1;
+    }
     ndm_acc A, B;
     const int nst = p / 4;
     for (int s0 = KS == 1 ? 0 : wv * NDM_U; s0 < nst; s0 += KS * NDM_U) {
@@ -1489,38 +1509,53 @@ __global__ __launch_bounds__(KS == 1 ? 256 : 64 * KS) void k_ndm_down(NdLev lv, 
         for (int q = 0; q < NDM_U; ++q)
             if (s0 + q < nst) A.step(a[q], x[q]);
     }
-    // four consecutive columns k0 + 4 kg .. + 3 per lane; b is a multiple of 4
-    for (int k0 = KS == 1 ? 0 : 16 * wv; k0 < b; k0 += KS * 16) {
-        const int k = k0 + 4 * kg;
-        const bool ok = k < b;
-        C a[4], x[4];
+    // four consecutive columns k0 + 4 kg .. + 3 per lane (b is a multiple of 4), of
+    // two groups of 16; the next two groups' cells are looked up meanwhile
+    auto look = [&](int k0, int (&n)[2][4]) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int n = ok ? gload_s(node + p + k + q) : -1;
-            a[q] = gload(Q + (ok ? k + q : 0));
-            x[q] = gload(xp + (long)max(n, 0) * 16 + l16);
-            if (n < 0) {
-                a[q] = mk<C>(R(0), R(0));
-                x[q] = a[q];
+        for (int g = 0; g < 2; ++g)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int k = k0 + KS * 16 * g + 4 * kg + q;
+                n[g][q] = node[p + min(k, b - 1)];
+            }
+    };
+    int n[2][4];
+    const int kb = KS == 1 ? 0 : 16 * wv;
+    if (b > 0) look(kb, n);
+    for (int k0 = kb; k0 < b; k0 += 2 * KS * 16) {
+        C a[2][4], x[2][4];
+        int nn[2][4];
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int k = k0 + KS * 16 * g + 4 * kg + q;
+                a[g][q] = gload(Q + min(k, b - 1));
+                x[g][q] = gload(xp + (long)max(n[g][q], 0) * 16 + l16);
+            }
+        look(k0 + 2 * KS * 16, nn);
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            if (g == 1 && k0 + KS * 16 >= b) break;  // uniform
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const bool ok = n[g][q] >= 0 && k0 + KS * 16 * g + 4 * kg + q < b;
+                B.step(csel(ok, a[g][q], mk<C>(0, 0)), csel(ok, x[g][q], mk<C>(0, 0)));
             }
         }
 #pragma unroll
-        for (int q = 0; q < 4; ++q) B.step(a[q], x[q]);
+        for (int g = 0; g < 2; ++g)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) n[g][q] = nn[g][q];
     }
     C z[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r)
         z[r] = mk<C>((A.rr[r] - A.ii[r]) - (B.rr[r] - B.ii[r]), A.ri[r] - B.ri[r]);
-    ndm_reduce<KS>(z, red, wv, lane);
-    if (KS > 1 && wv != 0) return;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int i = i0 + M::row(lane, r);
-        if (i < p) {
-            const int k = node[i];
-            if (k >= 0) gstore(xp + (long)k * 16 + l16, z[r]);
-        }
-    }
+    ndm_finish<KS>(z, red, wv, lane, [&](int r, C s) {
+        if (cell[r] >= 0) gstore(xp + (long)cell[r] * 16 + l16, s);
+    });
 }
 
 void launch_ndm_io(hipStream_t s, const NdVec& z, void* x, long N, int Nx, int na, bool pack) {
