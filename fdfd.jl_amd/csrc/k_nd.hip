@@ -1114,6 +1114,10 @@ void launch_nd_stat(hipStream_t s, const NdFac* fac, int B, int nfronts, double*
 // 3 to 11 each), against 490 us with v staged by the workgroup before it loads Q
 // and rows of X and Q in turn (leaves 26 and 111, levels 9 to 19).
 //
+// Grid row y is a solve of its own: the sideband factors of a modulated device are
+// applied in one launch a level (three on 500 x 200: 8.2 ms a solve, 10.9 one by one).
+// A lone solve passes its own arguments only.
+//
 // Upward step of a level: the separator values
 //   v = scaled right-hand side + children's updates
 // and the boundary update u = children's updates - Q^T v.  A task is CL boundary
@@ -1122,9 +1126,10 @@ void launch_nd_stat(hipStream_t s, const NdFac* fac, int B, int nfronts, double*
 // ---------------------------------------------------------------------------
 constexpr int UP_MU = 8;  // rows of Q a lane loads at a time
 
-template <int CL, int KW>
-__global__ __launch_bounds__(KW > 4 ? 64 * KW : 256) void k_nd_up(NdLev lv, const void* arena, NdVec z, int Nx,
-                                                                 int nchunk) {
+template <int CL, int KW, int NS>
+__global__ __launch_bounds__(KW > 4 ? 64 * KW : 256) void k_nd_up(NdLev lv, NdBatch<NS> bt, int Nx, int nchunk) {
+    const NdVec& z = bt.s[NS > 1 ? blockIdx.y : 0].z;
+    const void* arena = bt.s[NS > 1 ? blockIdx.y : 0].arena;
     constexpr int RG = 64 / CL, NW = KW > 4 ? KW : 4;  // row groups of a wave, waves
     __shared__ C vs[NW][64];
     __shared__ C red[KW > 1 ? KW : 1][CL];
@@ -1209,8 +1214,10 @@ __global__ __launch_bounds__(KW > 4 ? 64 * KW : 256) void k_nd_up(NdLev lv, cons
 // Downward step: x = X v - Q x_boundary.  A task is RW rows of one front, whose
 // columns (of X, then of Q) are spread over the lanes of KW waves; the sums over
 // the lanes are folded so that each exchange halves the rows a lane holds.
-template <int RW, int KW>
-__global__ __launch_bounds__(256) void k_nd_down(NdLev lv, const void* arena, NdVec z, int Nx, int nchunk) {
+template <int RW, int KW, int NS>
+__global__ __launch_bounds__(256) void k_nd_down(NdLev lv, NdBatch<NS> bt, int Nx, int nchunk) {
+    const NdVec& z = bt.s[NS > 1 ? blockIdx.y : 0].z;
+    const void* arena = bt.s[NS > 1 ? blockIdx.y : 0].arena;
     constexpr int MU = RW >= 8 ? 2 : 8 / RW;  // columns a lane takes at a time
     __shared__ C red[KW][RW];
     const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -1297,31 +1304,37 @@ __global__ __launch_bounds__(256) void k_nd_down(NdLev lv, const void* arena, Nd
 // 160 / 186 ms; a modulated device of 500 x 200: 10.6 / 10.5 / 11.4 / 11.8 ms.
 constexpr long ND_WAVES = 1024;
 
-void launch_nd_up(hipStream_t s, const NdLev& lv, const void* arena, const NdVec& z, int Nx) {
-    auto tasks = [&](int CL) { return (long)lv.cnt * std::max(1, (lv.b + CL - 1) / CL); };
+template <int NS>
+void launch_nd_up(hipStream_t s, const NdLev& lv, const NdBatch<NS>& bt, int nb, int Nx) {
+    auto chunks = [&](int CL) { return std::max(1, (lv.b + CL - 1) / CL); };
+    auto tasks = [&](int CL) { return (long)lv.cnt * chunks(CL) * nb; };
     auto go = [&](auto kern, int CL, int KW) {
-        const long n = tasks(CL);
-        const int per = KW > 1 ? 1 : 4, NT = KW > 4 ? 64 * KW : 256;
-        kern<<<(unsigned)((n + per - 1) / per), NT, 0, s>>>(lv, arena, z, Nx, (int)(n / lv.cnt));
+        const int n = lv.cnt * chunks(CL), per = KW > 1 ? 1 : 4, NT = KW > 4 ? 64 * KW : 256;
+        kern<<<dim3((n + per - 1) / per, nb), NT, 0, s>>>(lv, bt, Nx, chunks(CL));
     };
-    if (lv.p <= 16 && tasks(64) >= ND_WAVES) go(k_nd_up<64, 1>, 64, 1);
-    else if (tasks(32) >= ND_WAVES) go(k_nd_up<32, 1>, 32, 1);
-    else if (tasks(16) >= ND_WAVES) go(k_nd_up<16, 1>, 16, 1);
-    else if (lv.p <= 64 || tasks(16) * 4 >= ND_WAVES) go(k_nd_up<16, 4>, 16, 4);
-    else go(k_nd_up<8, 16>, 8, 16);
+    if (lv.p <= 16 && tasks(64) >= ND_WAVES) go(k_nd_up<64, 1, NS>, 64, 1);
+    else if (tasks(32) >= ND_WAVES) go(k_nd_up<32, 1, NS>, 32, 1);
+    else if (tasks(16) >= ND_WAVES) go(k_nd_up<16, 1, NS>, 16, 1);
+    else if (lv.p <= 64 || tasks(16) * 4 >= ND_WAVES) go(k_nd_up<16, 4, NS>, 16, 4);
+    else go(k_nd_up<8, 16, NS>, 8, 16);
 }
-void launch_nd_down(hipStream_t s, const NdLev& lv, const void* arena, const NdVec& z, int Nx) {
-    auto tasks = [&](int RW) { return (long)lv.cnt * ((lv.p + RW - 1) / RW); };
+template <int NS>
+void launch_nd_down(hipStream_t s, const NdLev& lv, const NdBatch<NS>& bt, int nb, int Nx) {
+    auto chunks = [&](int RW) { return (lv.p + RW - 1) / RW; };
+    auto tasks = [&](int RW) { return (long)lv.cnt * chunks(RW) * nb; };
     auto go = [&](auto kern, int RW, int KW) {
-        const long n = tasks(RW);
-        const int per = KW > 1 ? 1 : 4;
-        kern<<<(unsigned)((n + per - 1) / per), 256, 0, s>>>(lv, arena, z, Nx, (int)(n / lv.cnt));
+        const int n = lv.cnt * chunks(RW), per = KW > 1 ? 1 : 4;
+        kern<<<dim3((n + per - 1) / per, nb), 256, 0, s>>>(lv, bt, Nx, chunks(RW));
     };
-    if (tasks(8) >= ND_WAVES) go(k_nd_down<8, 1>, 8, 1);
-    else if (tasks(4) * 4 >= ND_WAVES) go(k_nd_down<4, 4>, 4, 4);
-    else if (tasks(2) * 4 >= ND_WAVES) go(k_nd_down<2, 4>, 2, 4);
-    else go(k_nd_down<1, 4>, 1, 4);
+    if (tasks(8) >= ND_WAVES) go(k_nd_down<8, 1, NS>, 8, 1);
+    else if (tasks(4) * 4 >= ND_WAVES) go(k_nd_down<4, 4, NS>, 4, 4);
+    else if (tasks(2) * 4 >= ND_WAVES) go(k_nd_down<2, 4, NS>, 2, 4);
+    else go(k_nd_down<1, 4, NS>, 1, 4);
 }
+template void launch_nd_up(hipStream_t, const NdLev&, const NdBatch<1>&, int, int);
+template void launch_nd_up(hipStream_t, const NdLev&, const NdBatch<ND_SOLVES>&, int, int);
+template void launch_nd_down(hipStream_t, const NdLev&, const NdBatch<1>&, int, int);
+template void launch_nd_down(hipStream_t, const NdLev&, const NdBatch<ND_SOLVES>&, int, int);
 
 // ---------------------------------------------------------------------------
 // The reduced solve for 2 .. 16 sources on MFMA (16 x 16 x 4).  Work vectors

@@ -119,6 +119,9 @@ extern "C" int fdfd_modulated_solve(fdfd_handle* hh, double omega, double Omega,
         return FDFD_OK;
     };
     auto prec = [&](const double2* v, double2* z) -> int {
+        // (a factor with a bad pivot is one by lines)
+        if (std::all_of(Fs.begin(), Fs.end(), [&](Factor* F) { return F->nd && F->nd == Fs[0]->nd; }))
+            return rt_nd_solve_each(h, Fs, v, z, h->prof.enabled);
         for (int j = 0; j < nf; ++j) {
             const int r = rt_prec_apply(h, Fs[j], 0, v + (long)j * N, z + (long)j * N);
             if (r) return r;

@@ -298,11 +298,9 @@ int rt_build_nd(Handle* h, const std::vector<Factor*>& Fs, std::vector<int>& bad
 // out = A'^-1 in or A'^-T in for na sources (source ridx[i] at ridx[i] * rs;
 // ridx null: one source).  S = U^-1 A' U gives A'^-1 = U S^-1 U^-1 and
 // A'^-T = U^-1 S^-1 U.
-int rt_nd_solve(Handle* h, Factor* F, int trans, const double2* in, double2* out, long rs,
-                const int* ridx, int na, bool prof) {
-    const NdPlan& P = *F->nd;
-    const long N = (long)P.Nx * P.Ny, per = P.vlen + P.ulen + N;
-    const size_t need = sizeof(double2) * (size_t)per * (na == 1 ? 1 : KMULTI);
+// work vectors of `count` solves, in the handle's buffer
+static int nd_vectors(Handle* h, long per, int count, double2** v) {
+    const size_t need = sizeof(double2) * (size_t)per * count;
     if (h->nd_vec_bytes < need) {
         if (h->nd_vec) {
             HIPCHK(h, hipStreamSynchronize(h->stream));
@@ -313,11 +311,27 @@ int rt_nd_solve(Handle* h, Factor* F, int trans, const double2* in, double2* out
         HIPCHK(h, hipMalloc(&h->nd_vec, need));
         h->nd_vec_bytes = need;
     }
-    double2* v = (double2*)h->nd_vec;
-    static_assert(KMULTI == 16, "the multi-source kernels hold 16 sources");
+    *v = (double2*)h->nd_vec;
+    return FDFD_OK;
+}
+
+// in -> out with the factor's scalings; v: its work vectors
+static NdVec nd_vec(const Factor* F, int trans, const double2* in, double2* out, long rs, const int* ridx, double2* v) {
+    const NdPlan& P = *F->nd;
     const double2 *ux = F->ndu, *uxi = ux + P.Nx, *uy = ux + 2 * P.Nx, *uyi = uy + P.Ny;
-    NdVec z{in, out, rs, ridx, v, v + P.vlen, v + P.vlen + P.ulen,
-            trans ? ux : uxi, trans ? uy : uyi, trans ? uxi : ux, trans ? uyi : uy};
+    return NdVec{in, out, rs, ridx, v, v + P.vlen, v + P.vlen + P.ulen,
+                 trans ? ux : uxi, trans ? uy : uyi, trans ? uxi : ux, trans ? uyi : uy};
+}
+
+int rt_nd_solve(Handle* h, Factor* F, int trans, const double2* in, double2* out, long rs,
+                const int* ridx, int na, bool prof) {
+    const NdPlan& P = *F->nd;
+    const long N = (long)P.Nx * P.Ny, per = P.vlen + P.ulen + N;
+    double2* v;
+    int rc = nd_vectors(h, per, na == 1 ? 1 : KMULTI, &v);
+    if (rc) return rc;
+    static_assert(KMULTI == 16, "the multi-source kernels hold 16 sources");
+    const NdVec z = nd_vec(F, trans, in, out, rs, ridx, v);
     const int nl = (int)P.lev.size();
     ProfScope* ps = prof ? new ProfScope(h, P_SWEEP, 0, 0) : nullptr;
     if (na > 1) {
@@ -326,14 +340,36 @@ int rt_nd_solve(Handle* h, Factor* F, int trans, const double2* in, double2* out
         for (int li = nl - 1; li >= 0; --li) launch_ndm_up(h->stream, P.lev[li], F->blocks, vp, up, xp);
         for (int li = 0; li < nl; ++li) launch_ndm_down(h->stream, P.lev[li], F->blocks, vp, xp);
         launch_ndm_io(h->stream, z, xp, N, P.Nx, na, false);
-        delete ps;
-        return FDFD_OK;
+    } else {
+        NdBatch<1> bt{};
+        bt.s[0].z = z;
+        bt.s[0].arena = F->blocks;
+        for (int li = nl - 1; li >= 0; --li) launch_nd_up(h->stream, P.lev[li], bt, 1, P.Nx);
+        for (int li = 0; li < nl; ++li) launch_nd_down(h->stream, P.lev[li], bt, 1, P.Nx);
     }
-    for (int li = nl - 1; li >= 0; --li) {
-        launch_nd_up(h->stream, P.lev[li], F->blocks, z, P.Nx);
-    }
-    for (int li = 0; li < nl; ++li) {
-        launch_nd_down(h->stream, P.lev[li], F->blocks, z, P.Nx);
+    delete ps;
+    return FDFD_OK;
+}
+
+// out_j = M_j^-1 in_j for the factors of one grid, N values apart
+int rt_nd_solve_each(Handle* h, const std::vector<Factor*>& Fs, const double2* in, double2* out, bool prof) {
+    const NdPlan& P = *Fs[0]->nd;
+    const long N = (long)P.Nx * P.Ny, per = P.vlen + P.ulen + N;
+    const int nf = (int)Fs.size(), nl = (int)P.lev.size();
+    double2* v;
+    int rc = nd_vectors(h, per, std::min(nf, ND_SOLVES), &v);
+    if (rc) return rc;
+    ProfScope* ps = prof ? new ProfScope(h, P_SWEEP, 0, 0) : nullptr;
+    for (int f0 = 0; f0 < nf; f0 += ND_SOLVES) {
+        const int nb = std::min(ND_SOLVES, nf - f0);
+        NdBatch<ND_SOLVES> bt{};
+        for (int q = 0; q < nb; ++q) {
+            const long o = (long)(f0 + q) * N;
+            bt.s[q].z = nd_vec(Fs[f0 + q], 0, in + o, out + o, 0, nullptr, v + q * per);
+            bt.s[q].arena = Fs[f0 + q]->blocks;
+        }
+        for (int li = nl - 1; li >= 0; --li) launch_nd_up(h->stream, P.lev[li], bt, nb, P.Nx);
+        for (int li = 0; li < nl; ++li) launch_nd_down(h->stream, P.lev[li], bt, nb, P.Nx);
     }
     delete ps;
     return FDFD_OK;

@@ -58,8 +58,16 @@ void launch_nd_invert(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, c
 void launch_nd_gemm(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, const void* F12,
                     const void* Sc, void* S, bool schur);
 void launch_nd_stat(hipStream_t s, const NdFac* fac, int B, int nfronts, double* out);
-void launch_nd_up(hipStream_t s, const NdLev& lv, const void* arena, const NdVec& z, int Nx);
-void launch_nd_down(hipStream_t s, const NdLev& lv, const void* arena, const NdVec& z, int Nx);
+// independent solves with factors of one tree, side by side
+constexpr int ND_SOLVES = 8;
+template <int N> struct NdBatch {
+    struct {
+        NdVec z;
+        const void* arena;
+    } s[N];
+};
+template <int N> void launch_nd_up(hipStream_t s, const NdLev& lv, const NdBatch<N>& bt, int nb, int Nx);
+template <int N> void launch_nd_down(hipStream_t s, const NdLev& lv, const NdBatch<N>& bt, int nb, int Nx);
 // several sources (at most 16): pack / unpack, one level up, one level down
 void launch_ndm_io(hipStream_t s, const NdVec& z, void* x, long N, int Nx, int na, bool pack);
 void launch_ndm_up(hipStream_t s, const NdLev& lv, const void* arena, void* vp, void* up, const void* x);

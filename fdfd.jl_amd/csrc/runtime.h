@@ -284,6 +284,7 @@ int rt_nd_prepare(Handle* h, int Nx, int Ny);
 // refinement failed on them is then tried once more)
 int rt_rebuild_by_lines(Handle* h, const std::vector<Factor*>& Fs);
 int rt_build_nd(Handle* h, const std::vector<Factor*>& Fs, std::vector<int>& bad);
+int rt_nd_solve_each(Handle* h, const std::vector<Factor*>& Fs, const double2* in, double2* out, bool prof);
 int rt_nd_solve(Handle* h, Factor* F, int trans, const double2* in, double2* out, long rs,
                 const int* ridx, int na, bool prof);
 size_t rt_factor_bytes(int n, int m, int precision, bool b3);

@@ -107,3 +107,20 @@ def test_leaf_fronts_of_every_size(monkeypatch, Nx, Ny):
             e.release(fid)
     finally:
         e.close()
+
+
+@pytest.mark.parametrize("K", [3, 4])
+def test_sideband_factors_side_by_side(K):
+    """Seven and nine sideband factors: fewer and more than one launch takes
+    (eight).  Same bar as the modulated solve's other tests, 1e-10 of the largest
+    sideband at a residual of 1e-13."""
+    from test_gpu_modulated import _check, _pair
+    from fdfd.modulated import solve_modulated
+    d, o = _pair(48, 40, 4, K, True, seed=20 + K)
+    e = Engine(0)
+    try:
+        fg, st = solve_modulated(d, precision="fp64", tol=1e-13, eng=e, return_stats=True)
+        assert st[0]["residual"] <= 1e-13
+        _check(fg[0], O.solve_modulated(o)[0], f"K={K}")
+    finally:
+        e.close()
