@@ -411,14 +411,18 @@ template <int NF> struct NdCells {
     int x[NF], y[NF];  // x < 0: no cell
     __device__ inline void load(const int* node, int n, const double2* coef, long N, int Nx) {
         for (int e = threadIdx.x; e < 3 * NF; e += 256) {
-            const int i = e % NF, pl = e / NF;
-            const int k = i < n ? node[i] : -1, kk = max(k, 0);
-            const C c = gload(coef + (long)(pl == 0 ? CC : pl == 1 ? CE : CN) * N + kk);
-            (pl == 0 ? cc : pl == 1 ? ce : cn)[i] = c;
-            if (pl == 0) {
-                x[i] = k < 0 ? -1 : k % Nx;
-                y[i] = kk / Nx;
-            }
+            const int i = e % NF;
+            put(i, e / NF, i < n ? node[i] : -1, coef, N, Nx);
+        }
+    }
+    // plane pl of row i, cell k
+    __device__ inline void put(int i, int pl, int k, const double2* coef, long N, int Nx) {
+        const int kk = max(k, 0);
+        const C c = gload(coef + (long)(pl == 0 ? CC : pl == 1 ? CE : CN) * N + kk);
+        (pl == 0 ? cc : pl == 1 ? ce : cn)[i] = c;
+        if (pl == 0) {
+            x[i] = k < 0 ? -1 : k % Nx;
+            y[i] = kk / Nx;
         }
     }
     // entry (i, j) of the symmetrised operator, a unit row where there is no cell
@@ -606,6 +610,155 @@ void launch_nd_front(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, in
     else if (lv.p <= 32) k_nd_front<2><<<g, 256, 0, s>>>(lv, fac, Nx, Ny, Sc, w, nch);
     else if (lv.p <= 48) k_nd_front<3><<<g, 256, 0, s>>>(lv, fac, Nx, Ny, Sc, w, nch);
     else k_nd_front<4><<<g, 256, 0, s>>>(lv, fac, Nx, Ny, Sc, w, nch);
+}
+
+// accumulators of a complex 16 x 16 tile: re = rr - ii, im = ri
+struct ndm_acc {
+    typename mfma_t<R>::acc rr = {0, 0, 0, 0}, ii = {0, 0, 0, 0}, ri = {0, 0, 0, 0};
+    __device__ inline void step(C a, C b) {
+        rr = mfma_t<R>::run(a.x, b.x, rr);
+        ii = mfma_t<R>::run(a.y, b.y, ii);
+        ri = mfma_t<R>::run(a.x, b.y, ri);
+        ri = mfma_t<R>::run(a.y, b.x, ri);
+    }
+};
+
+// ---------------------------------------------------------------------------
+// Small fronts whole, one workgroup each (p <= 16, b <= 16 BT): wave 0 gathers and
+// sweeps F11 while the others gather F12, both stay in LDS, then
+//   Q = X F12  and  S = F22 - F12^T Q
+// by 16 x 16 tiles.  The lowest levels have thousands of such fronts and do little
+// arithmetic: what counts is that S is written and the children's read once, and
+// that F12 never leaves the chip.  8192 fronts of 8 cells and 44 boundary cells (1024 x
+// 1024): 173 us, of which 110 at the copy rate; 332 us as assembly, Q and S in turn.
+// 16 cells with 92: 142 us against 184.
+// ---------------------------------------------------------------------------
+template <int BT>
+__global__ __launch_bounds__(256, 2) void k_nd_small(NdLev lv, const NdFac* fac, int Nx, int Ny, const void* Scv,
+                                                     void* Sv) {
+    constexpr int NF = 16 + 16 * BT, LC = 16 * BT + 1;
+    __shared__ NdCells<NF> cl;
+    __shared__ short cm[2][NF];  // places in the children; front rows: 16 for F11, then b
+    __shared__ C F12[16][LC], Qs[16][LC], X[16][17];
+    const int q = blockIdx.y, fr = blockIdx.x, p = lv.p, b = lv.b, f = p + b;
+    const NdFac F = fac[q];
+    const int t = threadIdx.x, lane = t & 63, l16 = lane & 15, g = lane >> 4;
+    const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
+    const long N = (long)Nx * Ny, job = (long)q * lv.cnt + fr;
+    const C* Sc = (const C*)Scv + ((long)q * lv.cnt * lv.nch + (long)fr * lv.nch) * lv.cb * lv.cb;
+    const int* node = lv.node + (long)fr * f;
+    const short* cmg = lv.cm + (long)fr * 2 * f;
+    // row r of the padded front -> index in the front, -1 outside
+    auto at = [&](int r) { return r < 16 ? (r < p ? r : -1) : (r - 16 < b ? p + r - 16 : -1); };
+    for (int e = t; e < 3 * NF; e += 256) {
+        const int r = e % NF, pl = e / NF, i = at(r), k = i >= 0 ? node[i] : -1;
+        cl.put(r, pl, k, F.coef, N, Nx);
+        if (pl > 0) cm[pl - 1][r] = i >= 0 && pl <= lv.nch ? cmg[(pl - 1) * f + i] : -1;
+    }
+    __syncthreads();
+    // the children's part of rows 4 v + g and column c: loaded (entry 0 where there is
+    // none) before any is used
+    auto kids = [&](int r0, int c, C (&o)[4]) {
+        const int n0 = cm[0][c], n1 = cm[1][c];
+        C a[4], d[4];
+        int m0[4], m1[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            m0[v] = cm[0][r0 + F64::row(lane, v)];
+            m1[v] = cm[1][r0 + F64::row(lane, v)];
+            a[v] = gload(Sc + (m0[v] >= 0 && n0 >= 0 ? (long)m0[v] * lv.cb + n0 : 0));
+            d[v] = gload(Sc + (m1[v] >= 0 && n1 >= 0 ? ((long)lv.cb + m1[v]) * lv.cb + n1 : 0));
+        }
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const bool k0 = m0[v] >= 0 && n0 >= 0, k1 = m1[v] >= 0 && n1 >= 0;
+            o[v] = mk<C>((k0 ? a[v].x : 0.0) + (k1 ? d[v].x : 0.0), (k0 ? a[v].y : 0.0) + (k1 ? d[v].y : 0.0));
+        }
+    };
+    if (wv == 0) {
+        C o[4];
+        kids(0, l16, o);
+        d4v mr, mi;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const C z = cl.entry(F64::row(lane, v), l16, Nx, Ny);
+            mr[v] = z.x + o[v].x;
+            mi[v] = z.y + o[v].y;
+        }
+        NdPiv pv;
+        nd_sweep16(mr, mi, p, X, pv);
+        C* Xg = (C*)F.arena + lv.offX + (long)fr * p * p;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int i = F64::row(lane, v);
+            const C z = mk<C>(mr[v], mi[v]);
+            X[i][l16] = z;
+            if (i < p && l16 < p) gstore(Xg + i * p + l16, z);
+        }
+        if (lane == 0) {
+            double* pst = F.pivstat + 3 * (long)(lv.stat + fr);
+            pst[0] = pv.mn;
+            pst[1] = pv.mx;
+            pst[2] = pv.bad ? 1.0 : 0.0;
+        }
+    } else {
+        for (int c = wv - 1; 16 * c < b; c += 3) {
+            C o[4];
+            kids(0, 16 + 16 * c + l16, o);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int i = F64::row(lane, v), j = 16 * c + l16;
+                const bool ok = i < p && j < b;
+                F12[i][j] = csel(ok, cadd(cl.entry(i, 16 + j, Nx, Ny), o[v]), mk<C>(0, 0));
+            }
+        }
+    }
+    __syncthreads();
+    const int nt = (b + 15) / 16;
+    C* Qg = (C*)F.arena + lv.offQ + (long)fr * p * b;
+    for (int c = wv; c < nt; c += 4) {
+        ndm_acc A;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) A.step(X[4 * s + g][l16], F12[4 * s + g][16 * c + l16]);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int i = F64::row(lane, v), j = 16 * c + l16;
+            const C z = mk<C>(A.rr[v] - A.ii[v], A.ri[v]);
+            Qs[i][j] = z;
+            if (i < p && j < b) gstore(Qg + i * b + j, z);
+        }
+    }
+    __syncthreads();
+    C* S = (C*)Sv + job * b * b;
+    for (int e = wv; e < nt * (nt + 1) / 2; e += 4) {
+        int I = 0;
+#pragma unroll
+        for (int u = 1; u < BT; ++u) I += e >= u * (u + 1) / 2;
+        const int J = e - I * (I + 1) / 2, j = 16 * J + l16;
+        C o[4];
+        kids(16 + 16 * I, 16 + j, o);
+        ndm_acc A;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) A.step(F12[4 * s + g][16 * I + l16], Qs[4 * s + g][j]);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int i = 16 * I + F64::row(lane, v);
+            const C z = csub(o[v], mk<C>(A.rr[v] - A.ii[v], A.ri[v]));
+            if (i < b && j < b) {
+                gstore(S + (long)i * b + j, z);
+                if (I != J) gstore(S + (long)j * b + i, z);  // (four lanes write 64 bytes)
+            }
+        }
+    }
+}
+
+bool launch_nd_small(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, int Nx, int Ny, const void* Sc,
+                     void* S) {
+    if (lv.p > 16 || lv.b == 0 || lv.b > 96) return false;
+    const dim3 g(lv.cnt, B);
+    if (lv.b <= 64) k_nd_small<4><<<g, 256, 0, s>>>(lv, fac, Nx, Ny, Sc, S);
+    else k_nd_small<6><<<g, 256, 0, s>>>(lv, fac, Nx, Ny, Sc, S);
+    return true;
 }
 
 // ---------------------------------------------------------------------------
@@ -1399,17 +1552,6 @@ __global__ __launch_bounds__(256) void k_ndm_gather(NdLev lv, C* vp, C* up, cons
     if (i < lv.p) gstore(vp + (lv.offV + (long)fr * lv.p + i) * 16 + s, v);
     else gstore(up + (lv.offU + (long)fr * lv.b + (i - lv.p)) * 16 + s, v);
 }
-
-// accumulators of a complex 16 x 16 tile: re = rr - ii, im = ri
-struct ndm_acc {
-    typename mfma_t<R>::acc rr = {0, 0, 0, 0}, ii = {0, 0, 0, 0}, ri = {0, 0, 0, 0};
-    __device__ inline void step(C a, C b) {
-        rr = mfma_t<R>::run(a.x, b.x, rr);
-        ii = mfma_t<R>::run(a.y, b.y, ii);
-        ri = mfma_t<R>::run(a.x, b.y, ri);
-        ri = mfma_t<R>::run(a.y, b.x, ri);
-    }
-};
 
 // f(r, value) for the tile's entries v = r of this wave's lanes; with KS waves their
 // tiles are added through LDS, entry r by wave r

@@ -255,6 +255,10 @@ int rt_build_nd(Handle* h, const std::vector<Factor*>& Fs, std::vector<int>& bad
             delete ps;
             continue;
         }
+        if (launch_nd_small(st, v, dfac, B, g.Nx, g.Ny, Sc, S)) {
+            delete ps;
+            continue;
+        }
         launch_nd_front(st, v, dfac, B, g.Nx, g.Ny, Sc, iw);
         delete ps;
         ps = scope(P_PANEL, 4 * p * p * p * nj, 0);

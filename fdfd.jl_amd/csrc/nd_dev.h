@@ -52,6 +52,9 @@ void launch_nd_maps(hipStream_t s, const NdMapArgs& a, int* node, short* cm);
 void launch_nd_symmetrise(hipStream_t s, double2* coef, double2* us, const double2* wx,
                           const double2* wy, int Nx, int Ny);
 void launch_nd_leaf(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, int Nx, int Ny, void* S);
+// a level of small fronts in one launch; false if they are not
+bool launch_nd_small(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, int Nx, int Ny, const void* Sc,
+                     void* S);
 void launch_nd_front(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, int Nx, int Ny, const void* Sc,
                      const NdInv& w);
 void launch_nd_invert(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, const NdInv& w);

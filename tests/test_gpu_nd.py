@@ -124,3 +124,11 @@ def test_sideband_factors_side_by_side(K):
         _check(fg[0], O.solve_modulated(o)[0], f"K={K}")
     finally:
         e.close()
+
+
+@pytest.mark.parametrize("Nx,Ny", [(17, 300), (17, 17), (26, 26), (32, 32), (34, 34), (36, 36), (100, 16)])
+def test_small_fronts_whole(monkeypatch, Nx, Ny):
+    """Levels of 4, 8, 12 and 16 separator cells with 16 to 84 boundary cells, on
+    both sides of 64, where the kernel of whole fronts changes size; one child or
+    two.  Same bar as the leaves'."""
+    test_leaf_fronts_of_every_size(monkeypatch, Nx, Ny)
