@@ -1,8 +1,9 @@
-"""Benchmark: TM solves/s at 1024^2 to 1e-10 relative residual, mixed
-(complex64 block factors + FP64 FGMRES refinement) vs plain FP64 block factors.
+"""Benchmark: TM solves/s at 1024^2 to 1e-10 relative residual, precision
+"mixed" vs "fp64" (both complex128 dissected factors + FP64 FGMRES refinement
+on this grid; the mixed-fp32* legs take the complex64 line reduction).
 
-One step = set eps (device-resident) -> assemble + factor (block cyclic
-reduction of the line ring) on the GPU -> refined solve of one source ->
+One step = set eps (device-resident) -> assemble + factor (nested dissection of
+the grid) on the GPU -> refined solve of one source ->
 field recovery (Ez, Hx, Hy) into a device-resident output.  Inputs are in
 HBM before the timed region starts.
 
@@ -250,7 +251,7 @@ def c3_leg(eng):
     _, st = eng.batch_solve(spec, precision="mixed", tol=1e-10, fetch=[])
     wall = time.perf_counter() - t0
     return {"workload": "3 grids (256^2, 384x512, 512^2) x 64 wavelengths (1.50-1.60 um) x 16 "
-                        "point sources, complex64 factors + FP64 FGMRES to 1e-10, one call",
+                        "point sources, precision mixed (dissected c128 factors) + FP64 FGMRES to 1e-10, one call",
             "solves": nsolve, "factorizations": 192, "wall_s": wall, "solves_per_s": nsolve / wall,
             "cold_wall_s": cold, "factor_ms": st["t_factor_ms"], "solve_ms": st["t_solve_ms"],
             "fgmres_its": st["iterations"], "worst_residual": st["residual"]}
@@ -324,10 +325,9 @@ def main():
     ap.add_argument("--no-legs", action="store_true",
                     help="skip every leg but the headline TM solves (profiling runs)")
     ap.add_argument("--precisions", default="mixed,fp64,mixed-fp32gemm,mixed-fp32",
-                    help="mixed: complex64 factors with fp16x3 GEMM and trailing products (default "
-                         "mixed path); mixed-fp32gemm: FP32 MFMA GEMMs, fp16x3 trailing updates; "
-                         "mixed-fp32: FP32 MFMA GEMMs and trailing updates; fp64: complex128 "
-                         "factors")
+                    help="mixed, fp64: dissected complex128 factors; mixed-fp32gemm, mixed-fp32: the "
+                         "line reduction with complex64 factors, FP32 MFMA GEMMs and fp16x3 or FP32 "
+                         "MFMA trailing updates")
     ap.add_argument("--probe-copy", type=int, default=0, metavar="MIB",
                     help="only run 4 device-to-device copies of MIB MiB (calibrates the "
                          "FETCH_SIZE / WRITE_SIZE counters against a known byte count)")
@@ -437,19 +437,15 @@ def main():
         kd = {"ms": 0.0, "launches": 1, "flops": 0.0, "bytes": 0.0}
     avg_s = kd["ms"] / kd["launches"] / 1e3
     # roofline of the dominant kernel against the published peak of the MFMA
-    # instructions it runs (fp16 for the split-operand GEMM, FP32 or FP64
-    # otherwise) or of HBM; achieved = algorithmic flops (8 n^3 per complex
-    # GEMM) or bytes per launch / average launch time
-    if head == "mixed":
-        ptype = "fp16" if (dom == "gemm" or dom == "trailing") else "fp32"
-    elif head.startswith("mixed"):
-        ptype = "fp32"
-    else:
-        ptype = "fp64"
+    # instructions it runs (FP64 for dissected factors, FP32 for the line
+    # reduction's legs) or of HBM; achieved = algorithmic flops (8 per complex
+    # multiply-add) or bytes per launch / average launch time
+    dissected = head in ("mixed", "fp64")
+    ptype = "fp64" if dissected else "fp32"
     mpeak = PEAK[ptype]
-    # executed MFMA work per algorithmic flop: fp16x3 forms each real product
-    # from three fp16 products
-    exec_factor = 3.0 if ptype == "fp16" else 1.0
+    # executed MFMA work per algorithmic flop: dissected products form a complex
+    # one from three real ones
+    exec_factor = 0.75 if dissected else 1.0
     per_launch_f = kd["flops"] / kd["launches"]
     per_launch_b = kd["bytes"] / kd["launches"]
     t_m = per_launch_f / mpeak
@@ -461,8 +457,8 @@ def main():
                 "peak_note": f"published dense {ptype} MFMA peak of MI355X",
                 "mfma_executed_tflops": exec_factor * achieved / 1e12,
                 "mfma_executed_frac": exec_factor * achieved / mpeak,
-                "executed_note": ("fp16x3 split products: 3 fp16 MFMA products per real "
-                                  "product" if exec_factor > 1 else "executed = algorithmic")}
+                "executed_note": ("three real MFMA products per complex product"
+                                  if exec_factor < 1 else "executed = algorithmic")}
         if per_launch_b > 0:
             roof["hbm_achieved_GBps"] = per_launch_b / avg_s / 1e9
             roof["flop_per_byte"] = per_launch_f / per_launch_b
@@ -481,10 +477,10 @@ def main():
     if os.path.exists(pmc):
         with open(pmc) as fh:
             P = json.load(fh)
-        rt = "float" if head.startswith("mixed") else "double"
-        trail = "k_trailing_h3" if head == "mixed" and n % 4 == 0 else "k_trailing<" + rt
-        prefix = {"gemm": "k_gemm_b3" if head == "mixed" else "k_gemm<" + rt,
-                  "trailing": trail, "solve": "k_mv<" + rt}.get(dom)
+        if dissected:
+            prefix = {"gemm": "k_nd_gemm", "solve": "k_nd_down"}.get(dom)
+        else:
+            prefix = {"gemm": "k_gemm<float", "trailing": "k_trailing<float", "solve": "k_mv<float"}.get(dom)
         for name, v in P["kernels"].items():
             if prefix and name.startswith(prefix):
                 roof["traffic"] = v["read_bytes"] + v["write_bytes"]
@@ -492,9 +488,11 @@ def main():
                 roof["traffic_source"] = os.path.relpath(pmc, ROOT)
                 break
     roof["avg_launch_us"] = avg_s * 1e6
-    # whole-factorization figure: F = 8 n^3 m real flops per factorization
-    roof["factor_tflops"] = 8.0 * n ** 3 * n / (R["factor_ms"] / 1e3) / 1e12
-    roof["factor_frac_fp32_peak"] = roof["factor_tflops"] * 1e12 / PEAK["fp32"]
+    # whole-factorization figure: the counted algorithmic flops of its products and
+    # inversions (no count without profiled steps)
+    fflops = sum(R["kernels"][k]["flops"] for k in ("gemm", "trailing", "panel") if k in R["kernels"])
+    roof["factor_tflops"] = fflops / max(1, a.profile_steps) / (R["factor_ms"] / 1e3) / 1e12
+    roof["factor_frac_peak"] = roof["factor_tflops"] * 1e12 / mpeak
     # the stencil / residual kernel (matrix-free operator apply, 64 B/cell)
     ks = R["kernels"]["stencil"]
     stencil = None
@@ -538,8 +536,7 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": ("c64 factors (GEMM and trailing products fp16x3 on row-scaled split operands, "
-                  "FP32 accumulation) + c128 refinement" if head == "mixed" else "c128"),
+        "dtype": "c128" if dissected else "c64 factors + c128 refinement",
         "data": "synthetic (seeded random-pixel coupler, generated in-process)",
         "config": {
             "workload": (f"TM driven solve, {n}x{n} cells, dl=0.02 um, 20-cell SC-PML, 600x600 "

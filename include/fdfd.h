@@ -121,11 +121,12 @@ int fdfd_set_eps_d(fdfd_handle* h, const void* d_eps);
 /* ---- factorization ------------------------------------------------------ */
 /* Assembles the TM (driven.jl:35) or TE (driven.jl:45) operator at angular
  * frequency omega (rad/s, normalised units c0/L0 as in device.jl:40) on the
- * device and factors it by block cyclic reduction of its ring of grid lines
- * (the y-periodic corner blocks close the ring): every reduction level
- * inverts every other line's dense block by Gauss-Jordan elimination with
- * threshold partial pivoting (|pivot| >= 0.1 x the column's largest
- * candidate) and folds its couplings into its neighbours with complex GEMMs.
+ * device and factors it by nested dissection of its torus of cells, or (a
+ * side below 16 cells, and where the options above select it) by block cyclic
+ * reduction of its ring of grid lines: every reduction level inverts every
+ * other line's dense block by Gauss-Jordan elimination with threshold partial
+ * pivoting (|pivot| >= 0.1 x the column's largest candidate) and folds its
+ * couplings into its neighbours with complex GEMMs.
  * The factorization is a direct solver of A.  Replaces lu(A) of
  * solver.jl:35. */
 int fdfd_factor(fdfd_handle* h, int pol, double omega, int precision,
