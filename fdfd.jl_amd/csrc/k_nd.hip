@@ -561,7 +561,7 @@ __global__ __launch_bounds__(256, 2) void k_nd_front(NdLev lv, const NdFac* fac,
         __syncthreads();
         nd_sweep<T>(mr, mi, np, s.w, F.pivstat + 3 * (long)(lv.stat + fr), false);
         const bool whole = p <= NB;
-        C* out = whole ? (C*)F.arena + lv.offX + (long)fr * p * p : (C*)w.D + job * NB * NB;
+        C* out = whole ? (C*)F.arena + lv.offX + (long)fr * p * p : (C*)w.D + job * 2 * NB * NB;
         const int ld = whole ? p : NB;
         nd_each_entry<T>([&](auto sc, int v, int i, int j, bool off) {
             const C z = mk<C>(mr[sc][v], mi[sc][v]);
@@ -574,6 +574,7 @@ __global__ __launch_bounds__(256, 2) void k_nd_front(NdLev lv, const NdFac* fac,
     }
     const int r0 = (e % nchunk) * ASM_ROWS, j0 = p > NB ? 0 : p, nr = min(ASM_ROWS, p - r0);
     C* Y = (C*)w.Y + job * p * p;
+    C* R = (C*)w.R + job * NB * p;
     C* G = (C*)w.F12 + job * p * b;
     for (int j = j0 + (int)threadIdx.x; j < f; j += 256) {
         const int kj = node[j], c0 = cm[j], c1 = lv.nch > 1 ? cm[f + j] : -1;
@@ -597,6 +598,7 @@ __global__ __launch_bounds__(256, 2) void k_nd_front(NdLev lv, const NdFac* fac,
             if (r < nr) {
                 if (j >= p) gstore(G + (long)i * b + (j - p), v);
                 else if (j <= (i | (NB - 1))) gstore(Y + (long)i * p + j, v);
+                if (j < NB && i >= NB && p > NB) gstore(R + (long)j * p + i, v);  // the first block row
             }
         }
     }
@@ -762,41 +764,40 @@ bool launch_nd_small(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, in
 }
 
 // ---------------------------------------------------------------------------
-// Separators longer than 64 cells: block sweeps of 64 on the lower tiles of Y.
-// For block k with inverse D^-1 and block row R_J = M_kJ (stored as tile
-// (k, J), or transposed as tile (J, k) for J > k):
-//   k_nd_bz : Z_J = D^-1 R_J; tile (k, J) <- Z_J, tile (J, k) <- -Z_J^T;
-//   k_nd_bu : M_IJ -= sigma_I R_I^T Z_J on the other lower tiles, sigma = -1 for
-//             swept blocks I < k; the first workgroup goes on to sweep tile
-//             (k + 1, k + 1), so the next D^-1 is ready when the other tiles
-//             are.
-// The chain of a block is the product for Z (by halves of a tile, 64 x 32), the
-// product on tile (k + 1, k + 1), on its lower 16 x 16 tiles in the layout of the
-// sweep, and the sweep (23 us).  It bounds a level of few fronts: 47 us a block
-// of the 1024-cell separators of a 1024 x 1024 grid, against 76 us with both
-// products and the sweep in k_nd_bz and the second product on the whole tile.
+// Separators longer than 64 cells: block sweeps of 64 on the lower tiles of Y,
+// one launch a block.  For block k with inverse D^-1 and block row R_J = M_kJ,
+// the workgroup of a lower tile (I, J), I, J != k, forms
+//   Z_J = D^-1 R_J  and  M_IJ -= sigma_I R_I^T Z_J, sigma = -1 for swept I < k,
+// Z_J once more for every I: the chip is mostly idle here, and a launch of its
+// own for Z was 12 us of the chain.  Tile (J, J)'s workgroup also writes Z_J to
+// tile (k, J), or -Z_J^T to (J, k) for J > k.  The first workgroup takes tile
+// (k + 1, k + 1) in the layout of the sweep and sweeps it: the next D^-1; the last
+// one writes its Z for it.  Block rows and inverses are kept twice, the next ones
+// written (by whoever updates a tile of block k + 1) while the present ones are
+// read.
+// The chain of a block is two products and the sweep (23 us).  It bounds a level
+// of few fronts: 45 us a block on a 1024 x 1024 grid (separators of 1024 cells
+// and less), 47 and a launch more with Z on its own, 76 with both products and the
+// sweep in one workgroup before the update's launch.  200 x 120: 35 us, 37.
 // ---------------------------------------------------------------------------
 // The operands of a product over 64 K rows, 64 rows by TN columns, staged 16 K
 // rows at a time through LDS; mm(kk) multiplies K rows kk .. kk + 3 of a stage.
 // pa(k, i) and pb(k, j) give an entry's address, clamped where oka / okb, which
-// zero it at the store to LDS, are false; keep(k, j, v) sees every entry of B
-// (KB: neighbouring threads read neighbouring k of B).
+// zero it at the store to LDS, are false.
 struct NdTile {
     double sAr[16][NB + 16], sAi[16][NB + 16], sBr[16][NB + 16], sBi[16][NB + 16];
 };
-template <bool KB, int TN, typename PA, typename PB, typename OA, typename OB, typename KP, typename MM>
+template <int TN, typename PA, typename PB, typename OA, typename OB, typename MM>
 __device__ __attribute__((always_inline)) inline void nd_staged(NdTile& s, PA&& pa, PB&& pb, OA&& oka, OB&& okb,
-                                                                KP&& keep, MM&& mm) {
+                                                                MM&& mm) {
     constexpr int NE = TN / 16;
     const int t = threadIdx.x;
     C ra[4], rb[NE];
-    auto kB = [&](int e) { return KB ? t & 15 : (t + 256 * e) / TN; };
-    auto jB = [&](int e) { return KB ? (t + 256 * e) >> 4 : (t + 256 * e) % TN; };
     auto load = [&](int k0) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) ra[e] = gload(pa(k0 + ((t + 256 * e) >> 6), t & 63));
 #pragma unroll
-        for (int e = 0; e < NE; ++e) rb[e] = gload(pb(k0 + kB(e), jB(e)));
+        for (int e = 0; e < NE; ++e) rb[e] = gload(pb(k0 + (t + 256 * e) / TN, t % TN));
     };
     load(0);
     for (int k0 = 0; k0 < NB; k0 += 16) {
@@ -810,11 +811,10 @@ __device__ __attribute__((always_inline)) inline void nd_staged(NdTile& s, PA&& 
         }
 #pragma unroll
         for (int e = 0; e < NE; ++e) {
-            const int k = kB(e), j = jB(e);
-            const C v = csel(okb(k0 + k, j), rb[e], mk<C>(0, 0));
-            s.sBr[k][j] = v.x;
-            s.sBi[k][j] = v.y;
-            keep(k0 + k, j, v);
+            const int k = (t + 256 * e) / TN, j = t % TN;
+            const bool ob = okb(k0 + k, j);
+            s.sBr[k][j] = ob ? rb[e].x : 0.0;
+            s.sBi[k][j] = ob ? rb[e].y : 0.0;
         }
         __syncthreads();
         if (k0 + 16 < NB) load(k0 + 16);
@@ -870,104 +870,132 @@ template <int TN> struct NdAcc {
     }
 };
 
-constexpr int ZC = 32;  // columns of Z per workgroup
-
-__global__ __launch_bounds__(256, 2) void k_nd_bz(NdLev lv, NdInv w, int k, int nb) {
-    __shared__ NdTile s;
-    const int per = (nb - 1) * (NB / ZC), fr = blockIdx.x / per, q = blockIdx.y, p = lv.p;
-    const int e = (int)blockIdx.x % per, Jb = e / (NB / ZC), J = Jb + (Jb >= k);
-    const long job = (long)q * lv.cnt + fr;
-    const int jc = J * NB + (e % (NB / ZC)) * ZC;  // first column
-    const int kw = min(NB, p - k * NB), jw = min(ZC, p - jc);
-    C* Y = (C*)w.Y + job * p * p;
-    C* Rb = (C*)w.R + job * NB * p + jc;
-    C* Zb = (C*)w.Z + job * NB * p + jc;
-    const C* D = (const C*)w.D + job * NB * NB;
-    const C zero = mk<C>(0, 0);
-    if (e == 0) {  // tile (k, k) <- D^-1
-        for (int i = threadIdx.x; i < NB * NB; i += 256) {
-            const int r = i >> 6, j = i & 63;
-            if (r < kw && j < kw) gstore(Y + (long)(k * NB + r) * p + k * NB + j, gload(D + i));
-        }
-    }
-    if (jw <= 0) return;
-    auto pd = [&](int kk, int i) { return D + kk * NB + i; };
-    auto okd = [&](int kk, int i) { return kk < kw && i < kw; };
-    auto okr = [&](int kk, int j) { return kk < kw && j < jw; };
-    auto keep = [&](int kk, int j, C v) {
-        if (j < jw) gstore(Rb + (long)kk * p + j, v);
-    };
-    NdAcc<ZC> A;
-    auto mm = [&](int kk) { A.mul(s, kk); };
-    const bool lower = J < k;
-    C* T = lower ? Y + (long)k * NB * p + jc : Y + (long)jc * p + k * NB;
-    if (lower)
-        nd_staged<false, ZC>(s, pd, [&](int kk, int j) { return T + (long)min(kk, kw - 1) * p + min(j, jw - 1); }, okd,
-                             okr, keep, mm);
-    else
-        nd_staged<true, ZC>(s, pd, [&](int kk, int j) { return T + (long)min(j, jw - 1) * p + min(kk, kw - 1); }, okd,
-                            okr, keep, mm);
-    // (the tile was read, by this workgroup alone, before the last barrier)
-    A.each([&](int i, int j, C z) {
-        if (j >= jw) return;
-        gstore(Zb + (long)i * p + j, i < kw ? z : zero);
-        if (i < kw) {
-            if (lower) gstore(T + (long)i * p + j, z);
-            else gstore(T + (long)j * p + i, cneg(z));
-        }
-    });
-}
-
-__global__ __launch_bounds__(256, 2) void k_nd_bu(NdLev lv, const NdFac* fac, NdInv w, int k, int nb, int ntile) {
+__global__ __launch_bounds__(256, 2) void k_nd_block(NdLev lv, const NdFac* fac, NdInv w, int k, int nb, int ntile) {
     __shared__ union {
         NdTile s;
         NdSweep<4> w;
     } u;
     NdTile& s = u.s;
-    const int fr = blockIdx.x / ntile, q = blockIdx.y, p = lv.p;
+    const int fr = blockIdx.x / (ntile + 1), q = blockIdx.y, p = lv.p;
     const long job = (long)q * lv.cnt + fr;
     // tile number -> (I, J), I >= J, over the blocks other than k; number 0 and
-    // that of (k + 1, k + 1) change places
-    int e = blockIdx.x % ntile;
-    const int en = k + 1 < nb ? k * (k + 3) / 2 : 0;
-    e = e == 0 ? en : e == en ? 0 : e;
+    // that of (k + 1, k + 1) change places, and the last workgroup does what that of
+    // (k + 1, k + 1) has no time for
+    const bool more = k + 1 < nb;
+    const int en = more ? k * (k + 3) / 2 : 0, e0 = blockIdx.x % (ntile + 1);
+    const bool extra = e0 == ntile;
+    const int e = e0 == 0 || extra ? en : e0 == en ? 0 : e0;
     int I = (int)((sqrtf(8.0f * e + 1.0f) - 1.0f) * 0.5f);
     while ((I + 1) * (I + 2) / 2 <= e) ++I;
     while (I * (I + 1) / 2 > e) --I;
     int J = e - I * (I + 1) / 2;
     I += I >= k;
     J += J >= k;
-    const int iw = min(NB, p - I * NB), jw = min(NB, p - J * NB);
-    C* Y = (C*)w.Y + job * p * p + (long)I * NB * p + J * NB;
-    const C* Rb = (const C*)w.R + job * NB * p + I * NB;
-    const C* Zb = (const C*)w.Z + job * NB * p + J * NB;
-    auto pa = [&](int kk, int i) { return Rb + (long)kk * p + min(i, iw - 1); };
-    auto pb = [&](int kk, int j) { return Zb + (long)kk * p + min(j, jw - 1); };
-    auto oka = [&](int, int i) { return i < iw; };
-    auto okb = [&](int, int j) { return j < jw; };
-    auto keep = [](int, int, C) {};
-    if (I != k + 1 || J != k + 1) {
+    const int kw = min(NB, p - k * NB), iw = min(NB, p - I * NB), jw = min(NB, p - J * NB);
+    C* Yf = (C*)w.Y + job * p * p;
+    C* Y = Yf + (long)I * NB * p + J * NB;
+    const C* R0 = (const C*)((k & 1) ? w.R1 : w.R) + job * NB * p;
+    C* R1 = (C*)((k & 1) ? w.R : w.R1) + job * NB * p;
+    const C* D = (const C*)w.D + (job * 2 + (k & 1)) * NB * NB;
+    C* Dn = (C*)w.D + (job * 2 + (~k & 1)) * NB * NB;
+    const int t = threadIdx.x, lane = t & 63, lr = lane & 15, lk = lane >> 4;
+    const int wv = __builtin_amdgcn_readfirstlane(t >> 6), wr = wv >> 1, wc = wv & 1;
+    // Z_J, this thread's entries
+    C z[2][2][4];
+    {
         NdAcc<NB> A;
-        nd_staged<false, NB>(s, pa, pb, oka, okb, keep, [&](int kk) { A.mul(s, kk); });
+        nd_staged<NB>(
+            s, [&](int kk, int i) { return D + kk * NB + i; },
+            [&](int kk, int j) { return R0 + (long)min(kk, kw - 1) * p + J * NB + min(j, jw - 1); },
+            [&](int kk, int i) { return kk < kw && i < kw; }, [&](int kk, int j) { return kk < kw && j < jw; },
+            [&](int kk) { A.mul(s, kk); });
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < 2; ++y)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    z[x][y][v] = mk<C>(A.c1[x][y][v] - A.c2[x][y][v],
+                                       A.c3[x][y][v] - A.c1[x][y][v] - A.c2[x][y][v]);
+    }
+    // sum over the 64 rows of R_I^T Z_J: R_I staged from memory, Z_J from registers
+    auto product = [&](auto&& mm) {
+        C ra[4];
+        auto load = [&](int k0) {
+#pragma unroll
+            for (int h = 0; h < 4; ++h)
+                ra[h] = gload(R0 + (long)min(k0 + ((t + 256 * h) >> 6), kw - 1) * p + I * NB + min(t & 63, iw - 1));
+        };
+        load(0);
+        static_for<0, 4>([&](auto sc) {
+            constexpr int st = decltype(sc)::value, k0 = 16 * st;
+            __syncthreads();  // the previous stage is consumed
+#pragma unroll
+            for (int h = 0; h < 4; ++h) {
+                const int kr = (t + 256 * h) >> 6, i = t & 63;
+                const bool ok = k0 + kr < kw && i < iw;
+                s.sAr[kr][i] = ok ? ra[h].x : 0.0;
+                s.sAi[kr][i] = ok ? ra[h].y : 0.0;
+            }
+            if (wr == (st >> 1)) {
+#pragma unroll
+                for (int y = 0; y < 2; ++y)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        s.sBr[F64::row(lane, v)][wc * 32 + y * 16 + lr] = z[st & 1][y][v].x;
+                        s.sBi[F64::row(lane, v)][wc * 32 + y * 16 + lr] = z[st & 1][y][v].y;
+                    }
+            }
+            __syncthreads();
+            if (st < 3) load(k0 + 16);
+#pragma unroll
+            for (int kk = 0; kk < 16; kk += 4) mm(kk);
+        });
+    };
+    // what else becomes of Z_J, by the workgroup of tile (J, J)
+    auto spread = [&]() {
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < 2; ++y)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int i = wr * 32 + x * 16 + F64::row(lane, v), j = wc * 32 + y * 16 + lr;
+                    if (i < kw && j < jw) {
+                        if (J < k) gstore(Yf + (long)(k * NB + i) * p + J * NB + j, z[x][y][v]);
+                        else gstore(Yf + (long)(J * NB + j) * p + k * NB + i, cneg(z[x][y][v]));
+                        if (more && J == k + 1) gstore(R1 + (long)j * p + k * NB + i, cneg(z[x][y][v]));
+                    }
+                }
+    };
+    if (extra) {
+        for (int i = t; i < NB * NB; i += 256) {  // tile (k, k) <- D^-1
+            const int r = i >> 6, j = i & 63;
+            if (r < kw && j < kw) gstore(Yf + (long)(k * NB + r) * p + k * NB + j, gload(D + i));
+        }
+        if (more) spread();
+        return;
+    }
+    if (!more || I != k + 1 || J != k + 1) {
+        NdAcc<NB> A;
+        product([&](int kk) { A.mul(s, kk); });
         const double sg = I < k ? 1.0 : -1.0;
-        A.each([&](int i, int j, C z) {
+        A.each([&](int i, int j, C v) {
             if (i < iw && j < jw) {
                 C* y = Y + (long)i * p + j;
-                gstore(y, cadd(gload(y), cscale(z, sg)));
+                const C m = cadd(gload(y), cscale(v, sg));
+                gstore(y, m);
+                if (more && I == k + 1) gstore(R1 + (long)i * p + J * NB + j, m);
+                else if (more && J == k + 1) gstore(R1 + (long)j * p + I * NB + i, m);
             }
         });
+        if (I == J) spread();
         return;
     }
     // the lower 16 x 16 tiles in the layout of the sweep
     constexpr int NS = NdSweep<4>::NS;
-    const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
     d4v mr[NS], mi[NS], c1[NS] = {}, c2[NS] = {}, c3[NS] = {};
-    nd_each_entry<4>([&](auto sc, int v, int i, int j, bool) {
-        const C y = gload(Y + (long)min(i, iw - 1) * p + min(j, iw - 1));
-        mr[sc][v] = y.x;
-        mi[sc][v] = y.y;
-    });
-    nd_staged<false, NB>(s, pa, pb, oka, okb, keep, [&](int kk) {
+    product([&](int kk) {
         nd_each_tile<4>([&](auto sc, int ti, int tj) {
             const double ar = s.sAr[kk + lk][16 * ti + lr], ai = s.sAi[kk + lk][16 * ti + lr];
             const double br = s.sBr[kk + lk][16 * tj + lr], bi = s.sBi[kk + lk][16 * tj + lr];
@@ -977,6 +1005,11 @@ __global__ __launch_bounds__(256, 2) void k_nd_bu(NdLev lv, const NdFac* fac, Nd
         });
     });
     nd_each_entry<4>([&](auto sc, int v, int i, int j, bool) {
+        const C y = gload(Y + (long)min(i, iw - 1) * p + min(j, iw - 1));
+        mr[sc][v] = y.x;
+        mi[sc][v] = y.y;
+    });
+    nd_each_entry<4>([&](auto sc, int v, int i, int j, bool) {
         const bool ok = i < iw && j < iw;
         const double re = c1[sc][v] - c2[sc][v], im = c3[sc][v] - c1[sc][v] - c2[sc][v];
         mr[sc][v] = ok ? mr[sc][v] - re : (i == j ? 1.0 : 0.0);
@@ -984,11 +1017,10 @@ __global__ __launch_bounds__(256, 2) void k_nd_bu(NdLev lv, const NdFac* fac, Nd
     });
     __syncthreads();
     nd_sweep<4>(mr, mi, iw, u.w, fac[q].pivstat + 3 * (long)(lv.stat + fr), true);
-    C* Dn = (C*)w.D + job * NB * NB;
     nd_each_entry<4>([&](auto sc, int v, int i, int j, bool off) {
-        const C z = mk<C>(mr[sc][v], mi[sc][v]);
-        gstore(Dn + i * NB + j, z);
-        if (off) gstore(Dn + j * NB + i, z);
+        const C x = mk<C>(mr[sc][v], mi[sc][v]);
+        gstore(Dn + i * NB + j, x);
+        if (off) gstore(Dn + j * NB + i, x);
     });
 }
 
@@ -1022,8 +1054,7 @@ void launch_nd_invert(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, c
     if (lv.p <= NB) return;
     const int nb = (lv.p + NB - 1) / NB, nt = (nb - 1) * nb / 2, np = (lv.p + 31) / 32;
     for (int k = 0; k < nb; ++k) {
-        k_nd_bz<<<dim3(lv.cnt * (nb - 1) * (NB / ZC), B), 256, 0, s>>>(lv, w, k, nb);
-        k_nd_bu<<<dim3(lv.cnt * nt, B), 256, 0, s>>>(lv, fac, w, k, nb, nt);
+        k_nd_block<<<dim3(lv.cnt * (nt + 1), B), 256, 0, s>>>(lv, fac, w, k, nb, nt);
     }
     k_nd_mirror<<<dim3(lv.cnt * np * np, B), 256, 0, s>>>(lv, fac, w, nb);
 }

@@ -87,7 +87,7 @@ void size_plan(NdPlan& P, const std::vector<nd::Level>& L) {
 // level and the Schur complements of two neighbouring levels
 struct Scratch {
     size_t bytes = 0;
-    size_t oY, oF12, oR, oZ, oD, oS[2], ofac, ostat;
+    size_t oY, oF12, oR, oR1, oD, oS[2], ofac, ostat;
     Scratch(const NdPlan& P, int B) {
         auto take = [&](size_t n) {
             const size_t o = bytes;
@@ -97,8 +97,8 @@ struct Scratch {
         oY = take(ELEM * P.maxY * B);
         oF12 = take(ELEM * P.maxF12 * B);
         oR = take(ELEM * P.maxp * 64 * B);
-        oZ = take(ELEM * P.maxp * 64 * B);
-        oD = take(ELEM * P.maxcnt * 64 * 64 * B);
+        oR1 = take(ELEM * P.maxp * 64 * B);
+        oD = take(ELEM * P.maxcnt * 2 * 64 * 64 * B);
         for (int k = 0; k < 2; ++k) oS[k] = take(ELEM * P.maxS[k] * B);
         ofac = take(sizeof(NdFac) * B);
         ostat = take(sizeof(double) * 3 * B);
@@ -238,7 +238,7 @@ int rt_build_nd(Handle* h, const std::vector<Factor*>& Fs, std::vector<int>& bad
     }
     NdFac* dfac = (NdFac*)(w + sc.ofac);
     COPY(h, dfac, fac.data(), sizeof(NdFac) * B, hipMemcpyHostToDevice);
-    const NdInv iw{w + sc.oY, w + sc.oF12, w + sc.oR, w + sc.oZ, w + sc.oD};
+    const NdInv iw{w + sc.oY, w + sc.oF12, w + sc.oR, w + sc.oR1, w + sc.oD};
     hipEvent_t e0, e1;
     HIPCHK(h, hipEventCreate(&e0));
     HIPCHK(h, hipEventCreate(&e1));

@@ -33,7 +33,7 @@ struct NdFac {
 // block, F12, the block row and its product of a block sweep (64 x p each) and
 // two 64 x 64 block inverses
 struct NdInv {
-    void *Y, *F12, *R, *Z, *D;
+    void *Y, *F12, *R, *R1, *D;
 };
 
 // vectors of a reduced solve: source ridx[s] (0 without a list) at in / out

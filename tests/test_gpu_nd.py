@@ -132,3 +132,10 @@ def test_small_fronts_whole(monkeypatch, Nx, Ny):
     both sides of 64, where the kernel of whole fronts changes size; one child or
     two.  Same bar as the leaves'."""
     test_leaf_fronts_of_every_size(monkeypatch, Nx, Ny)
+
+
+@pytest.mark.parametrize("Nx,Ny", [(66, 68), (128, 129), (132, 150), (193, 196), (257, 260)])
+def test_long_separators(monkeypatch, Nx, Ny):
+    """Separators swept in blocks of 64: two to five of them, the last one of 4
+    cells, nearly or quite full.  Same bar as the leaves'."""
+    test_leaf_fronts_of_every_size(monkeypatch, Nx, Ny)
