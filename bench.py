@@ -481,12 +481,12 @@ def main():
             prefix = {"gemm": "k_nd_gemm", "solve": "k_nd_down"}.get(dom)
         else:
             prefix = {"gemm": "k_gemm<float", "trailing": "k_trailing<float", "solve": "k_mv<float"}.get(dom)
-        for name, v in P["kernels"].items():
-            if prefix and name.startswith(prefix):
-                roof["traffic"] = v["read_bytes"] + v["write_bytes"]
-                roof["traffic_unit"] = "bytes/launch"
-                roof["traffic_source"] = os.path.relpath(pmc, ROOT)
-                break
+        ks = [v for name, v in P["kernels"].items() if prefix and name.startswith(prefix)]
+        if ks:  # over all launches of its variants
+            roof["traffic"] = (sum((v["read_bytes"] + v["write_bytes"]) * v["launches"] for v in ks) /
+                               sum(v["launches"] for v in ks))
+            roof["traffic_unit"] = "bytes/launch"
+            roof["traffic_source"] = os.path.relpath(pmc, ROOT)
     roof["avg_launch_us"] = avg_s * 1e6
     # whole-factorization figure: the counted algorithmic flops of its products and
     # inversions (no count without profiled steps)
