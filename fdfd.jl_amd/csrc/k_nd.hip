@@ -1260,7 +1260,7 @@ void launch_nd_gemm(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, con
 }
 
 // smallest and largest pivot and zero-pivot flag of each factor's fronts
-constexpr int STAT_T = 1024;  // (256, one load after another: 60 us for the 32767 fronts of 1024 x 1024)
+constexpr int STAT_T = 1024;  // (256, one load after another: 60 us for the 32767 fronts of 1024 x 1024; 17 so)
 __global__ __launch_bounds__(STAT_T) void k_nd_stat(const NdFac* fac, int nfronts, double* out) {
     const double* ps = fac[blockIdx.x].pivstat;
     double mn = __builtin_huge_val(), mx = 0, z = 0;
