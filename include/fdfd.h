@@ -391,9 +391,10 @@ int fdfd_get_tuning(fdfd_handle* h, int* knobs, int nknobs);
  *   FDFD_INJECT_SINGULAR        next factorization reports a zero pivot in
  *                               line block `arg` (FDFD_ERR_SINGULAR)
  *   FDFD_INJECT_NOCONV          next refined solve runs at most `arg` FGMRES
- *                               iterations and no restart (FDFD_ERR_NOCONV;
- *                               on factors of the line reduction unless that
- *                               reaches the tolerance)
+ *                               iterations and no restart (FDFD_ERR_NOCONV
+ *                               unless that reaches the tolerance; a dissected
+ *                               factor, of which one iteration would, answers
+ *                               only half of the cells in that solve)
  *   FDFD_INJECT_OOM             next factorization fails its storage
  *                               allocation (FDFD_ERR_OOM) */
 enum {
