@@ -78,6 +78,7 @@ int builder_init(Builder& B, Handle* h) {
         b.inject_arg = h->inject_arg;
         h->inject = 0;
     }
+    std::swap(b.inject_poor, h->inject_poor);
     b.use_graphs = false;
     b.gemm3m = h->gemm3m;
     b.mv_mfma = h->mv_mfma;
@@ -461,6 +462,7 @@ int fdfd_batch_run(fdfd_batch* b, int precision, double tol, fdfd_stats* stats) 
             (void)hipEventDestroy(e0);
             (void)hipEventDestroy(e1);
         }
+        for (Factor* F : Fs) pivot_fallback |= F->pivot_fallback;  // (rebuilt after a failed refinement)
         const double solve_s = secs(ts0, now());
         if (overlap) {
             worker.join();

@@ -299,13 +299,15 @@ int rt_build_factors(Handle* h, const std::vector<Factor*>& Fs) {
     if (inject == FDFD_INJECT_PIVOT_FALLBACK || inject == FDFD_INJECT_SINGULAR ||
         inject == FDFD_INJECT_OOM)
         h->inject = 0;
+    const int poor = h->inject_poor;
+    h->inject_poor = 0;
     if (inject == FDFD_INJECT_OOM)
         return fail(h, FDFD_ERR_OOM, "factor storage allocation failed (injected)");
     bool forms01 = true;
     for (Factor* F : Fs) forms01 = forms01 && F->form <= 1;
     if (forms01 && inject != FDFD_INJECT_SINGULAR && rt_nd_applies(h, g.Nx, g.Ny)) {
         std::vector<int> bad;
-        if ((rc = rt_build_nd(h, Fs, bad))) return rc;
+        if ((rc = rt_build_nd(h, Fs, bad, poor))) return rc;
         if (inject == FDFD_INJECT_PIVOT_FALLBACK && (bad.empty() || bad[0] != 0)) bad.insert(bad.begin(), 0);
         const double ms_nd = Fs[0]->t_factor_ms;
         float ms_redo = 0;

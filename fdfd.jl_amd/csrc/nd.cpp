@@ -202,7 +202,7 @@ int rt_nd_prepare(Handle* h, int Nx, int Ny) {
 
 // Builds Fs by nested dissection; `bad` receives the factors whose pivots
 // failed their check (their storage is kept, their result is not usable).
-int rt_build_nd(Handle* h, const std::vector<Factor*>& Fs, std::vector<int>& bad) {
+int rt_build_nd(Handle* h, const std::vector<Factor*>& Fs, std::vector<int>& bad, int poor) {
     const GridDesc& g = h->g;
     const int B = (int)Fs.size();
     const bool prof = h->prof.enabled;
@@ -272,6 +272,8 @@ int rt_build_nd(Handle* h, const std::vector<Factor*>& Fs, std::vector<int>& bad
         launch_nd_gemm(st, v, dfac, B, iw.F12, Sc, S, true);
         delete ps;
     }
+    if (poor > 0 && poor <= B)  // injected: nothing reaches the cells of the last separator
+        launch_zero(st, (double2*)Fs[poor - 1]->blocks + P->lev[0].offX, (long)P->lev[0].p * P->lev[0].p);
     double* dstat = (double*)(w + sc.ostat);
     launch_nd_stat(st, dfac, B, P->fronts, dstat);
     hipError_t le = hipGetLastError();

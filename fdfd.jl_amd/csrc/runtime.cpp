@@ -791,6 +791,7 @@ int fdfd_solve_d(fdfd_handle* hh, int factor_id, int nrhs, const void* d_src, vo
         stats->t_solve_ms = ms;
         stats->pivot_growth = F->pivot_growth;
         stats->singular_line = F->singular_line;
+        stats->pivot_fallback = F->pivot_fallback;
     }
     if (rc) return rc;
     if (hipGetLastError() != hipSuccess) return fail(h, FDFD_ERR_HIP, "kernel launch failed");
@@ -845,6 +846,7 @@ int fdfd_linsolve(fdfd_handle* hh, int factor_id, int transpose, int nrhs, const
         stats->t_factor_ms = F->t_factor_ms;
         stats->pivot_growth = F->pivot_growth;
         stats->singular_line = -1;
+        stats->pivot_fallback = F->pivot_fallback;
     }
     return FDFD_OK;
 }
@@ -948,6 +950,7 @@ int fdfd_solve_pullback_d(fdfd_handle* hh, int factor_id, const void* d_ez, cons
         stats->t_solve_ms = ms;
         stats->pivot_growth = F->pivot_growth;
         stats->singular_line = -1;
+        stats->pivot_fallback = F->pivot_fallback;
     }
     if (rc) return rc;
     if (hipGetLastError() != hipSuccess) return fail(h, FDFD_ERR_HIP, "kernel launch failed");
@@ -1007,8 +1010,11 @@ int fdfd_profile_read(fdfd_handle* hh, int kernel, double* total_ms, long long* 
 int fdfd_debug_inject(fdfd_handle* hh, int what, int arg) {
     Handle* h = H(hh);
     if (!h) return FDFD_ERR_INVALID;
-    if (what < FDFD_INJECT_NONE || what > FDFD_INJECT_OOM)
+    if (what < FDFD_INJECT_NONE || what > FDFD_INJECT_POOR_FACTOR)
         return fail(h, FDFD_ERR_INVALID, "unknown injection");
+    if (what == FDFD_INJECT_POOR_FACTOR || what == FDFD_INJECT_NONE)
+        h->inject_poor = what == FDFD_INJECT_NONE ? 0 : 1 + std::max(arg, 0);
+    if (what == FDFD_INJECT_POOR_FACTOR) return FDFD_OK;
     h->inject = what;
     h->inject_arg = arg;
     return FDFD_OK;

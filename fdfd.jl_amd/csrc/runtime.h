@@ -100,6 +100,7 @@ struct Handle {
     bool full_pivot_search = false;
     // one-shot failure injection (fdfd_debug_inject): FDFD_INJECT_* and its argument
     int inject = 0, inject_arg = 0;
+    int inject_poor = 0;               // FDFD_INJECT_POOR_FACTOR: 1 + the factor's index in its build
     bool use_graphs = true;            // FDFD_GRAPHS=0 disables graph replay
     int gemm3m = 1;                    // three-multiplication complex GEMM (FDFD_GEMM3M=0: four)
     int mv_mfma = 1;                   // multi-source reduced-solve products on MFMA (FDFD_MV_MFMA=0: VALU)
@@ -283,7 +284,8 @@ int rt_nd_prepare(Handle* h, int Nx, int Ny);
 // rebuilds the dissected factors among Fs by the line reduction (a solve whose
 // refinement failed on them is then tried once more)
 int rt_rebuild_by_lines(Handle* h, const std::vector<Factor*>& Fs);
-int rt_build_nd(Handle* h, const std::vector<Factor*>& Fs, std::vector<int>& bad);
+// poor: the factor (1 + index) left without its last separator, 0 for none
+int rt_build_nd(Handle* h, const std::vector<Factor*>& Fs, std::vector<int>& bad, int poor);
 int rt_nd_solve_each(Handle* h, const std::vector<Factor*>& Fs, const double2* in, double2* out, bool prof);
 int rt_nd_solve(Handle* h, Factor* F, int trans, const double2* in, double2* out, long rs,
                 const int* ridx, int na, bool prof);

@@ -15,7 +15,7 @@ FDFD_TM, FDFD_TE = 1, 2
 FDFD_FP64, FDFD_FP32_IR = 0, 1
 FDFD_WHICH_LM, FDFD_WHICH_LR = 0, 1
 (FDFD_INJECT_NONE, FDFD_INJECT_PIVOT_FALLBACK, FDFD_INJECT_SINGULAR, FDFD_INJECT_NOCONV,
- FDFD_INJECT_OOM) = range(5)
+ FDFD_INJECT_OOM, FDFD_INJECT_POOR_FACTOR) = range(6)
 
 STATUS = {
     0: "FDFD_OK", -1: "FDFD_ERR_INVALID", -2: "FDFD_ERR_OOM", -3: "FDFD_ERR_SINGULAR",

@@ -90,7 +90,8 @@ typedef struct {
     int nconv;             /* converged eigenpairs (eigenfrequency)         */
     int pivot_fallback;    /* 1: a pivot outside the candidate window won a
                               step and the factorization was redone with the
-                              full-column pivot search                       */
+                              full-column pivot search, or a dissected factor
+                              was rebuilt by the line reduction              */
 } fdfd_stats;
 
 /* ---- library / handle --------------------------------------------------- */
@@ -396,13 +397,20 @@ int fdfd_get_tuning(fdfd_handle* h, int* knobs, int nknobs);
  *                               factor, of which one iteration would, answers
  *                               only half of the cells in that solve)
  *   FDFD_INJECT_OOM             next factorization fails its storage
- *                               allocation (FDFD_ERR_OOM) */
+ *                               allocation (FDFD_ERR_OOM)
+ *   FDFD_INJECT_POOR_FACTOR     next factorization: factor `arg` of the build,
+ *                               if dissected, loses its last separator, so that
+ *                               no refinement on it converges and the solve
+ *                               rebuilds it by the line reduction
+ *                               (stats.pivot_fallback); may be armed beside
+ *                               one of the others */
 enum {
     FDFD_INJECT_NONE = 0,
     FDFD_INJECT_PIVOT_FALLBACK = 1,
     FDFD_INJECT_SINGULAR = 2,
     FDFD_INJECT_NOCONV = 3,
-    FDFD_INJECT_OOM = 4
+    FDFD_INJECT_OOM = 4,
+    FDFD_INJECT_POOR_FACTOR = 5
 };
 int fdfd_debug_inject(fdfd_handle* h, int what, int arg);
 

@@ -1,6 +1,9 @@
 """What happens when the refinement on a dissected factor fails: an injected cut
-is a failure by its residual, not by decree.  Grids and tolerances are those of
-the error-path tests (96 x 80 cells, 1e-12)."""
+is a failure by its residual, not by decree; a factor that no refinement converges
+on (FDFD_INJECT_POOR_FACTOR) is rebuilt by the line reduction and the solve
+repeated, for one source, several, transposed, coupled sidebands and batches.
+Grids and tolerances are those of the error-path tests (96 x 80 cells, residual
+1e-12, fields 1e-10)."""
 import re
 
 import numpy as np
@@ -8,7 +11,7 @@ import pytest
 
 import fdfd_oracle as O
 from fdfd import core
-from fdfd._lib import FDFD_INJECT_NOCONV, FDFDError
+from fdfd._lib import FDFD_INJECT_NOCONV, FDFD_INJECT_POOR_FACTOR, FDFDError
 from fdfd.solve import Engine
 
 pytestmark = pytest.mark.gpu
@@ -70,5 +73,101 @@ def test_cut_that_suffices_is_no_failure(monkeypatch, small):
         e.debug_inject(FDFD_INJECT_NOCONV, 30)
         _, st = e.solve_fields(fid, d.src, tol=1e-12)
         assert st["residual"] <= 1e-12
+    finally:
+        e.close()
+
+
+def _field_err(f, ref):
+    return np.linalg.norm(f - ref) / np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_poor_factor_is_rebuilt_for_one_source(monkeypatch, small, precision):
+    d, om, ref = small
+    e = _engine(monkeypatch, "nd", d)
+    try:
+        e.debug_inject(FDFD_INJECT_POOR_FACTOR)
+        fid, fst = e.factor(O.TM, om, precision)
+        f, st = e.solve_fields(fid, d.src, tol=1e-12)
+        print(precision, st, flush=True)
+        assert fst["pivot_fallback"] == 0 and st["pivot_fallback"] == 1
+        assert st["residual"] <= 1e-12 and _field_err(f[:, :, :, 0], ref.data) <= 1e-10
+        f, again = e.solve_fields(fid, d.src, tol=1e-12)  # on the rebuilt factor
+        assert again["iterations"] < 30 and _field_err(f[:, :, :, 0], ref.data) <= 1e-10
+        e.release(fid)
+        fid, _ = e.factor(O.TM, om, precision)  # one-shot
+        _, st = e.solve_fields(fid, d.src, tol=1e-12)
+        assert st["pivot_fallback"] == 0
+    finally:
+        e.close()
+
+
+def test_poor_factor_is_rebuilt_for_transposed_solves(monkeypatch, small):
+    d, om, _ = small
+    b = O.rhs(om, d.src)
+    A = O.assemble(d.grid, d.eps_r, om, O.TM)
+    e = _engine(monkeypatch, "nd", d)
+    try:
+        e.debug_inject(FDFD_INJECT_POOR_FACTOR)
+        fid, _ = e.factor(O.TM, om, "fp64")
+        x, st = e.linsolve(fid, b, transpose=True, tol=1e-12)
+        assert st["pivot_fallback"] == 1
+        assert np.linalg.norm(b - A.T @ x) <= 1e-11 * np.linalg.norm(b)
+    finally:
+        e.close()
+
+
+def test_poor_factor_is_rebuilt_for_several_sources(monkeypatch, small):
+    d, om, ref = small
+    src = np.stack([d.src, np.zeros_like(d.src), np.roll(d.src, 7, axis=1)], axis=2)
+    e = _engine(monkeypatch, "nd", d)
+    try:
+        e.debug_inject(FDFD_INJECT_POOR_FACTOR)
+        fid, _ = e.factor(O.TM, om, "mixed")
+        f, st = e.solve_fields(fid, src, tol=1e-12)
+        assert st["pivot_fallback"] == 1 and st["residual"] <= 1e-12
+        assert _field_err(f[:, :, :, 0], ref.data) <= 1e-10 and not f[:, :, :, 1].any()
+        x, _ = O.linear_solve(O.assemble(d.grid, d.eps_r, om, O.TM), O.rhs(om, src[:, :, 2]))
+        assert _field_err(f[:, :, 0, 2].ravel(order="F"), x) <= 1e-10
+    finally:
+        e.close()
+
+
+@pytest.mark.parametrize("poor", [0, 1, 2])
+def test_poor_sideband_factor_is_rebuilt(monkeypatch, poor):
+    from test_gpu_modulated import _check, _pair
+    from fdfd.modulated import solve_modulated
+    monkeypatch.delenv("FDFD_METHOD", raising=False)
+    d, o = _pair(48, 40, 4, 1, True, seed=11)
+    e = Engine(0)
+    try:
+        e.debug_inject(FDFD_INJECT_POOR_FACTOR, poor)
+        fg, st = solve_modulated(d, precision="fp64", tol=1e-13, eng=e, return_stats=True)
+        assert st[0]["pivot_fallback"] == 1 and st[0]["residual"] <= 1e-13
+        _check(fg[0], O.solve_modulated(o)[0], f"poor sideband {poor}")
+    finally:
+        e.close()
+
+
+@pytest.mark.parametrize("poor", [0, 2])
+def test_poor_factor_is_rebuilt_inside_a_batch(monkeypatch, poor):
+    """Two jobs are two groups: the second is factored by the builder's thread
+    while the first group's solve rebuilds its poor factor."""
+    monkeypatch.delenv("FDFD_METHOD", raising=False)
+    oms = np.array([O.omega_of_wavelength(l) for l in (1.50, 1.54, 1.58)])
+    ds = [O.random_pixel_device(96, 80, 10, 1.55, 7), O.random_pixel_device(72, 88, 10, 1.55, 8)]
+    e = Engine(0)
+    try:
+        e.debug_inject(FDFD_INJECT_POOR_FACTOR, poor)
+        srcs = [np.stack([d.src, np.roll(d.src, 5, axis=1)], axis=2) for d in ds]
+        res, st = e.batch_solve([(_cgrid(d.grid), O.TM, d.eps_r, oms, s) for d, s in zip(ds, srcs)],
+                                precision="mixed", tol=1e-12)
+        assert st["pivot_fallback"] == 1 and st["residual"] <= 1e-12
+        for d, s, r in zip(ds, srcs, res):
+            for o, w in enumerate(oms):
+                A = O.assemble(d.grid, d.eps_r, float(w), O.TM)
+                for k in range(2):
+                    x, _ = O.linear_solve(A, O.rhs(float(w), s[:, :, k]))
+                    assert _field_err(r[o, k, :, :, 0].ravel(order="F"), x) <= 1e-10, (o, k)
     finally:
         e.close()
