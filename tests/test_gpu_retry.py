@@ -11,7 +11,8 @@ import pytest
 
 import fdfd_oracle as O
 from fdfd import core
-from fdfd._lib import FDFD_INJECT_NOCONV, FDFD_INJECT_POOR_FACTOR, FDFDError
+from fdfd._lib import (FDFD_INJECT_NOCONV, FDFD_INJECT_PIVOT_FALLBACK, FDFD_INJECT_POOR_FACTOR,
+                       FDFDError)
 from fdfd.solve import Engine
 
 pytestmark = pytest.mark.gpu
@@ -169,5 +170,24 @@ def test_poor_factor_is_rebuilt_inside_a_batch(monkeypatch, poor):
                 for k in range(2):
                     x, _ = O.linear_solve(A, O.rhs(float(w), s[:, :, k]))
                     assert _field_err(r[o, k, :, :, 0].ravel(order="F"), x) <= 1e-10, (o, k)
+    finally:
+        e.close()
+
+
+@pytest.mark.parametrize("poor", [1, 2])
+def test_poor_sideband_beside_a_line_factor(monkeypatch, poor):
+    """Sideband 0 fails its pivot check and is a line factor from the start;
+    another one is poor."""
+    from test_gpu_modulated import _check, _pair
+    from fdfd.modulated import solve_modulated
+    monkeypatch.delenv("FDFD_METHOD", raising=False)
+    d, o = _pair(48, 40, 4, 1, True, seed=11)
+    e = Engine(0)
+    try:
+        e.debug_inject(FDFD_INJECT_PIVOT_FALLBACK)
+        e.debug_inject(FDFD_INJECT_POOR_FACTOR, poor)
+        fg, st = solve_modulated(d, precision="fp64", tol=1e-13, eng=e, return_stats=True)
+        assert st[0]["residual"] <= 1e-13
+        _check(fg[0], O.solve_modulated(o)[0], f"poor sideband {poor} beside a line factor")
     finally:
         e.close()
