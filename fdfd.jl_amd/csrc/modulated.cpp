@@ -132,11 +132,8 @@ extern "C" int fdfd_modulated_solve(fdfd_handle* hh, double omega, double Omega,
     double resid = 0;
     const bool injected = h->inject == FDFD_INJECT_NOCONV;
     rc = rt_gmres_op(h, NF, apply, prec, V, Zk, b, x, tol, MF_MAX_RESTARTS, &iters, &restarts, &resid);
-    const bool dissected = std::any_of(Fs.begin(), Fs.end(), [](Factor* F) { return F->nd != nullptr; });
-    if (rc == FDFD_ERR_NOCONV && dissected && !injected) {  // once more on line-reduction factors
-        if ((rc = rt_rebuild_by_lines(h, Fs))) return done(rc);
+    if (!injected && rt_retry_by_lines(h, Fs, &rc))
         rc = rt_gmres_op(h, NF, apply, prec, V, Zk, b, x, tol, MF_MAX_RESTARTS, &iters, &restarts, &resid);
-    }
     if (rc == FDFD_OK) {
         // fields per sideband: Hx = -Syf dyf ez / (i wn mu0'), Hy = Sxf dxf ez / (i wn mu0')
         for (int j = 0; j < nf && rc == FDFD_OK; ++j) {

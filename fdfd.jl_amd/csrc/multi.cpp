@@ -406,8 +406,7 @@ int rt_gmres_multi(Handle* h, Factor* F, int nr, const double2* B, double2* X, d
                    int* iters, double* worst) {
     const double before = *worst;
     int rc = gmres_multi(h, F, nr, B, X, tol, iters, worst);
-    if (rc == FDFD_ERR_NOCONV && F->nd) {
-        if ((rc = rt_rebuild_by_lines(h, {F}))) return rc;
+    if (rt_retry_by_lines(h, {F}, &rc)) {
         *worst = before;
         rc = gmres_multi(h, F, nr, B, X, tol, iters, worst);
     }

@@ -491,6 +491,16 @@ int rt_gmres_op(Handle* h, long N,
     return fail(h, FDFD_ERR_NOCONV, buf);
 }
 
+bool rt_retry_by_lines(Handle* h, const std::vector<Factor*>& Fs, int* rc) {
+    if (*rc != FDFD_ERR_NOCONV || std::none_of(Fs.begin(), Fs.end(), [](Factor* F) { return F->nd != nullptr; }))
+        return false;
+    const std::string why = h->err;
+    const int r = rt_rebuild_by_lines(h, Fs);
+    if (r == FDFD_ERR_OOM) h->err = why;  // no room for factors by lines: the solve failed as it did
+    else if (r) *rc = r;
+    return r == FDFD_OK;
+}
+
 // FGMRES on one factor's operator A' (or A'^T), preconditioned by the factor.
 // A dissected factor on which it fails above the residual `accept` (that the
 // caller would take) is rebuilt by the line reduction and the solve repeated.
@@ -514,11 +524,9 @@ static int gmres(Handle* h, Factor* F, int trans, const double2* b, double2* x, 
     };
     int rc = rt_gmres_op(h, N, apply, prec, h->V, h->Zk, b, x, tol, max_restarts, &st.iters,
                          &st.restarts, &st.resid);
-    if (rc == FDFD_ERR_NOCONV && F->nd && !injected && st.resid > accept) {
-        if ((rc = rt_rebuild_by_lines(h, {F}))) return rc;
+    if (!injected && st.resid > accept && rt_retry_by_lines(h, {F}, &rc))
         rc = rt_gmres_op(h, N, apply, prec, h->V, h->Zk, b, x, tol, max_restarts, &st.iters,
                          &st.restarts, &st.resid);
-    }
     return rc;
 }
 

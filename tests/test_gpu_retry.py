@@ -11,8 +11,8 @@ import pytest
 
 import fdfd_oracle as O
 from fdfd import core
-from fdfd._lib import (FDFD_INJECT_NOCONV, FDFD_INJECT_PIVOT_FALLBACK, FDFD_INJECT_POOR_FACTOR,
-                       FDFDError)
+from fdfd._lib import (FDFD_INJECT_NOCONV, FDFD_INJECT_OOM, FDFD_INJECT_PIVOT_FALLBACK,
+                       FDFD_INJECT_POOR_FACTOR, FDFDError)
 from fdfd.solve import Engine
 
 pytestmark = pytest.mark.gpu
@@ -189,5 +189,25 @@ def test_poor_sideband_beside_a_line_factor(monkeypatch, poor):
         fg, st = solve_modulated(d, precision="fp64", tol=1e-13, eng=e, return_stats=True)
         assert st[0]["residual"] <= 1e-13
         _check(fg[0], O.solve_modulated(o)[0], f"poor sideband {poor} beside a line factor")
+    finally:
+        e.close()
+
+
+@pytest.mark.parametrize("nsrc", [1, 3])
+def test_no_room_for_line_factors(monkeypatch, small, nsrc):
+    """Where the line factor cannot be had, the solve has failed to converge and says
+    so, with its residual; a later one, with memory back, rebuilds and succeeds."""
+    d, om, ref = small
+    src = np.stack([d.src] * nsrc, axis=2)
+    e = _engine(monkeypatch, "nd", d)
+    try:
+        e.debug_inject(FDFD_INJECT_POOR_FACTOR)
+        fid, _ = e.factor(O.TM, om, "fp64")
+        e.debug_inject(FDFD_INJECT_OOM)
+        with pytest.raises(FDFDError) as ei:
+            e.solve_fields(fid, src, tol=1e-12)
+        assert ei.value.code == -4 and _residual(str(ei.value)) > 1e-12
+        f, st = e.solve_fields(fid, src, tol=1e-12)
+        assert st["pivot_fallback"] == 1 and _field_err(f[:, :, :, 0], ref.data) <= 1e-10
     finally:
         e.close()
