@@ -281,6 +281,9 @@ struct StencilOp {
 void launch_stencil(hipStream_t s, double2* y, const double2* x, const StencilOp& op,
                     int transpose, const double2* b, long rs = 0, const int* ridx = nullptr,
                     int na = 1);
+// y = |A| |x| + |b|
+void launch_stencil_abs(hipStream_t s, double2* y, const double2* x, const StencilOp& op, int transpose,
+                        const double2* b);
 // several right-hand sides per launch (k_multi.hip): sources ridx[0..na) of
 // buffers whose source r starts at r * rs; the matrix-vector step runs on the
 // matrix cores (16 sources per chunk, inputs packed into `pack`, at least

@@ -241,7 +241,8 @@ __device__ inline StW st_weights(int i, int j, int Nx, int Ny, const double2* sx
 }
 }  // namespace
 
-template <int POL, int FORM, bool TRANS>
+// ABS: y = |A| |x| + |b| (entrywise magnitudes), what rounding in b - A x scales with
+template <int POL, int FORM, bool TRANS, bool ABS>
 __global__ __launch_bounds__(256) void k_stencil(double2* __restrict__ y, const double2* __restrict__ x,
                                                  const double2* __restrict__ eps,
                                                  const double2* sxf, const double2* sxb,
@@ -298,23 +299,27 @@ __global__ __launch_bounds__(256) void k_stencil(double2* __restrict__ y, const 
         const double2 xw = xs[ly + 1][lx], xe = xs[ly + 1][lx + 2];
         const double2 xsn = xs[ly][lx + 1], xn = xs[ly + 2][lx + 1];
         double2 acc;
+        auto mul = [](double2 w, double2 v) -> double2 {
+            return ABS ? make_double2(hypot(w.x, w.y) * hypot(v.x, v.y), 0.0) : cmul(w, v);
+        };
         const StW W = weights(i, j, 0, 0);
         if (!TRANS) {
-            acc = cmul(W.c, xc);
-            acc = cadd(acc, cmul(W.w, xw));
-            acc = cadd(acc, cmul(W.e, xe));
-            acc = cadd(acc, cmul(W.s, xsn));
-            acc = cadd(acc, cmul(W.n, xn));
+            acc = mul(W.c, xc);
+            acc = cadd(acc, mul(W.w, xw));
+            acc = cadd(acc, mul(W.e, xe));
+            acc = cadd(acc, mul(W.s, xsn));
+            acc = cadd(acc, mul(W.n, xn));
         } else {
             const int im = (i == 0) ? Nx - 1 : i - 1, ip = (i + 1 == Nx) ? 0 : i + 1;
             const int jm = (j == 0) ? Ny - 1 : j - 1, jp = (j + 1 == Ny) ? 0 : j + 1;
-            acc = cmul(W.c, xc);
-            acc = cadd(acc, cmul(weights(im, j, -1, 0).e, xw));
-            acc = cadd(acc, cmul(weights(ip, j, 1, 0).w, xe));
-            acc = cadd(acc, cmul(weights(i, jm, 0, -1).n, xsn));
-            acc = cadd(acc, cmul(weights(i, jp, 0, 1).s, xn));
+            acc = mul(W.c, xc);
+            acc = cadd(acc, mul(weights(im, j, -1, 0).e, xw));
+            acc = cadd(acc, mul(weights(ip, j, 1, 0).w, xe));
+            acc = cadd(acc, mul(weights(i, jm, 0, -1).n, xsn));
+            acc = cadd(acc, mul(weights(i, jp, 0, 1).s, xn));
         }
-        y[k] = b ? csub(b[k], acc) : acc;
+        if (ABS && b) acc.x += hypot(b[k].x, b[k].y);
+        y[k] = b && !ABS ? csub(b[k], acc) : acc;
     }
 }
 
@@ -322,7 +327,7 @@ void launch_stencil(hipStream_t s, double2* y, const double2* x, const StencilOp
                     int transpose, const double2* b, long rs, const int* ridx, int na) {
     const dim3 grid((op.Nx + ST_TX - 1) / ST_TX, (op.Ny + ST_TY - 1) / ST_TY, ridx ? na : 1);
 #define ST_LAUNCH(P, F, T)                                                                     \
-    k_stencil<P, F, T><<<grid, 256, 0, s>>>(y, x, op.eps, op.sxf, op.sxb, op.syf, op.syb, op.Nx, \
+    k_stencil<P, F, T, false><<<grid, 256, 0, s>>>(y, x, op.eps, op.sxf, op.sxb, op.syf, op.syb, op.Nx, \
                                             op.Ny, op.ry, op.kdiag, b, rs, ridx)
     if (op.form == 1) {
         if (transpose) ST_LAUNCH(1, 1, true);
@@ -335,6 +340,18 @@ void launch_stencil(hipStream_t s, double2* y, const double2* x, const StencilOp
         else ST_LAUNCH(2, 0, false);
     }
 #undef ST_LAUNCH
+}
+
+void launch_stencil_abs(hipStream_t s, double2* y, const double2* x, const StencilOp& op, int transpose,
+                        const double2* b) {
+    const dim3 grid((op.Nx + ST_TX - 1) / ST_TX, (op.Ny + ST_TY - 1) / ST_TY);
+    auto go = [&](auto kern) {
+        kern<<<grid, 256, 0, s>>>(y, x, op.eps, op.sxf, op.sxb, op.syf, op.syb, op.Nx, op.Ny, op.ry, op.kdiag, b, 0,
+                                  nullptr);
+    };
+    if (op.form == 1) go(transpose ? k_stencil<1, 1, true, true> : k_stencil<1, 1, false, true>);
+    else if (op.pol == 1) go(transpose ? k_stencil<1, 0, true, true> : k_stencil<1, 0, false, true>);
+    else go(transpose ? k_stencil<2, 0, true, true> : k_stencil<2, 0, false, true>);
 }
 
 // y = a * x

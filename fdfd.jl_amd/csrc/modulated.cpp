@@ -132,7 +132,7 @@ extern "C" int fdfd_modulated_solve(fdfd_handle* hh, double omega, double Omega,
     double resid = 0;
     const bool injected = h->inject == FDFD_INJECT_NOCONV;
     rc = rt_gmres_op(h, NF, apply, prec, V, Zk, b, x, tol, MF_MAX_RESTARTS, &iters, &restarts, &resid);
-    if (!injected && rt_retry_by_lines(h, Fs, &rc))
+    if (!injected && rt_retry_by_lines(h, Fs, 0, {{b, x, resid}}, V, &rc))
         rc = rt_gmres_op(h, NF, apply, prec, V, Zk, b, x, tol, MF_MAX_RESTARTS, &iters, &restarts, &resid);
     if (rc == FDFD_OK) {
         // fields per sideband: Hx = -Syf dyf ez / (i wn mu0'), Hy = Sxf dxf ez / (i wn mu0')

@@ -160,7 +160,7 @@ static void launch_solve_multi(Handle* h, Factor* F, long rs, const int* ridx, i
 }
 
 static int gmres_multi(Handle* h, Factor* F, int nr, const double2* B, double2* X, double tol,
-                       int* iters, double* worst) {
+                       int* iters, double* worst, std::vector<Unsolved>& left) {
     if (nr < 1 || nr > KMULTI) return fail(h, FDFD_ERR_INVALID, "1 <= sources <= 16 per multi solve");
     if (F->form != 0 && F->form != 1)
         return fail(h, FDFD_ERR_INVALID, "multi-source solves take driven or sideband factors");
@@ -386,7 +386,9 @@ static int gmres_multi(Handle* h, Factor* F, int nr, const double2* B, double2* 
     int failed = 0;
     for (int r = 0; r < nr; ++r) {
         w = std::max(w, resid[r]);
-        if (state[r] != 1) ++failed;
+        if (state[r] == 1) continue;
+        ++failed;
+        left.push_back({B + (long)r * N, X + (long)r * N, resid[r]});
     }
     *worst = std::max(*worst, w);
     HIPCHK(h, hipGetLastError());
@@ -405,10 +407,11 @@ static int gmres_multi(Handle* h, Factor* F, int nr, const double2* B, double2* 
 int rt_gmres_multi(Handle* h, Factor* F, int nr, const double2* B, double2* X, double tol,
                    int* iters, double* worst) {
     const double before = *worst;
-    int rc = gmres_multi(h, F, nr, B, X, tol, iters, worst);
-    if (rt_retry_by_lines(h, {F}, &rc)) {
+    std::vector<Unsolved> left;
+    int rc = gmres_multi(h, F, nr, B, X, tol, iters, worst, left);
+    if (rt_retry_by_lines(h, {F}, 0, left, h->mV, &rc)) {
         *worst = before;
-        rc = gmres_multi(h, F, nr, B, X, tol, iters, worst);
+        rc = gmres_multi(h, F, nr, B, X, tol, iters, worst, left);
     }
     return rc;
 }

@@ -283,10 +283,17 @@ void rt_nd_bytes(int Nx, int Ny, size_t* arena, size_t* scratch);
 int rt_nd_prepare(Handle* h, int Nx, int Ny);
 // rebuilds the dissected factors among Fs by the line reduction
 int rt_rebuild_by_lines(Handle* h, const std::vector<Factor*>& Fs);
+// a system that a refinement left with the relative residual resid
+struct Unsolved {
+    const double2 *b, *x;
+    double resid;
+};
 // after a solve on Fs that returned *rc: true if its refinement failed on dissected
-// factors, which are rebuilt by lines now, and it is to be repeated; else *rc is its
-// result (FDFD_ERR_NOCONV as it was where line factors do not fit in memory)
-bool rt_retry_by_lines(Handle* h, const std::vector<Factor*>& Fs, int* rc);
+// factors above what rounding allows; they are rebuilt by lines now, and it is to be
+// repeated.  Else *rc is its result (FDFD_ERR_NOCONV as it was where line factors
+// do not fit in memory).  w: work, as long as b
+bool rt_retry_by_lines(Handle* h, const std::vector<Factor*>& Fs, int trans, const std::vector<Unsolved>& left,
+                       double2* w, int* rc);
 // poor: the factor (1 + index) left without its last separator, 0 for none
 int rt_build_nd(Handle* h, const std::vector<Factor*>& Fs, std::vector<int>& bad, int poor);
 int rt_nd_solve_each(Handle* h, const std::vector<Factor*>& Fs, const double2* in, double2* out, bool prof);

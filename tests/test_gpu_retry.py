@@ -211,3 +211,46 @@ def test_no_room_for_line_factors(monkeypatch, small, nsrc):
         assert st["pivot_fallback"] == 1 and _field_err(f[:, :, :, 0], ref.data) <= 1e-10
     finally:
         e.close()
+
+
+@pytest.mark.parametrize("pol", [O.TM, O.TE])
+@pytest.mark.parametrize("tol", [1e-16, 1e-18])
+@pytest.mark.parametrize("npml", [0, 10])
+def test_tolerance_below_rounding_keeps_the_factor(monkeypatch, pol, tol, npml):
+    """A residual of a few 1e-15 is what rounding leaves of any solve here, so lower
+    tolerances fail (they did on line factors too) and the factor is not to blame:
+    it stays, whether one source asked, several, or the transposed system."""
+    d = O.random_pixel_device(96, 80, npml, 1.55, 7)
+    om = float(d.omega[0])
+    b = O.rhs(om, d.src) if npml else O.rhs(om, np.roll(d.src, 30, axis=0))
+    src = b.reshape(d.grid.N, order="F") / (1j * om)
+    e = _engine(monkeypatch, "nd", d)
+    try:
+        fid, _ = e.factor(pol, om, "fp64")
+        calls = [lambda t: e.solve_fields(fid, src, tol=t)[1],
+                 lambda t: e.solve_fields(fid, np.stack([src, np.roll(src, 3, axis=1)], axis=2), tol=t)[1],
+                 lambda t: e.linsolve(fid, b, tol=t)[1],
+                 lambda t: e.linsolve(fid, b, transpose=True, tol=t)[1]]
+        for call in calls:
+            with pytest.raises(FDFDError) as ei:
+                call(tol)
+            assert ei.value.code == -4 and _residual(str(ei.value)) <= 1e-11
+            assert call(1e-10)["pivot_fallback"] == 0
+    finally:
+        e.close()
+
+
+def test_tolerance_below_rounding_keeps_sideband_factors(monkeypatch):
+    from test_gpu_modulated import _pair
+    from fdfd.modulated import solve_modulated
+    monkeypatch.delenv("FDFD_METHOD", raising=False)
+    d, _ = _pair(48, 40, 4, 1, True, seed=11)
+    e = Engine(0)
+    rcs = []
+    e._chk = rcs.append  # the statistics of the failed solve, in place of its error
+    try:
+        _, st = solve_modulated(d, precision="fp64", tol=1e-18, eng=e, return_stats=True)
+        print(rcs, st, flush=True)
+        assert rcs[-1] == -4 and 0 < st[0]["residual"] <= 1e-13 and st[0]["pivot_fallback"] == 0
+    finally:
+        e.close()
