@@ -159,6 +159,9 @@ static void launch_solve_multi(Handle* h, Factor* F, long rs, const int* ridx, i
     }
 }
 
+// the larger residual, or the one that is not a number
+static double worse(double a, double b) { return std::isnan(a) || b <= a ? a : b; }
+
 static int gmres_multi(Handle* h, Factor* F, int nr, const double2* B, double2* X, double tol,
                        int* iters, double* worst, std::vector<Unsolved>& left) {
     if (nr < 1 || nr > KMULTI) return fail(h, FDFD_ERR_INVALID, "1 <= sources <= 16 per multi solve");
@@ -278,8 +281,8 @@ static int gmres_multi(Handle* h, Factor* F, int nr, const double2* B, double2* 
                 resid[r] = beta[q] / bnorm[r];
                 if (resid[r] <= tol) state[r] = 1;
                 // no restart left, or a whole cycle that gained less than 10%: the
-                // rounding floor of the operator
-                else if (rs == max_restarts || resid[r] > 0.9 * prev[r]) state[r] = 2;
+                // rounding floor of the operator, or not finite
+                else if (rs == max_restarts || !(resid[r] <= 0.9 * prev[r])) state[r] = 2;
                 if (state[r] == 0) inv.push_back(make_double2(1.0 / beta[q], 0.0));
             }
         }
@@ -358,7 +361,7 @@ static int gmres_multi(Handle* h, Factor* F, int nr, const double2* B, double2* 
                 ++*iters;
                 s.jdone = j + 1;
                 const double est = std::abs(s.gv[j + 1]);
-                if (!(est <= 0.5 * tol || hn[q] == 0)) still.push_back(r);
+                if (!(est <= 0.5 * tol || hn[q] == 0) && std::isfinite(hn[q])) still.push_back(r);
             }
             if (!still.empty() && (rc = scale(W, W, hinv))) return rc;
             it = still;
@@ -385,12 +388,12 @@ static int gmres_multi(Handle* h, Factor* F, int nr, const double2* B, double2* 
     double w = 0;
     int failed = 0;
     for (int r = 0; r < nr; ++r) {
-        w = std::max(w, resid[r]);
+        w = worse(w, resid[r]);
         if (state[r] == 1) continue;
         ++failed;
         left.push_back({B + (long)r * N, X + (long)r * N, resid[r]});
     }
-    *worst = std::max(*worst, w);
+    *worst = worse(*worst, w);
     HIPCHK(h, hipGetLastError());
     if (failed) {
         char buf[200];

@@ -272,8 +272,11 @@ int rt_build_nd(Handle* h, const std::vector<Factor*>& Fs, std::vector<int>& bad
         launch_nd_gemm(st, v, dfac, B, iw.F12, Sc, S, true);
         delete ps;
     }
-    if (poor > 0 && poor <= B)  // injected: nothing reaches the cells of the last separator
-        launch_zero(st, (double2*)Fs[poor - 1]->blocks + P->lev[0].offX, (long)P->lev[0].p * P->lev[0].p);
+    if (poor != 0 && std::abs(poor) <= B) {  // injected: the inverse of the last separator
+        double2* X = (double2*)Fs[std::abs(poor) - 1]->blocks + P->lev[0].offX;
+        const double a = poor > 0 ? 0.0 : std::numeric_limits<double>::quiet_NaN();
+        launch_scale_copy(st, X, X, make_double2(a, 0), (long)P->lev[0].p * P->lev[0].p);
+    }
     double* dstat = (double*)(w + sc.ostat);
     launch_nd_stat(st, dfac, B, P->fronts, dstat);
     hipError_t le = hipGetLastError();

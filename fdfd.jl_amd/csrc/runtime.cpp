@@ -426,8 +426,9 @@ int rt_gmres_op(Handle* h, long N,
             if (resid <= tol) return FDFD_OK;
             if (rs == max_restarts) break;
             // a whole restart cycle that gains less than 10% has reached the
-            // rounding floor of the operator: stop instead of cycling
-            if (resid > 0.9 * prev) break;
+            // rounding floor of the operator, and one that is not finite will
+            // not get better: stop instead of cycling
+            if (!(resid <= 0.9 * prev)) break;
             ++*restarts;
             launch_scale_copy(h->stream, V, V, make_double2(1.0 / beta, 0), N);
         }
@@ -477,7 +478,7 @@ int rt_gmres_op(Handle* h, long N,
             ++*iters;
             jdone = j + 1;
             const double est = std::abs(gv[j + 1]);
-            if (est <= 0.5 * tol || hn == 0) break;
+            if (est <= 0.5 * tol || hn == 0 || !std::isfinite(hn)) break;
             launch_scale_copy(h->stream, w, w, make_double2(1.0 / hn, 0), N);
         }
         // y = H^-1 g, x += Z y
@@ -560,7 +561,7 @@ static int gmres(Handle* h, Factor* F, int trans, const double2* b, double2* x, 
     };
     int rc = rt_gmres_op(h, N, apply, prec, h->V, h->Zk, b, x, tol, max_restarts, &st.iters,
                          &st.restarts, &st.resid);
-    if (!injected && st.resid > accept && rt_retry_by_lines(h, {F}, trans, {{b, x, st.resid}}, h->V, &rc))
+    if (!injected && !(st.resid <= accept) && rt_retry_by_lines(h, {F}, trans, {{b, x, st.resid}}, h->V, &rc))
         rc = rt_gmres_op(h, N, apply, prec, h->V, h->Zk, b, x, tol, max_restarts, &st.iters,
                          &st.restarts, &st.resid);
     return rc;
@@ -812,7 +813,7 @@ int fdfd_solve_d(fdfd_handle* hh, int factor_id, int nrhs, const void* d_src, vo
         rc = gmres(h, F, 0, h->bvec, h->xvec, tol, MAX_RESTARTS, s1);
         st.iters += s1.iters;
         st.restarts += s1.restarts;
-        worst = std::max(worst, s1.resid);
+        worst = std::max(s1.resid, worst);  // (not a number: stays)
         if (rc) break;
         // field recovery: TM w = 1/(i omega mu0'), TE w = 1/(i omega eps0')
         double c = (F->pol == FDFD_TM) ? mu0n : eps0n;
@@ -877,7 +878,7 @@ int fdfd_linsolve(fdfd_handle* hh, int factor_id, int transpose, int nrhs, const
         SolveStats s1;
         int rc = gmres(h, F, transpose ? 1 : 0, h->bvec, h->xvec, tol, MAX_RESTARTS, s1);
         st.iters += s1.iters;
-        worst = std::max(worst, s1.resid);
+        worst = std::max(s1.resid, worst);  // (not a number: stays)
         if (rc) return rc;
         HIPCHK(h, hipMemcpyAsync(x + (long)r * N, h->xvec, sizeof(double2) * N,
                                  hipMemcpyDeviceToHost, h->stream));
@@ -1057,7 +1058,7 @@ int fdfd_debug_inject(fdfd_handle* hh, int what, int arg) {
     if (what < FDFD_INJECT_NONE || what > FDFD_INJECT_POOR_FACTOR)
         return fail(h, FDFD_ERR_INVALID, "unknown injection");
     if (what == FDFD_INJECT_POOR_FACTOR || what == FDFD_INJECT_NONE)
-        h->inject_poor = what == FDFD_INJECT_NONE ? 0 : 1 + std::max(arg, 0);
+        h->inject_poor = what == FDFD_INJECT_NONE ? 0 : arg < 0 ? arg : 1 + arg;
     if (what == FDFD_INJECT_POOR_FACTOR) return FDFD_OK;
     h->inject = what;
     h->inject_arg = arg;

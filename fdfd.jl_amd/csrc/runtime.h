@@ -100,7 +100,7 @@ struct Handle {
     bool full_pivot_search = false;
     // one-shot failure injection (fdfd_debug_inject): FDFD_INJECT_* and its argument
     int inject = 0, inject_arg = 0;
-    int inject_poor = 0;               // FDFD_INJECT_POOR_FACTOR: 1 + the factor's index in its build
+    int inject_poor = 0;               // FDFD_INJECT_POOR_FACTOR: 1 + the factor's index in its build, < 0 for NaN
     bool use_graphs = true;            // FDFD_GRAPHS=0 disables graph replay
     int gemm3m = 1;                    // three-multiplication complex GEMM (FDFD_GEMM3M=0: four)
     int mv_mfma = 1;                   // multi-source reduced-solve products on MFMA (FDFD_MV_MFMA=0: VALU)
@@ -294,7 +294,8 @@ struct Unsolved {
 // do not fit in memory).  w: work, as long as b
 bool rt_retry_by_lines(Handle* h, const std::vector<Factor*>& Fs, int trans, const std::vector<Unsolved>& left,
                        double2* w, int* rc);
-// poor: the factor (1 + index) left without its last separator, 0 for none
+// poor: 1 + the index of the factor whose last separator's inverse is zero (negative: not
+// a number), 0 for none
 int rt_build_nd(Handle* h, const std::vector<Factor*>& Fs, std::vector<int>& bad, int poor);
 int rt_nd_solve_each(Handle* h, const std::vector<Factor*>& Fs, const double2* in, double2* out, bool prof);
 int rt_nd_solve(Handle* h, Factor* F, int trans, const double2* in, double2* out, long rs,

@@ -399,8 +399,10 @@ int fdfd_get_tuning(fdfd_handle* h, int* knobs, int nknobs);
  *   FDFD_INJECT_OOM             next factorization fails its storage
  *                               allocation (FDFD_ERR_OOM)
  *   FDFD_INJECT_POOR_FACTOR     next factorization: factor `arg` of the build,
- *                               if dissected, loses its last separator, so that
- *                               no refinement on it converges and the solve
+ *                               if dissected, has zeros for the inverse of its
+ *                               last separator (factor -1 - `arg`, for `arg` < 0,
+ *                               values that are not numbers), so that no
+ *                               refinement on it converges and the solve
  *                               rebuilds it by the line reduction
  *                               (stats.pivot_fallback); may be armed beside
  *                               one of the others */

@@ -254,3 +254,46 @@ def test_tolerance_below_rounding_keeps_sideband_factors(monkeypatch):
         assert rcs[-1] == -4 and 0 < st[0]["residual"] <= 1e-13 and st[0]["pivot_fallback"] == 0
     finally:
         e.close()
+
+
+@pytest.mark.parametrize("nsrc", [1, 3])
+def test_factor_that_is_not_finite_is_rebuilt(monkeypatch, small, nsrc):
+    """Residuals that are not numbers end the refinement at once (it used to restart
+    40 times on them) and the factor is rebuilt."""
+    d, om, ref = small
+    e = _engine(monkeypatch, "nd", d)
+    try:
+        e.debug_inject(FDFD_INJECT_POOR_FACTOR, -1)
+        fid, _ = e.factor(O.TM, om, "fp64")
+        f, st = e.solve_fields(fid, np.stack([d.src] * nsrc, axis=2), tol=1e-12)
+        print(st, flush=True)
+        assert st["pivot_fallback"] == 1 and st["iterations"] <= 5 * nsrc
+        assert _field_err(f[:, :, :, nsrc - 1], ref.data) <= 1e-10
+        e.debug_inject(FDFD_INJECT_POOR_FACTOR, -1)
+        fid, _ = e.factor(O.TM, om, "fp64")
+        b = O.rhs(om, d.src)
+        x, st = e.linsolve(fid, b, transpose=True, tol=1e-12)
+        A = O.assemble(d.grid, d.eps_r, om, O.TM)
+        assert st["pivot_fallback"] == 1 and np.linalg.norm(b - A.T @ x) <= 1e-11 * np.linalg.norm(b)
+    finally:
+        e.close()
+
+
+@pytest.mark.parametrize("nsrc", [1, 3])
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+def test_source_that_is_not_finite_keeps_the_factor(monkeypatch, small, nsrc, value):
+    d, om, ref = small
+    src = np.stack([d.src] * nsrc, axis=2)
+    src[40, 40, 0] = value
+    e = _engine(monkeypatch, "nd", d)
+    chk, rcs = e._chk, []
+    try:
+        fid, _ = e.factor(O.TM, om, "fp64")
+        e._chk = rcs.append  # the statistics of the failed solve, in place of its error
+        _, st = e.solve_fields(fid, src, tol=1e-12)
+        e._chk = chk
+        assert rcs == [-4] and not np.isfinite(st["residual"]) and st["iterations"] <= 5 * nsrc
+        f, st = e.solve_fields(fid, d.src, tol=1e-12)
+        assert st["pivot_fallback"] == 0 and _field_err(f[:, :, :, 0], ref.data) <= 1e-10
+    finally:
+        e.close()
