@@ -153,7 +153,7 @@ __device__ inline double2 nd_entry(const double2* coef, long N, int Nx, int Ny, 
 __device__ inline C nd_rcp(C z) {
     // 1 / z from one hardware reciprocal of |z|^2 (about half the bits) and one
     // step r (1 + e + e^2), e = 1 - n r (the entries are scaled to O(1) and grow
-    // by 1e6 or so: no range handling)
+    // by 1e6 or so: no range handling; NdPiv reports what is outside)
     const double n = fma(z.x, z.x, z.y * z.y), r0 = rcp_hw(n);
     const double e = fma(-n, r0, 1.0), r = fma(r0, fma(e, e, e), r0);
     return mk<C>(z.x * r, -z.y * r);
@@ -166,7 +166,7 @@ __device__ inline C cfma(C a, C b, C c) {
 using F64 = mfma_t<double>;
 
 // smallest and largest 2 x 2 pivot determinant (|re| + |im|), and whether one was
-// zero or not finite
+// out of the range that nd_rcp, which squares it, inverts
 struct NdPiv {
     double mn = 1e300, mx = 0;
     bool bad = false;
@@ -174,7 +174,7 @@ struct NdPiv {
         const double m = cabs1(det);
         mn = fmin(mn, m);
         mx = fmax(mx, m);
-        bad = bad || !(m > 0 && m < 1e300);
+        bad = bad || !(m > 1e-140 && m < 1e140);
     }
 };
 

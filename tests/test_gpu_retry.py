@@ -297,3 +297,27 @@ def test_source_that_is_not_finite_keeps_the_factor(monkeypatch, small, nsrc, va
         assert st["pivot_fallback"] == 0 and _field_err(f[:, :, :, 0], ref.data) <= 1e-10
     finally:
         e.close()
+
+
+@pytest.mark.parametrize("cells", [2, 4])
+@pytest.mark.parametrize("value", [1e70, 1e82, 1e120])
+def test_pivots_out_of_range(monkeypatch, value, cells):
+    """Permittivities that take the last pivot blocks out of the range their
+    reciprocal works in (squares up to 1e308), with no later pivot to show it: the
+    factor is one by lines, as it would have been without the dissection.  The
+    cells are the last ones eliminated, on the column that cuts the torus."""
+    d = O.random_pixel_device(96, 80, 10, 1.55, 7)
+    d.eps_r[-1, -cells:] = value
+    om = float(d.omega[0])
+    b = O.rhs(om, d.src)
+    b[np.real(d.eps_r.ravel(order="F")) > 1e50] = 0
+    e = _engine(monkeypatch, "nd", d)
+    try:
+        fid, fst = e.factor(O.TM, om, "fp64")
+        x, st = e.linsolve(fid, b, tol=1e-11)
+        res = np.linalg.norm(b - O.assemble(d.grid, d.eps_r, om, O.TM) @ x) / np.linalg.norm(b)
+        print(f"eps {value:.0e} in {cells} cells: fallback {fst['pivot_fallback']} its {st['iterations']} res {res:.1e}",
+              flush=True)
+        assert fst["pivot_fallback"] == (1 if value > 1e80 else 0) and res <= 1e-10
+    finally:
+        e.close()
