@@ -19,6 +19,8 @@
 namespace fdfd {
 
 int fail(Handle* h, int code, const std::string& msg) {
+    // reported here: the check after the next call's launches is to find its own errors
+    if (code == FDFD_ERR_OOM || code == FDFD_ERR_HIP) (void)hipGetLastError();
     if (h) h->err = msg;
     return code;
 }

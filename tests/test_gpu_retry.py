@@ -4,6 +4,7 @@ on (FDFD_INJECT_POOR_FACTOR) is rebuilt by the line reduction and the solve
 repeated, for one source, several, transposed, coupled sidebands and batches.
 Grids and tolerances are those of the error-path tests (96 x 80 cells, residual
 1e-12, fields 1e-10)."""
+import ctypes as C
 import re
 
 import numpy as np
@@ -319,5 +320,24 @@ def test_pivots_out_of_range(monkeypatch, value, cells):
         print(f"eps {value:.0e} in {cells} cells: fallback {fst['pivot_fallback']} its {st['iterations']} res {res:.1e}",
               flush=True)
         assert fst["pivot_fallback"] == (1 if value > 1e80 else 0) and res <= 1e-10
+    finally:
+        e.close()
+
+
+def test_allocation_failure_leaves_no_error_behind(monkeypatch, small):
+    """A batch whose results do not fit (10000 wavelengths at 1024 x 1024, 500 GB) is
+    refused, and the next call does not report that again."""
+    d, om, ref = small
+    e = _engine(monkeypatch, "nd", d)
+    g = core.Grid(0.02, (8, 8), (0.0, 1024 * 0.02), (0.0, 1024 * 0.02))
+    try:
+        with pytest.raises(FDFDError) as ei:
+            e.batch_solve([(g, O.TM, np.ones(g.N), om * np.linspace(1, 1.1, 10000), np.ones(g.N))], keep=False)
+        assert ei.value.code == -2
+        e.set_grid(_cgrid(d.grid))
+        e.set_eps(d.eps_r)
+        fid, _ = e.factor(O.TM, om, "fp64")
+        f, _ = e.solve_fields(fid, d.src, tol=1e-12)
+        assert _field_err(f[:, :, :, 0], ref.data) <= 1e-10
     finally:
         e.close()
