@@ -87,7 +87,9 @@ PinOut pin_out(void* base) {
 }  // namespace
 
 int ensure_multi_work(Handle* h, long N, int k) {
-    if (!h->msmall) {
+    if (!h->mpin) {
+        if (h->msmall) (void)hipFree(h->msmall);
+        h->msmall = nullptr;
         HIPCHK(h, hipMalloc(&h->msmall, msmall_bytes()));
         HIPCHK(h, hipHostMalloc(&h->mpin, pin_bytes(), hipHostMallocDefault));
     }

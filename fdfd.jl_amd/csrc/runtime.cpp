@@ -76,6 +76,7 @@ int ensure_factor_work(Handle* h, int n, int nch) {
     dfree(h->win); dfree(h->verr);
     h->used = h->piv = h->win = h->verr = nullptr;
     h->Vbuf = h->LU = h->Zb = nullptr;
+    h->work_n = h->work_ch = 0;  // (an allocation below may fail)
     const int NBmax = VMAX;
     HIPCHK(h, hipMalloc(&h->used, sizeof(int) * nch * n));
     HIPCHK(h, hipMalloc(&h->piv, sizeof(int) * nch * NBmax));
@@ -108,6 +109,7 @@ int ensure_solve_work(Handle* h, long N) {
                      (void**)&h->Zk, (void**)&h->tmp, (void**)&h->tmp2, (void**)&h->bvec,
                      (void**)&h->xvec};
     for (auto b : bufs) { dfree(*b); *b = nullptr; }
+    h->work_N = 0;  // (an allocation below may fail)
     HIPCHK(h, hipMalloc(&h->g_mid, sizeof(double2) * N * KMULTI));
     HIPCHK(h, hipMalloc(&h->x_out, sizeof(double2) * N * KMULTI));
     HIPCHK(h, hipMalloc(&h->V, sizeof(double2) * N * (KDIM + 1)));
@@ -116,7 +118,8 @@ int ensure_solve_work(Handle* h, long N) {
     HIPCHK(h, hipMalloc(&h->tmp2, sizeof(double2) * N));
     HIPCHK(h, hipMalloc(&h->bvec, sizeof(double2) * N));
     HIPCHK(h, hipMalloc(&h->xvec, sizeof(double2) * N));
-    if (!h->dpart) {
+    if (!h->hpin) {  // the last of these
+        for (void** b : {(void**)&h->dpart, (void**)&h->rpart, (void**)&h->hdev}) { dfree(*b); *b = nullptr; }
         h->nblk = 512;
         HIPCHK(h, hipMalloc(&h->dpart, sizeof(double2) * h->nblk * (KDIM + 2)));
         HIPCHK(h, hipMalloc(&h->rpart, sizeof(double) * h->nblk));

@@ -341,3 +341,33 @@ def test_allocation_failure_leaves_no_error_behind(monkeypatch, small):
         assert _field_err(f[:, :, :, 0], ref.data) <= 1e-10
     finally:
         e.close()
+
+
+def test_work_that_does_not_fit_is_allocated_again(monkeypatch, small):
+    """A factorization whose work does not fit (1024 lines of 700000 cells) frees the
+    work of smaller ones; they get theirs anew."""
+    d, om, ref = small
+    e = _engine(monkeypatch, "bcr", d)
+    hip = C.CDLL("libamdhip64.so")
+    hip.hipMalloc.argtypes = [C.POINTER(C.c_void_p), C.c_size_t]
+    hip.hipFree.argtypes = [C.c_void_p]
+    try:
+        for again in (False, True):
+            if again:
+                g = core.Grid(0.02, (8, 8), (0.0, 1024 * 0.02), (0.0, 700000 * 0.02))
+                e.set_grid(g)
+                eps = C.c_void_p()  # (its values are not looked at)
+                assert hip.hipMalloc(C.byref(eps), 16 * len(g)) == 0
+                e._chk(e.lib.fdfd_set_eps_d(e.h, eps))
+                assert hip.hipFree(eps) == 0
+                with pytest.raises(FDFDError) as ei:
+                    e.factor(O.TM, om, "fp64")
+                assert ei.value.code == -2
+                e.set_grid(_cgrid(d.grid))
+                e.set_eps(d.eps_r)
+            fid, _ = e.factor(O.TM, om, "fp64")
+            f, _ = e.solve_fields(fid, d.src, tol=1e-12)
+            assert _field_err(f[:, :, :, 0], ref.data) <= 1e-10
+            e.release(fid)
+    finally:
+        e.close()
