@@ -19,6 +19,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <map>
 #include <numeric>
 #include <thread>
 #include <vector>
@@ -207,20 +208,28 @@ int fdfd_batch_run(fdfd_batch* b, int precision, double tol, fdfd_stats* stats) 
     for (auto& kv : h->factors) rt_free_factor(h, kv.second);
     h->factors.clear();
     h->has_grid = h->has_eps = false;
-    // largest factors first (the slab below is sized by them)
+    // largest factors first (the slab below is sized by them); the sizes once for
+    // each grid shape
+    struct Size {
+        bool nd;
+        size_t factor, scratch;  // bytes of a factor, and of what its build adds
+    };
+    std::map<std::pair<int, int>, Size> sizes;
+    std::vector<const Size*> size(b->jobs.size());
+    for (size_t ji = 0; ji < b->jobs.size(); ++ji) {
+        const GridDesc& g = b->jobs[ji].g;
+        auto it = sizes.find({g.Nx, g.Ny});
+        if (it == sizes.end()) {
+            Size s{rt_nd_applies(h, g.Nx, g.Ny), 0, 0};
+            if (s.nd) rt_nd_bytes(h, g.Nx, g.Ny, &s.factor, &s.scratch);
+            else s.factor = rt_factor_bytes(std::min(g.Nx, g.Ny), std::max(g.Nx, g.Ny), precision, h->gemm_b3 != 0);
+            it = sizes.emplace(std::make_pair(g.Nx, g.Ny), s).first;
+        }
+        size[ji] = &it->second;
+    }
     std::vector<int> order(b->jobs.size());
     std::iota(order.begin(), order.end(), 0);
-    auto fbytes = [&](const BatchJob& j) {
-        const int n = std::min(j.g.Nx, j.g.Ny), m = std::max(j.g.Nx, j.g.Ny);
-        if (rt_nd_applies(h, j.g.Nx, j.g.Ny)) {
-            size_t arena = 0, scratch = 0;
-            rt_nd_bytes(j.g.Nx, j.g.Ny, &arena, &scratch);
-            return arena;
-        }
-        return rt_factor_bytes(n, m, precision, h->gemm_b3 != 0);
-    };
-    std::stable_sort(order.begin(), order.end(),
-                     [&](int a, int c) { return fbytes(b->jobs[a]) > fbytes(b->jobs[c]); });
+    std::stable_sort(order.begin(), order.end(), [&](int a, int c) { return size[a]->factor > size[c]->factor; });
     // Memory plan: result buffers first, then a slab of two halves for the
     // factor arenas of the largest group of frequencies (one half is solved
     // while the next group is factored into the other), reused by every group
@@ -265,10 +274,9 @@ int fdfd_batch_run(fdfd_batch* b, int precision, double tol, fdfd_stats* stats) 
     for (size_t ji = 0; ji < b->jobs.size(); ++ji) {
         const BatchJob& job = b->jobs[ji];
         const int n = std::min(job.g.Nx, job.g.Ny), m = std::max(job.g.Nx, job.g.Ny);
-        size_t sb = 0, ss = 0;
-        size_t scratch = 0;
-        if (rt_nd_applies(h, job.g.Nx, job.g.Ny)) {
-            rt_nd_bytes(job.g.Nx, job.g.Ny, &sb, &scratch);
+        size_t sb = size[ji]->factor, ss = 0;
+        const size_t scratch = size[ji]->scratch;
+        if (size[ji]->nd) {
             if ((rc = rt_nd_prepare(h, job.g.Nx, job.g.Ny))) {
                 free_results(b);
                 return rc;

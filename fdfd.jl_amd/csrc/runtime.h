@@ -279,7 +279,7 @@ int rt_prec_apply(Handle* h, Factor* F, int trans, const double2* in, double2* o
 // nested dissection (nd.cpp)
 constexpr int ND_MIN_LINE = 16;  // shorter lines: line reduction
 bool rt_nd_applies(const Handle* h, int Nx, int Ny);
-void rt_nd_bytes(int Nx, int Ny, size_t* arena, size_t* scratch);
+void rt_nd_bytes(const Handle* h, int Nx, int Ny, size_t* arena, size_t* scratch);
 int rt_nd_prepare(Handle* h, int Nx, int Ny);
 // rebuilds the dissected factors among Fs by the line reduction
 int rt_rebuild_by_lines(Handle* h, const std::vector<Factor*>& Fs);
