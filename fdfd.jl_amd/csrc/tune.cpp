@@ -1,4 +1,4 @@
-// Autotuner for the factorization's kernel variants.
+// Autotuner for the kernel variants of the line reduction.
 //
 // No counterpart in the reference (its solver choice is the FDFD_SOLVER
 // switch of src/solver/solver.jl:10).  The variant knobs of a handle are:
@@ -10,7 +10,10 @@
 // fdfd_autotune times a whole step (assemble + factor + refined solve of a
 // point source to 1e-10) for every candidate on the handle's current grid
 // and eps, keeps the fastest on the handle, and, when FDFD_TUNE_CACHE names a
-// file, records it there.  Handles created later look that file up by
+// file, records it there.  Where the handle dissects this grid (rt_nd_applies) it
+// goes on doing so, and the step time reported is the dissection's, timed like the
+// candidates; the variants then are those of its line factors (full-vector modes,
+// short lines, factors rebuilt after a failed refinement).  Handles created later look that file up by
 // (n, m, precision, pol) when they factor, unless switches were forced by
 // the environment.  The file is plain text, one entry per line:
 //   n m precision pol gemm_b3 trail_h3 fuse_panels gemm_waves gemm3m ms
@@ -145,13 +148,10 @@ extern "C" int fdfd_autotune(fdfd_handle* hh, int pol, double omega, int precisi
     int rc = stream_copy(h, dsrc, src.data(), sizeof(double2) * N, hipMemcpyHostToDevice);
     const Knobs start = get_knobs(h);
     Knobs best = start;
-    double best_ms = 1e300;
+    double best_ms = 1e300, nd_ms = 1e300;
     const bool nd_was_off = h->nd_off;
-    h->nd_off = true;  // the variants are the line reduction's
-    for (const Knobs& k : candidates(precision)) {
-        if (rc) break;
-        set_knobs(h, k);
-        h->tuned_explicitly = true;  // no cache lookup while timing
+    // the better of two steps with the present settings, in ms
+    auto step = [&]() {
         double t_best = 1e300;
         for (int rep = 0; rep < 2 && rc == FDFD_OK; ++rep) {
             const auto t0 = std::chrono::steady_clock::now();
@@ -166,10 +166,17 @@ extern "C" int fdfd_autotune(fdfd_handle* hh, int pol, double omega, int precisi
                                   std::chrono::steady_clock::now() - t0).count();
             t_best = std::min(t_best, ms);
         }
-        if (rc == FDFD_ERR_NOCONV) {  // a variant that cannot reach the tolerance is skipped
-            rc = FDFD_OK;
-            continue;
-        }
+        if (rc != FDFD_ERR_NOCONV) return t_best;
+        rc = FDFD_OK;  // a variant that cannot reach the tolerance is skipped
+        return 1e300;
+    };
+    h->tuned_explicitly = true;  // no cache lookup while timing
+    if (rc == FDFD_OK && rt_nd_applies(h, g.Nx, g.Ny)) nd_ms = step();
+    h->nd_off = true;  // the variants are the line reduction's
+    for (const Knobs& k : candidates(precision)) {
+        if (rc) break;
+        set_knobs(h, k);
+        const double t_best = step();
         if (t_best < best_ms) {
             best_ms = t_best;
             best = k;
@@ -183,7 +190,8 @@ extern "C" int fdfd_autotune(fdfd_handle* hh, int pol, double omega, int precisi
     if (rc) return rc;
     if (stats) {
         memset(stats, 0, sizeof(*stats));
-        stats->t_factor_ms = best_ms;  // the winning step time (factor + refined solve)
+        // the step time (factor + refined solve) of this grid from now on
+        stats->t_factor_ms = nd_ms < 1e300 ? nd_ms : best_ms;
         stats->singular_line = -1;
     }
     const char* path = std::getenv("FDFD_TUNE_CACHE");

@@ -223,9 +223,10 @@ class Engine:
         self._chk(self.lib.fdfd_set_tuning(self.h, panel_width, int(force_full_search)))
 
     def autotune(self, pol: int, omega: float, precision="mixed"):
-        """Time every factorization variant on the current grid and eps and keep
-        the fastest (fdfd_autotune); recorded in FDFD_TUNE_CACHE if set.
-        Returns (knobs, winning step ms)."""
+        """Time every variant of the line reduction on the current grid and eps and
+        keep the fastest (fdfd_autotune); recorded in FDFD_TUNE_CACHE if set.
+        Returns (knobs, step ms from now on: the winner's, or the dissection's
+        where the grid is dissected)."""
         st = fdfd_stats()
         self._chk(self.lib.fdfd_autotune(self.h, int(pol), float(omega), PRECISIONS[precision],
                                          C.byref(st)))

@@ -359,10 +359,11 @@ end
 """
     autotune!(d::Device, pol=TM; precision=:mixed) -> NamedTuple
 
-Times every variant of the factorization kernels on `d`'s grid and `ϵᵣ` at
+Times every variant of the line reduction's kernels on `d`'s grid and `ϵᵣ` at
 `d.ω[1]` (`fdfd_autotune`) and keeps the fastest on the handle; with
 `ENV["FDFD_TUNE_CACHE"]` naming a file the choice is recorded there and read
-by later handles.  No counterpart in the reference.
+by later handles.  Grids that are dissected stay so, and the step time is the
+dissection's.  No counterpart in the reference.
 """
 function autotune!(d::FDFD.Device, pol::FDFD.Polarization=FDFD.TM; precision::Symbol=:mixed,
                    handle::Handle=default_handle())
