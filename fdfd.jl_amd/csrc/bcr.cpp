@@ -164,7 +164,7 @@ static int* blk_e(const Factor* F, int id) {
 // first panel leaves them, are formed by the window panel for its window and
 // by the Z build's check blocks for every row, and its pivot rows by the Z
 // build); the full search runs single panels.
-void rt_launch_gj(Handle* h, const LineJob* J, int nj, int n, bool fp64, bool h3, bool full, bool prof) {
+static void launch_gj(Handle* h, const LineJob* J, int nj, int n, bool fp64, bool h3, bool full, bool prof) {
     hipStream_t st = h->stream;
     const size_t elem = fp64 ? sizeof(double2) : sizeof(float2);
     const int NB = h->panel_width ? h->panel_width : PMAX;
@@ -541,7 +541,7 @@ int rt_build_factors(Handle* h, const std::vector<Factor*>& Fs) {
                 }
             } else {
                 launch_gjreset(st, T.lj + ol, nj, n);
-                rt_launch_gj(h, T.lj + ol, nj, n, fp64, h->trail_h3 != 0, full, prof);
+                launch_gj(h, T.lj + ol, nj, n, fp64, h->trail_h3 != 0, full, prof);
                 ol += nj;
             }
         }

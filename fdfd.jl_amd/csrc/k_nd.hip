@@ -1025,7 +1025,7 @@ __global__ __launch_bounds__(256, 2) void k_nd_block(NdLev lv, const NdFac* fac,
 }
 
 // X (whole) from the lower tiles of Y
-__global__ __launch_bounds__(256) void k_nd_mirror(NdLev lv, const NdFac* fac, NdInv w, int nb) {
+__global__ __launch_bounds__(256) void k_nd_mirror(NdLev lv, const NdFac* fac, NdInv w) {
     __shared__ C tile[32][33];
     const int q = blockIdx.y, p = lv.p, np = (p + 31) / 32;
     const int fr = blockIdx.x / (np * np), e = blockIdx.x % (np * np), I = e / np, J = e % np;
@@ -1056,7 +1056,7 @@ void launch_nd_invert(hipStream_t s, const NdLev& lv, const NdFac* fac, int B, c
     for (int k = 0; k < nb; ++k) {
         k_nd_block<<<dim3(lv.cnt * (nt + 1), B), 256, 0, s>>>(lv, fac, w, k, nb, nt);
     }
-    k_nd_mirror<<<dim3(lv.cnt * np * np, B), 256, 0, s>>>(lv, fac, w, nb);
+    k_nd_mirror<<<dim3(lv.cnt * np * np, B), 256, 0, s>>>(lv, fac, w);
 }
 
 // ---------------------------------------------------------------------------
@@ -1528,9 +1528,8 @@ template void launch_nd_down(hipStream_t, const NdLev&, const NdBatch<ND_SOLVES>
 // ones), so a row of 16 sources is one contiguous piece of every gather and
 // the product's B operand; the factor streams straight into the A operand, so
 // it is read once for all sources.  With one wave a tile of 16 outputs, a
-// CU's four SIMDs consume about 16 B of factor a clock in FP32 and FP64
-// alike, above its share of the memory rate, so the products cost no more than
-// the stream.  Levels with few tiles split K over KS waves of a workgroup.
+// CU's four SIMDs consume about 16 B of factor a clock, above its share of the
+// memory rate, so the products cost no more than the stream.  Levels with few tiles split K over KS waves of a workgroup.
 // ---------------------------------------------------------------------------
 // x[k][s] = scale_k in_s[k] (PACK), or out_s[k] = scale_k x[k][s]
 template <bool PACK>
@@ -1574,7 +1573,7 @@ __global__ __launch_bounds__(256) void k_ndm_gather(NdLev lv, C* vp, C* up, cons
     if (e >= (long)lv.cnt * f) return;
     const int s = threadIdx.x & 15, fr = (int)(e / f), i = (int)(e % f);
     const int k = lv.node[e];
-    C v = mk<C>(R(0), R(0));
+    C v = mk<C>(0, 0);
     if (k >= 0) {
         if (i < lv.p) v = gload(x + (long)k * 16 + s);
         const C* uc = up + (lv.offUc + (long)fr * lv.nch * lv.cb) * 16;

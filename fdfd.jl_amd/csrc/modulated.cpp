@@ -8,8 +8,8 @@
 //   block (j, j+1) += 0.5 wn_j^2 conj(T_deps), block (j+1, j) += 0.5 wn_{j+1}^2 T_deps,
 // with b = i w src in the centre block, and solves it with lu(A)\b.
 //
-// Here every sideband operator A_j is factored by the block cyclic reduction
-// (all 2K+1 at once, batched), and the coupled system is solved by FP64
+// Here every sideband operator A_j is factored (nested dissection or the line
+// reduction, rt_nd_applies; all 2K+1 at once, batched), and the coupled system is solved by FP64
 // flexible GMRES on the exact coupled operator (stencils + the diagonal
 // sideband coupling, k_mf_couple), right-preconditioned by the block
 // diagonal of the factors.  The coupling is diagonal and usually weak next to

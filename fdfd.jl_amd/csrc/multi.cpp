@@ -4,10 +4,9 @@
 // driven.jl:11-55; dolinearsolve, solver.jl:35).  Sources that share a
 // factorization (one frequency, many sources) are solved together here: each
 // FGMRES(30) iteration applies the preconditioner (the reduced solve of the
-// block cyclic reduction) to every active source in one pass over the factor
-// blocks, the operator to all of them in one stencil launch, and does the
-// CGS2 orthogonalisation of all of them with one host round trip per
-// reduction.  Every source keeps its own Krylov basis, Hessenberg matrix,
+// dissection or of the line reduction) to every active source in one pass over
+// the factor, the operator to all of them in one stencil launch, and does the
+// CGS2 orthogonalisation of all of them with one host round trip.  Every source keeps its own Krylov basis, Hessenberg matrix,
 // restarts and convergence test; the arithmetic per source is that of the
 // single-source FGMRES in runtime.cpp.  A source that converges (or
 // stagnates) drops out of the launches.

@@ -3,14 +3,14 @@
 // The torus of cells is dissected by nd_plan.h; every tree level is one batch
 // of equal-sized fronts (k_nd.hip).  Leaves are eliminated in registers; a
 // level above assembles [F11 | F12] from the operator and its children's
-// Schur complements, inverts F11 by symmetric block sweeps, and forms Q = X F12 and the Schur complement
-// F22 - F12^T Q on MFMA.
+// Schur complements, inverts F11 by symmetric block sweeps, and forms
+// Q = X F12 and the Schur complement F22 - F12^T Q on MFMA.
 //
 // Against the block cyclic reduction of the lines (bcr.cpp) this takes of
 // the order of N^1.5 operations and N log N storage instead of n^3 m and
 // n^2 m, at the price of a fixed pivot order (4 x 4 blocks).  A factor with a
-// pivot that is zero or not finite is rebuilt by the line reduction, and so is
-// one on which the refinement does not converge.
+// pivot block that cannot be inverted is rebuilt by the line reduction, and so is
+// one on which the refinement stalls above what rounding allows.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -83,8 +83,9 @@ void size_plan(NdPlan& P, const std::vector<nd::Level>& L) {
     P.arena = off;
 }
 
-// scratch of B factors built together: Gauss-Jordan work of the largest
-// level and the Schur complements of two neighbouring levels
+// scratch of B factors built together: separators, F12, block rows and inverses
+// (NdInv) of the largest level, and the Schur complements of two neighbouring
+// levels
 struct Scratch {
     size_t bytes = 0;
     size_t oY, oF12, oR, oR1, oD, oS[2], ofac, ostat;
@@ -311,9 +312,6 @@ int rt_build_nd(Handle* h, const std::vector<Factor*>& Fs, std::vector<int>& bad
     return FDFD_OK;
 }
 
-// out = A'^-1 in or A'^-T in for na sources (source ridx[i] at ridx[i] * rs;
-// ridx null: one source).  S = U^-1 A' U gives A'^-1 = U S^-1 U^-1 and
-// A'^-T = U^-1 S^-1 U.
 // work vectors of `count` solves, in the handle's buffer
 static int nd_vectors(Handle* h, long per, int count, double2** v) {
     const size_t need = sizeof(double2) * (size_t)per * count;
@@ -339,6 +337,9 @@ static NdVec nd_vec(const Factor* F, int trans, const double2* in, double2* out,
                  trans ? ux : uxi, trans ? uy : uyi, trans ? uxi : ux, trans ? uyi : uy};
 }
 
+// out = A'^-1 in or A'^-T in for na sources (source ridx[i] at ridx[i] * rs;
+// ridx null: one source).  S = U^-1 A' U gives A'^-1 = U S^-1 U^-1 and
+// A'^-T = U^-1 S^-1 U.
 int rt_nd_solve(Handle* h, Factor* F, int trans, const double2* in, double2* out, long rs,
                 const int* ridx, int na, bool prof) {
     const NdPlan& P = *F->nd;

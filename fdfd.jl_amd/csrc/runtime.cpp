@@ -1,6 +1,6 @@
 // Host runtime and C ABI of libfdfd: handle lifecycle, operator assembly,
-// FP64 flexible GMRES refinement, field recovery, adjoint gradient.  The
-// block cyclic reduction factorization and its solve are in bcr.cpp,
+// FP64 flexible GMRES refinement, field recovery, adjoint gradient.  Nested
+// dissection is in nd.cpp, the block cyclic reduction of the lines in bcr.cpp,
 // shift-invert Arnoldi in eigen.cpp, batched solves in batch.cpp.
 //
 // Reference path replaced: solve(d::Device, pol) (src/solver/driven.jl:4-59)

@@ -36,8 +36,9 @@ struct Prof {
     double bytes[P_COUNT] = {0};
 };
 
-// Factors of one operator (pol, omega) on the handle's grid: the blocks of
-// the block cyclic reduction and its reduced-solve program.
+// Factors of one operator (pol, omega) on the handle's grid: the fronts of the
+// dissection, or the blocks of the block cyclic reduction and its reduced-solve
+// program.
 struct Factor {
     int id = 0, pol = 1, precision = 0;
     double omega = 0;
@@ -277,7 +278,13 @@ int rt_build_factors(Handle* h, const std::vector<Factor*>& Fs);
 int rt_build_factor(Handle* h, Factor* F);
 int rt_prec_apply(Handle* h, Factor* F, int trans, const double2* in, double2* out);
 // nested dissection (nd.cpp)
-constexpr int ND_MIN_LINE = 16;  // shorter lines: line reduction
+// Shorter lines: line reduction.  On both sides of it a step (factor and solve) takes,
+// dissected and by lines, plain FP64: 16 x 200 0.36 and 0.90 ms, 16 x 50000 2.2 and
+// 35 ms, 64 x 6000 1.7 and 8.0 ms; 15 x 200 0.35 and 0.91 ms, 15 x 50000 2.7 and 36 ms,
+// 4 x 200 0.28 and 0.72 ms.  So the limit costs grids of 4 to 15 lines half their
+// time and more; these were never dissected, and only solves of several
+// sources on one factor would not gain there (8 to 15 x 3000: the same time).
+constexpr int ND_MIN_LINE = 16;
 bool rt_nd_applies(const Handle* h, int Nx, int Ny);
 void rt_nd_bytes(const Handle* h, int Nx, int Ny, size_t* arena, size_t* scratch);
 int rt_nd_prepare(Handle* h, int Nx, int Ny);
