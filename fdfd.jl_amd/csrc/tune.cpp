@@ -171,7 +171,6 @@ extern "C" int fdfd_autotune(fdfd_handle* hh, int pol, double omega, int precisi
         return 1e300;
     };
     h->tuned_explicitly = true;  // no cache lookup while timing
-    if (rc == FDFD_OK && rt_nd_applies(h, g.Nx, g.Ny)) nd_ms = step();
     h->nd_off = true;  // the variants are the line reduction's
     for (const Knobs& k : candidates(precision)) {
         if (rc) break;
@@ -183,6 +182,13 @@ extern "C" int fdfd_autotune(fdfd_handle* hh, int pol, double omega, int precisi
         }
     }
     h->nd_off = nd_was_off;
+    // the dissection last, when whatever the allocations before it set off in the
+    // driver (clearing of freed memory) has passed, and after a step that makes its
+    // tree and work
+    if (rc == FDFD_OK && rt_nd_applies(h, g.Nx, g.Ny)) {
+        (void)step();
+        if (rc == FDFD_OK) nd_ms = step();
+    }
     (void)hipFree(dsrc);
     (void)hipFree(dout);
     set_knobs(h, rc ? start : best);
